@@ -521,6 +521,52 @@ int lattice_hip_sparse_quantized_conv_features_sorted_fragments(
     const int32_t* reorder_rows, int out_capacity, void* out, const void* bias,
     int epilogue, void* workspace, size_t workspace_bytes, void* stream);
 
+/* Streamed matrix-core conv over the sorted view for the channel counts and
+ * types the entries above refuse (no counterpart in the reference): float32
+ * (16x16x4 MFMAs, every product and sum in binary32), float16 and bfloat16
+ * features whose rows are whole 16-byte pieces (c_in % 4 == 0 for float32,
+ * % 8 otherwise), any c_out, K <= 32; feats, map and fragments under 4 GiB
+ * each (lattice_hip_conv_padded_supported: 1 when the shape is taken).  Same
+ * sum, output rows, bias, epilogue, workspace and tile order as
+ * lattice_hip_sparse_conv_features_sorted_fragments; feats and fragments
+ * 16-byte aligned.
+ * fragments holds lattice_hip_conv_padded_fragments_bytes(...) bytes, the
+ * weight in the kernel's fragment order, zero past its channels:
+ *  - lattice_hip_conv_padded_fragments from a float weight of
+ *    (weight_c_in, weight_c_out) channels in either layout; role: the weight
+ *    itself (c_in, c_out = weight_c_in, weight_c_out), or the weight of the
+ *    input gradient (c_in, c_out = weight_c_out, weight_c_in: the conv then
+ *    reads the cotangent), with its offsets as they are (over a transposed
+ *    view) or reversed (over a submanifold relation's own view);
+ *  - lattice_hip_quantized_padded_fragments from packed codes, scales and
+ *    biases (float16/bfloat16); the conv then takes their bits (0 for float
+ *    weights). */
+typedef enum {
+    LATTICE_FRAGMENTS_FORWARD = 0,
+    LATTICE_FRAGMENTS_TRANSPOSED = 1,
+    LATTICE_FRAGMENTS_MIRRORED = 2
+} lattice_fragment_role;
+int lattice_hip_conv_padded_supported(int dtype, int n_in, int c_in, int c_out,
+                                      int kernel_count, int out_capacity);
+size_t lattice_hip_conv_padded_fragments_bytes(int dtype, int kernel_count,
+                                               int c_in, int c_out);
+int lattice_hip_conv_padded_fragments(int dtype, const void* weights,
+                                      int weight_layout, int kernel_count,
+                                      int weight_c_in, int weight_c_out,
+                                      int role, void* fragments,
+                                      size_t fragments_bytes, void* stream);
+int lattice_hip_quantized_padded_fragments(
+    int dtype, const uint32_t* weights, const void* scales,
+    const void* biases, int kernel_count, int c_in, int c_out,
+    int storage_c_in, int group_size, int bits, void* fragments,
+    size_t fragments_bytes, void* stream);
+int lattice_hip_sparse_conv_features_padded(
+    int dtype, const void* feats, int n_in, int c_in, const void* fragments,
+    int bits, int kernel_count, int c_out,
+    const int32_t* sorted_kv_out_in_map, const int32_t* tile_masks,
+    const int32_t* reorder_rows, int out_capacity, void* out, const void* bias,
+    int epilogue, void* workspace, size_t workspace_bytes, void* stream);
+
 /* Input gradient of the float conv (SparseConvFeaturesInputGrad,
  * primitive.cpp:192-260, 597-639; cpu/algorithms.cpp:355-410):
  * grad[in, ci] = sum over the edges of input row `in` in the input-grouped

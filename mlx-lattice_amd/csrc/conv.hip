@@ -341,6 +341,16 @@ template <> struct MfmaOps<__bf16> {
         return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
     }
 };
+// float32: a 16-byte piece holds four channels, one per 16x16x4 MFMA (lane
+// group lg contributes channel 4 lg + e of the 16-channel step to the e-th).
+template <> struct MfmaOps<float> {
+    typedef float4_t vec;
+    __device__ static float4_t mfma(vec a, vec b, float4_t c) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[e], b[e], c, 0, 0, 0);
+        return c;
+    }
+};
 
 // Tile and pipeline shape of the matrix-core kernel.
 //   C_OUT      output channels (the block covers all of them);
@@ -1177,6 +1187,8 @@ __device__ inline void static_for_range(F& f, int lo, int hi) {
     }
 }
 
+constexpr int kOrderTileRows = 128;  // rows of the tiles a tile order ranks
+
 constexpr int gcd_int(int a, int b) { return b == 0 ? a : gcd_int(b, a % b); }
 
 // Vector-memory ops a streamed stage j issues: the row indices of a trip
@@ -1193,25 +1205,29 @@ constexpr int stream_wait_a(int p, int la, int li, int nch, int nbd) {
 }
 constexpr int lcm_int(int a, int b) { return a / gcd_int(a, b) * b; }
 
-// Tile of the streamed kernel: C_OUT output channels per block (a column
-// half when C_out = 256), its 4 waves in WR row groups x 4 / WR column
-// groups of 32 columns.
-template <int C_OUT_, int WR_, int LA_ = 2, int OCC_ = 3>
+// Tile of the streamed kernel: ROWS sorted rows x C_OUT output channels per
+// block (a column tile when the conv has more), its 4 waves in WR row groups
+// x 4 / WR column groups of 32 columns.  T_ is the feature type: a 16-byte
+// piece holds PE channels, a 128-byte row line (a stage's chunk) CHUNK.
+template <typename T_, int C_OUT_, int WR_, int ROWS_ = 128, int LA_ = 2, int OCC_ = 3>
 struct StreamShape {
+    using T = T_;
     static constexpr int C_OUT = C_OUT_;
     static constexpr int WAVES = 4;
     static constexpr int THREADS = WAVES * 64;
     static constexpr int WR = WR_;
     static constexpr int WC = WAVES / WR_;
-    static constexpr int ROWS = 128;          // tile rows (the tile order's 128-row tiles)
+    static constexpr int ROWS = ROWS_;        // 128 (the tile order's tiles) or 64 (their halves)
     static constexpr int WROWS = ROWS / WR;   // rows per wave
     static constexpr int WCOLS = C_OUT / WC;  // columns per wave
     static constexpr int RB = WROWS / 16;     // 16-row MFMA blocks per wave
     static constexpr int CB = WCOLS / 16;     // 16-column MFMA blocks per wave
-    static constexpr int CHUNK = 64;          // input channels per stage
-    static constexpr int ST = CHUNK / 32;     // 32-channel MFMA steps per stage
-    static constexpr int GATHER = ROWS * (CHUNK / 8) / THREADS;  // row-line copies per thread and stage
-    static constexpr int ABUF = ROWS * CHUNK;  // halves of one A buffer
+    static constexpr int PE = 16 / static_cast<int>(sizeof(T));  // channels per 16-byte piece
+    static constexpr int CHUNK = 8 * PE;      // input channels per stage: 64 (32 for float32)
+    static constexpr int STEP = 4 * PE;       // input channels per MFMA fragment: 32 (16 for float32)
+    static constexpr int ST = CHUNK / STEP;   // fragments per stage
+    static constexpr int GATHER = ROWS * 8 / THREADS;  // row-line copies per thread and stage
+    static constexpr int ABUF = ROWS * CHUNK;  // elements of one A buffer
     static constexpr int OCC = OCC_;           // blocks per CU
     // A copies lead by LA stages (a ring of LA + 1 buffers).  LA = 2 at
     // three blocks per CU measured fastest: LA = 3 or 4 at two blocks per
@@ -1222,7 +1238,7 @@ struct StreamShape {
     static constexpr int LB = 2;               // B loads lead by LB stages
     static constexpr int LI = LA_ + 1;         // row-index loads lead by LI stages
     static constexpr int READ_AHEAD = 2;       // 16-row fragment reads in flight
-    static_assert(WCOLS == 32 && WROWS % 16 == 0 && GATHER == 4, "stream tile shape");
+    static_assert(WCOLS == 32 && WROWS % 16 == 0 && (GATHER == 4 || GATHER == 2), "stream tile shape");
 };
 
 // Fragment (k, ks, cg, cb) of a weight: the 16 x 32 block of output
@@ -1257,6 +1273,49 @@ weight_fragments(const T* __restrict__ w, int K, int c_in, int c_out, T* __restr
     }
 }
 
+// Fragments of a weight whose channels do not fill them (the PAD instances):
+// 16 x STEP blocks (STEP = 32 input channels, 16 for float32; lane (lr, lg)
+// holds 16 bytes: W[co][k][ci .. ci + PE - 1] with co = cg*32 + cb*16 + lr,
+// ci = ks*STEP + lg*PE) in (k, ks, cg, cb) order, zeros past C_out and C_in.
+// role (LATTICE_FRAGMENTS_*): the weight itself, or that of the input
+// gradient: its channels swapped, and for a submanifold relation its offsets
+// reversed too.  One launch per weight version; bound by its own size.
+template <typename T>
+__global__ void __launch_bounds__(256)
+padded_weight_fragments(const T* __restrict__ w, WeightIndex widx, int role, int c_in, int c_out,
+                        T* __restrict__ frag) {
+    constexpr int PE = 16 / static_cast<int>(sizeof(T));
+    const int ksteps = (c_in + 4 * PE - 1) / (4 * PE);
+    const int ncg = (c_out + 31) / 32;
+    const long long pieces = static_cast<long long>(widx.K) * ksteps * ncg * 128;
+    for (long long p = static_cast<long long>(blockIdx.x) * blockDim.x + threadIdx.x; p < pieces;
+         p += static_cast<long long>(gridDim.x) * blockDim.x) {
+        const int lane = static_cast<int>(p % 64);
+        long long f = p / 64;
+        const int cb = static_cast<int>(f % 2);
+        f /= 2;
+        const int cg = static_cast<int>(f % ncg);
+        f /= ncg;
+        const int ks = static_cast<int>(f % ksteps);
+        const int k = static_cast<int>(f / ksteps);
+        const int co = cg * 32 + cb * 16 + (lane & 15);
+        const int ci = (ks * 4 + (lane >> 4)) * PE;
+        const int ksrc = role == LATTICE_FRAGMENTS_MIRRORED ? widx.K - 1 - k : k;
+        union {
+            uint4 q;
+            T v[PE];
+        } r;
+        r.q = uint4{0u, 0u, 0u, 0u};
+#pragma unroll
+        for (int e = 0; e < PE; ++e) {
+            if (co < c_out && ci + e < c_in) {
+                r.v[e] = role == LATTICE_FRAGMENTS_FORWARD ? w[widx(ksrc, ci + e, co)] : w[widx(ksrc, co, ci + e)];
+            }
+        }
+        reinterpret_cast<uint4*>(frag)[p] = r.q;
+    }
+}
+
 // Packed fragment of a quantized weight (lattice_hip_quantized_weight_
 // fragments): the 16 bytes of lane (lr, lg) of fragment (k, ks, cg, cb)
 // hold the codes of W[co][k][ci .. ci + 7] (co = cg*32 + cb*16 + lr,
@@ -1267,15 +1326,16 @@ weight_fragments(const T* __restrict__ w, int K, int c_in, int c_out, T* __restr
 // one rounding to T (packed fp16 math as in PackedB::load).
 // Packed fragments of a quantized weight (layout above dequant_fragment):
 // w (K, packed_words, c_out) uint32 codes, scales / biases (K, groups,
-// c_out) of type T.
-template <typename T>
+// c_out) of type T.  PAD: channel counts that do not fill the fragments;
+// pieces past C_out or C_in hold zero codes, scale and bias.
+template <typename T, bool PAD = false>
 __global__ void __launch_bounds__(256)
 packed_weight_fragments(const uint32_t* __restrict__ w, const T* __restrict__ scales, const T* __restrict__ biases,
                         int K, int c_in, int c_out, int packed_words, int groups, int group_size, int bits,
                         uint4* __restrict__ frag) {
-    const int ksteps = c_in / 32;
-    const int ncg = c_out / 32;
-    const long long pieces = static_cast<long long>(K) * c_in * c_out / 8;
+    const int ksteps = PAD ? (c_in + 31) / 32 : c_in / 32;
+    const int ncg = PAD ? (c_out + 31) / 32 : c_out / 32;
+    const long long pieces = static_cast<long long>(K) * ksteps * ncg * 128;
     for (long long p = static_cast<long long>(blockIdx.x) * blockDim.x + threadIdx.x; p < pieces;
          p += static_cast<long long>(gridDim.x) * blockDim.x) {
         const int lane = static_cast<int>(p % 64);
@@ -1288,6 +1348,10 @@ packed_weight_fragments(const uint32_t* __restrict__ w, const T* __restrict__ sc
         const int k = static_cast<int>(f / ksteps);
         const int co = cg * 32 + cb * 16 + (lane & 15);
         const int ci = ks * 32 + (lane >> 4) * 8;
+        if (PAD && (co >= c_out || ci >= c_in)) {
+            frag[p] = uint4{0u, 0u, 0u, 0u};
+            continue;
+        }
         const long long wbase = static_cast<long long>(k) * packed_words * c_out + co;
         const long long sidx = (static_cast<long long>(k) * groups + ci / group_size) * c_out + co;
         uint4 r;
@@ -1345,12 +1409,106 @@ __device__ inline typename MfmaOps<T>::vec dequant_fragment(typename MfmaOps<T>:
     return out;
 }
 
-template <typename T, typename S, int NCH, int QB>
+// Store of a finished tile whose columns may end inside it (PAD): column
+// tile col0 .. of an output with c_out columns.  16-bit tiles are staged in
+// the idle A ring (one row after the other, 16 bytes apart in the banks) and
+// leave as 16-byte stores where rows are 16-byte aligned, float32 lanes hold
+// four consecutive columns and store them directly; other column counts
+// store value by value.
+template <typename T, typename S, int RB, int CB>
+__device__ inline void stream_store_padded(const float4_t (&acc)[RB][CB], T* stage, const Epilogue<T>& epi, int col0,
+                                           int c_out, int row0, int wr, int wc, int rows,
+                                           const int32_t* __restrict__ reorder_rows, T* __restrict__ out) {
+    const int lane = lane_id();
+    const int lr = lane & 15;
+    const int lg = lane >> 4;
+    const bool whole = (reinterpret_cast<uintptr_t>(out) | (static_cast<unsigned>(c_out) * sizeof(T))) % 16 == 0;
+    float bcol[CB][4];
+#pragma unroll
+    for (int cb = 0; cb < CB; ++cb)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int co = col0 + wc * S::WCOLS + cb * 16 + lg * 4 + q;
+            bcol[cb][q] = epi.bias != nullptr && co < c_out ? static_cast<float>(epi.bias[co]) : 0.0f;
+        }
+    if constexpr (sizeof(T) == 4) {
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb) {
+            const int sr = row0 + wr * S::WROWS + rb * 16 + lr;
+            if (sr >= rows) continue;
+            const long long orow = reorder_rows != nullptr ? reorder_rows[sr] : sr;
+#pragma unroll
+            for (int cb = 0; cb < CB; ++cb) {
+                const int co = col0 + wc * S::WCOLS + cb * 16 + lg * 4;
+                float4_t v;
+#pragma unroll
+                for (int q = 0; q < 4; ++q) v[q] = epi.finish(acc[rb][cb][q], bcol[cb][q]);
+                T* const dst = out + orow * c_out + co;
+                if (whole) {
+                    if (co < c_out) *reinterpret_cast<float4_t*>(dst) = v;
+                } else {
+#pragma unroll
+                    for (int q = 0; q < 4; ++q)
+                        if (co + q < c_out) dst[q] = v[q];
+                }
+            }
+        }
+    } else {
+        constexpr int LDW = S::C_OUT + 8;
+        static_assert(S::ROWS * LDW <= (S::LA + 1) * S::ABUF, "the staged tile fits the A ring");
+        __syncthreads();
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb) {
+            const int r = wr * S::WROWS + rb * 16 + lr;
+#pragma unroll
+            for (int cb = 0; cb < CB; ++cb) {
+                T v[4];
+#pragma unroll
+                for (int q = 0; q < 4; ++q) v[q] = epi.finish(acc[rb][cb][q], bcol[cb][q]);
+                *reinterpret_cast<uint2*>(stage + r * LDW + wc * S::WCOLS + cb * 16 + lg * 4) =
+                    *reinterpret_cast<const uint2*>(v);
+            }
+        }
+        __syncthreads();
+        const int cols = min(S::C_OUT, c_out - col0);
+        if (whole) {
+            const int cpr = cols / 8;  // 16-byte pieces per row
+            for (int i = threadIdx.x; i < S::ROWS * cpr; i += S::THREADS) {
+                const int r = i / cpr;
+                const int piece = i - r * cpr;
+                if (row0 + r < rows) {
+                    const long long orow = reorder_rows != nullptr ? reorder_rows[row0 + r] : row0 + r;
+                    __builtin_nontemporal_store(*reinterpret_cast<const u32x4v_t*>(stage + r * LDW + piece * 8),
+                                                reinterpret_cast<u32x4v_t*>(out + orow * c_out + col0 + piece * 8));
+                }
+            }
+        } else {
+            for (int i = threadIdx.x; i < S::ROWS * cols; i += S::THREADS) {
+                const int r = i / cols;
+                const int c = i - r * cols;
+                if (row0 + r < rows) {
+                    const long long orow = reorder_rows != nullptr ? reorder_rows[row0 + r] : row0 + r;
+                    out[orow * c_out + col0 + c] = stage[r * LDW + c];
+                }
+            }
+        }
+    }
+}
+
+// PAD: channel counts that do not fill the tiles.  The fragments are padded
+// with zeros to whole 32-column groups and whole fragments of input
+// channels, a copy's pieces past C_in wrap past the buffer's range (zeros, no
+// memory access), a wave whose 32 columns all lie past C_out issues no
+// MFMAs, and the store guards the columns.  The chunks of an offset are then
+// stages of their own (NCH = 1; each loads its row indices), so one instance
+// serves every C_in.
+template <typename T, typename S, int NCH, int QB, bool PAD = false>
 __global__ void __launch_bounds__(S::THREADS, S::OCC)
 conv_igemm_stream(const T* __restrict__ feats, int n_in, int c_in, const T* __restrict__ wfrag, int kernel_count,
                   int c_out_total, const int32_t* __restrict__ kv_map, const int32_t* __restrict__ tile_masks,
                   const int32_t* __restrict__ reorder_rows, int rows, const int32_t* __restrict__ block_order,
                   T* __restrict__ out, Epilogue<T> epi, int halves) {
+    static_assert(!PAD || NCH == 1, "padded chunks are stages of their own");
     using V = typename MfmaOps<T>::vec;
     constexpr int RB = S::RB;
     constexpr int CB = S::CB;
@@ -1370,11 +1528,18 @@ conv_igemm_stream(const T* __restrict__ feats, int n_in, int c_in, const T* __re
     const int col0 = wc * S::WCOLS;
     // Longest-first tile order; with C_out = 256 consecutive blocks take the
     // two column halves of one tile (the second finds its rows in L2).
-    const int slot = halves > 1 ? static_cast<int>(blockIdx.x) / 2 : static_cast<int>(blockIdx.x);
-    const int half = halves > 1 ? static_cast<int>(blockIdx.x & 1u) : 0;
-    const int cg = half * (S::C_OUT / S::WCOLS) + wc;  // 32-column group of the weight
-    const int out_ld = S::C_OUT * halves;
-    const int tile = block_order != nullptr ? block_order[slot] : slot;
+    // (PAD: any number of column tiles).  The order ranks 128-row tiles;
+    // 64-row tiles take their two halves in turn.
+    const int slot = PAD ? static_cast<int>(blockIdx.x) / halves
+                         : halves > 1 ? static_cast<int>(blockIdx.x) / 2 : static_cast<int>(blockIdx.x);
+    const int half = PAD ? static_cast<int>(blockIdx.x) % halves : halves > 1 ? static_cast<int>(blockIdx.x & 1u) : 0;
+    const int ncg = PAD ? (c_out_total + 31) / 32 : c_out_total / S::WCOLS;  // 32-column groups of the weight
+    const int cg_own = half * (S::C_OUT / S::WCOLS) + wc;
+    const bool idle = PAD && cg_own >= ncg;
+    const int cg = idle ? ncg - 1 : cg_own;
+    const int out_ld = PAD ? c_out_total : S::C_OUT * halves;
+    constexpr int TPO = kOrderTileRows / S::ROWS;  // tiles per entry of the order
+    const int tile = block_order != nullptr ? block_order[slot / TPO] * TPO + slot % TPO : slot;
     const int row0 = tile * S::ROWS;
     const int quarters = ((rows + 63) / 64) * 4;
     // Offset masks of the wave's 16-row blocks and of the whole tile.
@@ -1385,9 +1550,10 @@ conv_igemm_stream(const T* __restrict__ feats, int n_in, int c_in, const T* __re
         const int qi = row0 / 16 + q;
         const uint32_t m = qi < quarters ? static_cast<uint32_t>(tile_masks[qi]) : 0u;
         bmask |= m;
-        if (q / RB == wr) qm[q % RB] = m;
+        if (q / RB == wr) qm[q % RB] = idle ? 0u : m;
     }
-    const int ntrips = __popc(bmask);
+    const int nch = PAD ? (c_in + S::CHUNK - 1) / S::CHUNK : NCH;
+    const int ntrips = PAD ? __popc(bmask) * nch : __popc(bmask);
 
     float4_t acc[RB][CB];
 #pragma unroll
@@ -1397,14 +1563,14 @@ conv_igemm_stream(const T* __restrict__ feats, int n_in, int c_in, const T* __re
 
     if (ntrips > 0) {
         const int gp = (lane & 7) ^ ((lane >> 3) & 7);  // piece it copies (its slot ^ row % 8)
-        const int ksteps = c_in / 32;
-        const int ncg = c_out_total / S::WCOLS;
-        const bool partial = (c_in % S::CHUNK) != 0;  // the last chunk holds 32 channels
+        const int ksteps = PAD ? (c_in + S::STEP - 1) / S::STEP : c_in / S::STEP;
+        const bool partial = !PAD && (c_in % S::CHUNK) != 0;  // the last chunk holds 32 channels
         const u32x4v_t frs = raw_rsrc(feats, static_cast<unsigned>(static_cast<long long>(n_in) * c_in * sizeof(T)));
         const u32x4v_t krs =
             raw_rsrc(kv_map, static_cast<unsigned>(static_cast<long long>(kernel_count) * rows * sizeof(int32_t)));
         const u32x4v_t wrs = raw_rsrc(
-            wfrag, static_cast<unsigned>(static_cast<long long>(kernel_count) * c_in * c_out_total * sizeof(T)));
+            wfrag, PAD ? static_cast<unsigned>(static_cast<long long>(kernel_count) * ksteps * ncg * 2048)
+                       : static_cast<unsigned>(static_cast<long long>(kernel_count) * c_in * c_out_total * sizeof(T)));
         const unsigned lds0 = static_cast<unsigned>(reinterpret_cast<unsigned long long>(lds));
 
         constexpr int LA = S::LA, LB = S::LB, LI = S::LI;
@@ -1423,9 +1589,20 @@ conv_igemm_stream(const T* __restrict__ feats, int n_in, int c_in, const T* __re
         // Offset ring: kr[i] is the offset of trip t + i (t = the block's
         // first trip); past the last trip it repeats the last offset, whose
         // prefetched operands are never used.
+        // PAD: an entry is offset | chunk << 8.
         uint32_t rem = bmask;
         int klast = 0;
         auto pop = [&]() {
+            if constexpr (PAD) {
+                const int ch = (klast >> 8) + 1;
+                if (ch < nch && rem != bmask) {
+                    klast += 1 << 8;
+                } else if (rem) {
+                    klast = __builtin_ctz(rem);
+                    rem &= rem - 1;
+                }
+                return klast;
+            }
             if (rem) {
                 klast = __builtin_ctz(rem);
                 rem &= rem - 1;
@@ -1436,27 +1613,37 @@ conv_igemm_stream(const T* __restrict__ feats, int n_in, int c_in, const T* __re
 #pragma unroll
         for (int i = 0; i < R; ++i) kr[i] = pop();
 
-        // Lanes j and j + 32 load the index of copy row j of the wave.
+        // Lane j (mod 8 G) loads the index of copy row j of the wave.
         auto idx_load = [&](int& raw, int k) {
-            const int r = min(row0 + wave * (8 * G) + (lane & 31), rows - 1);
-            raw = asm_load_i32(krs, static_cast<unsigned>((k * rows + r) * 4));
+            const int r = min(row0 + wave * (8 * G) + (lane & (8 * G - 1)), rows - 1);
+            const int ko = PAD ? k & 255 : k;
+            raw = asm_load_i32(krs, static_cast<unsigned>(ko) * static_cast<unsigned>(rows) * 4u +
+                                        static_cast<unsigned>(r) * 4u);
         };
-        // Copy i of this lane reads row 8 i + lane / 8 of the wave's 32.
+        // Copy i of this lane reads row 8 i + lane / 8 of the wave's 8 G.
         auto idx_expand = [&](int (&d)[G], int raw) {
 #pragma unroll
             for (int i = 0; i < G; ++i) d[i] = __builtin_amdgcn_ds_bpermute((8 * i + (lane >> 3)) << 2, raw);
         };
         auto b_load = [&](V (&b)[CB][ST], int k, int ch, int cb, int st) {
+            const int ko = PAD ? k & 255 : k;
+            const int co = PAD ? k >> 8 : ch;
             b[cb][st] = asm_load_b128<V>(
-                wrs, static_cast<unsigned>(fragment_piece(k, ch * ST + st, cg, cb, lane, ksteps, ncg) * 16));
+                wrs, static_cast<unsigned>(fragment_piece(ko, co * ST + st, cg, cb, lane, ksteps, ncg) * 16));
         };
-        auto a_copy = [&](const int (&d)[G], int ch, int buf, int i) {
-            const int ci = ch * S::CHUNK;
-            // a partial last chunk copies its four pieces twice
-            const int off = (partial && ch == NCH - 1 && gp >= 4) ? (gp - 4) * 8 : gp * 8;
+        auto a_copy = [&](const int (&d)[G], int k, int ch, int buf, int i) {
             const unsigned dst = lds0 + buf * ABYTES + (wave * (8 * G) + 8 * i) * S::CHUNK * sizeof(T);
             const unsigned row = static_cast<unsigned>(d[i]) * static_cast<unsigned>(c_in * sizeof(T));
-            asm_copy_b128(frs, row + (ci + off) * sizeof(T), __builtin_amdgcn_readfirstlane(dst));
+            if constexpr (PAD) {
+                const int c = (k >> 8) * S::CHUNK + gp * S::PE;
+                asm_copy_b128(frs, c < c_in ? row + c * static_cast<unsigned>(sizeof(T)) : 0xfffffff0u,
+                              __builtin_amdgcn_readfirstlane(dst));
+            } else {
+                const int ci = ch * S::CHUNK;
+                // a partial last chunk copies its four pieces twice
+                const int off = (partial && ch == NCH - 1 && gp >= 4) ? (gp - 4) * 8 : gp * 8;
+                asm_copy_b128(frs, row + (ci + off) * sizeof(T), __builtin_amdgcn_readfirstlane(dst));
+            }
         };
 
         // Memory ops of stage j: the trip's row indices when stage j + LI
@@ -1479,7 +1666,7 @@ conv_igemm_stream(const T* __restrict__ feats, int n_in, int c_in, const T* __re
                     idx_expand(d, raw[(u / NCH) % NRS]);
                 }
 #pragma unroll
-                for (int i = 0; i < G; ++i) a_copy(d, u % NCH, u, i);
+                for (int i = 0; i < G; ++i) a_copy(d, kr[u / NCH], u % NCH, u, i);
             }
         }
 #pragma unroll
@@ -1505,9 +1692,10 @@ conv_igemm_stream(const T* __restrict__ feats, int n_in, int c_in, const T* __re
             static_assert(LB == 2, "W_B counts one stage between a B load and its use");
             V (&bcur)[CB][ST] = b[p % NBS];
             V (&bfill)[CB][ST] = b[(p + LB) % NBS];
-            const int k = kr[p / NCH];
+            const int k = PAD ? kr[p / NCH] & 255 : kr[p / NCH];
             const int k_i = kr[(p + LI) / NCH];
             const int k_b = kr[(p + LB) / NCH];
+            const int k_a = kr[(p + LA) / NCH];
             const int abuf_fill = buf == 0 ? LA : buf - 1;  // (s + LA) % (LA + 1)
             if constexpr ((p + LA) % NCH == 0) {
                 int& ra = raw[((p + LA) / NCH) % NRS];
@@ -1529,15 +1717,15 @@ conv_igemm_stream(const T* __restrict__ feats, int n_in, int c_in, const T* __re
                 } else if constexpr (q < NI + NB) {
                     b_load(bfill, k_b, (p + LB) % NCH, (q - NI) / ST, (q - NI) % ST);
                 } else {
-                    a_copy(d, (p + LA) % NCH, abuf_fill, q - NI - NB);
+                    a_copy(d, k_a, (p + LA) % NCH, abuf_fill, q - NI - NB);
                 }
             };
-            const int nst = (partial && ch == NCH - 1) ? 1 : ST;
+            const int nst = PAD ? min(ST, ksteps - (kr[p / NCH] >> 8) * ST) : (partial && ch == NCH - 1) ? 1 : ST;
             const T* arow = lds + buf * S::ABUF + (wr * S::WROWS + lr) * S::CHUNK;
             auto read_a = [&](V (&a)[ST], int rb) {
 #pragma unroll
                 for (int st = 0; st < ST; ++st) {
-                    a[st] = *reinterpret_cast<const V*>(arow + rb * 16 * S::CHUNK + (((st * 4 + lg) ^ (lr & 7)) * 8));
+                    a[st] = *reinterpret_cast<const V*>(arow + rb * 16 * S::CHUNK + (((st * 4 + lg) ^ (lr & 7)) * S::PE));
                 }
             };
             constexpr int RA = S::READ_AHEAD;
@@ -1582,6 +1770,9 @@ conv_igemm_stream(const T* __restrict__ feats, int n_in, int c_in, const T* __re
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     }
 
+    if constexpr (PAD) {
+        stream_store_padded<T, S>(acc, lds, epi, half * S::C_OUT, c_out_total, row0, wr, wc, rows, reorder_rows, out);
+    } else {
     // The finished tile goes through LDS (the A ring is free once every
     // wave's copies have landed) so that it leaves as 16-byte stores of
     // whole output rows to out[reorder_rows[row]], non-temporal (streamed
@@ -1623,6 +1814,7 @@ conv_igemm_stream(const T* __restrict__ feats, int n_in, int c_in, const T* __re
                 *reinterpret_cast<const u32x4v_t*>(stage + r * LDW + piece * 8),
                 reinterpret_cast<u32x4v_t*>(ohalf + static_cast<long long>(orow) * out_ld + piece * 8));
         }
+    }
     }
 }
 
@@ -1956,7 +2148,6 @@ int launch_expand(const T* feats, int n_in, const int32_t* active, int c_in, con
 // order.
 constexpr int kScheduleThreads = 1024;
 constexpr int kMaxScheduledTiles = 32768;
-constexpr int kOrderTileRows = 128;  // rows of the tiles a tile order ranks
 
 template <int QUARTERS>
 __global__ void __launch_bounds__(kScheduleThreads)
@@ -2112,13 +2303,72 @@ int launch_stream(const T* feats, int n_in, int c_in, const T* frag, int K, int 
         LATTICE_LAUNCH_CHECK();
     }
     if (c_out == 64) {
-        launch_stream_shape<T, StreamShape<64, 2>, QB>(feats, n_in, c_in, frag, K, c_out, kv_map, tile_masks,
+        launch_stream_shape<T, StreamShape<T, 64, 2>, QB>(feats, n_in, c_in, frag, K, c_out, kv_map, tile_masks,
                                                    reorder_rows, rows, schedule, out, epi, 1, stream);
     } else {
-        launch_stream_shape<T, StreamShape<128, 1>, QB>(feats, n_in, c_in, frag, K, c_out, kv_map, tile_masks,
+        launch_stream_shape<T, StreamShape<T, 128, 1>, QB>(feats, n_in, c_in, frag, K, c_out, kv_map, tile_masks,
                                                     reorder_rows, rows, schedule, out, epi, c_out == 256 ? 2 : 1,
                                                     stream);
     }
+    LATTICE_LAUNCH_CHECK();
+    return LATTICE_OK;
+}
+
+// Shapes the padded instances of the streamed kernel take: every feature
+// type (packed weights: fp16/bf16), input rows of whole 16-byte pieces, any
+// C_out, K <= 32.  The kernel reads its map, weight and rows at 32-bit byte
+// offsets (with the wrapped -1 rows above the table's end), and a row's copy
+// past C_in asks for an offset no table reaches.
+bool padded_shape_ok(int dtype, long long n_in, int c_in, int c_out, int K, long long rows) {
+    const int size = dtype == LATTICE_F32 ? 4 : 2;
+    const long long row_bytes = static_cast<long long>(c_in) * size;
+    const long long limit = 1ll << 32;
+    const long long step = 64 / size;
+    if (c_in <= 0 || c_out <= 0 || K <= 0 || K > 32 || n_in < 0 || rows < 0) return false;
+    const long long frag = ((c_in + step - 1) / step) * ((static_cast<long long>(c_out) + 31) / 32) * 2048 * K;
+    return row_bytes % 16 == 0 && (n_in + 1) * row_bytes <= limit && 4ll * K * rows < limit && frag < limit &&
+           c_in <= 8192;
+}
+
+size_t padded_fragments_bytes(int dtype, int K, int c_in, int c_out) {
+    const int step = dtype == LATTICE_F32 ? 16 : 32;
+    return static_cast<size_t>(K) * ((c_in + step - 1) / step) * ((c_out + 31) / 32) * 2048;
+}
+
+template <typename T, typename S, int QB>
+void launch_padded_shape(const T* feats, int n_in, int c_in, const T* frag, int K, int c_out, const int32_t* kv_map,
+                         const int32_t* tile_masks, const int32_t* reorder_rows, int rows, const int32_t* order,
+                         T* out, Epilogue<T> epi, hipStream_t stream) {
+    // an order's 128-row tiles are two 64-row ones
+    const int tiles = (rows + kOrderTileRows - 1) / kOrderTileRows * (kOrderTileRows / S::ROWS);
+    const int columns = (c_out + S::C_OUT - 1) / S::C_OUT;
+    conv_igemm_stream<T, S, 1, QB, true><<<static_cast<unsigned>(tiles) * columns, S::THREADS, 0, stream>>>(
+        feats, n_in, c_in, frag, K, c_out, kv_map, tile_masks, reorder_rows, rows, order, out, epi, columns);
+}
+
+template <typename T, int QB = 0>
+int launch_padded(const T* feats, int n_in, int c_in, const T* frag, int K, int c_out, const int32_t* kv_map,
+                  const int32_t* tile_masks, const int32_t* reorder_rows, int rows, int32_t* schedule, bool ready,
+                  T* out, Epilogue<T> epi, hipStream_t stream) {
+    if (rows <= 0) return LATTICE_OK;
+    const int tiles = (rows + kOrderTileRows - 1) / kOrderTileRows;
+    if (tiles > kMaxScheduledTiles) schedule = nullptr;
+    if (schedule != nullptr && !ready) {
+        schedule_tiles<kOrderTileRows / 16><<<1, kScheduleThreads, 0, stream>>>(tile_masks, rows, tiles, schedule);
+        LATTICE_LAUNCH_CHECK();
+    }
+    constexpr int ROWS = sizeof(T) == 4 ? 64 : 128;
+#define LATTICE_PADDED(C, WR)                                                                                      \
+    launch_padded_shape<T, StreamShape<T, C, WR, ROWS>, QB>(feats, n_in, c_in, frag, K, c_out, kv_map, tile_masks, \
+                                                            reorder_rows, rows, schedule, out, epi, stream)
+    if (c_out <= 32) {
+        LATTICE_PADDED(32, 4);
+    } else if (c_out <= 64) {
+        LATTICE_PADDED(64, 2);
+    } else {
+        LATTICE_PADDED(128, 1);
+    }
+#undef LATTICE_PADDED
     LATTICE_LAUNCH_CHECK();
     return LATTICE_OK;
 }
@@ -2339,6 +2589,129 @@ extern "C" int lattice_hip_sparse_conv_features_sorted_fragments(
                                  static_cast<const __bf16*>(weight_fragments), kernel_count, c_out,
                                  sorted_kv_out_in_map, tile_masks, reorder_rows, out_capacity, schedule, ready,
                                  static_cast<__bf16*>(out), epilogue_of<__bf16>(bias, epilogue), stream);
+}
+
+// ------------------------------- streamed conv, channels padded to tiles --
+
+extern "C" int lattice_hip_conv_padded_supported(int dtype, int n_in, int c_in, int c_out, int kernel_count,
+                                                 int out_capacity) {
+    if (dtype != LATTICE_F32 && dtype != LATTICE_F16 && dtype != LATTICE_BF16) return 0;
+    return padded_shape_ok(dtype, n_in, c_in, c_out, kernel_count, out_capacity) ? 1 : 0;
+}
+
+extern "C" size_t lattice_hip_conv_padded_fragments_bytes(int dtype, int kernel_count, int c_in, int c_out) {
+    if (lattice_hip_conv_padded_supported(dtype, 0, c_in, c_out, kernel_count, 0) == 0) return 0;
+    return padded_fragments_bytes(dtype, kernel_count, c_in, c_out);
+}
+
+extern "C" int lattice_hip_conv_padded_fragments(int dtype, const void* weights, int weight_layout, int kernel_count,
+                                                 int weight_c_in, int weight_c_out, int role, void* fragments,
+                                                 size_t fragments_bytes_given, void* stream_ptr) {
+    LATTICE_REQUIRE(role == LATTICE_FRAGMENTS_FORWARD || role == LATTICE_FRAGMENTS_TRANSPOSED ||
+                        role == LATTICE_FRAGMENTS_MIRRORED,
+                    "unknown fragment role.");
+    LATTICE_REQUIRE(weight_layout == LATTICE_WEIGHT_KERNEL_MAJOR || weight_layout == LATTICE_WEIGHT_DENSE_5D,
+                    "weights must have shape (K, C_in, C_out) or (C_out, Kx, Ky, Kz, C_in).");
+    const bool swap = role != LATTICE_FRAGMENTS_FORWARD;
+    const int c_in = swap ? weight_c_out : weight_c_in;
+    const int c_out = swap ? weight_c_in : weight_c_out;
+    const size_t need = lattice_hip_conv_padded_fragments_bytes(dtype, kernel_count, c_in, c_out);
+    if (need == 0) {
+        set_error("padded weight fragments need input rows of whole 16-byte pieces and K <= 32.");
+        return LATTICE_ERROR_UNSUPPORTED;
+    }
+    LATTICE_REQUIRE(weights != nullptr && fragments != nullptr, "weight fragment pointers must be non-null.");
+    LATTICE_REQUIRE(fragments_bytes_given >= need, "weight fragment buffer too small.");
+    LATTICE_REQUIRE(reinterpret_cast<uintptr_t>(fragments) % 16 == 0, "weight fragments must be 16-byte aligned.");
+    hipStream_t stream = as_stream(stream_ptr);
+    const WeightIndex widx{weight_layout, kernel_count, weight_c_in, weight_c_out};
+    const unsigned grid = grid_for(static_cast<long long>(need / 16), 256, 1u << 14);
+    if (dtype == LATTICE_F32) {
+        padded_weight_fragments<float><<<grid, 256, 0, stream>>>(static_cast<const float*>(weights), widx, role, c_in,
+                                                                 c_out, static_cast<float*>(fragments));
+    } else if (dtype == LATTICE_F16) {
+        padded_weight_fragments<_Float16><<<grid, 256, 0, stream>>>(static_cast<const _Float16*>(weights), widx, role,
+                                                                    c_in, c_out, static_cast<_Float16*>(fragments));
+    } else {
+        padded_weight_fragments<__bf16><<<grid, 256, 0, stream>>>(static_cast<const __bf16*>(weights), widx, role,
+                                                                  c_in, c_out, static_cast<__bf16*>(fragments));
+    }
+    LATTICE_LAUNCH_CHECK();
+    return LATTICE_OK;
+}
+
+extern "C" int lattice_hip_quantized_padded_fragments(int dtype, const uint32_t* weights, const void* scales,
+                                                      const void* biases, int kernel_count, int c_in, int c_out,
+                                                      int storage_c_in, int group_size, int bits, void* fragments,
+                                                      size_t fragments_bytes_given, void* stream_ptr) {
+    const size_t need =
+        dtype == LATTICE_F32 ? 0 : lattice_hip_conv_padded_fragments_bytes(dtype, kernel_count, c_in, c_out);
+    if (need == 0) {
+        set_error("padded quantized fragments need fp16/bf16 scales, c_in % 8 == 0 and K <= 32.");
+        return LATTICE_ERROR_UNSUPPORTED;
+    }
+    LATTICE_REQUIRE(bits == 4 || bits == 8, "quantized weight bits must be 4 or 8.");
+    LATTICE_REQUIRE(group_size == 32 || group_size == 64 || group_size == 128,
+                    "quantized weight group_size must be 32, 64, or 128.");
+    LATTICE_REQUIRE(storage_c_in >= c_in && storage_c_in % group_size == 0,
+                    "quantized weight channel metadata is invalid.");
+    LATTICE_REQUIRE(weights != nullptr && scales != nullptr && biases != nullptr && fragments != nullptr,
+                    "quantized weight fragment pointers must be non-null.");
+    LATTICE_REQUIRE(fragments_bytes_given >= need, "quantized weight fragment buffer too small.");
+    LATTICE_REQUIRE(reinterpret_cast<uintptr_t>(fragments) % 16 == 0, "weight fragments must be 16-byte aligned.");
+    hipStream_t stream = as_stream(stream_ptr);
+    const unsigned grid = grid_for(static_cast<long long>(need / 16), 256, 1u << 14);
+    const int packed_words = storage_c_in * bits / 32;
+    const int groups = storage_c_in / group_size;
+    if (dtype == LATTICE_F16) {
+        packed_weight_fragments<_Float16, true><<<grid, 256, 0, stream>>>(
+            weights, static_cast<const _Float16*>(scales), static_cast<const _Float16*>(biases), kernel_count, c_in,
+            c_out, packed_words, groups, group_size, bits, static_cast<uint4*>(fragments));
+    } else {
+        packed_weight_fragments<__bf16, true><<<grid, 256, 0, stream>>>(
+            weights, static_cast<const __bf16*>(scales), static_cast<const __bf16*>(biases), kernel_count, c_in,
+            c_out, packed_words, groups, group_size, bits, static_cast<uint4*>(fragments));
+    }
+    LATTICE_LAUNCH_CHECK();
+    return LATTICE_OK;
+}
+
+extern "C" int lattice_hip_sparse_conv_features_padded(
+    int dtype, const void* feats, int n_in, int c_in, const void* fragments, int bits, int kernel_count, int c_out,
+    const int32_t* sorted_kv_out_in_map, const int32_t* tile_masks, const int32_t* reorder_rows, int out_capacity,
+    void* out, const void* bias, int epilogue, void* workspace, size_t workspace_bytes, void* stream_ptr) {
+    LATTICE_REQUIRE((epilogue & ~LATTICE_EPILOGUE_RELU) == 0, "unknown conv epilogue flags.");
+    int rc = check_dtype(dtype);
+    if (rc != LATTICE_OK) return rc;
+    LATTICE_REQUIRE(bits == 0 || ((bits == 4 || bits == 8) && dtype != LATTICE_F32),
+                    "fragments hold dense weights (bits 0), or 4- or 8-bit codes for float16/bfloat16 features.");
+    LATTICE_REQUIRE(n_in >= 0 && out_capacity >= 0, "feats must have shape (N, C_in).");
+    if (!padded_shape_ok(dtype, n_in, c_in, c_out, kernel_count, out_capacity)) {
+        set_error("the padded streamed conv needs input rows of whole 16-byte pieces, K <= 32 and feats, map and "
+                  "fragments under 4 GiB each.");
+        return LATTICE_ERROR_UNSUPPORTED;
+    }
+    LATTICE_REQUIRE(sorted_kv_out_in_map && tile_masks && out && fragments && (feats || n_in == 0),
+                    "conv pointers must be non-null.");
+    LATTICE_REQUIRE((reinterpret_cast<uintptr_t>(feats) | reinterpret_cast<uintptr_t>(fragments)) % 16 == 0,
+                    "the padded streamed conv needs 16-byte aligned features and fragments.");
+    int32_t* schedule = nullptr;
+    bool ready = false;
+    rc = conv_schedule(workspace, workspace_bytes, out_capacity, &schedule, &ready);
+    if (rc != LATTICE_OK) return rc;
+    hipStream_t stream = as_stream(stream_ptr);
+#define LATTICE_PADDED_CALL(T, QB)                                                                                  \
+    launch_padded<T, QB>(static_cast<const T*>(feats), n_in, c_in, static_cast<const T*>(fragments), kernel_count,  \
+                         c_out, sorted_kv_out_in_map, tile_masks, reorder_rows, out_capacity, schedule, ready,     \
+                         static_cast<T*>(out), epilogue_of<T>(bias, epilogue), stream)
+    if (dtype == LATTICE_F32) return LATTICE_PADDED_CALL(float, 0);
+    if (dtype == LATTICE_F16) {
+        if (bits == 0) return LATTICE_PADDED_CALL(_Float16, 0);
+        return bits == 4 ? LATTICE_PADDED_CALL(_Float16, 4) : LATTICE_PADDED_CALL(_Float16, 8);
+    }
+    if (bits == 0) return LATTICE_PADDED_CALL(__bf16, 0);
+    return bits == 4 ? LATTICE_PADDED_CALL(__bf16, 4) : LATTICE_PADDED_CALL(__bf16, 8);
+#undef LATTICE_PADDED_CALL
 }
 
 extern "C" size_t lattice_hip_quantized_weight_fragments_bytes(int dtype, int kernel_count, int c_in, int c_out) {

@@ -2,12 +2,13 @@
 (mlx_lattice/ops/_relation_exec.py:19-250).
 
 Route policy (this build's, the reference routes by Metal capability):
-fp16/bf16 features with ``C_in % 32 == 0``, ``C_out`` in {16, 32, 64, 128,
-256} and at most 32 kernel offsets run the matrix-core implicit GEMM over the
-mask-sorted view, for every relation kind whose edges fit the dense
-(out_row, offset) map; everything else (fp32, small or odd channel counts)
-runs the CSR bandwidth kernel.  Both routes compute the same sum with an fp32
-accumulator.
+features with at most 32 kernel offsets run a matrix-core implicit GEMM over
+the mask-sorted view, for every relation kind whose edges fit the dense
+(out_row, offset) map: fp16/bf16 with ``C_in % 32 == 0`` and ``C_out`` in
+{16, 32, 64, 128, 256} on the kernels tuned for those, other channel counts
+and fp32 on the streamed kernel's padded instances (rows of whole 16-byte
+pieces); everything else runs the CSR bandwidth kernel.  All routes compute
+the same sum with an fp32 accumulator.
 """
 
 from __future__ import annotations
@@ -65,6 +66,55 @@ def _small_dense_map(dtype: torch.dtype, c_in: int, c_out: int,
             or not relation.dense_map_exact):
         return None
     return view.out_in_map
+
+
+# lattice_fragment_role: the weight of a padded conv
+_FORWARD, _TRANSPOSED, _MIRRORED = 0, 1, 2
+
+
+def _padded_eligible(feats: torch.Tensor, c_out: int,
+                     relation: KernelRelation, rows: int) -> bool:
+    """Whether a conv of ``feats`` with ``c_out`` output channels and
+    ``rows`` output rows takes the streamed kernel's padded instances: types
+    and channel counts the sorted entries refuse, in rows of whole 16-byte
+    pieces (``ext.conv_padded_supported``: sizes and alignment)."""
+    return (relation.n_kernels is not None and relation.n_kernels <= 32
+            and feats.ndim == 2
+            and ext.conv_padded_supported(feats, c_out, relation.n_kernels,
+                                          rows))
+
+
+def _padded_forward(feats: torch.Tensor, c_in: int, c_out: int,
+                    relation: KernelRelation) -> bool:
+    """The forward conv's use of the padded instances.  Rows of at most 16
+    channels with 16 or 32 outputs have kernels of their own (a lane per
+    row, the dense map), which a relation used once runs faster than it
+    sorts its view.  Expanded relations keep the CSR route in fp32: their
+    rows hold one edge each or few, so the view costs more than it saves."""
+    if not relation.dense_map_exact:
+        return False
+    if feats.dtype == torch.float32 and relation.contract.kind in (
+            'transposed', 'generative'):
+        return False
+    if (c_in <= 16 and c_out in (16, 32)
+            and relation.sorted_implicit_gemm is None):
+        return False
+    return _padded_eligible(feats, c_out, relation, relation.n_out_capacity)
+
+
+def _padded_fragments(weight: torch.Tensor, role: int) -> torch.Tensor:
+    """The padded conv's fragment-ordered copy of a float weight, or of its
+    input gradient's weight, cached with the weight."""
+    return _cached_weight(weight, ('padded', role),
+                          lambda w: ext.conv_padded_fragments(w, role))
+
+
+def _padded_conv(feats, fragments, bits, c_out, view, rows, relation,
+                 bias=None, relu=False) -> torch.Tensor:
+    return ext.sparse_conv_features_padded(
+        feats, fragments, bits, c_out, view.sorted_kv_out_in_map,
+        view.reorder_rows, view.tile_masks, rows, relation.n_kernels,
+        bias=bias, tile_order=view.tile_order(), relu=relu)
 
 
 _EXPAND_CHANNELS = (32, 64, 128, 256)
@@ -232,6 +282,16 @@ def sparse_conv_input_grad_from_relation(cot: torch.Tensor,
             None, None, None, None, None, None, None, None, None,
             in_capacity, relation.n_kernels, tile_order=view.tile_order(),
             weight_fragments=_weight_fragments(transposed))
+    c_in = int(weight.shape[1] if weight.ndim == 3 else weight.shape[4])
+    if (relation.contract.kind != 'target' and relation.transposed_map_exact
+            and _padded_eligible(cot, c_in, relation, in_capacity)):
+        mirrored = _mirror_symmetric(relation)
+        view = (relation.require_sorted_implicit_gemm() if mirrored
+                else relation.require_transposed_sorted_implicit_gemm())
+        fragments = _padded_fragments(weight,
+                                      _MIRRORED if mirrored else _TRANSPOSED)
+        return _padded_conv(cot, fragments, 0, c_in, view, in_capacity,
+                            relation)
     input_csr = relation.input_csr
     return ext.sparse_conv_input_grad(
         cot, weight, relation.edges.out_rows, relation.edges.kernel_ids,
@@ -275,6 +335,13 @@ def _conv_features(feats: torch.Tensor, weight: torch.Tensor,
                                                          relu=relu)
     dense = (_small_dense_map(feats.dtype, int(feats.shape[1]), c_out,
                               relation) if feats.ndim == 2 else None)
+    c_in = int(weight.shape[1] if weight.ndim == 3 else weight.shape[4])
+    if (dense is None and feats.ndim == 2 and c_in == int(feats.shape[1])
+            and feats.dtype == weight.dtype
+            and _padded_forward(feats, c_in, c_out, relation)):
+        return _padded_conv(feats, _padded_fragments(weight, _FORWARD), 0,
+                            c_out, relation.require_sorted_implicit_gemm(),
+                            relation.n_out_capacity, relation, bias, relu)
     return ext.sparse_conv_features_csr(
         feats, weight, relation.edges.in_rows, relation.edges.kernel_ids,
         relation.counts, relation.output_csr.row_offsets,
@@ -337,6 +404,16 @@ def sparse_quantized_conv_features_from_relation(
     else:
         dense = _small_dense_map(feats.dtype, weight.in_channels,
                                  weight.out_channels, relation)
+        if (dense is None and feats.dtype != torch.float32
+                and feats.ndim == 2
+                and int(feats.shape[1]) == weight.in_channels
+                and feats.dtype == weight.scales.dtype
+                and _padded_forward(feats, weight.in_channels,
+                                    weight.out_channels, relation)):
+            return _padded_conv(
+                feats, _quantized_fragments(weight, padded=True), weight.bits,
+                weight.out_channels, relation.require_sorted_implicit_gemm(),
+                relation.n_out_capacity, relation, bias, relu)
     return ext.sparse_quantized_conv_features(
         feats, weight.weight, weight.scales, weight.biases,
         relation.edges.in_rows, relation.edges.out_rows,
@@ -430,17 +507,21 @@ def _weight_fragments(weight5d: torch.Tensor) -> torch.Tensor:
     return _cached_weight(weight5d, 'fragments', ext.conv_weight_fragments)
 
 
-def _quantized_fragments(weight: QuantizedWeight) -> torch.Tensor:
+def _quantized_fragments(weight: QuantizedWeight,
+                         padded: bool = False) -> torch.Tensor:
     """The streamed matrix-core conv's fragment-ordered packed copy of a
     quantized weight (``ext.quantized_weight_fragments``: codes, scale and
     bias per 16-byte piece, dequantised in the kernel; empty when the shape
     takes the other matrix-core kernel), cached with the packed words and
     rebuilt when they, the scales or the biases change."""
-    kind = ('quantized fragments', id(weight.scales), weight.scales._version,
+    kind = ('padded quantized fragments' if padded else 'quantized fragments',
+            id(weight.scales), weight.scales._version,
             id(weight.biases), weight.biases._version)
+    fragments = (ext.quantized_padded_fragments if padded
+                 else ext.quantized_weight_fragments)
 
     def make(words):
-        return ext.quantized_weight_fragments(
+        return fragments(
             words, weight.scales, weight.biases, weight.in_channels,
             weight.out_channels, weight.storage_in_channels,
             weight.group_size, weight.bits)

@@ -212,6 +212,16 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("in_edge_ids"), py::arg("kernel_row_offsets"), py::arg("kernel_edge_ids"), py::arg("out_capacity"),
         py::arg("n_kernels"), py::arg("store_sorted") = false, py::kw_only(), py::arg("bias") = py::none(),
         py::arg("tile_order") = py::none(), py::arg("relu") = false, py::arg("weight_fragments") = py::none());
+    m.def("conv_padded_supported", &ln::conv_padded_supported, py::arg("feats"), py::arg("out_channels"),
+          py::arg("n_kernels"), py::arg("out_capacity"));
+    m.def("conv_padded_fragments", &ln::conv_padded_fragments, py::arg("weights"), py::arg("role"));
+    m.def("quantized_padded_fragments", &ln::quantized_padded_fragments, py::arg("weights"), py::arg("scales"),
+          py::arg("biases"), py::arg("in_channels"), py::arg("out_channels"), py::arg("storage_in_channels"),
+          py::arg("group_size"), py::arg("bits"));
+    m.def("sparse_conv_features_padded", &ln::sparse_conv_features_padded, py::arg("feats"), py::arg("fragments"),
+          py::arg("bits"), py::arg("out_channels"), py::arg("sorted_kv_out_in_map"), py::arg("reorder_rows"),
+          py::arg("tile_masks"), py::arg("out_capacity"), py::arg("n_kernels"), py::kw_only(),
+          py::arg("bias") = py::none(), py::arg("tile_order") = py::none(), py::arg("relu") = false);
     m.def("conv_weight_fragments", &ln::conv_weight_fragments, py::arg("weights"),
           "Fragment-ordered copy of a 5D fp16/bf16 weight for the streamed matrix-core conv (empty when the shape "
           "does not take it).");

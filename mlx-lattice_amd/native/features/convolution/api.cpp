@@ -1,5 +1,6 @@
 #include "features/convolution/api.h"
 
+#include <climits>
 #include <stdexcept>
 #include <string>
 
@@ -332,9 +333,11 @@ at::Tensor conv_weight_fragments(const at::Tensor& weights_in) {
     return frag;
 }
 
-at::Tensor quantized_weight_fragments(const at::Tensor& weights_in, const at::Tensor& scales_in,
-                                      const at::Tensor& biases_in, int in_channels, int out_channels,
-                                      int storage_in_channels, int group_size, int bits) {
+namespace {
+
+at::Tensor quantized_fragments(const at::Tensor& weights_in, const at::Tensor& scales_in,
+                               const at::Tensor& biases_in, int in_channels, int out_channels,
+                               int storage_in_channels, int group_size, int bits, bool padded) {
     if (weights_in.dim() != 3 || weights_in.scalar_type() != at::kUInt32) {
         throw std::invalid_argument("packed weights must be a three-dimensional uint32 array.");
     }
@@ -362,18 +365,115 @@ at::Tensor quantized_weight_fragments(const at::Tensor& weights_in, const at::Te
     int dtype = -1;
     if (scales_in.scalar_type() == at::kHalf) dtype = LATTICE_F16;
     if (scales_in.scalar_type() == at::kBFloat16) dtype = LATTICE_BF16;
-    const size_t bytes =
-        dtype < 0 ? 0 : lattice_hip_quantized_weight_fragments_bytes(dtype, k, in_channels, out_channels);
+    const size_t bytes = dtype < 0 ? 0
+                         : padded  ? lattice_hip_conv_padded_fragments_bytes(dtype, k, in_channels, out_channels)
+                                   : lattice_hip_quantized_weight_fragments_bytes(dtype, k, in_channels, out_channels);
     at::Tensor frag = at::empty({static_cast<int64_t>(bytes / 2)}, scales_in.options());
     if (bytes == 0) return frag;
     const at::Tensor weights = weights_in.contiguous();
     const at::Tensor scales = scales_in.contiguous();
     const at::Tensor biases = biases_in.contiguous();
-    check_status(lattice_hip_quantized_weight_fragments(
+    const auto make = padded ? lattice_hip_quantized_padded_fragments : lattice_hip_quantized_weight_fragments;
+    check_status(make(
         dtype, reinterpret_cast<const uint32_t*>(weights.data_ptr()), scales.data_ptr(), biases.data_ptr(), k,
         in_channels, out_channels, storage_in_channels, group_size, bits, frag.data_ptr(), bytes,
         current_stream(weights)));
     return frag;
+}
+
+}  // namespace
+
+at::Tensor quantized_weight_fragments(const at::Tensor& weights, const at::Tensor& scales, const at::Tensor& biases,
+                                      int in_channels, int out_channels, int storage_in_channels, int group_size,
+                                      int bits) {
+    return quantized_fragments(weights, scales, biases, in_channels, out_channels, storage_in_channels, group_size,
+                               bits, false);
+}
+
+at::Tensor quantized_padded_fragments(const at::Tensor& weights, const at::Tensor& scales, const at::Tensor& biases,
+                                      int in_channels, int out_channels, int storage_in_channels, int group_size,
+                                      int bits) {
+    return quantized_fragments(weights, scales, biases, in_channels, out_channels, storage_in_channels, group_size,
+                               bits, true);
+}
+
+bool conv_padded_supported(const at::Tensor& feats, int out_channels, int n_kernels, int out_capacity) {
+    if (feats.dim() != 2 || feats.size(0) > INT_MAX || feats.size(1) > INT_MAX) return false;
+    int dtype = -1;
+    if (feats.scalar_type() == at::kFloat) dtype = LATTICE_F32;
+    if (feats.scalar_type() == at::kHalf) dtype = LATTICE_F16;
+    if (feats.scalar_type() == at::kBFloat16) dtype = LATTICE_BF16;
+    if (dtype < 0) return false;
+    // a strided view is copied to a fresh (aligned) tensor by the conv
+    if (feats.is_contiguous() && reinterpret_cast<uintptr_t>(feats.data_ptr()) % 16 != 0) return false;
+    return lattice_hip_conv_padded_supported(dtype, static_cast<int>(feats.size(0)), static_cast<int>(feats.size(1)),
+                                             out_channels, n_kernels, out_capacity) != 0;
+}
+
+at::Tensor conv_padded_fragments(const at::Tensor& weights_in, int role) {
+    if (weights_in.dim() != 5 && weights_in.dim() != 3) {
+        throw std::invalid_argument("weights must have shape (K, C_in, C_out) or (C_out, Kx, Ky, Kz, C_in).");
+    }
+    require_device(weights_in, "weights");
+    const at::Tensor weights = weights_in.contiguous();
+    const bool mapped = weights.dim() == 3;
+    const int c_out = static_cast<int>(out_channels_of(weights));
+    const int c_in = static_cast<int>(mapped ? weights.size(1) : weights.size(4));
+    const int k = static_cast<int>(mapped ? weights.size(0) : weights.size(1) * weights.size(2) * weights.size(3));
+    const int dtype = dtype_code(weights, "conv_padded_fragments");
+    const bool swap = role != LATTICE_FRAGMENTS_FORWARD;
+    const size_t bytes = lattice_hip_conv_padded_fragments_bytes(dtype, k, swap ? c_out : c_in, swap ? c_in : c_out);
+    at::Tensor frag = at::empty({static_cast<int64_t>(bytes / weights.element_size())}, weights.options());
+    check_status(lattice_hip_conv_padded_fragments(
+        dtype, weights.data_ptr(), mapped ? LATTICE_WEIGHT_KERNEL_MAJOR : LATTICE_WEIGHT_DENSE_5D, k, c_in, c_out,
+        role, frag.data_ptr(), bytes, current_stream(weights)));
+    return frag;
+}
+
+at::Tensor sparse_conv_features_padded(const at::Tensor& feats_in, const at::Tensor& fragments, int bits,
+                                       int out_channels, const at::Tensor& sorted_kv_out_in_map,
+                                       const at::Tensor& reorder_rows, const at::Tensor& tile_masks,
+                                       int out_capacity, int n_kernels, const std::optional<at::Tensor>& bias,
+                                       const std::optional<at::Tensor>& tile_order, bool relu) {
+    const char* op = "sparse_conv_features_padded";
+    if (feats_in.dim() != 2) throw std::invalid_argument("feats must have shape (N, C_in).");
+    const int dtype = dtype_code(feats_in, op);
+    if (out_capacity < 0 || n_kernels <= 0 || out_channels <= 0) {
+        throw std::invalid_argument("out_capacity must be nonnegative and n_kernels must be positive.");
+    }
+    require_i32_vector(reorder_rows, "reorder_rows must have shape (N_out,) and int32 dtype.");
+    require_i32_vector(tile_masks, "tile_masks must have shape (ceil(N_out / 64) * 4,) and int32 dtype.");
+    if (sorted_kv_out_in_map.dim() != 2 || sorted_kv_out_in_map.scalar_type() != at::kInt ||
+        sorted_kv_out_in_map.size(0) != n_kernels || sorted_kv_out_in_map.size(1) != out_capacity ||
+        reorder_rows.size(0) != out_capacity || tile_masks.size(0) != ((out_capacity + 63) / 64) * 4) {
+        throw std::invalid_argument("sorted convolution view shape must match out_capacity and n_kernels.");
+    }
+    require_device(feats_in, "feats");
+    require_device(fragments, "fragments");
+    require_device(sorted_kv_out_in_map, "sorted_kv_out_in_map");
+    require_device(reorder_rows, "reorder_rows");
+    require_device(tile_masks, "tile_masks");
+    const at::Tensor feats = feats_in.contiguous();
+    const int c_in = static_cast<int>(feats.size(1));
+    const size_t frag_bytes = lattice_hip_conv_padded_fragments_bytes(dtype, n_kernels, c_in, out_channels);
+    if (!fragments.is_contiguous() ||
+        static_cast<size_t>(fragments.numel()) * fragments.element_size() < frag_bytes ||
+        fragments.scalar_type() != feats.scalar_type()) {
+        throw std::invalid_argument("fragments must be the padded fragments of this conv's weight.");
+    }
+    at::Tensor out = at::empty({out_capacity, out_channels}, feats.options());
+    const at::Tensor kv = sorted_kv_out_in_map.contiguous();
+    const at::Tensor tiles = tile_masks.contiguous();
+    const at::Tensor order = reorder_rows.contiguous();
+    size_t ws_bytes = 0;
+    at::Tensor ws = schedule_workspace(tile_order, out_capacity, feats, &ws_bytes);
+    at::Tensor bias_keep;
+    const void* b = bias_ptr(bias, feats, out_channels, &bias_keep);
+    check_status(lattice_hip_sparse_conv_features_padded(
+        dtype, feats.data_ptr(), static_cast<int>(feats.size(0)), c_in, fragments.data_ptr(), bits, n_kernels,
+        out_channels, ci32(kv), ci32(tiles), ci32(order), out_capacity, out.data_ptr(), b,
+        relu ? LATTICE_EPILOGUE_RELU : LATTICE_EPILOGUE_NONE, ws.data_ptr(), ws_bytes, current_stream(feats)));
+    return out;
 }
 
 at::Tensor conv_tile_order(const at::Tensor& tile_masks, int out_capacity) {

@@ -49,6 +49,23 @@ at::Tensor sparse_conv_features_sorted_implicit_gemm(const at::Tensor& feats, co
 // weight's shape does not take that route.
 at::Tensor conv_weight_fragments(const at::Tensor& weights);
 
+// The streamed conv for the types and channel counts the sorted entry does
+// not take (lattice_hip_sparse_conv_features_padded): whether a contiguous
+// `feats` and the shape qualify; the fragments of a float weight (role:
+// lattice_fragment_role) or of a packed one; the conv over a sorted view.
+bool conv_padded_supported(const at::Tensor& feats, int out_channels, int n_kernels, int out_capacity);
+at::Tensor conv_padded_fragments(const at::Tensor& weights, int role);
+at::Tensor quantized_padded_fragments(const at::Tensor& weights, const at::Tensor& scales, const at::Tensor& biases,
+                                      int in_channels, int out_channels, int storage_in_channels, int group_size,
+                                      int bits);
+at::Tensor sparse_conv_features_padded(const at::Tensor& feats, const at::Tensor& fragments, int bits,
+                                       int out_channels, const at::Tensor& sorted_kv_out_in_map,
+                                       const at::Tensor& reorder_rows, const at::Tensor& tile_masks,
+                                       int out_capacity, int n_kernels,
+                                       const std::optional<at::Tensor>& bias = std::nullopt,
+                                       const std::optional<at::Tensor>& tile_order = std::nullopt,
+                                       bool relu = false);
+
 at::Tensor sparse_quantized_conv_features(const at::Tensor& feats, const at::Tensor& weights,
                                           const at::Tensor& scales, const at::Tensor& biases,
                                           const at::Tensor& in_rows, const at::Tensor& out_rows,

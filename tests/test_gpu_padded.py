@@ -1,0 +1,188 @@
+"""The streamed conv's padded instances: float32, and channel counts that do
+not fill the tiles, against the fp64 edge sum over the oracle's relation.
+
+Bounds: a sum of L products in binary32, in any order, is off by at most
+(L + 1) 2^-24 sum|f w|; a 16-bit result then rounds once (2^-11 or 2^-8 of
+its value), and once more after the bias."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+from helpers import to_np
+from oracle import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+DEV = 'cuda'
+HALF_ULP = {torch.float32: 2.0 ** -24, torch.float16: 2.0 ** -11,
+            torch.bfloat16: 2.0 ** -8}
+
+
+def _cloud(rows, seed):
+    """Distinct voxels on the faces of a box and scattered around it, so
+    that rows use one to all of the 27 offsets."""
+    rng = np.random.default_rng(seed)
+    side = max(3, int(np.ceil((rows / 2) ** (1 / 3))))
+    dense = np.stack(np.meshgrid(*[np.arange(side)] * 3, indexing='ij'),
+                     -1).reshape(-1, 3)[:(rows + 1) // 2]
+    far = rng.integers(100, 100 + 4 * side, (8 * rows + 8, 3))
+    pts = np.concatenate([dense, np.unique(far, axis=0)])
+    pts = np.concatenate([pts[:len(dense)],
+                          rng.permutation(pts[len(dense):])])[:rows]
+    pts = pts[rng.permutation(len(pts))]
+    return np.concatenate([np.zeros((len(pts), 1), np.int64), pts],
+                          1).astype(np.int32), rng
+
+
+def _bound(feats, weight, rel, ref, dtype, c_in, bias):
+    mag = O.conv_features_fp64(np.abs(feats), O.mapped_weight(np.abs(weight)),
+                               rel)
+    terms = 27 * c_in + 1
+    out = terms * 2.0 ** -24 * mag
+    if dtype != torch.float32 or bias:
+        out = out + 2 * HALF_ULP[dtype] * (np.abs(ref) + 0.5 * bias) + 1e-7
+    return out + 1e-30
+
+
+def _check(actual, ref, bound, what):
+    err = np.abs(actual - ref)
+    assert np.isfinite(actual).all(), what
+    assert (err <= bound).all(), (what, float((err / bound).max()))
+
+
+@pytest.mark.parametrize('dtype,c_in,c_out,rows', [
+    (torch.float32, 4, 1, 1),          # one row, one column
+    (torch.float32, 20, 33, 63),       # partial chunk; one column past 32
+    (torch.float32, 32, 32, 64),       # whole chunk, whole column group
+    (torch.float32, 36, 64, 65),       # a row past the 64-row tile
+    (torch.float32, 64, 130, 129),     # two column tiles, odd columns
+    (torch.float32, 96, 96, 3001),
+    (torch.float16, 8, 24, 127),
+    (torch.float16, 40, 65, 129),      # columns with no 16-byte rows
+    (torch.float16, 96, 96, 3001),
+    (torch.bfloat16, 72, 200, 1000),   # two column tiles, the last partial
+    (torch.bfloat16, 320, 48, 500),    # five chunks
+])
+def test_padded_conv_matches_fp64(dtype, c_in, c_out, rows):
+    from mlx_lattice_amd import SparseTensor, ops
+    from mlx_lattice_amd._native import ext
+
+    coords, rng = _cloud(rows, 3 * c_in + c_out)
+    f = torch.as_tensor(rng.standard_normal((rows, c_in))).to(DEV, dtype)
+    w = torch.as_tensor(rng.standard_normal((c_out, 3, 3, 3, c_in))
+                        / np.sqrt(9 * c_in)).to(DEV, dtype)
+    b = torch.as_tensor(rng.standard_normal(c_out)).to(DEV, dtype)
+    print(f'padded {dtype} {c_in}->{c_out} rows={rows}', flush=True)
+    x = SparseTensor(torch.as_tensor(coords).to(DEV), f)
+    rel = x.coord_manager.submanifold_kernel_relation(x.coord_key,
+                                                      kernel_size=3)
+    view = rel.require_sorted_implicit_gemm()
+    plain = ext.sparse_conv_features_padded(
+        f, ext.conv_padded_fragments(w, 0), 0, c_out,
+        view.sorted_kv_out_in_map, view.reorder_rows, view.tile_masks, rows,
+        27)
+    orel = O.kernel_relation(coords, kernel_size=3)
+    fd, wd = to_np(f.double()), to_np(w.double())
+    ref = O.conv_features_fp64(fd, O.mapped_weight(wd), orel)
+    _check(to_np(plain.double()), ref,
+           _bound(fd, wd, orel, ref, dtype, c_in, 0.0), 'plain')
+    # the operator takes this route (bit for bit), bias and ReLU included;
+    # a mapped weight is the same weight
+    for weight in (w, w.permute(1, 2, 3, 4, 0).reshape(27, c_in, c_out)):
+        y = ops.subm_conv3d(x, weight.contiguous(), kernel_size=3)
+        assert torch.equal(y.feats, plain)
+    y = ops.subm_conv3d(x, w, b, kernel_size=3, activation='relu')
+    assert torch.equal(y.feats, torch.relu(plain + b))
+    # a strided view of the features gives the same; rows that do not start
+    # at 16 bytes are refused here and run on the CSR route
+    wide = torch.cat([f, f], 1)
+    assert torch.equal(
+        ops.subm_conv3d(x.replace(feats=wide[:, :c_in]), w).feats, plain)
+    flat = torch.empty(rows * c_in + 1, dtype=dtype, device=DEV)
+    off = flat[1:].view(rows, c_in)
+    off.copy_(f)
+    assert not ext.conv_padded_supported(off, c_out, 27, rows)
+    y = ops.subm_conv3d(x.replace(feats=off), w)
+    _check(to_np(y.feats.double()), ref,
+           _bound(fd, wd, orel, ref, dtype, c_in, 0.0), 'misaligned')
+    torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize('dtype,bits,c_in,c_out', [
+    (torch.float16, 4, 96, 96), (torch.float16, 8, 40, 24),
+    (torch.bfloat16, 4, 288, 48), (torch.bfloat16, 8, 64, 96)])
+def test_padded_quantized_conv_matches_the_unpacked_weight(dtype, bits, c_in,
+                                                           c_out):
+    from mlx_lattice_amd import SparseTensor, dequantize_weight, ops
+    from mlx_lattice_amd import quantize_weight
+
+    rows = 777
+    coords, rng = _cloud(rows, bits + c_in)
+    f = torch.as_tensor(rng.standard_normal((rows, c_in))).to(DEV, dtype)
+    q = quantize_weight(torch.as_tensor(
+        rng.standard_normal((c_out, 3, 3, 3, c_in)) / np.sqrt(9 * c_in)).to(
+            DEV, dtype), group_size=32, bits=bits)
+    print(f'padded int{bits} {dtype} {c_in}->{c_out}', flush=True)
+    x = SparseTensor(torch.as_tensor(coords).to(DEV), f)
+    y = ops.subm_conv3d(x, q, kernel_size=3)
+    torch.cuda.synchronize()
+    # codes * scale + bias before the rounding of dequantize_weight: the
+    # kernel rounds once to the feature type, half an ulp of the weight
+    wd = to_np(dequantize_weight(q).double())
+    orel = O.kernel_relation(coords, kernel_size=3)
+    fd = to_np(f.double())
+    ref = O.conv_features_fp64(fd, O.mapped_weight(wd), orel)
+    mag = O.conv_features_fp64(np.abs(fd), O.mapped_weight(np.abs(wd)), orel)
+    bound = _bound(fd, wd, orel, ref, dtype, c_in, 0.0)
+    _check(to_np(y.feats.double()), ref,
+           bound + 2 * HALF_ULP[dtype] * mag, f'int{bits}')
+
+
+@pytest.mark.parametrize('dtype,c_in,c_out', [
+    (torch.float32, 64, 64), (torch.float32, 12, 20),
+    (torch.bfloat16, 96, 96)])
+@pytest.mark.parametrize('op', ['subm', 'down', 'up'])
+def test_padded_input_grad_matches_fp64(op, dtype, c_in, c_out):
+    """Over the forward view with the mirrored weight (submanifold), and the
+    transposed view (strided and transposed convs)."""
+    from mlx_lattice_amd import SparseTensor, ops
+
+    rows = 900 if op != 'up' else 150
+    coords, rng = _cloud(rows, 7 + c_in)
+    f = torch.as_tensor(rng.standard_normal((rows, c_in))).to(
+        DEV, dtype).requires_grad_()
+    w = torch.as_tensor(rng.standard_normal((c_out, 3, 3, 3, c_in))
+                        / np.sqrt(9 * c_in)).to(DEV, dtype)
+    x = SparseTensor(torch.as_tensor(coords).to(DEV), f,
+                     stride=2 if op == 'up' else 1)
+    print(f'padded input grad {op} {dtype} {c_in}->{c_out}', flush=True)
+    if op == 'subm':
+        y = ops.subm_conv3d(x, w, kernel_size=3)
+        rel = O.kernel_relation(coords, kernel_size=3)
+    elif op == 'down':
+        y = ops.conv3d(x, w, kernel_size=3, stride=2, padding=1)
+        rel = O.kernel_relation(coords, kernel_size=3, stride=2, padding=1)
+    else:
+        y = ops.conv_transpose3d(x, w, kernel_size=3, stride=2)
+        rel = O.transposed_kernel_relation(coords, kernel_size=3, stride=2)
+    cot = torch.as_tensor(rng.standard_normal(tuple(y.feats.shape))).to(
+        DEV, dtype)
+    grad, = torch.autograd.grad(y.feats, f, cot)
+    torch.cuda.synchronize()
+    e = int(rel['counts'][0])
+    i, o, k = (rel[n][:e] for n in ('in_rows', 'out_rows', 'kernel_ids'))
+    wk = to_np(w.double()).reshape(c_out, 27, c_in)
+    cd = to_np(cot.double())
+    ref = np.zeros((rows, c_in))
+    mag = np.zeros((rows, c_in))
+    for j in range(27):
+        at = k == j
+        np.add.at(ref, i[at], cd[o[at]] @ wk[:, j])
+        np.add.at(mag, i[at], np.abs(cd[o[at]]) @ np.abs(wk[:, j]))
+    bound = (27 * c_out + 1) * 2.0 ** -24 * mag + 1e-30
+    if dtype != torch.float32:
+        bound = bound + 2 * HALF_ULP[dtype] * np.abs(ref) + 1e-7
+    _check(to_np(grad.double()), ref, bound, op)
