@@ -6,8 +6,9 @@
 //    accumulator; lanes of a row read the same feature values (broadcast)
 //    and consecutive output channels of the weight (coalesced).  Follows
 //    the output-stationary loop of cpu/algorithms.cpp:180-302 and, for packed
-//    weights, cpu/quantized.cpp:64-141.  Used for fp32, for channel counts
-//    that do not tile the matrix cores, and for small problems.
+//    weights, cpu/quantized.cpp:64-141.  Used for input rows
+//    that are not whole 16-byte pieces, K > 32 and relations the dense map
+//    cannot hold.
 //  * Implicit-GEMM route (MFMA path): output rows are visited in the
 //    mask-sorted order of the sorted view (core/relations/views.py:467-510),
 //    64 rows per 256-thread block.  For every kernel offset that any row of
@@ -1501,7 +1502,13 @@ __device__ inline void stream_store_padded(const float4_t (&acc)[RB][CB], T* sta
 // memory access), a wave whose 32 columns all lie past C_out issues no
 // MFMAs, and the store guards the columns.  The chunks of an offset are then
 // stages of their own (NCH = 1; each loads its row indices), so one instance
-// serves every C_in.
+// serves every C_in.  float32 runs the same pipeline on 16x16x4 MFMAs, where
+// it is bound by the matrix cores (a stage's MFMAs take eight times as long
+// per byte gathered), so its tiles are 64 rows: twice the blocks to fill the
+// chip, and half the longest block.  Measured against the CSR kernels, whose
+// lanes load both factors of every product: 96 -> 96 bf16 over 150,001 rows
+// (4.6 edges each) 19,300 -> 45 us; 64 -> 64 float32 over 60,001 rows 3,000
+// -> 55 us, its input gradient 629 -> 55 us.
 template <typename T, typename S, int NCH, int QB, bool PAD = false>
 __global__ void __launch_bounds__(S::THREADS, S::OCC)
 conv_igemm_stream(const T* __restrict__ feats, int n_in, int c_in, const T* __restrict__ wfrag, int kernel_count,
