@@ -607,10 +607,10 @@ int lattice_hip_build_transposed_implicit_gemm_map(
  * grad[k, ci, co] = sum over the edges of offset k in the kernel-grouped CSR
  * (kernel_row_offsets [K + 1], kernel_edge_ids) of
  * feats[in_rows[e], ci] * cot[out_rows[e], co], fp32 accumulator, one
- * rounding, written in `weight_layout`.  fp16/bf16 with c_in and c_out
- * multiples of 8 run on the matrix cores and need the workspace
- * (lattice_hip_conv_weight_grad_workspace_bytes, 0 for other shapes); the
- * result is deterministic.  Other shapes take a lane-per-weight kernel. */
+ * rounding, written in `weight_layout`.  With the workspace
+ * (lattice_hip_conv_weight_grad_workspace_bytes) it runs on the matrix
+ * cores (float32 on 16x16x4 MFMAs, every product and sum in binary32),
+ * deterministically; without one, one lane per weight value. */
 size_t lattice_hip_conv_weight_grad_workspace_bytes(int dtype,
                                                     int kernel_count,
                                                     int c_in, int c_out,

@@ -29,8 +29,12 @@
 //    fragments (8 consecutive edges per lane) with transposing LDS reads
 //    and accumulates in fp32.  Each block writes its partial tile; a second
 //    kernel sums an offset's partials in a fixed order and rounds once, so
-//    results are deterministic.  Other dtypes and shapes take a
-//    one-lane-per-weight kernel.
+//    results are deterministic.  float32 contracts on 16x16x4 MFMAs over the
+//    same steps; rows that are not whole 16-byte pieces are loaded value by
+//    value.  Callers without a workspace take a one-lane-per-weight kernel,
+//    whose lanes walk all of an offset's edges through three dependent
+//    loads each: 64 -> 64 float32 over 60,001 rows (280k edges) 31,000 us
+//    there, 42 us (plus 18 us of reduction) here.
 
 #include <hip/hip_bf16.h>
 #include <hip/hip_fp16.h>
@@ -169,6 +173,12 @@ template <> struct GradMfma<__bf16> {
     }
 };
 
+// float32 contracts four edges per MFMA (16x16x4); the pieces are four
+// channels.
+template <> struct GradMfma<float> {
+    typedef float4_t vec;
+};
+
 constexpr int kWgEdges = 64;   // edges per staged step (two 32-edge MFMA steps)
 
 // LDS rows of a weight-gradient step: one row per edge, the operand's
@@ -180,8 +190,16 @@ __device__ inline int wg_swizzle(int r, int pieces) {
     return (2 * (r & 1) + 4 * ((r >> 1) & 1) + 8 * (((r >> 3) ^ r) & 1)) & (pieces - 1);
 }
 
-template <int TC>
-__device__ inline int wg_piece_slot(int r, int q) { return r * TC + ((q ^ wg_swizzle(r, TC / 8)) << 3); }
+// float32 rows are read one 4-byte value per lane, 16 channels of four rows
+// at a time: rows 16 floats apart in the banks spread them over all 64.
+template <typename T, int TC>
+constexpr int wg_row = sizeof(T) == 4 ? TC + 16 : TC;  // elements per staged row
+
+template <typename T, int TC>
+__device__ inline int wg_piece_slot(int r, int q) {
+    if constexpr (sizeof(T) == 4) return r * wg_row<T, TC> + q * 4;
+    return r * TC + ((q ^ wg_swizzle(r, TC / 8)) << 3);
+}
 
 typedef short short4_t __attribute__((ext_vector_type(4)));
 
@@ -201,7 +219,7 @@ __device__ inline V wg_fragment(const T* lds, int ks, int c0, int lane) {
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
         const int r = 32 * ks + 8 * g + 4 * t + (s >> 2);
-        const T* src = lds + wg_piece_slot<TC>(r, q) + 4 * (s & 1);
+        const T* src = lds + wg_piece_slot<T, TC>(r, q) + 4 * (s & 1);
         h[t] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
             (__attribute__((address_space(3))) short4_t*)(src));
     }
@@ -245,7 +263,9 @@ __device__ inline void wg_share(const int32_t* koff, int K, int slots, int k, in
 // Block (launch index): XCD x = index mod 8, then (tile, slot) from
 // index / 8; channel tile TCI x TCO, four waves of (TCI/2) x (TCO/2).  Per
 // step of 64 edges the block stages both operands into edge-major LDS rows.
-template <typename T, int TCI, int TCO>
+// VEC: rows are whole 16-byte pieces (16-byte loads); otherwise every value
+// is loaded by itself.
+template <typename T, int TCI, int TCO, bool VEC>
 __global__ void __launch_bounds__(256, 3)
 weight_grad_mfma(const T* __restrict__ feats, int n_in, int c_in, const T* __restrict__ cot, int n_out, int c_out,
                  const int32_t* __restrict__ in_rows, const int32_t* __restrict__ out_rows,
@@ -255,8 +275,9 @@ weight_grad_mfma(const T* __restrict__ feats, int n_in, int c_in, const T* __res
     using V = typename GradMfma<T>::vec;
     constexpr int MB = TCI / 32;  // 16-row blocks per wave
     constexpr int NB = TCO / 32;  // 16-column blocks per wave
-    __shared__ __align__(16) T a_t[kWgEdges * TCI];
-    __shared__ __align__(16) T b_t[kWgEdges * TCO];
+    constexpr int PE = 16 / static_cast<int>(sizeof(T));  // channels per 16-byte piece
+    __shared__ __align__(16) T a_t[kWgEdges * wg_row<T, TCI>];
+    __shared__ __align__(16) T b_t[kWgEdges * wg_row<T, TCO>];
     const int x = static_cast<int>(blockIdx.x) % kXcds;
     const int q = static_cast<int>(blockIdx.x) / kXcds;
     const int tile = q % tiles;
@@ -305,11 +326,11 @@ weight_grad_mfma(const T* __restrict__ feats, int n_in, int c_in, const T* __res
 #pragma unroll
         for (int n = 0; n < NB; ++n) acc[a][n] = float4_t{0.f, 0.f, 0.f, 0.f};
 
-    // Thread t stages edges t/8 and t/8 + 32 of the step: 8-channel pieces
-    // t%8 + 8i of their feature rows (i < TCI/64) and cotangent rows
-    // (i < TCO/64), so a wave's loads cover eight whole 128-byte row lines.
-    constexpr int PA = TCI / 64;
-    constexpr int PB = TCO / 64;
+    // Thread t stages edges t/8 and t/8 + 32 of the step: pieces t%8 + 8i of
+    // their feature rows (i < PA) and cotangent rows (i < PB), so a wave's
+    // loads cover eight whole 128-byte row lines.
+    constexpr int PA = TCI / (8 * PE);
+    constexpr int PB = TCO / (8 * PE);
     const int j = threadIdx.x >> 3;
     const int p = threadIdx.x & 7;
     V av[2][PA], bv[2][PB];
@@ -352,21 +373,41 @@ weight_grad_mfma(const T* __restrict__ feats, int n_in, int c_in, const T* __res
             ro[h] = ok ? rout[h] : -1;
         }
     };
+    // Channels c .. of a row (VEC: one load; c past the row re-reads its
+    // start, masked when the piece is staged).
+    auto load_piece = [&](const T* row, int c, int channels) {
+        if constexpr (VEC) {
+            return *reinterpret_cast<const V*>(row + (c < channels ? c : 0));
+        } else {
+            V v;
+#pragma unroll
+            for (int e = 0; e < PE; ++e) v[e] = row[min(c + e, channels - 1)];
+            return v;
+        }
+    };
+    auto staged_piece = [&](V v, bool ok, int c, int channels) {
+        if constexpr (!VEC) {
+#pragma unroll
+            for (int e = 0; e < PE; ++e)
+                if (c + e >= channels) v[e] = T(0);
+        }
+        return ok ? v : V{};
+    };
     auto gather = [&](const int (&ri)[2], const int (&ro)[2]) {
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
             const long long rin = ri[h] >= 0 ? ri[h] : 0, rout = ro[h] >= 0 ? ro[h] : 0;
 #pragma unroll
             for (int i = 0; i < PA; ++i) {
-                const int c = ci0 + 8 * (p + 8 * i);
+                const int c = ci0 + PE * (p + 8 * i);
                 aok[h][i] = ri[h] >= 0 && c < c_in;
-                av[h][i] = *reinterpret_cast<const V*>(feats + rin * c_in + (c < c_in ? c : 0));
+                av[h][i] = load_piece(feats + rin * c_in, c, c_in);
             }
 #pragma unroll
             for (int i = 0; i < PB; ++i) {
-                const int c = co0 + 8 * (p + 8 * i);
+                const int c = co0 + PE * (p + 8 * i);
                 bok[h][i] = ro[h] >= 0 && c < c_out;
-                bv[h][i] = *reinterpret_cast<const V*>(cot + rout * c_out + (c < c_out ? c : 0));
+                bv[h][i] = load_piece(cot + rout * c_out, c, c_out);
             }
         }
     };
@@ -390,10 +431,12 @@ weight_grad_mfma(const T* __restrict__ feats, int n_in, int c_in, const T* __res
         for (int h = 0; h < 2; ++h) {
 #pragma unroll
             for (int i = 0; i < PA; ++i)
-                *reinterpret_cast<V*>(a_t + wg_piece_slot<TCI>(j + 32 * h, p + 8 * i)) = aok[h][i] ? av[h][i] : V{};
+                *reinterpret_cast<V*>(a_t + wg_piece_slot<T, TCI>(j + 32 * h, p + 8 * i)) =
+                    staged_piece(av[h][i], aok[h][i], ci0 + PE * (p + 8 * i), c_in);
 #pragma unroll
             for (int i = 0; i < PB; ++i)
-                *reinterpret_cast<V*>(b_t + wg_piece_slot<TCO>(j + 32 * h, p + 8 * i)) = bok[h][i] ? bv[h][i] : V{};
+                *reinterpret_cast<V*>(b_t + wg_piece_slot<T, TCO>(j + 32 * h, p + 8 * i)) =
+                    staged_piece(bv[h][i], bok[h][i], co0 + PE * (p + 8 * i), c_out);
         }
         __syncthreads();
         issue_rows(ev, rin, rout);                   // row indices of step s+2
@@ -406,19 +449,38 @@ weight_grad_mfma(const T* __restrict__ feats, int n_in, int c_in, const T* __res
             __builtin_amdgcn_sched_barrier(0);
             gather(ri, ro);  // rows of step s+1
             __builtin_amdgcn_sched_barrier(0);
+            if constexpr (sizeof(T) == 4) {
+                // lane (lr, g): channel lr of edge 4 ks + g
 #pragma unroll
-            for (int ks = 0; ks < 2; ++ks) {
-                V af[MB], bf[NB];
+                for (int ks = 0; ks < kWgEdges / 4; ++ks) {
+                    float af[MB], bf[NB];
 #pragma unroll
-                for (int m = 0; m < MB; ++m)
-                    af[m] = wg_fragment<V, TCI>(a_t, ks, (TCI / 2) * wm + 16 * m, lane);
+                    for (int m = 0; m < MB; ++m)
+                        af[m] = a_t[(4 * ks + g) * wg_row<T, TCI> + (TCI / 2) * wm + 16 * m + lr];
 #pragma unroll
-                for (int n = 0; n < NB; ++n)
-                    bf[n] = wg_fragment<V, TCO>(b_t, ks, (TCO / 2) * wn + 16 * n, lane);
+                    for (int n = 0; n < NB; ++n)
+                        bf[n] = b_t[(4 * ks + g) * wg_row<T, TCO> + (TCO / 2) * wn + 16 * n + lr];
 #pragma unroll
-                for (int m = 0; m < MB; ++m)
+                    for (int m = 0; m < MB; ++m)
 #pragma unroll
-                    for (int n = 0; n < NB; ++n) acc[m][n] = GradMfma<T>::mfma(af[m], bf[n], acc[m][n]);
+                        for (int n = 0; n < NB; ++n)
+                            acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x4f32(af[m], bf[n], acc[m][n], 0, 0, 0);
+                }
+            } else {
+#pragma unroll
+                for (int ks = 0; ks < 2; ++ks) {
+                    V af[MB], bf[NB];
+#pragma unroll
+                    for (int m = 0; m < MB; ++m)
+                        af[m] = wg_fragment<V, TCI>(a_t, ks, (TCI / 2) * wm + 16 * m, lane);
+#pragma unroll
+                    for (int n = 0; n < NB; ++n)
+                        bf[n] = wg_fragment<V, TCO>(b_t, ks, (TCO / 2) * wn + 16 * n, lane);
+#pragma unroll
+                    for (int m = 0; m < MB; ++m)
+#pragma unroll
+                        for (int n = 0; n < NB; ++n) acc[m][n] = GradMfma<T>::mfma(af[m], bf[n], acc[m][n]);
+                }
             }
             edges_of(evr_n, evv_n, ev_next);
         }
@@ -511,8 +573,7 @@ weight_grad_reduce(const float* __restrict__ partial, const int32_t* __restrict_
 
 // One lane per weight entry (k, ci, co), co fastest: the kernel-grouped
 // edges of k in order with an fp32 accumulator (eval_weight_grad_typed's
-// loop).  Used for fp32 and for channel counts the matrix-core kernel does
-// not take.
+// loop).  Used by callers that bring no workspace.
 template <typename T>
 __global__ void __launch_bounds__(256)
 weight_grad_simple(const T* __restrict__ feats, int n_in, const T* __restrict__ cot, int n_out,
@@ -553,10 +614,10 @@ int check_grad_dtype(int dtype) {
 // XCD's 32 CUs: one round, so the blocks of an XCD move together).
 constexpr int kWgEdgesPerBlock = 2048;
 constexpr int kWgMaxSlots = 96;
-int weight_grad_slots(int edge_capacity, int kernel_count) {
+int weight_grad_slots(int edge_capacity, int kernel_count, int tiles) {
     const long long want =
         (static_cast<long long>(edge_capacity) + kXcds * kWgEdgesPerBlock - 1) / (kXcds * kWgEdgesPerBlock);
-    return static_cast<int>(std::max<long long>(kernel_count, std::min<long long>(kWgMaxSlots, want)));
+    return static_cast<int>(std::max<long long>(kernel_count, std::min<long long>(kWgMaxSlots / tiles, want)));
 }
 
 // Channel tiles of the matrix-core weight gradient: 128-channel tiles where
@@ -566,25 +627,35 @@ struct WgTiles {
     int tci, tco, tiles_ci, tiles_co;
     int tiles() const { return tiles_ci * tiles_co; }
 };
-WgTiles wg_tiles(int c_in, int c_out) {
+// float32 takes tiles of 64 or 32: its MFMAs, a sixteenth of the 16-bit
+// rate, cost more than a second gather of the rows, so padding to 128 or 64
+// costs more than more tiles do (wider tiles' staged rows would also leave
+// room for fewer blocks per CU).
+// Rows that are not whole 16-byte pieces (vec false) take the narrow tile of
+// their type: value by value, the wide tiles' loads spill.
+WgTiles wg_tiles(int dtype, int c_in, int c_out, bool vec) {
     WgTiles t;
-    t.tci = c_in > 64 ? 128 : 64;
-    t.tco = c_out > 64 ? 128 : 64;
+    const int wide = dtype == LATTICE_F32 ? 64 : 128;
+    t.tci = vec && c_in > wide / 2 ? wide : wide / 2;
+    t.tco = vec && c_out > wide / 2 ? wide : wide / 2;
     t.tiles_ci = (c_in + t.tci - 1) / t.tci;
     t.tiles_co = (c_out + t.tco - 1) / t.tco;
     return t;
 }
 
-// One fp32 partial matrix (every channel tile, in fragment order) per block
-// slot.
-size_t weight_grad_partial_bytes(int edge_capacity, int kernel_count, int c_in, int c_out) {
-    const WgTiles t = wg_tiles(c_in, c_out);
-    return static_cast<size_t>(kXcds) * weight_grad_slots(edge_capacity, kernel_count) * t.tiles() * t.tci * t.tco *
-           sizeof(float);
+// Block slots of the launch: one round of blocks per XCD whatever the number
+// of channel tiles in float32 (its partial matrices would otherwise grow with
+// their square); 16-bit tiles each take a round of their own.
+int wg_slots(int dtype, int edge_capacity, int kernel_count, const WgTiles& t) {
+    return weight_grad_slots(edge_capacity, kernel_count, dtype == LATTICE_F32 ? std::min(t.tiles(), 4) : 1);
 }
 
-bool weight_grad_mfma_ok(int dtype, int c_in, int c_out) {
-    return (dtype == LATTICE_F16 || dtype == LATTICE_BF16) && c_in % 8 == 0 && c_out % 8 == 0;
+// One fp32 partial matrix (every channel tile, in fragment order) per block
+// slot; wide tiles (vec) need the most.
+size_t weight_grad_partial_bytes(int dtype, int edge_capacity, int kernel_count, int c_in, int c_out) {
+    const WgTiles t = wg_tiles(dtype, c_in, c_out, true);
+    return static_cast<size_t>(kXcds) * wg_slots(dtype, edge_capacity, kernel_count, t) * t.tiles() * t.tci * t.tco *
+           sizeof(float);
 }
 
 template <typename T>
@@ -606,33 +677,40 @@ int launch_weight_grad(int dtype, const void* feats, int n_in, const void* cot, 
                        const int32_t* in_rows, const int32_t* out_rows, const int32_t* counts, int edge_capacity,
                        const int32_t* koff, const int32_t* kedges, void* grad, void* workspace,
                        size_t workspace_bytes, hipStream_t stream) {
-    if (weight_grad_mfma_ok(dtype, widx.c_in, widx.c_out) && workspace != nullptr) {
-        if constexpr (!std::is_same<T, float>::value) {
-            const int slots = weight_grad_slots(edge_capacity, widx.K);
-            const size_t need = weight_grad_partial_bytes(edge_capacity, widx.K, widx.c_in, widx.c_out);
-            LATTICE_REQUIRE(workspace_bytes >= need, "weight gradient workspace too small.");
-            float* partial = static_cast<float*>(workspace);
-            const WgTiles wt = wg_tiles(widx.c_in, widx.c_out);
-            const int tci = wt.tci, tco = wt.tco, tiles_co = wt.tiles_co, tiles = wt.tiles();
-            const unsigned grid = static_cast<unsigned>(kXcds) * slots * tiles;
-#define LATTICE_WG_LAUNCH(A, B)                                                                                 \
-    weight_grad_mfma<T, A, B><<<grid, 256, 0, stream>>>(static_cast<const T*>(feats), n_in, widx.c_in,          \
-                                                        static_cast<const T*>(cot), n_out, widx.c_out, in_rows,  \
-                                                        out_rows, counts, edge_capacity, koff, kedges, widx.K,   \
-                                                        tiles, tiles_co, slots, partial)
-            if (tci == 128 && tco == 128) LATTICE_WG_LAUNCH(128, 128);
-            else if (tci == 128) LATTICE_WG_LAUNCH(128, 64);
-            else if (tco == 128) LATTICE_WG_LAUNCH(64, 128);
-            else LATTICE_WG_LAUNCH(64, 64);
+    const size_t need = weight_grad_partial_bytes(dtype, edge_capacity, widx.K, widx.c_in, widx.c_out);
+    // Without its workspace (or, for float32 and odd channel counts, with a
+    // smaller one) the call runs one lane per weight value.
+    const bool sixteens = dtype != LATTICE_F32 && widx.c_in % 8 == 0 && widx.c_out % 8 == 0;
+    if (workspace != nullptr && (sixteens || workspace_bytes >= need)) {
+        LATTICE_REQUIRE(workspace_bytes >= need, "weight gradient workspace too small.");
+        float* partial = static_cast<float*>(workspace);
+        const bool vec = (reinterpret_cast<uintptr_t>(feats) | reinterpret_cast<uintptr_t>(cot) |
+                          (static_cast<uintptr_t>(widx.c_in) * sizeof(T)) |
+                          (static_cast<uintptr_t>(widx.c_out) * sizeof(T))) %
+                             16 ==
+                         0;
+        const WgTiles wt = wg_tiles(dtype, widx.c_in, widx.c_out, vec);
+        const int slots = wg_slots(dtype, edge_capacity, widx.K, wt);
+        const int tci = wt.tci, tco = wt.tco, tiles_co = wt.tiles_co, tiles = wt.tiles();
+        const unsigned grid = static_cast<unsigned>(kXcds) * slots * tiles;
+#define LATTICE_WG_LAUNCH(A, B, VEC)                                                                            \
+    weight_grad_mfma<T, A, B, VEC><<<grid, 256, 0, stream>>>(                                                   \
+        static_cast<const T*>(feats), n_in, widx.c_in, static_cast<const T*>(cot), n_out, widx.c_out, in_rows,   \
+        out_rows, counts, edge_capacity, koff, kedges, widx.K, tiles, tiles_co, slots, partial)
+        constexpr int W = sizeof(T) == 4 ? 64 : 128;
+        if (!vec) LATTICE_WG_LAUNCH(W / 2, W / 2, false);
+        else if (tci == W && tco == W) LATTICE_WG_LAUNCH(W, W, true);
+        else if (tci == W) LATTICE_WG_LAUNCH(W, W / 2, true);
+        else if (tco == W) LATTICE_WG_LAUNCH(W / 2, W, true);
+        else LATTICE_WG_LAUNCH(W / 2, W / 2, true);
 #undef LATTICE_WG_LAUNCH
-            LATTICE_LAUNCH_CHECK();
-            const long long pieces = static_cast<long long>(tiles) * tci * tco / 4;
-            const dim3 rgrid(grid_for(pieces, 256, 256), static_cast<unsigned>(widx.K));
-            weight_grad_reduce<T><<<rgrid, 256, 0, stream>>>(partial, koff, slots, widx, tci, tco, tiles, tiles_co,
-                                                             static_cast<T*>(grad));
-            LATTICE_LAUNCH_CHECK();
-            return LATTICE_OK;
-        }
+        LATTICE_LAUNCH_CHECK();
+        const long long pieces = static_cast<long long>(tiles) * tci * tco / 4;
+        const dim3 rgrid(grid_for(pieces, 256, 256), static_cast<unsigned>(widx.K));
+        weight_grad_reduce<T><<<rgrid, 256, 0, stream>>>(partial, koff, slots, widx, tci, tco, tiles, tiles_co,
+                                                         static_cast<T*>(grad));
+        LATTICE_LAUNCH_CHECK();
+        return LATTICE_OK;
     }
     const long long total = static_cast<long long>(widx.K) * widx.c_in * widx.c_out;
     weight_grad_simple<T><<<grid_for(total, 256, 1u << 16), 256, 0, stream>>>(
@@ -714,8 +792,9 @@ extern "C" int lattice_hip_build_transposed_implicit_gemm_map(const int32_t* in_
 
 extern "C" size_t lattice_hip_conv_weight_grad_workspace_bytes(int dtype, int kernel_count, int c_in, int c_out,
                                                                 int edge_capacity) {
-    if (!weight_grad_mfma_ok(dtype, c_in, c_out) || kernel_count <= 0) return 0;
-    return weight_grad_partial_bytes(edge_capacity, kernel_count, c_in, c_out);
+    if (dtype != LATTICE_F32 && dtype != LATTICE_F16 && dtype != LATTICE_BF16) return 0;
+    if (kernel_count <= 0 || c_in <= 0 || c_out <= 0) return 0;
+    return weight_grad_partial_bytes(dtype, edge_capacity, kernel_count, c_in, c_out);
 }
 
 extern "C" int lattice_hip_sparse_conv_weight_grad(int dtype, const void* feats, int n_in, int c_in, const void* cot,

@@ -186,3 +186,58 @@ def test_padded_input_grad_matches_fp64(op, dtype, c_in, c_out):
     if dtype != torch.float32:
         bound = bound + 2 * HALF_ULP[dtype] * np.abs(ref) + 1e-7
     _check(to_np(grad.double()), ref, bound, op)
+
+
+@pytest.mark.parametrize('dtype,c_in,c_out,rows', [
+    (torch.float32, 64, 64, 3001),     # whole tiles
+    (torch.float32, 32, 64, 700),      # a narrow and a wide tile
+    (torch.float32, 4, 16, 65),        # most of a tile is padding
+    (torch.float32, 100, 72, 500),     # several tiles, the last partial
+    (torch.float32, 5, 3, 64),         # rows of no whole 16-byte piece
+    (torch.float32, 33, 64, 1),        # one edge
+    (torch.float16, 20, 96, 700),      # 40-byte rows
+    (torch.bfloat16, 130, 5, 300),
+])
+def test_weight_grad_matches_fp64(dtype, c_in, c_out, rows):
+    """The matrix-core weight gradient of float32 and of rows that are not
+    whole 16-byte pieces; also on features that start off a 16-byte border,
+    and with a mapped weight."""
+    from mlx_lattice_amd import SparseTensor
+    from mlx_lattice_amd.ops._relation_exec import (
+        sparse_conv_weight_grad_from_relation,
+    )
+
+    coords, rng = _cloud(rows, 11 + c_in)
+    f = torch.as_tensor(rng.standard_normal((rows, c_in))).to(DEV, dtype)
+    cot = torch.as_tensor(rng.standard_normal((rows, c_out))).to(DEV, dtype)
+    w = torch.zeros((c_out, 3, 3, 3, c_in), dtype=dtype, device=DEV)
+    print(f'weight grad {dtype} {c_in}->{c_out} rows={rows}', flush=True)
+    x = SparseTensor(torch.as_tensor(coords).to(DEV), f)
+    rel = x.coord_manager.submanifold_kernel_relation(x.coord_key,
+                                                      kernel_size=3)
+    grad = sparse_conv_weight_grad_from_relation(f, cot, w, rel)
+    flat = torch.empty(rows * c_in + 1, dtype=dtype, device=DEV)
+    off = flat[1:].view(rows, c_in)
+    off.copy_(f)
+    shifted = sparse_conv_weight_grad_from_relation(off, cot, w, rel)
+    mapped = sparse_conv_weight_grad_from_relation(
+        f, cot, torch.zeros((27, c_in, c_out), dtype=dtype, device=DEV), rel)
+    torch.cuda.synchronize()
+    orel = O.kernel_relation(coords, kernel_size=3)
+    e = int(orel['counts'][0])
+    i, o, k = (orel[n][:e] for n in ('in_rows', 'out_rows', 'kernel_ids'))
+    fd, cd = to_np(f.double()), to_np(cot.double())
+    ref = np.zeros((27, c_out, c_in))
+    mag = np.zeros((27, c_out, c_in))
+    for j in range(27):
+        at = k == j
+        ref[j] = cd[o[at]].T @ fd[i[at]]
+        mag[j] = (at.sum() + 1) * 2.0 ** -24 * (
+            np.abs(cd[o[at]]).T @ np.abs(fd[i[at]]))
+    bound = mag + 1e-30
+    if dtype != torch.float32:
+        bound = bound + 2 * HALF_ULP[dtype] * np.abs(ref) + 1e-7
+    for got, what in ((grad, '5D'), (shifted, 'off a 16-byte border')):
+        got = to_np(got.double()).reshape(c_out, 27, c_in).transpose(1, 0, 2)
+        _check(got, ref, bound, what)
+    _check(to_np(mapped.double()).transpose(0, 2, 1), ref, bound, 'mapped')
