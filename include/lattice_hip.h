@@ -623,6 +623,31 @@ int lattice_hip_sparse_conv_weight_grad(
     const int32_t* kernel_edge_ids, void* grad, void* workspace,
     size_t workspace_bytes, void* stream);
 
+/* The edges of a relation grouped by offset (write_relation_grouped_view,
+ * relation_views_detail.h:84-120), for relations whose edges run in
+ * (out_row, offset) order and whose row masks hold one bit per edge: the
+ * forward, submanifold and target builds' row_masks [rows], row_offsets
+ * [rows + 1] and in_rows [edge_capacity], K <= 32.  Writes
+ * kernel_row_offsets [K + 1] and, each when non-NULL, pairs
+ * [edge_capacity][2] (input row, output row) and kernel_edge_ids
+ * [edge_capacity], both defined on their first kernel_row_offsets[K]
+ * entries; the same grouping, in the same order, as
+ * lattice_hip_build_relation_grouped_views.  The weight gradient over the
+ * pairs is that of the entry above (the same result bit for bit). */
+size_t lattice_hip_kernel_pairs_workspace_bytes(int rows);
+int lattice_hip_build_kernel_pairs(const int32_t* row_masks,
+                                   const int32_t* row_offsets,
+                                   const int32_t* in_rows, int rows,
+                                   int kernel_count, int edge_capacity,
+                                   int32_t* kernel_row_offsets, int32_t* pairs,
+                                   int32_t* kernel_edge_ids, void* workspace,
+                                   size_t workspace_bytes, void* stream);
+int lattice_hip_sparse_conv_weight_grad_pairs(
+    int dtype, const void* feats, int n_in, int c_in, const void* cot,
+    int out_capacity, int c_out, int weight_layout, int kernel_count,
+    const int32_t* pairs, int edge_capacity, const int32_t* kernel_row_offsets,
+    void* grad, void* workspace, size_t workspace_bytes, void* stream);
+
 /* Sparse pooling over a kernel relation (SparsePoolFeatures,
  * pooling/cpu/algorithms.cpp:180-242; binding sparse_pool_features,
  * bindings/pooling.cpp:15-66).  mode 0 sum, 1 max, 2 avg; fp32 features

@@ -157,6 +157,134 @@ transposed_masks(const int32_t* __restrict__ in_out_map, int in_capacity, int K,
     }
 }
 
+// ------------------------------------------ edges grouped by the offset --
+//
+// A relation whose edges run in (out_row, offset) order and whose row masks
+// hold one bit per edge groups by offset without a sort: the edges of offset
+// k are the rows with bit k, in row order, and row r's is number
+// popcount(mask & below k) of its run.  group_count counts the bits of every
+// 1024-row block, group_scan places the blocks (offset by offset), and
+// group_emit writes each edge's (input row, output row) pair and, when asked
+// for, its id.  The masks, the run starts and the input rows are read once
+// and the groups written once, against radix passes over the relation's
+// whole capacity (K slots per row, used or not): 200k rows, 2.1M edges, both
+// sorted groupings 440 us, the pairs 27 us (count 5, scan 5, emit 17).
+constexpr int kGroupRows = 1024;   // rows per block, 64 per wave
+constexpr int kGroupWaves = kGroupRows / kWave;
+constexpr int kGroupBins = 32;     // offsets per block counter row
+
+// counts of the wave's 64 masks: lane k (< 32) gets the rows with bit k
+__device__ inline int wave_bit_counts(uint32_t mask, int K, int lane) {
+    int mine = 0;
+    for (int k = 0; k < K; ++k) {
+        const int c = __popcll(ballot((mask >> k) & 1u));
+        mine = lane == k ? c : mine;
+    }
+    return mine;
+}
+
+__global__ void __launch_bounds__(kGroupRows)
+group_count(const int32_t* __restrict__ row_masks, int rows, int K, int32_t* __restrict__ block_counts) {
+    __shared__ int32_t wave_counts[kGroupWaves][kGroupBins];
+    const int lane = lane_id();
+    const int wave = threadIdx.x / kWave;
+    const long long row = static_cast<long long>(blockIdx.x) * kGroupRows + threadIdx.x;
+    const uint32_t mask = row < rows ? static_cast<uint32_t>(row_masks[row]) : 0u;
+    const int c = wave_bit_counts(mask, K, lane);
+    if (lane < kGroupBins) wave_counts[wave][lane] = c;
+    __syncthreads();
+    if (threadIdx.x < kGroupBins) {
+        int sum = 0;
+#pragma unroll
+        for (int w = 0; w < kGroupWaves; ++w) sum += wave_counts[w][threadIdx.x];
+        block_counts[static_cast<long long>(blockIdx.x) * kGroupBins + threadIdx.x] = sum;
+    }
+}
+
+// One workgroup: thread (segment, k) sums its run of blocks, the segments
+// and offsets are scanned in LDS, and the counts become places in turn.
+__global__ void __launch_bounds__(1024)
+group_scan(int32_t* __restrict__ block_counts, int blocks, int K, int32_t* __restrict__ offsets) {
+    constexpr int kSegments = 1024 / kGroupBins;
+    __shared__ int32_t sums[kSegments][kGroupBins];
+    __shared__ int32_t base[kGroupBins];
+    const int k = threadIdx.x % kGroupBins;
+    const int seg = threadIdx.x / kGroupBins;
+    const int per = (blocks + kSegments - 1) / kSegments;
+    const int lo = min(seg * per, blocks), hi = min(lo + per, blocks);
+    int sum = 0;
+    for (int b = lo; b < hi; ++b) sum += block_counts[static_cast<long long>(b) * kGroupBins + k];
+    sums[seg][k] = sum;
+    __syncthreads();
+    if (threadIdx.x < kGroupBins) {
+        int run = 0;
+        for (int i = 0; i < kSegments; ++i) {
+            const int v = sums[i][threadIdx.x];
+            sums[i][threadIdx.x] = run;
+            run += v;
+        }
+        base[threadIdx.x] = run;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        int run = 0;
+        for (int i = 0; i < kGroupBins; ++i) {
+            const int v = base[i];
+            base[i] = run;
+            if (i <= K) offsets[i] = run;
+            run += v;
+        }
+        if (K == kGroupBins) offsets[K] = run;
+    }
+    __syncthreads();
+    int run = base[k] + sums[seg][k];
+    for (int b = lo; b < hi; ++b) {
+        int32_t* c = block_counts + static_cast<long long>(b) * kGroupBins + k;
+        const int v = *c;
+        *c = run;
+        run += v;
+    }
+}
+
+__global__ void __launch_bounds__(kGroupRows)
+group_emit(const int32_t* __restrict__ row_masks, const int32_t* __restrict__ row_offsets,
+           const int32_t* __restrict__ in_rows, int rows, int K, int edge_capacity,
+           const int32_t* __restrict__ block_places, int2* __restrict__ pairs, int32_t* __restrict__ edge_ids) {
+    __shared__ int32_t place[kGroupWaves][kGroupBins];
+    const int lane = lane_id();
+    const int wave = threadIdx.x / kWave;
+    const long long row = static_cast<long long>(blockIdx.x) * kGroupRows + threadIdx.x;
+    const uint32_t mask = row < rows ? static_cast<uint32_t>(row_masks[row]) : 0u;
+    const int first = row < rows ? row_offsets[row] : 0;
+    const int c = wave_bit_counts(mask, K, lane);
+    if (lane < kGroupBins) place[wave][lane] = c;
+    __syncthreads();
+    if (threadIdx.x < kGroupBins) {
+        int run = block_places[static_cast<long long>(blockIdx.x) * kGroupBins + threadIdx.x];
+#pragma unroll
+        for (int w = 0; w < kGroupWaves; ++w) {
+            const int v = place[w][threadIdx.x];
+            place[w][threadIdx.x] = run;
+            run += v;
+        }
+    }
+    __syncthreads();
+    for (int k = 0; k < K; ++k) {
+        const bool has = (mask >> k) & 1u;
+        const uint64_t b = ballot(has);
+        if (has) {
+            const int pos = place[wave][k] + lanes_below(b);
+            const int e = first + __popc(mask & ((1u << k) - 1u));
+            if (pos >= 0 && pos < edge_capacity && e >= 0 && e < edge_capacity) {
+                if (pairs != nullptr) pairs[pos] = make_int2(in_rows[e], static_cast<int>(row));
+                if (edge_ids != nullptr) edge_ids[pos] = e;
+            }
+        }
+    }
+}
+
+size_t group_blocks(int rows) { return (static_cast<size_t>(std::max(rows, 0)) + kGroupRows - 1) / kGroupRows; }
+
 // --------------------------------------- weight gradient (matrix cores) --
 
 template <typename T> struct GradMfma;
@@ -264,14 +392,16 @@ __device__ inline void wg_share(const int32_t* koff, int K, int slots, int k, in
 // index / 8; channel tile TCI x TCO, four waves of (TCI/2) x (TCO/2).  Per
 // step of 64 edges the block stages both operands into edge-major LDS rows.
 // VEC: rows are whole 16-byte pieces (16-byte loads); otherwise every value
-// is loaded by itself.
-template <typename T, int TCI, int TCO, bool VEC>
+// is loaded by itself.  PAIRS: the grouped edges come as (input row, output
+// row) pairs, one 8-byte load each, instead of as ids into the edge arrays
+// (two dependent loads, the second of neighbours a row's degree apart).
+template <typename T, int TCI, int TCO, bool VEC, bool PAIRS>
 __global__ void __launch_bounds__(256, 3)
 weight_grad_mfma(const T* __restrict__ feats, int n_in, int c_in, const T* __restrict__ cot, int n_out, int c_out,
                  const int32_t* __restrict__ in_rows, const int32_t* __restrict__ out_rows,
                  const int32_t* __restrict__ counts, int edge_capacity, const int32_t* __restrict__ koff,
-                 const int32_t* __restrict__ kedges, int K, int tiles, int tiles_co, int slots,
-                 float* __restrict__ partial) {
+                 const int32_t* __restrict__ kedges, const int2* __restrict__ kpairs, int K, int tiles, int tiles_co,
+                 int slots, float* __restrict__ partial) {
     using V = typename GradMfma<T>::vec;
     constexpr int MB = TCI / 32;  // 16-row blocks per wave
     constexpr int NB = TCO / 32;  // 16-column blocks per wave
@@ -306,7 +436,7 @@ weight_grad_mfma(const T* __restrict__ feats, int n_in, int c_in, const T* __res
     if (k < 0) return;  // a spare slot: no partial tile is read for it
     const int ci0 = (tile / tiles_co) * TCI;
     const int co0 = (tile % tiles_co) * TCO;
-    const int E = min(counts[0], edge_capacity);
+    const int E = PAIRS ? edge_capacity : min(counts[0], edge_capacity);
     const int lo_k = koff[k];
     const long long n_k = koff[k + 1] - lo_k;
     const int lo = lo_k + static_cast<int>(n_k * x / kXcds);
@@ -349,7 +479,7 @@ weight_grad_mfma(const T* __restrict__ feats, int n_in, int c_in, const T* __res
         for (int h = 0; h < 2; ++h) {
             const int cur = base + j + 32 * h;
             evv[h] = cur < hi;
-            evr[h] = kedges[min(cur, last_edge)];
+            evr[h] = PAIRS ? cur : kedges[min(cur, last_edge)];
         }
     };
     auto edges_of = [&](const int (&evr)[2], const bool (&evv)[2], int (&ev)[2]) {
@@ -360,8 +490,14 @@ weight_grad_mfma(const T* __restrict__ feats, int n_in, int c_in, const T* __res
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
             const int e = ev[h] >= 0 && ev[h] < E ? ev[h] : 0;
-            rin[h] = in_rows[e];
-            rout[h] = out_rows[e];
+            if constexpr (PAIRS) {
+                const int2 io = kpairs[e];
+                rin[h] = io.x;
+                rout[h] = io.y;
+            } else {
+                rin[h] = in_rows[e];
+                rout[h] = out_rows[e];
+            }
         }
     };
     auto rows_of = [&](const int (&ev)[2], const int (&rin)[2], const int (&rout)[2], int (&ri)[2], int (&ro)[2]) {
@@ -675,7 +811,7 @@ void launch_input_grad(const void* cot, int out_capacity, const void* weights, G
 template <typename T>
 int launch_weight_grad(int dtype, const void* feats, int n_in, const void* cot, int n_out, GradWeightIndex widx,
                        const int32_t* in_rows, const int32_t* out_rows, const int32_t* counts, int edge_capacity,
-                       const int32_t* koff, const int32_t* kedges, void* grad, void* workspace,
+                       const int32_t* koff, const int32_t* kedges, const int2* kpairs, void* grad, void* workspace,
                        size_t workspace_bytes, hipStream_t stream) {
     const size_t need = weight_grad_partial_bytes(dtype, edge_capacity, widx.K, widx.c_in, widx.c_out);
     // Without its workspace (or, for float32 and odd channel counts, with a
@@ -693,10 +829,15 @@ int launch_weight_grad(int dtype, const void* feats, int n_in, const void* cot, 
         const int slots = wg_slots(dtype, edge_capacity, widx.K, wt);
         const int tci = wt.tci, tco = wt.tco, tiles_co = wt.tiles_co, tiles = wt.tiles();
         const unsigned grid = static_cast<unsigned>(kXcds) * slots * tiles;
-#define LATTICE_WG_LAUNCH(A, B, VEC)                                                                            \
-    weight_grad_mfma<T, A, B, VEC><<<grid, 256, 0, stream>>>(                                                   \
+#define LATTICE_WG_KERNEL(A, B, VEC, PAIRS)                                                                     \
+    weight_grad_mfma<T, A, B, VEC, PAIRS><<<grid, 256, 0, stream>>>(                                            \
         static_cast<const T*>(feats), n_in, widx.c_in, static_cast<const T*>(cot), n_out, widx.c_out, in_rows,   \
-        out_rows, counts, edge_capacity, koff, kedges, widx.K, tiles, tiles_co, slots, partial)
+        out_rows, counts, edge_capacity, koff, kedges, kpairs, widx.K, tiles, tiles_co, slots, partial)
+#define LATTICE_WG_LAUNCH(A, B, VEC)                                     \
+    do {                                                                 \
+        if (kpairs != nullptr) LATTICE_WG_KERNEL(A, B, VEC, true);       \
+        else LATTICE_WG_KERNEL(A, B, VEC, false);                        \
+    } while (0)
         constexpr int W = sizeof(T) == 4 ? 64 : 128;
         if (!vec) LATTICE_WG_LAUNCH(W / 2, W / 2, false);
         else if (tci == W && tco == W) LATTICE_WG_LAUNCH(W, W, true);
@@ -704,6 +845,7 @@ int launch_weight_grad(int dtype, const void* feats, int n_in, const void* cot, 
         else if (tco == W) LATTICE_WG_LAUNCH(W / 2, W, true);
         else LATTICE_WG_LAUNCH(W / 2, W / 2, true);
 #undef LATTICE_WG_LAUNCH
+#undef LATTICE_WG_KERNEL
         LATTICE_LAUNCH_CHECK();
         const long long pieces = static_cast<long long>(tiles) * tci * tco / 4;
         const dim3 rgrid(grid_for(pieces, 256, 256), static_cast<unsigned>(widx.K));
@@ -712,6 +854,7 @@ int launch_weight_grad(int dtype, const void* feats, int n_in, const void* cot, 
         LATTICE_LAUNCH_CHECK();
         return LATTICE_OK;
     }
+    LATTICE_REQUIRE(kpairs == nullptr, "weight gradient workspace too small.");
     const long long total = static_cast<long long>(widx.K) * widx.c_in * widx.c_out;
     weight_grad_simple<T><<<grid_for(total, 256, 1u << 16), 256, 0, stream>>>(
         static_cast<const T*>(feats), n_in, static_cast<const T*>(cot), n_out, in_rows, out_rows, counts,
@@ -816,15 +959,80 @@ extern "C" int lattice_hip_sparse_conv_weight_grad(int dtype, const void* feats,
     GradWeightIndex widx{weight_layout, kernel_count, c_in, c_out};
     if (dtype == LATTICE_F32) {
         return launch_weight_grad<float>(dtype, feats, n_in, cot, out_capacity, widx, in_rows, out_rows, counts,
-                                         edge_capacity, kernel_row_offsets, kernel_edge_ids, grad, workspace,
+                                         edge_capacity, kernel_row_offsets, kernel_edge_ids, nullptr, grad, workspace,
                                          workspace_bytes, stream);
     }
     if (dtype == LATTICE_F16) {
         return launch_weight_grad<_Float16>(dtype, feats, n_in, cot, out_capacity, widx, in_rows, out_rows, counts,
-                                            edge_capacity, kernel_row_offsets, kernel_edge_ids, grad, workspace,
+                                            edge_capacity, kernel_row_offsets, kernel_edge_ids, nullptr, grad, workspace,
                                             workspace_bytes, stream);
     }
     return launch_weight_grad<__bf16>(dtype, feats, n_in, cot, out_capacity, widx, in_rows, out_rows, counts,
-                                      edge_capacity, kernel_row_offsets, kernel_edge_ids, grad, workspace,
+                                      edge_capacity, kernel_row_offsets, kernel_edge_ids, nullptr, grad, workspace,
                                       workspace_bytes, stream);
+}
+
+extern "C" size_t lattice_hip_kernel_pairs_workspace_bytes(int rows) {
+    return aligned_bytes(std::max<size_t>(group_blocks(rows), 1) * kGroupBins * sizeof(int32_t)) + 256;
+}
+
+extern "C" int lattice_hip_build_kernel_pairs(const int32_t* row_masks, const int32_t* row_offsets,
+                                              const int32_t* in_rows, int rows, int kernel_count, int edge_capacity,
+                                              int32_t* kernel_row_offsets, int32_t* pairs, int32_t* kernel_edge_ids,
+                                              void* workspace, size_t workspace_bytes, void* stream_ptr) {
+    LATTICE_REQUIRE(rows >= 0 && edge_capacity >= 0 && kernel_count > 0 && kernel_count <= kGroupBins,
+                    "kernel pairs need nonnegative capacities and K <= 32.");
+    LATTICE_REQUIRE(kernel_row_offsets != nullptr, "kernel pair pointers must be non-null.");
+    LATTICE_REQUIRE(rows == 0 || edge_capacity == 0 ||
+                        (row_masks && row_offsets && in_rows && (pairs || kernel_edge_ids)),
+                    "kernel pair pointers must be non-null.");
+    LATTICE_REQUIRE(reinterpret_cast<uintptr_t>(pairs) % 8 == 0, "kernel pairs must be 8-byte aligned.");
+    LATTICE_REQUIRE(workspace != nullptr && workspace_bytes >= lattice_hip_kernel_pairs_workspace_bytes(rows),
+                    "kernel pairs workspace too small.");
+    hipStream_t stream = as_stream(stream_ptr);
+    if (rows == 0 || edge_capacity == 0) return fill_i32(kernel_row_offsets, kernel_count + 1, 0, stream);
+    Workspace ws{static_cast<char*>(workspace), workspace_bytes};
+    const int blocks = static_cast<int>(group_blocks(rows));
+    int32_t* places = ws.take<int32_t>(static_cast<size_t>(blocks) * kGroupBins);
+    LATTICE_REQUIRE(places != nullptr, "kernel pairs workspace too small.");
+    group_count<<<blocks, kGroupRows, 0, stream>>>(row_masks, rows, kernel_count, places);
+    LATTICE_LAUNCH_CHECK();
+    group_scan<<<1, 1024, 0, stream>>>(places, blocks, kernel_count, kernel_row_offsets);
+    LATTICE_LAUNCH_CHECK();
+    group_emit<<<blocks, kGroupRows, 0, stream>>>(row_masks, row_offsets, in_rows, rows, kernel_count, edge_capacity,
+                                                  places, reinterpret_cast<int2*>(pairs), kernel_edge_ids);
+    LATTICE_LAUNCH_CHECK();
+    return LATTICE_OK;
+}
+
+extern "C" int lattice_hip_sparse_conv_weight_grad_pairs(int dtype, const void* feats, int n_in, int c_in,
+                                                         const void* cot, int out_capacity, int c_out,
+                                                         int weight_layout, int kernel_count, const int32_t* pairs,
+                                                         int edge_capacity, const int32_t* kernel_row_offsets,
+                                                         void* grad, void* workspace, size_t workspace_bytes,
+                                                         void* stream_ptr) {
+    int rc = check_grad_dtype(dtype);
+    if (rc != LATTICE_OK) return rc;
+    LATTICE_REQUIRE(n_in >= 0 && out_capacity >= 0 && c_in > 0 && c_out > 0 && kernel_count > 0 && edge_capacity >= 0,
+                    "gradient shapes must be positive.");
+    LATTICE_REQUIRE(weight_layout == LATTICE_WEIGHT_KERNEL_MAJOR || weight_layout == LATTICE_WEIGHT_DENSE_5D,
+                    "weights must have shape (K, C_in, C_out) or (C_out, Kx, Ky, Kz, C_in).");
+    LATTICE_REQUIRE(grad && kernel_row_offsets && pairs && workspace, "gradient pointers must be non-null.");
+    LATTICE_REQUIRE(reinterpret_cast<uintptr_t>(pairs) % 8 == 0, "kernel pairs must be 8-byte aligned.");
+    hipStream_t stream = as_stream(stream_ptr);
+    GradWeightIndex widx{weight_layout, kernel_count, c_in, c_out};
+    const int2* p = reinterpret_cast<const int2*>(pairs);
+    if (dtype == LATTICE_F32) {
+        return launch_weight_grad<float>(dtype, feats, n_in, cot, out_capacity, widx, nullptr, nullptr, nullptr,
+                                         edge_capacity, kernel_row_offsets, nullptr, p, grad, workspace,
+                                         workspace_bytes, stream);
+    }
+    if (dtype == LATTICE_F16) {
+        return launch_weight_grad<_Float16>(dtype, feats, n_in, cot, out_capacity, widx, nullptr, nullptr, nullptr,
+                                            edge_capacity, kernel_row_offsets, nullptr, p, grad, workspace,
+                                            workspace_bytes, stream);
+    }
+    return launch_weight_grad<__bf16>(dtype, feats, n_in, cot, out_capacity, widx, nullptr, nullptr, nullptr,
+                                      edge_capacity, kernel_row_offsets, nullptr, p, grad, workspace, workspace_bytes,
+                                      stream);
 }

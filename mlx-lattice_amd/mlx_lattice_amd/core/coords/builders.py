@@ -251,6 +251,14 @@ def _kernel_relation_from_native(
         def grouped_views():
             return _ext().build_relation_grouped_views(
                 in_rows, kernel_ids, counts, in_capacity, n_kernels)
+    # The build's own row masks hold one bit per edge, in edge order.
+    kernel_groups = None
+    if implicit is not None and len(offsets) <= 32:
+        row_masks = implicit.row_masks
+
+        def kernel_groups(edge_ids):
+            return _ext().build_kernel_pairs(row_masks, row_offsets, in_rows,
+                                             len(offsets), edge_ids)
     return KernelRelation(
         in_rows, out_rows, kernel_ids, row_offsets=row_offsets,
         counts=counts, in_row_offsets=in_row_offsets,
@@ -262,7 +270,8 @@ def _kernel_relation_from_native(
         source_active_rows=source_active_rows, target_coords=target_coords,
         target_active_rows=target_active_rows, stride=stride,
         padding=padding, kind=kind, implicit_gemm=implicit,
-        grouped_views=grouped_views, repeated_edges=repeated_edges,
+        grouped_views=grouped_views, kernel_groups=kernel_groups,
+        repeated_edges=repeated_edges,
         direct_expansion=direct_expansion, repeated_coords=repeated_coords,
         block_table=block_table)
 

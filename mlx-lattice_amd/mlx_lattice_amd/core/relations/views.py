@@ -239,6 +239,11 @@ class KernelRelation:
     _input_csr: RelationCSRView | None
     _kernel_csr: RelationCSRView | None
     _grouped_views: Callable[[], tuple] | None
+    # Builds the edges grouped by offset without a sort (dense-map relations
+    # of at most 32 offsets): called with whether to return the edge ids or
+    # the (input row, output row) pairs.
+    _kernel_groups: Callable[[bool], tuple] | None
+    _kernel_pairs: tuple[torch.Tensor, torch.Tensor] | None
     implicit_gemm: RelationImplicitGemmView | None = None
     sorted_implicit_gemm: RelationSortedImplicitGemmView | None = None
     transposed_sorted_implicit_gemm: RelationSortedImplicitGemmView | None = None
@@ -289,6 +294,7 @@ class KernelRelation:
         implicit_gemm: RelationImplicitGemmView | None = None,
         sorted_implicit_gemm: RelationSortedImplicitGemmView | None = None,
         grouped_views: Callable[[], tuple] | None = None,
+        kernel_groups: Callable[[bool], tuple] | None = None,
         repeated_edges: bool | torch.Tensor | None = None,
         direct_expansion: bool = False,
         repeated_coords: torch.Tensor | None = None,
@@ -298,7 +304,8 @@ class KernelRelation:
         not, is called on first access of ``input_csr`` / ``kernel_csr`` and
         returns ``(in_row_offsets, in_edge_ids, kernel_row_offsets,
         kernel_edge_ids)``; the forward convolution never reads those
-        views, so they are only built for consumers that do."""
+        views, so they are only built for consumers that do.
+        ``kernel_groups`` likewise builds the grouping by offset alone."""
         device = in_rows.device
         if counts is None:
             counts = torch.tensor(
@@ -355,6 +362,9 @@ class KernelRelation:
             else RelationCSRView(kernel_row_offsets, kernel_edge_ids))
         object.__setattr__(self, '_grouped_views',
                            grouped_views if lazy_views else None)
+        object.__setattr__(self, '_kernel_groups',
+                           kernel_groups if lazy_views else None)
+        object.__setattr__(self, '_kernel_pairs', None)
         object.__setattr__(self, 'implicit_gemm', implicit_gemm)
         object.__setattr__(self, 'sorted_implicit_gemm', sorted_implicit_gemm)
         object.__setattr__(self, 'transposed_sorted_implicit_gemm', None)
@@ -379,16 +389,30 @@ class KernelRelation:
     @property
     def kernel_csr(self) -> RelationCSRView:
         """Edges grouped by kernel offset (stable in edge order)."""
-        if self._kernel_csr is None:
+        if self._kernel_csr is None and self._kernel_groups is not None:
+            k_offsets, _, k_ids = self._kernel_groups(True)
+            object.__setattr__(self, '_kernel_csr',
+                               RelationCSRView(k_offsets, k_ids))
+        elif self._kernel_csr is None:
             self._materialize_grouped_views()
         return self._kernel_csr
+
+    def kernel_pairs(self) -> tuple[torch.Tensor, torch.Tensor] | None:
+        """(offsets (K + 1,), pairs (E, 2)): the (input row, output row) of
+        every edge, grouped by kernel offset in the order of ``kernel_csr``,
+        built on first use; None for relations that group by a sort."""
+        if self._kernel_pairs is None and self._kernel_groups is not None:
+            k_offsets, pairs, _ = self._kernel_groups(False)
+            object.__setattr__(self, '_kernel_pairs', (k_offsets, pairs))
+        return self._kernel_pairs
 
     def _materialize_grouped_views(self) -> None:
         in_offsets, in_ids, k_offsets, k_ids = self._grouped_views()
         object.__setattr__(self, '_input_csr',
                            RelationCSRView(in_offsets, in_ids))
-        object.__setattr__(self, '_kernel_csr',
-                           RelationCSRView(k_offsets, k_ids))
+        if self._kernel_csr is None:
+            object.__setattr__(self, '_kernel_csr',
+                               RelationCSRView(k_offsets, k_ids))
 
     @property
     def edge_capacity(self) -> int:

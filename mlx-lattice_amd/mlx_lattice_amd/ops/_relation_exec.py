@@ -305,8 +305,13 @@ def sparse_conv_weight_grad_from_relation(feats: torch.Tensor,
                                           relation: KernelRelation,
                                           ) -> torch.Tensor:
     """Weight gradient in ``weight``'s shape (make_sparse_conv_features_
-    weight_grad, primitive.cpp:641-680) over the kernel-grouped CSR."""
+    weight_grad, primitive.cpp:641-680) over the edges grouped by offset
+    (pairs where the relation groups without a sort, else the CSR)."""
     _require_static(relation)
+    pairs = relation.kernel_pairs()
+    if pairs is not None:
+        return ext.sparse_conv_weight_grad_pairs(
+            feats, cot, weight, pairs[1], pairs[0], relation.n_kernels)
     kernel_csr = relation.kernel_csr
     return ext.sparse_conv_weight_grad(
         feats, cot, weight, relation.edges.in_rows, relation.edges.out_rows,

@@ -212,6 +212,12 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("in_edge_ids"), py::arg("kernel_row_offsets"), py::arg("kernel_edge_ids"), py::arg("out_capacity"),
         py::arg("n_kernels"), py::arg("store_sorted") = false, py::kw_only(), py::arg("bias") = py::none(),
         py::arg("tile_order") = py::none(), py::arg("relu") = false, py::arg("weight_fragments") = py::none());
+    m.def("build_kernel_pairs", &ln::build_kernel_pairs, py::arg("row_masks"), py::arg("row_offsets"),
+          py::arg("in_rows"), py::arg("n_kernels"), py::arg("edge_ids"),
+          "Return (kernel_row_offsets, pairs, kernel_edge_ids); edge_ids picks the ids, else the pairs.");
+    m.def("sparse_conv_weight_grad_pairs", &ln::sparse_conv_weight_grad_pairs, py::arg("feats"),
+          py::arg("cotangent"), py::arg("weights"), py::arg("pairs"), py::arg("kernel_row_offsets"),
+          py::arg("n_kernels"));
     m.def("conv_padded_supported", &ln::conv_padded_supported, py::arg("feats"), py::arg("out_channels"),
           py::arg("n_kernels"), py::arg("out_capacity"));
     m.def("conv_padded_fragments", &ln::conv_padded_fragments, py::arg("weights"), py::arg("role"));

@@ -736,4 +736,75 @@ at::Tensor sparse_conv_weight_grad(const at::Tensor& feats_in, const at::Tensor&
     return grad;
 }
 
+std::tuple<at::Tensor, std::optional<at::Tensor>, std::optional<at::Tensor>> build_kernel_pairs(
+    const at::Tensor& row_masks_in, const at::Tensor& row_offsets, const at::Tensor& in_rows, int n_kernels,
+    bool edge_ids) {
+    if (row_masks_in.dim() != 2 || row_masks_in.size(1) != 1 || row_masks_in.scalar_type() != at::kInt) {
+        throw std::invalid_argument("row_masks must have shape (N_out, 1) and int32 dtype.");
+    }
+    require_i32_vector(row_offsets, "row_offsets must be a one-dimensional int32 array.");
+    require_i32_vector(in_rows, "relation rows must be one-dimensional int32 arrays.");
+    if (n_kernels <= 0 || n_kernels > 32) throw std::invalid_argument("kernel pairs need 1 to 32 offsets.");
+    if (row_offsets.size(0) != row_masks_in.size(0) + 1) {
+        throw std::invalid_argument("row_offsets length must match the masks' rows + 1.");
+    }
+    require_device(row_masks_in, "row_masks");
+    require_device(row_offsets, "row_offsets");
+    require_device(in_rows, "in_rows");
+    const at::Tensor masks = row_masks_in.contiguous();
+    const at::Tensor offsets = row_offsets.contiguous();
+    const at::Tensor in = in_rows.contiguous();
+    const int rows = static_cast<int>(masks.size(0));
+    const int edges = static_cast<int>(in.size(0));
+    at::Tensor groups = empty_i32({n_kernels + 1}, in);
+    std::optional<at::Tensor> pairs, ids;
+    if (edge_ids) ids = empty_i32({edges}, in);
+    else pairs = empty_i32({edges, 2}, in);
+    at::Tensor ws = workspace(lattice_hip_kernel_pairs_workspace_bytes(rows), in);
+    check_status(lattice_hip_build_kernel_pairs(ci32(masks), ci32(offsets), ci32(in), rows, n_kernels, edges,
+                                                i32(groups), pairs ? i32(*pairs) : nullptr, ids ? i32(*ids) : nullptr,
+                                                ws.data_ptr(), static_cast<size_t>(ws.numel()), current_stream(in)));
+    return {groups, pairs, ids};
+}
+
+at::Tensor sparse_conv_weight_grad_pairs(const at::Tensor& feats_in, const at::Tensor& cot_in,
+                                         const at::Tensor& weights, const at::Tensor& pairs,
+                                         const at::Tensor& kernel_row_offsets, int n_kernels) {
+    const char* op = "sparse_conv_weight_grad";
+    validate_weights(feats_in, weights, n_kernels, op);
+    const int64_t c_out = out_channels_of(weights);
+    if (cot_in.dim() != 2 || cot_in.size(1) != c_out) {
+        throw std::invalid_argument("cotangent must have shape (N_out, C_out).");
+    }
+    if (cot_in.scalar_type() != feats_in.scalar_type()) {
+        throw std::invalid_argument(std::string(op) + " cotangent must match feats dtype.");
+    }
+    require_i32_vector(kernel_row_offsets, "plan row_offsets must be one-dimensional int32 arrays.");
+    if (kernel_row_offsets.size(0) != n_kernels + 1) {
+        throw std::invalid_argument("kernel_row_offsets length must match n_kernels + 1.");
+    }
+    if (pairs.dim() != 2 || pairs.size(1) != 2 || pairs.scalar_type() != at::kInt || !pairs.is_contiguous()) {
+        throw std::invalid_argument("pairs must be a contiguous (E, 2) int32 array.");
+    }
+    require_device(cot_in, "cotangent");
+    require_device(pairs, "pairs");
+    require_device(kernel_row_offsets, "kernel_row_offsets");
+    const at::Tensor feats = feats_in.contiguous();
+    const at::Tensor cot = cot_in.contiguous();
+    const int dtype = dtype_code(feats, op);
+    const int c_in = static_cast<int>(feats.size(1));
+    const int edges = static_cast<int>(pairs.size(0));
+    at::Tensor grad = at::empty(weights.sizes(), cot.options());
+    if (edges == 0) return grad.zero_();
+    const size_t ws_bytes =
+        lattice_hip_conv_weight_grad_workspace_bytes(dtype, n_kernels, c_in, static_cast<int>(c_out), edges);
+    at::Tensor ws = workspace(ws_bytes, feats);
+    check_status(lattice_hip_sparse_conv_weight_grad_pairs(
+        dtype, feats.data_ptr(), static_cast<int>(feats.size(0)), c_in, cot.data_ptr(), static_cast<int>(cot.size(0)),
+        static_cast<int>(c_out), weights.dim() == 3 ? LATTICE_WEIGHT_KERNEL_MAJOR : LATTICE_WEIGHT_DENSE_5D,
+        n_kernels, ci32(pairs), edges, ci32(kernel_row_offsets), grad.data_ptr(), ws.data_ptr(), ws_bytes,
+        current_stream(feats)));
+    return grad;
+}
+
 }  // namespace lattice_native

@@ -49,6 +49,17 @@ at::Tensor sparse_conv_features_sorted_implicit_gemm(const at::Tensor& feats, co
 // weight's shape does not take that route.
 at::Tensor conv_weight_fragments(const at::Tensor& weights);
 
+// Edges of a dense-map relation grouped by offset without a sort
+// (lattice_hip_build_kernel_pairs): (kernel_row_offsets, pairs (E, 2) or
+// none, kernel_edge_ids (E,) or none), and the weight gradient over the
+// pairs.
+std::tuple<at::Tensor, std::optional<at::Tensor>, std::optional<at::Tensor>> build_kernel_pairs(
+    const at::Tensor& row_masks, const at::Tensor& row_offsets, const at::Tensor& in_rows, int n_kernels,
+    bool edge_ids);
+at::Tensor sparse_conv_weight_grad_pairs(const at::Tensor& feats, const at::Tensor& cotangent,
+                                         const at::Tensor& weights, const at::Tensor& pairs,
+                                         const at::Tensor& kernel_row_offsets, int n_kernels);
+
 // The streamed conv for the types and channel counts the sorted entry does
 // not take (lattice_hip_sparse_conv_features_padded): whether a contiguous
 // `feats` and the shape qualify; the fragments of a float weight (role:
