@@ -672,6 +672,16 @@ int lattice_hip_sparse_pool_features_grad(
     int edge_capacity, const int32_t* row_offsets, const int32_t* counts,
     const int32_t* in_row_offsets, const int32_t* in_edge_ids,
     int out_capacity, float* grad, void* stream);
+/* The same gradient for a relation in which each input row feeds at most
+ * one output row (the stride is at least the kernel's extent on every axis;
+ * the reference's input_exclusive), from the output rows' edges: no
+ * input-grouped CSR.  in_active_rows: the device count of active input rows
+ * the relation was built with. */
+int lattice_hip_sparse_pool_features_grad_exclusive(
+    int mode, const float* cot, const float* feats, const float* pooled,
+    int n_in, const int32_t* in_active_rows, int channels,
+    const int32_t* in_rows, int edge_capacity, const int32_t* row_offsets,
+    const int32_t* counts, int out_capacity, float* grad, void* stream);
 
 /* Per-batch global pooling (global_sum_pool / global_avg_pool /
  * global_max_pool, ops/pool.py:139-236): out[b, c] reduces rows

@@ -455,14 +455,16 @@ def _pool_features(feats, relation, input_exclusive, mode):
 
 class _SparsePoolFeatures(torch.autograd.Function):
     """Pooling with the reference's vjp (pooling/primitive.cpp:109-160):
-    the gradient walks the input-grouped CSR; max routes the cotangent to
-    the inputs equal to the pooled value, split over ties."""
+    max routes the cotangent to the inputs equal to the pooled value, split
+    over ties.  A relation whose inputs feed at most one output each writes
+    it from the output rows; others walk the input-grouped CSR."""
 
     @staticmethod
     def forward(ctx, feats, relation, input_exclusive, mode):
         pooled = _pool_features(feats, relation, input_exclusive, mode)
         ctx.relation = relation
         ctx.mode = mode
+        ctx.input_exclusive = input_exclusive
         ctx.save_for_backward(feats, pooled)
         return pooled
 
@@ -470,6 +472,13 @@ class _SparsePoolFeatures(torch.autograd.Function):
     def backward(ctx, grad_out):
         feats, pooled = ctx.saved_tensors
         relation = ctx.relation
+        active = relation.contract.source_active_rows
+        if ctx.input_exclusive and active is not None:
+            grad = ext.sparse_pool_features_grad_exclusive(
+                grad_out.contiguous(), feats, pooled, relation.edges.in_rows,
+                relation.output_csr.row_offsets, relation.counts, active,
+                ctx.mode)
+            return grad, None, None, None
         input_csr = relation.input_csr
         grad = ext.sparse_pool_features_grad(
             grad_out.contiguous(), feats, pooled, relation.edges.in_rows,

@@ -292,6 +292,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
           py::arg("weights"));
     m.def("interpolate_point_features_grad", &ln::interpolate_point_features_grad, py::arg("point_grad"),
           py::arg("weights"), py::arg("voxel_offsets"), py::arg("entry_ids"), py::arg("voxel_rows"));
+    m.def("sparse_pool_features_grad_exclusive", &ln::sparse_pool_features_grad_exclusive, py::arg("cotangent"),
+          py::arg("feats"), py::arg("pooled"), py::arg("in_rows"), py::arg("row_offsets"), py::arg("counts"),
+          py::arg("in_active_rows"), py::arg("reduce"));
     m.def("global_pool", &ln::global_pool, py::arg("feats"), py::arg("batch_counts"), py::arg("mode"),
           "Per-batch global pooling: (B, C).");
 }

@@ -23,6 +23,13 @@ at::Tensor sparse_pool_features_grad(const at::Tensor& cotangent, const at::Tens
                                      const at::Tensor& counts, const at::Tensor& in_row_offsets,
                                      const at::Tensor& in_edge_ids, const std::string& reduce);
 
+// The gradient of a relation in which each input row feeds at most one
+// output row (lattice_hip_sparse_pool_features_grad_exclusive).
+at::Tensor sparse_pool_features_grad_exclusive(const at::Tensor& cotangent, const at::Tensor& feats,
+                                               const at::Tensor& pooled, const at::Tensor& in_rows,
+                                               const at::Tensor& row_offsets, const at::Tensor& counts,
+                                               const at::Tensor& in_active_rows, const std::string& reduce);
+
 // Per-batch global pooling of rows grouped by batch_counts: (B, C) float32.
 at::Tensor global_pool(const at::Tensor& feats, const std::vector<int64_t>& batch_counts, const std::string& mode);
 

@@ -103,6 +103,42 @@ at::Tensor sparse_pool_features_grad(const at::Tensor& cot_in, const at::Tensor&
     return grad;
 }
 
+at::Tensor sparse_pool_features_grad_exclusive(const at::Tensor& cot_in, const at::Tensor& feats_in,
+                                               const at::Tensor& pooled_in, const at::Tensor& in_rows,
+                                               const at::Tensor& row_offsets, const at::Tensor& counts,
+                                               const at::Tensor& in_active_rows, const std::string& reduce) {
+    const int mode = reduce_code(reduce, "reduce must be 'sum', 'max', or 'avg'.");
+    if (feats_in.dim() != 2 || cot_in.dim() != 2 || pooled_in.dim() != 2) {
+        throw std::invalid_argument("feats, pooled and cotangent must have shape (N, C).");
+    }
+    if (feats_in.scalar_type() != at::kFloat || cot_in.scalar_type() != at::kFloat ||
+        pooled_in.scalar_type() != at::kFloat) {
+        throw std::invalid_argument("sparse_pool_features currently supports float32 feats.");
+    }
+    if (cot_in.sizes() != pooled_in.sizes() || cot_in.size(1) != feats_in.size(1)) {
+        throw std::invalid_argument("cotangent must match the pooled output shape.");
+    }
+    validate_relation(in_rows, in_rows, in_rows, row_offsets, counts);
+    if (row_offsets.size(0) != cot_in.size(0) + 1) {
+        throw std::invalid_argument("row_offsets length must match out_capacity + 1.");
+    }
+    if (in_active_rows.dim() != 1 || in_active_rows.size(0) != 1 || in_active_rows.scalar_type() != at::kInt) {
+        throw std::invalid_argument("active_rows must have shape (1,) and int32 dtype.");
+    }
+    require_device(feats_in, "feats");
+    require_device(in_active_rows, "active_rows");
+    const at::Tensor cot = cot_in.contiguous();
+    const at::Tensor feats = feats_in.contiguous();
+    const at::Tensor pooled = pooled_in.contiguous();
+    at::Tensor grad = at::empty(feats.sizes(), feats.options());
+    check_status(lattice_hip_sparse_pool_features_grad_exclusive(
+        mode, cot.data_ptr<float>(), feats.data_ptr<float>(), pooled.data_ptr<float>(),
+        static_cast<int>(feats.size(0)), ci32(in_active_rows), static_cast<int>(feats.size(1)), ci32(in_rows),
+        static_cast<int>(in_rows.size(0)), ci32(row_offsets), ci32(counts), static_cast<int>(cot.size(0)),
+        grad.data_ptr<float>(), current_stream(feats)));
+    return grad;
+}
+
 at::Tensor global_pool(const at::Tensor& feats_in, const std::vector<int64_t>& batch_counts,
                        const std::string& mode) {
     const int code = reduce_code(mode, "mode must be 'sum', 'max', or 'avg'.");
