@@ -343,6 +343,17 @@ int lattice_hip_build_sorted_implicit_gemm_view(
     int32_t* sorted_kv_out_in_map, int32_t* tile_masks, void* workspace,
     size_t workspace_bytes, void* stream);
 
+/* The same view with the rows left in their order (no counterpart in the
+ * reference): one launch instead of a sort, reorder_rows the identity.  The
+ * conv entries over a sorted view take it and give the same result; their
+ * tiles then visit more offsets, which a launch of few tiles does not
+ * notice. */
+int lattice_hip_build_tiled_view(const int32_t* out_in_map,
+                                 const int32_t* row_masks, int rows,
+                                 int kernel_count, int32_t* reorder_rows,
+                                 int32_t* kv_out_in_map, int32_t* tile_masks,
+                                 void* stream);
+
 /* Float sparse conv over the output CSR (cpu/algorithms.cpp:180-302):
  * out[o] = sum_{e in CSR(o)} feats[in_rows[e]] @ W[kernel_ids[e]] with an
  * fp32 accumulator; rows >= counts[1] are zero.  feats [n_in, c_in];

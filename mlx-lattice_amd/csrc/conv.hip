@@ -1189,6 +1189,7 @@ __device__ inline void static_for_range(F& f, int lo, int hi) {
 }
 
 constexpr int kOrderTileRows = 128;  // rows of the tiles a tile order ranks
+constexpr int kXcds = 8;
 
 constexpr int gcd_int(int a, int b) { return b == 0 ? a : gcd_int(b, a % b); }
 
@@ -1218,7 +1219,7 @@ struct StreamShape {
     static constexpr int THREADS = WAVES * 64;
     static constexpr int WR = WR_;
     static constexpr int WC = WAVES / WR_;
-    static constexpr int ROWS = ROWS_;        // 128 (the tile order's tiles) or 64 (their halves)
+    static constexpr int ROWS = ROWS_;        // 128 (the tile order's tiles), 64 or 32
     static constexpr int WROWS = ROWS / WR;   // rows per wave
     static constexpr int WCOLS = C_OUT / WC;  // columns per wave
     static constexpr int RB = WROWS / 16;     // 16-row MFMA blocks per wave
@@ -1239,7 +1240,7 @@ struct StreamShape {
     static constexpr int LB = 2;               // B loads lead by LB stages
     static constexpr int LI = LA_ + 1;         // row-index loads lead by LI stages
     static constexpr int READ_AHEAD = 2;       // 16-row fragment reads in flight
-    static_assert(WCOLS == 32 && WROWS % 16 == 0 && (GATHER == 4 || GATHER == 2), "stream tile shape");
+    static_assert(WCOLS == 32 && WROWS % 16 == 0 && (GATHER == 4 || GATHER == 2 || GATHER == 1), "stream tile shape");
 };
 
 // Fragment (k, ks, cg, cb) of a weight: the 16 x 32 block of output
@@ -1504,11 +1505,11 @@ __device__ inline void stream_store_padded(const float4_t (&acc)[RB][CB], T* sta
 // stages of their own (NCH = 1; each loads its row indices), so one instance
 // serves every C_in.  float32 runs the same pipeline on 16x16x4 MFMAs, where
 // it is bound by the matrix cores (a stage's MFMAs take eight times as long
-// per byte gathered), so its tiles are 64 rows: twice the blocks to fill the
-// chip, and half the longest block.  Measured against the CSR kernels, whose
-// lanes load both factors of every product: 96 -> 96 bf16 over 150,001 rows
-// (4.6 edges each) 19,300 -> 45 us; 64 -> 64 float32 over 60,001 rows 3,000
-// -> 55 us, its input gradient 629 -> 55 us.
+// per byte gathered), so its tiles are small: more blocks to fill the
+// chip, and half the longest block (launch_padded).  Measured against the
+// CSR kernels, whose lanes load both factors of every product: 96 -> 96 bf16
+// over 150,001 rows (4.6 edges each) 19,300 -> 43 us; 64 -> 64 float32 over
+// 60,001 rows 3,000 -> 46 us, its input gradient 629 -> 46 us.
 template <typename T, typename S, int NCH, int QB, bool PAD = false>
 __global__ void __launch_bounds__(S::THREADS, S::OCC)
 conv_igemm_stream(const T* __restrict__ feats, int n_in, int c_in, const T* __restrict__ wfrag, int kernel_count,
@@ -1536,10 +1537,24 @@ conv_igemm_stream(const T* __restrict__ feats, int n_in, int c_in, const T* __re
     // Longest-first tile order; with C_out = 256 consecutive blocks take the
     // two column halves of one tile (the second finds its rows in L2).
     // (PAD: any number of column tiles).  The order ranks 128-row tiles;
-    // 64-row tiles take their two halves in turn.
-    const int slot = PAD ? static_cast<int>(blockIdx.x) / halves
-                         : halves > 1 ? static_cast<int>(blockIdx.x) / 2 : static_cast<int>(blockIdx.x);
-    const int half = PAD ? static_cast<int>(blockIdx.x) % halves : halves > 1 ? static_cast<int>(blockIdx.x & 1u) : 0;
+    // smaller tiles take their parts in turn.
+    int slot = static_cast<int>(blockIdx.x);
+    int half = 0;
+    if (halves > 1) {
+        // Launch indices go round the XCDs: the column tiles of a row tile
+        // are eight apart, on one XCD, whose L2 the first fills with the
+        // gathered rows for the others.
+        const int tiles = static_cast<int>(gridDim.x) / halves;
+        const int full = tiles & ~(kXcds - 1);
+        const int b = static_cast<int>(blockIdx.x);
+        if (b < full * halves) {
+            slot = b / (kXcds * halves) * kXcds + b % kXcds;
+            half = b / kXcds % halves;
+        } else {
+            slot = full + (b - full * halves) / halves;
+            half = (b - full * halves) % halves;
+        }
+    }
     const int ncg = PAD ? (c_out_total + 31) / 32 : c_out_total / S::WCOLS;  // 32-column groups of the weight
     const int cg_own = half * (S::C_OUT / S::WCOLS) + wc;
     const bool idle = PAD && cg_own >= ncg;
@@ -2298,29 +2313,6 @@ void launch_stream_shape(const T* feats, int n_in, int c_in, const T* frag, int 
     }
 }
 
-template <typename T, int QB = 0>
-int launch_stream(const T* feats, int n_in, int c_in, const T* frag, int K, int c_out, const int32_t* kv_map,
-                  const int32_t* tile_masks, const int32_t* reorder_rows, int rows, int32_t* schedule, bool ready,
-                  T* out, Epilogue<T> epi, hipStream_t stream) {
-    if (rows <= 0) return LATTICE_OK;
-    const int tiles = (rows + kOrderTileRows - 1) / kOrderTileRows;
-    if (tiles > kMaxScheduledTiles) schedule = nullptr;
-    if (schedule != nullptr && !ready) {
-        schedule_tiles<kOrderTileRows / 16><<<1, kScheduleThreads, 0, stream>>>(tile_masks, rows, tiles, schedule);
-        LATTICE_LAUNCH_CHECK();
-    }
-    if (c_out == 64) {
-        launch_stream_shape<T, StreamShape<T, 64, 2>, QB>(feats, n_in, c_in, frag, K, c_out, kv_map, tile_masks,
-                                                   reorder_rows, rows, schedule, out, epi, 1, stream);
-    } else {
-        launch_stream_shape<T, StreamShape<T, 128, 1>, QB>(feats, n_in, c_in, frag, K, c_out, kv_map, tile_masks,
-                                                    reorder_rows, rows, schedule, out, epi, c_out == 256 ? 2 : 1,
-                                                    stream);
-    }
-    LATTICE_LAUNCH_CHECK();
-    return LATTICE_OK;
-}
-
 // Shapes the padded instances of the streamed kernel take: every feature
 // type (packed weights: fp16/bf16), input rows of whole 16-byte pieces, any
 // C_out, K <= 32.  The kernel reads its map, weight and rows at 32-bit byte
@@ -2346,11 +2338,23 @@ template <typename T, typename S, int QB>
 void launch_padded_shape(const T* feats, int n_in, int c_in, const T* frag, int K, int c_out, const int32_t* kv_map,
                          const int32_t* tile_masks, const int32_t* reorder_rows, int rows, const int32_t* order,
                          T* out, Epilogue<T> epi, hipStream_t stream) {
-    // an order's 128-row tiles are two 64-row ones
+    // an order's 128-row tiles are two 64-row or four 32-row ones
     const int tiles = (rows + kOrderTileRows - 1) / kOrderTileRows * (kOrderTileRows / S::ROWS);
     const int columns = (c_out + S::C_OUT - 1) / S::C_OUT;
     conv_igemm_stream<T, S, 1, QB, true><<<static_cast<unsigned>(tiles) * columns, S::THREADS, 0, stream>>>(
         feats, n_in, c_in, frag, K, c_out, kv_map, tile_masks, reorder_rows, rows, order, out, epi, columns);
+}
+
+// Few rows: a launch of at most about two 128-row tiles per CU lasts as long
+// as its longest tile (27 offsets, however sorted), and half a tile's stages
+// are shorter.  64-row tiles measured 128 -> 128 fp16 at 8,000 / 32,000
+// rows (10.5 edges each) 29 -> 20 / 33 -> 26 us and 64 -> 64 15 -> 10 / 15
+// -> 14 us, but 73 -> 79 us at 128,000; with two column tiles (256 -> 256)
+// 53 -> 34 us at 8,000 and 71 -> 82 us at 32,000 rows.
+constexpr long long kFewRows = 65536;
+bool few_rows(int rows, int c_out) {
+    const long long columns = (static_cast<long long>(c_out) + 127) / 128;
+    return rows * columns * columns <= kFewRows;
 }
 
 template <typename T, int QB = 0>
@@ -2364,18 +2368,68 @@ int launch_padded(const T* feats, int n_in, int c_in, const T* frag, int K, int 
         schedule_tiles<kOrderTileRows / 16><<<1, kScheduleThreads, 0, stream>>>(tile_masks, rows, tiles, schedule);
         LATTICE_LAUNCH_CHECK();
     }
-    constexpr int ROWS = sizeof(T) == 4 ? 64 : 128;
-#define LATTICE_PADDED(C, WR)                                                                                      \
+#define LATTICE_PADDED(C, WR, ROWS)                                                                                \
     launch_padded_shape<T, StreamShape<T, C, WR, ROWS>, QB>(feats, n_in, c_in, frag, K, c_out, kv_map, tile_masks, \
                                                             reorder_rows, rows, schedule, out, epi, stream)
-    if (c_out <= 32) {
-        LATTICE_PADDED(32, 4);
+    // Tile rows.  float32 is bound by its MFMAs: 32-row tiles (no more
+    // gathers, a shorter longest tile) measured fastest at every size for
+    // more than 32 columns (64 -> 64 over 60,001 / 128,000 rows 53 -> 46 /
+    // 149 -> 147 us against 64-row tiles, 128 -> 128 154 -> 126 / 229 -> 197
+    // us), and 64 rows below (32 -> 32 at 128,000 rows 49 against 62 us).
+    // 16 bits: 64 rows for few rows, and for one column tile of more than
+    // 64 (96 -> 96 over 150,001 / 128,000 rows 48 -> 43 / 75 -> 73 us).
+    if constexpr (sizeof(T) == 4) {
+        if (c_out <= 32) {
+            LATTICE_PADDED(32, 4, 64);
+        } else if (c_out <= 64) {
+            LATTICE_PADDED(64, 2, 32);
+        } else {
+            LATTICE_PADDED(128, 1, 32);
+        }
+    } else if (few_rows(rows, c_out) || (c_out > 64 && c_out <= 128)) {
+        if (c_out <= 32) {
+            LATTICE_PADDED(32, 4, 64);
+        } else if (c_out <= 64) {
+            LATTICE_PADDED(64, 2, 64);
+        } else {
+            LATTICE_PADDED(128, 1, 64);
+        }
+    } else if (c_out <= 32) {
+        LATTICE_PADDED(32, 4, 128);
     } else if (c_out <= 64) {
-        LATTICE_PADDED(64, 2);
+        LATTICE_PADDED(64, 2, 128);
     } else {
-        LATTICE_PADDED(128, 1);
+        LATTICE_PADDED(128, 1, 128);
     }
 #undef LATTICE_PADDED
+    LATTICE_LAUNCH_CHECK();
+    return LATTICE_OK;
+}
+
+template <typename T, int QB = 0>
+int launch_stream(const T* feats, int n_in, int c_in, const T* frag, int K, int c_out, const int32_t* kv_map,
+                  const int32_t* tile_masks, const int32_t* reorder_rows, int rows, int32_t* schedule, bool ready,
+                  T* out, Epilogue<T> epi, hipStream_t stream) {
+    if (rows <= 0) return LATTICE_OK;
+    // These shapes' fragments are the padded ones, with nothing to pad.
+    if (few_rows(rows, c_out)) {
+        return launch_padded<T, QB>(feats, n_in, c_in, frag, K, c_out, kv_map, tile_masks, reorder_rows, rows, schedule,
+                                    ready, out, epi, stream);
+    }
+    const int tiles = (rows + kOrderTileRows - 1) / kOrderTileRows;
+    if (tiles > kMaxScheduledTiles) schedule = nullptr;
+    if (schedule != nullptr && !ready) {
+        schedule_tiles<kOrderTileRows / 16><<<1, kScheduleThreads, 0, stream>>>(tile_masks, rows, tiles, schedule);
+        LATTICE_LAUNCH_CHECK();
+    }
+    if (c_out == 64) {
+        launch_stream_shape<T, StreamShape<T, 64, 2>, QB>(feats, n_in, c_in, frag, K, c_out, kv_map, tile_masks,
+                                                   reorder_rows, rows, schedule, out, epi, 1, stream);
+    } else {
+        launch_stream_shape<T, StreamShape<T, 128, 1>, QB>(feats, n_in, c_in, frag, K, c_out, kv_map, tile_masks,
+                                                    reorder_rows, rows, schedule, out, epi, c_out == 256 ? 2 : 1,
+                                                    stream);
+    }
     LATTICE_LAUNCH_CHECK();
     return LATTICE_OK;
 }

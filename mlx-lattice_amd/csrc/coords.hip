@@ -1327,7 +1327,7 @@ constexpr int kGatherRows = 64;
 __global__ void __launch_bounds__(kThreads)
 gather_sorted(const int32_t* __restrict__ out_in_map, const int32_t* __restrict__ row_masks, int rows, int K,
               const int32_t* __restrict__ order, int32_t* __restrict__ sorted_map, int32_t* __restrict__ kv_map,
-              int32_t* __restrict__ tile_masks) {
+              int32_t* __restrict__ tile_masks, int32_t* __restrict__ identity) {
     __shared__ int32_t tile[kGatherRows * 33];
     __shared__ int32_t src_rows[kGatherRows];
     const int row0 = blockIdx.x * kGatherRows;
@@ -1335,8 +1335,13 @@ gather_sorted(const int32_t* __restrict__ out_in_map, const int32_t* __restrict_
     if (threadIdx.x < kGatherRows) {
         // the quarter masks of this 64-row tile: OR of 16 sorted row masks
         // (rows past the end count as 0)
-        const int src = threadIdx.x < n ? order[row0 + threadIdx.x] : -1;
-        if (threadIdx.x < n) src_rows[threadIdx.x] = src;
+        // (order null: the rows as they are, which `identity` then records)
+        const int at = row0 + static_cast<int>(threadIdx.x);
+        const int src = threadIdx.x >= n ? -1 : order != nullptr ? order[at] : at;
+        if (threadIdx.x < n) {
+            src_rows[threadIdx.x] = src;
+            if (identity != nullptr) identity[at] = at;
+        }
         int m = src >= 0 ? row_masks[src] : 0;
 #pragma unroll
         for (int off = 1; off < 16; off <<= 1) m |= __shfl_xor(m, off, 16);
@@ -1388,7 +1393,21 @@ extern "C" int lattice_hip_build_sorted_implicit_gemm_view(const int32_t* out_in
     int rc = radix_sort_indices(keys, rows, kernel_count, nullptr, reorder_rows, ws, stream);
     if (rc != LATTICE_OK) return rc;
     gather_sorted<<<tiles, kThreads, 0, stream>>>(out_in_map, row_masks, rows, kernel_count, reorder_rows,
-                                                  sorted_out_in_map, sorted_kv_out_in_map, tile_masks);
+                                                  sorted_out_in_map, sorted_kv_out_in_map, tile_masks, nullptr);
+    LATTICE_LAUNCH_CHECK();
+    return LATTICE_OK;
+}
+
+extern "C" int lattice_hip_build_tiled_view(const int32_t* out_in_map, const int32_t* row_masks, int rows,
+                                            int kernel_count, int32_t* reorder_rows, int32_t* kv_out_in_map,
+                                            int32_t* tile_masks, void* stream_ptr) {
+    LATTICE_REQUIRE(kernel_count > 0 && kernel_count <= 32, "tiled views support K <= 32.");
+    LATTICE_REQUIRE(rows >= 0, "out_in_map must have shape (N_out, K).");
+    if (rows == 0) return LATTICE_OK;
+    LATTICE_REQUIRE(out_in_map && row_masks && reorder_rows && kv_out_in_map && tile_masks,
+                    "tiled view pointers must be non-null.");
+    gather_sorted<<<(rows + kGatherRows - 1) / kGatherRows, kThreads, 0, as_stream(stream_ptr)>>>(
+        out_in_map, row_masks, rows, kernel_count, nullptr, nullptr, kv_out_in_map, tile_masks, reorder_rows);
     LATTICE_LAUNCH_CHECK();
     return LATTICE_OK;
 }

@@ -21,6 +21,13 @@ RelationKind = Literal['forward', 'target', 'submanifold', 'transposed',
                        'generative']
 
 _INDEX_DTYPES = (torch.int32, torch.int64)
+# Rows whose 128-row tiles all start at once, one per CU.
+_ONE_ROUND_ROWS = 256 * 128
+# Rows, weight bytes per offset and their product up to which convs take the
+# rows in their own order (conv_view).
+_TILED_ROWS = 32768
+_TILED_WEIGHT_BYTES = 16384
+_TILED_WORK = 16384 * 16384
 
 
 @dataclass(frozen=True, slots=True)
@@ -114,10 +121,13 @@ class RelationSortedImplicitGemmView:
             raise ValueError(
                 'reorder_rows must have one row per sorted_out_in_map row.')
 
-    def tile_order(self) -> torch.Tensor:
+    def tile_order(self) -> torch.Tensor | None:
         """Longest-first order of the view's 128-row tiles for the
         matrix-core conv, computed on first use and kept with the view so
-        repeated convs over it skip their per-call schedule."""
+        repeated convs over it skip their per-call schedule; None when the
+        tiles all start at once."""
+        if int(self.reorder_rows.shape[0]) <= _ONE_ROUND_ROWS:
+            return None
         if self._tile_order is None:
             from mlx_lattice_amd._native import ext
 
@@ -247,6 +257,9 @@ class KernelRelation:
     implicit_gemm: RelationImplicitGemmView | None = None
     sorted_implicit_gemm: RelationSortedImplicitGemmView | None = None
     transposed_sorted_implicit_gemm: RelationSortedImplicitGemmView | None = None
+    # The unsorted views of small relations (conv_view).
+    _tiled: RelationSortedImplicitGemmView | None = None
+    _transposed_tiled: RelationSortedImplicitGemmView | None = None
     # Transposed relations only: whether two edges share (out_row, kernel_id)
     # (a repeated input coordinate).  The builder hands over its device
     # status word, copied to pinned memory at build time (a _StatusWord) and
@@ -368,6 +381,8 @@ class KernelRelation:
         object.__setattr__(self, 'implicit_gemm', implicit_gemm)
         object.__setattr__(self, 'sorted_implicit_gemm', sorted_implicit_gemm)
         object.__setattr__(self, 'transposed_sorted_implicit_gemm', None)
+        object.__setattr__(self, '_tiled', None)
+        object.__setattr__(self, '_transposed_tiled', None)
         object.__setattr__(
             self, 'repeated_edges',
             _StatusWord(repeated_edges)
@@ -573,6 +588,46 @@ class KernelRelation:
         object.__setattr__(self, 'sorted_implicit_gemm', sorted_view)
         return sorted_view
 
+    def conv_view(self, weight_bytes: int) -> RelationSortedImplicitGemmView:
+        """The view a matrix-core conv whose weight has ``weight_bytes`` per
+        offset reads: the mask-sorted one, or, for few rows and channels, the
+        rows in their own order (one launch instead of a sort; the result is
+        the same).  Such a launch lasts as long as its longest tile, which
+        sorting hardly shortens: the sorted view takes 44 us to build and the
+        other 9, and a conv over it runs 1 us longer for 64 -> 64 fp16 at
+        16,000 rows and 3 at 32,000, 6 for 16 -> 32 fp32 at 32,000 and 7 for
+        64 -> 64 fp32 at 16,000, but 30 for 128 -> 128 fp32."""
+        if (self.sorted_implicit_gemm is not None
+                or self.contract.kind not in ('forward', 'submanifold',
+                                              'target')
+                or not _tiled_pays(self.n_out_capacity, weight_bytes)):
+            return self.require_sorted_implicit_gemm()
+        if self._tiled is None:
+            view = self.require_implicit_gemm()
+            object.__setattr__(self, '_tiled', _tiled_view(
+                view.out_in_map, view.row_masks))
+        return self._tiled
+
+    def transposed_conv_view(self, weight_bytes: int,
+                             ) -> RelationSortedImplicitGemmView:
+        """``conv_view`` of the transposed relation."""
+        if (self.transposed_sorted_implicit_gemm is not None
+                or self.contract.kind not in ('forward', 'submanifold')
+                or self.n_in_capacity is None
+                or not _tiled_pays(self.n_in_capacity, weight_bytes)
+                or self.n_kernels is None or self.n_kernels > 32):
+            return self.require_transposed_sorted_implicit_gemm()
+        if self._transposed_tiled is None:
+            from mlx_lattice_amd._native import ext
+
+            in_out_map, row_masks, _ = ext.build_transposed_implicit_gemm_map(
+                self.edges.in_rows, self.edges.out_rows,
+                self.edges.kernel_ids, self.counts, int(self.n_in_capacity),
+                int(self.n_kernels))
+            object.__setattr__(self, '_transposed_tiled',
+                               _tiled_view(in_out_map, row_masks))
+        return self._transposed_tiled
+
     def require_transposed_sorted_implicit_gemm(
             self) -> RelationSortedImplicitGemmView:
         """Mask-sorted view of the transposed relation (input row -> output
@@ -611,6 +666,21 @@ class KernelRelation:
 
 
 # ---------------------------------------------------------------- helpers --
+
+
+def _tiled_pays(rows: int, weight_bytes: int) -> bool:
+    return (rows <= _TILED_ROWS and weight_bytes <= _TILED_WEIGHT_BYTES
+            and rows * weight_bytes <= _TILED_WORK)
+
+
+def _tiled_view(out_in_map: torch.Tensor, row_masks: torch.Tensor,
+                ) -> RelationSortedImplicitGemmView:
+    from mlx_lattice_amd._native import ext
+
+    order, rows, kv_map, tiles = ext.build_tiled_view(out_in_map, row_masks)
+    return RelationSortedImplicitGemmView(
+        sorted_out_in_map=rows, sorted_kv_out_in_map=kv_map,
+        reorder_rows=order, tile_masks=tiles)
 
 
 def _validate_row_array(value: torch.Tensor, *, name: str) -> None:

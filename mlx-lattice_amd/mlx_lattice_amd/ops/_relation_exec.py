@@ -86,20 +86,22 @@ def _padded_eligible(feats: torch.Tensor, c_out: int,
 
 def _padded_forward(feats: torch.Tensor, c_in: int, c_out: int,
                     relation: KernelRelation) -> bool:
-    """The forward conv's use of the padded instances.  Rows of at most 16
-    channels with 16 or 32 outputs have kernels of their own (a lane per
-    row, the dense map), which a relation used once runs faster than it
-    sorts its view.  Expanded relations keep the CSR route in fp32: their
-    rows hold one edge each or few, so the view costs more than it saves."""
+    """The forward conv's use of the padded instances.  Expanded relations
+    keep the CSR route in fp32: their rows hold one edge each or few, so the
+    view costs more than it saves."""
     if not relation.dense_map_exact:
         return False
     if feats.dtype == torch.float32 and relation.contract.kind in (
             'transposed', 'generative'):
         return False
-    if (c_in <= 16 and c_out in (16, 32)
-            and relation.sorted_implicit_gemm is None):
-        return False
     return _padded_eligible(feats, c_out, relation, relation.n_out_capacity)
+
+
+def _offset_bytes(weight: torch.Tensor) -> int:
+    """Bytes of the weight of one offset."""
+    c_in = weight.shape[1] if weight.ndim == 3 else weight.shape[4]
+    c_out = weight.shape[2] if weight.ndim == 3 else weight.shape[0]
+    return int(c_in) * int(c_out) * weight.element_size()
 
 
 def _padded_fragments(weight: torch.Tensor, role: int) -> torch.Tensor:
@@ -266,7 +268,7 @@ def sparse_conv_input_grad_from_relation(cot: torch.Tensor,
     _require_static(relation)
     if _input_grad_matrix_core_eligible(cot, weight, relation):
         if _mirror_symmetric(relation):
-            view = relation.require_sorted_implicit_gemm()
+            view = relation.conv_view(_offset_bytes(weight))
             mirrored = _mirrored_weight(weight)
             return ext.sparse_conv_features_sorted_implicit_gemm(
                 cot, mirrored, view.sorted_out_in_map,
@@ -274,7 +276,7 @@ def sparse_conv_input_grad_from_relation(cot: torch.Tensor,
                 None, None, None, None, None, None, None, None, None,
                 in_capacity, relation.n_kernels, tile_order=view.tile_order(),
                 weight_fragments=_weight_fragments(mirrored))
-        view = relation.require_transposed_sorted_implicit_gemm()
+        view = relation.transposed_conv_view(_offset_bytes(weight))
         transposed = _transposed_weight(weight)
         return ext.sparse_conv_features_sorted_implicit_gemm(
             cot, transposed, view.sorted_out_in_map,
@@ -286,8 +288,9 @@ def sparse_conv_input_grad_from_relation(cot: torch.Tensor,
     if (relation.contract.kind != 'target' and relation.transposed_map_exact
             and _padded_eligible(cot, c_in, relation, in_capacity)):
         mirrored = _mirror_symmetric(relation)
-        view = (relation.require_sorted_implicit_gemm() if mirrored
-                else relation.require_transposed_sorted_implicit_gemm())
+        size = _offset_bytes(weight)
+        view = (relation.conv_view(size) if mirrored
+                else relation.transposed_conv_view(size))
         fragments = _padded_fragments(weight,
                                       _MIRRORED if mirrored else _TRANSPOSED)
         return _padded_conv(cot, fragments, 0, c_in, view, in_capacity,
@@ -345,7 +348,7 @@ def _conv_features(feats: torch.Tensor, weight: torch.Tensor,
             and feats.dtype == weight.dtype
             and _padded_forward(feats, c_in, c_out, relation)):
         return _padded_conv(feats, _padded_fragments(weight, _FORWARD), 0,
-                            c_out, relation.require_sorted_implicit_gemm(),
+                            c_out, relation.conv_view(_offset_bytes(weight)),
                             relation.n_out_capacity, relation, bias, relu)
     return ext.sparse_conv_features_csr(
         feats, weight, relation.edges.in_rows, relation.edges.kernel_ids,
@@ -370,7 +373,9 @@ def sparse_conv_features_sorted_from_relation(feats: torch.Tensor,
         raise ValueError(
             'sorted implicit GEMM is not supported for this relation, '
             'feature tensor, or weight tensor.')
-    view = relation.require_sorted_implicit_gemm()
+    # rows stored in sorted order need the sorted view
+    view = (relation.require_sorted_implicit_gemm() if store_sorted
+            else relation.conv_view(_offset_bytes(weight)))
     w5 = _matrix_core_weight(weight)
     return ext.sparse_conv_features_sorted_implicit_gemm(
         feats, w5, view.sorted_out_in_map,
@@ -396,16 +401,18 @@ def sparse_quantized_conv_features_from_relation(
         raise ValueError('quantized weight kernel rows must match the relation.')
     device = feats.device
     kv = reorder = tiles = _empty_i32(device)
-    order = None
+    order = fragments = None
     dense = None
     if _matrix_core_eligible(feats.dtype, weight.in_channels,
                              weight.out_channels, relation,
                              int(feats.shape[0])):
-        view = relation.require_sorted_implicit_gemm()
+        view = relation.conv_view(
+            weight.in_channels * weight.out_channels * 2)
         kv = view.sorted_kv_out_in_map
         reorder = view.reorder_rows
         tiles = view.tile_masks
         order = view.tile_order()
+        fragments = _quantized_fragments(weight)
     else:
         dense = _small_dense_map(feats.dtype, weight.in_channels,
                                  weight.out_channels, relation)
@@ -417,7 +424,8 @@ def sparse_quantized_conv_features_from_relation(
                                     weight.out_channels, relation)):
             return _padded_conv(
                 feats, _quantized_fragments(weight, padded=True), weight.bits,
-                weight.out_channels, relation.require_sorted_implicit_gemm(),
+                weight.out_channels, relation.conv_view(
+                    weight.in_channels * weight.out_channels * 2),
                 relation.n_out_capacity, relation, bias, relu)
     return ext.sparse_quantized_conv_features(
         feats, weight.weight, weight.scales, weight.biases,
@@ -427,8 +435,7 @@ def sparse_quantized_conv_features_from_relation(
         relation.n_out_capacity, relation.n_kernels, weight.in_channels,
         weight.out_channels, weight.storage_in_channels, weight.group_size,
         weight.bits, bias=bias, tile_order=order, relu=relu,
-        weight_fragments=(_quantized_fragments(weight)
-                          if order is not None else None),
+        weight_fragments=fragments,
         out_in_map=dense)
 
 

@@ -177,6 +177,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("out_in_map"), py::arg("row_masks"),
         "Return (reorder_rows, sorted_out_in_map, sorted_kv_out_in_map, tile_masks).");
 
+    m.def("build_tiled_view", &ln::make_tiled_view, py::arg("out_in_map"), py::arg("row_masks"),
+          "The tuple of build_sorted_implicit_gemm_view with the rows left in their order.");
+
     m.def("sparse_conv_features", &ln::sparse_conv_features, py::arg("feats"), py::arg("weights"),
           py::arg("in_rows"), py::arg("out_rows"), py::arg("kernel_ids"), py::arg("counts"), py::arg("row_offsets"),
           py::arg("in_row_offsets"), py::arg("in_edge_ids"), py::arg("kernel_row_offsets"),

@@ -214,9 +214,13 @@ at::Tensor sparse_conv_features_expand(const at::Tensor& feats_in, const at::Ten
     return out;
 }
 
+// Row capacity up to which a conv's 128-row tiles all start at once, one per
+// CU: their order is then irrelevant and the schedule launch saved.
+constexpr int kOneRoundRows = 256 * 128;
+
 // The matrix-core conv's tile schedule: the caller's precomputed order
 // (conv_tile_order, flagged LATTICE_CONV_ORDER_READY), or a fresh workspace
-// the conv fills itself.
+// the conv fills itself (null: tiles in order, for one round of tiles).
 at::Tensor schedule_workspace(const std::optional<at::Tensor>& tile_order, int out_capacity, const at::Tensor& like,
                               size_t* bytes) {
     const size_t need = lattice_hip_conv_workspace_bytes(out_capacity);
@@ -230,9 +234,15 @@ at::Tensor schedule_workspace(const std::optional<at::Tensor>& tile_order, int o
         *bytes = need | LATTICE_CONV_ORDER_READY;
         return t;
     }
+    if (out_capacity <= kOneRoundRows) {
+        *bytes = 0;
+        return {};
+    }
     *bytes = need;
     return workspace(need, like);
 }
+
+void* schedule_ptr(const at::Tensor& ws) { return ws.defined() ? ws.data_ptr() : nullptr; }
 
 at::Tensor sparse_conv_features_sorted_implicit_gemm(const at::Tensor& feats_in, const at::Tensor& weights_in,
                                                      const at::Tensor& sorted_out_in_map,
@@ -299,7 +309,7 @@ at::Tensor sparse_conv_features_sorted_implicit_gemm(const at::Tensor& feats_in,
         check_status(lattice_hip_sparse_conv_features_sorted_fragments(
             dtype, feats.data_ptr(), static_cast<int>(feats.size(0)), c_in, frag.data_ptr(), n_kernels,
             static_cast<int>(c_out), ci32(kv), ci32(tiles), store_sorted ? nullptr : ci32(order), out_capacity,
-            out.data_ptr(), b, relu ? LATTICE_EPILOGUE_RELU : LATTICE_EPILOGUE_NONE, ws.data_ptr(), ws_bytes,
+            out.data_ptr(), b, relu ? LATTICE_EPILOGUE_RELU : LATTICE_EPILOGUE_NONE, schedule_ptr(ws), ws_bytes,
             current_stream(feats)));
         return out;
     }
@@ -307,7 +317,7 @@ at::Tensor sparse_conv_features_sorted_implicit_gemm(const at::Tensor& feats_in,
         dtype_code(feats, op), feats.data_ptr(), static_cast<int>(feats.size(0)), static_cast<int>(feats.size(1)),
         weights.data_ptr(), LATTICE_WEIGHT_DENSE_5D, n_kernels, static_cast<int>(c_out), ci32(kv), ci32(tiles),
         store_sorted ? nullptr : ci32(order), out_capacity, out.data_ptr(), b,
-        relu ? LATTICE_EPILOGUE_RELU : LATTICE_EPILOGUE_NONE, ws.data_ptr(), ws_bytes,
+        relu ? LATTICE_EPILOGUE_RELU : LATTICE_EPILOGUE_NONE, schedule_ptr(ws), ws_bytes,
         current_stream(feats)));
     return out;
 }
@@ -472,7 +482,7 @@ at::Tensor sparse_conv_features_padded(const at::Tensor& feats_in, const at::Ten
     check_status(lattice_hip_sparse_conv_features_padded(
         dtype, feats.data_ptr(), static_cast<int>(feats.size(0)), c_in, fragments.data_ptr(), bits, n_kernels,
         out_channels, ci32(kv), ci32(tiles), ci32(order), out_capacity, out.data_ptr(), b,
-        relu ? LATTICE_EPILOGUE_RELU : LATTICE_EPILOGUE_NONE, ws.data_ptr(), ws_bytes, current_stream(feats)));
+        relu ? LATTICE_EPILOGUE_RELU : LATTICE_EPILOGUE_NONE, schedule_ptr(ws), ws_bytes, current_stream(feats)));
     return out;
 }
 
@@ -607,7 +617,7 @@ at::Tensor sparse_quantized_conv_features(const at::Tensor& feats_in, const at::
         check_status(lattice_hip_sparse_quantized_conv_features_sorted_fragments(
             dtype, feats.data_ptr(), static_cast<int>(feats.size(0)), in_channels, frag.data_ptr(), bits, n_kernels,
             out_channels, ci32(kv), ci32(tiles), ci32(order), out_capacity, out.data_ptr(), b,
-            relu ? LATTICE_EPILOGUE_RELU : LATTICE_EPILOGUE_NONE, ws.data_ptr(), ws_bytes, current_stream(feats)));
+            relu ? LATTICE_EPILOGUE_RELU : LATTICE_EPILOGUE_NONE, schedule_ptr(ws), ws_bytes, current_stream(feats)));
         return out;
     }
     check_status(lattice_hip_sparse_quantized_conv_features(
@@ -616,7 +626,7 @@ at::Tensor sparse_quantized_conv_features(const at::Tensor& feats_in, const at::
         n_kernels, out_channels, storage_in_channels, group_size, bits, ci32(in_rows), ci32(kernel_ids),
         ci32(counts), static_cast<int>(in_rows.size(0)), ci32(row_offsets), has_plan ? ci32(kv) : nullptr,
         has_plan ? ci32(tiles) : nullptr, has_plan ? ci32(order) : nullptr, out_capacity, out.data_ptr(), b,
-        relu ? LATTICE_EPILOGUE_RELU : LATTICE_EPILOGUE_NONE, has_plan ? ws.data_ptr() : nullptr, ws_bytes,
+        relu ? LATTICE_EPILOGUE_RELU : LATTICE_EPILOGUE_NONE, schedule_ptr(ws), ws_bytes,
         current_stream(feats)));
     return out;
 }

@@ -331,4 +331,26 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor, at::Tensor> make_sorted_implicit_
     return {reorder, kv.t(), kv, tiles};
 }
 
+std::tuple<at::Tensor, at::Tensor, at::Tensor, at::Tensor> make_tiled_view(const at::Tensor& out_in_map_in,
+                                                                           const at::Tensor& row_masks_in) {
+    if (out_in_map_in.dim() != 2 || out_in_map_in.scalar_type() != at::kInt) {
+        throw std::invalid_argument("out_in_map must have shape (Nout, K) and int32 dtype.");
+    }
+    if (row_masks_in.dim() != 2 || row_masks_in.scalar_type() != at::kInt ||
+        row_masks_in.size(0) != out_in_map_in.size(0) || row_masks_in.size(1) != 1) {
+        throw std::invalid_argument("row_masks must have one word per out_in_map row.");
+    }
+    require_on_device({{&out_in_map_in, "out_in_map"}, {&row_masks_in, "row_masks"}});
+    const at::Tensor map = out_in_map_in.contiguous();
+    const at::Tensor masks = row_masks_in.contiguous();
+    const int rows = static_cast<int>(map.size(0));
+    const int K = static_cast<int>(map.size(1));
+    at::Tensor reorder = empty_i32({rows}, map);
+    at::Tensor kv = empty_i32({K, rows}, map);
+    at::Tensor tiles = empty_i32({((rows + 63) / 64) * 4}, map);
+    check_status(lattice_hip_build_tiled_view(ci32(map), ci32(masks), rows, K, i32(reorder), i32(kv), i32(tiles),
+                                              current_stream(map)));
+    return {reorder, kv.t(), kv, tiles};
+}
+
 }  // namespace lattice_native

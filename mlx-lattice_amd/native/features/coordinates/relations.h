@@ -77,4 +77,8 @@ std::tuple<at::Tensor, at::Tensor> make_relation_implicit_gemm_view(
 std::tuple<at::Tensor, at::Tensor, at::Tensor, at::Tensor> make_sorted_implicit_gemm_view(
     const at::Tensor& out_in_map, const at::Tensor& row_masks);
 
+// The same tuple with the rows in their order (lattice_hip_build_tiled_view).
+std::tuple<at::Tensor, at::Tensor, at::Tensor, at::Tensor> make_tiled_view(const at::Tensor& out_in_map,
+                                                                           const at::Tensor& row_masks);
+
 }  // namespace lattice_native
