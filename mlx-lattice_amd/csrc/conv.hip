@@ -1411,6 +1411,25 @@ __device__ inline typename MfmaOps<T>::vec dequant_fragment(typename MfmaOps<T>:
     return out;
 }
 
+// The same as two fragments whose sum is the fp32 weight but for 2^-16 (bf16)
+// or 2^-21 (fp16) of it: the padded instances contract both, as the edge
+// kernel contracts fp32 weights (one fragment alone raises the error of a
+// bf16 96 -> 96 int4 conv against 64 bits from 1.7e-3 to 2.3e-3).
+template <typename T, int QB>
+__device__ inline void dequant_fragments(typename MfmaOps<T>::vec raw, typename MfmaOps<T>::vec& hi,
+                                         typename MfmaOps<T>::vec& lo) {
+    const uint4 r = __builtin_bit_cast(uint4, raw);
+    const float sc = static_cast<float>(__builtin_bit_cast(T, static_cast<uint16_t>(r.z & 0xFFFFu)));
+    const float bi = static_cast<float>(__builtin_bit_cast(T, static_cast<uint16_t>(r.z >> 16)));
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        const uint32_t q = QB == 4 ? (r.x >> (4 * j)) & 15u : ((j < 4 ? r.x : r.y) >> (8 * (j & 3))) & 255u;
+        const float w = static_cast<float>(q) * sc + bi;
+        hi[j] = static_cast<T>(w);
+        lo[j] = static_cast<T>(w - static_cast<float>(hi[j]));
+    }
+}
+
 // Store of a finished tile whose columns may end inside it (PAD): column
 // tile col0 .. of an output with c_out columns.  16-bit tiles are staged in
 // the idle A ring (one row after the other, 16 bytes apart in the banks) and
@@ -1725,7 +1744,14 @@ conv_igemm_stream(const T* __restrict__ feats, int n_in, int c_in, const T* __re
                 idx_expand(d, ra);
             }
             wait_vm_b<W_B>(bcur);
-            if constexpr (QB != 0) {
+            constexpr bool SPLIT = PAD && QB != 0;
+            V blo[SPLIT ? CB : 1][SPLIT ? ST : 1];
+            if constexpr (SPLIT) {
+#pragma unroll
+                for (int cb = 0; cb < CB; ++cb)
+#pragma unroll
+                    for (int st = 0; st < ST; ++st) dequant_fragments<T, QB>(bcur[cb][st], bcur[cb][st], blo[cb][st]);
+            } else if constexpr (QB != 0) {
 #pragma unroll
                 for (int cb = 0; cb < CB; ++cb)
 #pragma unroll
@@ -1767,6 +1793,8 @@ conv_igemm_stream(const T* __restrict__ feats, int n_in, int c_in, const T* __re
                             for (int cb = 0; cb < CB; ++cb) {
                                 // transposed product: lane (lr, lg) accumulates
                                 // row rb*16 + lr, columns cb*16 + lg*4 .. + 3
+                                if constexpr (SPLIT)
+                                    acc[rb][cb] = MfmaOps<T>::mfma(blo[cb][st], af[rb % (RA + 1)][st], acc[rb][cb]);
                                 acc[rb][cb] = MfmaOps<T>::mfma(bcur[cb][st], af[rb % (RA + 1)][st], acc[rb][cb]);
                             }
                         }
@@ -2378,6 +2406,8 @@ int launch_padded(const T* feats, int n_in, int c_in, const T* frag, int K, int 
     // us), and 64 rows below (32 -> 32 at 128,000 rows 49 against 62 us).
     // 16 bits: 64 rows for few rows, and for one column tile of more than
     // 64 (96 -> 96 over 150,001 / 128,000 rows 48 -> 43 / 75 -> 73 us).
+    // Packed weights hold two fragments a piece, for which 128 rows and 128
+    // columns have no registers left: 64 rows.
     if constexpr (sizeof(T) == 4) {
         if (c_out <= 32) {
             LATTICE_PADDED(32, 4, 64);
@@ -2386,7 +2416,7 @@ int launch_padded(const T* feats, int n_in, int c_in, const T* frag, int K, int 
         } else {
             LATTICE_PADDED(128, 1, 32);
         }
-    } else if (few_rows(rows, c_out) || (c_out > 64 && c_out <= 128)) {
+    } else if (QB != 0 || few_rows(rows, c_out) || (c_out > 64 && c_out <= 128)) {
         if (c_out <= 32) {
             LATTICE_PADDED(32, 4, 64);
         } else if (c_out <= 64) {
@@ -2394,12 +2424,14 @@ int launch_padded(const T* feats, int n_in, int c_in, const T* frag, int K, int 
         } else {
             LATTICE_PADDED(128, 1, 64);
         }
-    } else if (c_out <= 32) {
-        LATTICE_PADDED(32, 4, 128);
-    } else if (c_out <= 64) {
-        LATTICE_PADDED(64, 2, 128);
-    } else {
-        LATTICE_PADDED(128, 1, 128);
+    } else if constexpr (QB == 0) {
+        if (c_out <= 32) {
+            LATTICE_PADDED(32, 4, 128);
+        } else if (c_out <= 64) {
+            LATTICE_PADDED(64, 2, 128);
+        } else {
+            LATTICE_PADDED(128, 1, 128);
+        }
     }
 #undef LATTICE_PADDED
     LATTICE_LAUNCH_CHECK();

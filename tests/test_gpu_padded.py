@@ -7,6 +7,8 @@ its value), and once more after the bias."""
 
 from __future__ import annotations
 
+import dataclasses
+
 import numpy as np
 import pytest
 import torch
@@ -129,16 +131,17 @@ def test_padded_quantized_conv_matches_the_unpacked_weight(dtype, bits, c_in,
     x = SparseTensor(torch.as_tensor(coords).to(DEV), f)
     y = ops.subm_conv3d(x, q, kernel_size=3)
     torch.cuda.synchronize()
-    # codes * scale + bias before the rounding of dequantize_weight: the
-    # kernel rounds once to the feature type, half an ulp of the weight
-    wd = to_np(dequantize_weight(q).double())
+    # codes * scale + bias unrounded: the kernel contracts a weight as two
+    # fragments, the second holding what the first's rounding leaves
+    wd = to_np(dequantize_weight(dataclasses.replace(
+        q, scales=q.scales.float(), biases=q.biases.float())).double())
     orel = O.kernel_relation(coords, kernel_size=3)
     fd = to_np(f.double())
     ref = O.conv_features_fp64(fd, O.mapped_weight(wd), orel)
     mag = O.conv_features_fp64(np.abs(fd), O.mapped_weight(np.abs(wd)), orel)
     bound = _bound(fd, wd, orel, ref, dtype, c_in, 0.0)
     _check(to_np(y.feats.double()), ref,
-           bound + 2 * HALF_ULP[dtype] * mag, f'int{bits}')
+           bound + 4 * HALF_ULP[dtype] ** 2 * mag, f'int{bits}')
 
 
 @pytest.mark.parametrize('dtype,c_in,c_out', [
