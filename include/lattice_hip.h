@@ -307,6 +307,34 @@ int lattice_hip_interpolate_point_features_grad(const float* point_grad,
                                                 int voxel_rows, float* out,
                                                 void* stream);
 
+/* The same builds without the edges: out_coords (forward), counts[1], the
+ * dense map, the masks and the status word, for callers that read the map
+ * alone (the matrix-core convs); in_rows, out_rows, kernel_ids and
+ * row_offsets are ignored (may be NULL) and counts[0] is left as it is.
+ * lattice_hip_build_map_edges writes them later from the map and the masks,
+ * the same values: in_rows, out_rows, kernel_ids [out_capacity * K],
+ * row_offsets [out_capacity + 1] and counts[0] of `out`. */
+int lattice_hip_build_kernel_map_with_table(
+    const int32_t* coords, int rows, const int32_t* active_rows,
+    const int kernel_size[3], const int stride[3], const int padding[3],
+    const int dilation[3], const lattice_relation_outputs* out, void* table,
+    size_t table_bytes, void* workspace, size_t workspace_bytes,
+    void* stream);
+int lattice_hip_build_target_kernel_map(
+    const int32_t* coords, int rows, const int32_t* active_rows,
+    const int32_t* target_coords, int target_rows,
+    const int32_t* target_active_rows, const int kernel_size[3],
+    const int stride[3], const int padding[3], const int dilation[3],
+    const lattice_relation_outputs* out, void* workspace,
+    size_t workspace_bytes, void* stream);
+size_t lattice_hip_map_edges_workspace_bytes(int out_capacity);
+int lattice_hip_build_map_edges(const int32_t* out_in_map,
+                                const int32_t* row_masks, int out_capacity,
+                                int kernel_count,
+                                const lattice_relation_outputs* out,
+                                void* workspace, size_t workspace_bytes,
+                                void* stream);
+
 /* Grouped CSR views of a relation: write_relation_grouped_view
  * (relation_views_detail.h:84-120; relations.cpp:438-476).  Stable
  * partition of the active edge ids by input row and by kernel offset:
@@ -635,24 +663,31 @@ int lattice_hip_sparse_conv_weight_grad(
     size_t workspace_bytes, void* stream);
 
 /* The edges of a relation grouped by offset (write_relation_grouped_view,
- * relation_views_detail.h:84-120), for relations whose edges run in
- * (out_row, offset) order and whose row masks hold one bit per edge: the
- * forward, submanifold and target builds' row_masks [rows], row_offsets
- * [rows + 1] and in_rows [edge_capacity], K <= 32.  Writes
+ * relation_views_detail.h:84-120), for relations with a dense map whose row
+ * masks hold one bit per edge (the forward, submanifold and target builds,
+ * edges in (out_row, offset) order), K <= 32: row_masks [rows].  Writes
  * kernel_row_offsets [K + 1] and, each when non-NULL, pairs
- * [edge_capacity][2] (input row, output row) and kernel_edge_ids
- * [edge_capacity], both defined on their first kernel_row_offsets[K]
- * entries; the same grouping, in the same order, as
+ * [edge_capacity][2] (input row, output row), which reads out_in_map
+ * [rows, K], and kernel_edge_ids [edge_capacity], which reads row_offsets
+ * [rows + 1]; both are defined on their first kernel_row_offsets[K] entries,
+ * the same grouping, in the same order, as
  * lattice_hip_build_relation_grouped_views.  The weight gradient over the
- * pairs is that of the entry above (the same result bit for bit). */
+ * pairs is that of the entry above (the same result bit for bit).
+ * lattice_hip_build_transposed_map_from_dense is
+ * lattice_hip_build_transposed_implicit_gemm_map reading the dense map
+ * instead of the edges. */
 size_t lattice_hip_kernel_pairs_workspace_bytes(int rows);
 int lattice_hip_build_kernel_pairs(const int32_t* row_masks,
-                                   const int32_t* row_offsets,
-                                   const int32_t* in_rows, int rows,
+                                   const int32_t* out_in_map,
+                                   const int32_t* row_offsets, int rows,
                                    int kernel_count, int edge_capacity,
                                    int32_t* kernel_row_offsets, int32_t* pairs,
                                    int32_t* kernel_edge_ids, void* workspace,
                                    size_t workspace_bytes, void* stream);
+int lattice_hip_build_transposed_map_from_dense(
+    const int32_t* out_in_map, int out_capacity, int in_capacity,
+    int kernel_count, int32_t* in_out_map, int32_t* row_masks,
+    int32_t* status, void* stream);
 int lattice_hip_sparse_conv_weight_grad_pairs(
     int dtype, const void* feats, int n_in, int c_in, const void* cot,
     int out_capacity, int c_out, int weight_layout, int kernel_count,

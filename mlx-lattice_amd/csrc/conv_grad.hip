@@ -129,6 +129,21 @@ transposed_map(const int32_t* __restrict__ in_rows, const int32_t* __restrict__ 
     }
 }
 
+// The same from the dense map: entry (row, k) -> in.
+__global__ void __launch_bounds__(256)
+transposed_dense_map(const int32_t* __restrict__ out_in_map, long long entries, int K, int in_capacity,
+                     int32_t* __restrict__ in_out_map, int32_t* __restrict__ status) {
+    for (long long i = static_cast<long long>(blockIdx.x) * blockDim.x + threadIdx.x; i < entries;
+         i += static_cast<long long>(gridDim.x) * blockDim.x) {
+        const int in = out_in_map[i];
+        if (in < 0 || in >= in_capacity) continue;
+        const long long row = i / K;
+        const int k = static_cast<int>(i - row * K);
+        const int prev = atomicCAS(&in_out_map[static_cast<long long>(in) * K + k], -1, static_cast<int>(row));
+        if (prev != -1 && status != nullptr) atomicOr(status, LATTICE_STATUS_REPEATED_PAIR);
+    }
+}
+
 // Offset bits of each input row, from its row of the transposed map.  A
 // block takes `rows_per_block` consecutive rows, copies their contiguous
 // map rows into LDS with coalesced loads, and one lane per row then reads
@@ -246,16 +261,24 @@ group_scan(int32_t* __restrict__ block_counts, int blocks, int K, int32_t* __res
     }
 }
 
+// A wave emits its 64 rows; their map rows pass through its own LDS, 16
+// offsets at a time (coalesced reads, which the lanes then take offset by
+// offset).  Reading the map by lane instead touches 64 lines per load.
+constexpr int kEmitOffsets = 16;
+
 __global__ void __launch_bounds__(kGroupRows)
-group_emit(const int32_t* __restrict__ row_masks, const int32_t* __restrict__ row_offsets,
-           const int32_t* __restrict__ in_rows, int rows, int K, int edge_capacity,
+group_emit(const int32_t* __restrict__ row_masks, const int32_t* __restrict__ out_in_map,
+           const int32_t* __restrict__ row_offsets, int rows, int K, int edge_capacity,
            const int32_t* __restrict__ block_places, int2* __restrict__ pairs, int32_t* __restrict__ edge_ids) {
+    constexpr int kStride = kEmitOffsets + 1;
     __shared__ int32_t place[kGroupWaves][kGroupBins];
+    __shared__ int32_t stage[kGroupWaves][kWave * kStride];
     const int lane = lane_id();
     const int wave = threadIdx.x / kWave;
     const long long row = static_cast<long long>(blockIdx.x) * kGroupRows + threadIdx.x;
+    const long long row0 = row - lane;
+    const int wave_rows = static_cast<int>(max(0ll, min(static_cast<long long>(kWave), rows - row0)));
     const uint32_t mask = row < rows ? static_cast<uint32_t>(row_masks[row]) : 0u;
-    const int first = row < rows ? row_offsets[row] : 0;
     const int c = wave_bit_counts(mask, K, lane);
     if (lane < kGroupBins) place[wave][lane] = c;
     __syncthreads();
@@ -269,17 +292,39 @@ group_emit(const int32_t* __restrict__ row_masks, const int32_t* __restrict__ ro
         }
     }
     __syncthreads();
-    for (int k = 0; k < K; ++k) {
-        const bool has = (mask >> k) & 1u;
-        const uint64_t b = ballot(has);
-        if (has) {
-            const int pos = place[wave][k] + lanes_below(b);
-            const int e = first + __popc(mask & ((1u << k) - 1u));
-            if (pos >= 0 && pos < edge_capacity && e >= 0 && e < edge_capacity) {
-                if (pairs != nullptr) pairs[pos] = make_int2(in_rows[e], static_cast<int>(row));
-                if (edge_ids != nullptr) edge_ids[pos] = e;
+    const int first = edge_ids != nullptr && row < rows ? row_offsets[row] : 0;
+    for (int k0 = 0; k0 < K; k0 += kEmitOffsets) {
+        const int n = min(kEmitOffsets, K - k0);
+        if (pairs != nullptr) {
+            const int step_rows = kWave / n;
+            const int step_k = kWave % n;
+            int r = lane / n;
+            int k = lane % n;
+            while (r < wave_rows) {
+                stage[wave][r * kStride + k] = out_in_map[(row0 + r) * K + k0 + k];
+                r += step_rows;
+                k += step_k;
+                if (k >= n) {
+                    k -= n;
+                    ++r;
+                }
             }
         }
+        __syncthreads();
+        for (int j = 0; j < n; ++j) {
+            const int k = k0 + j;
+            const bool has = (mask >> k) & 1u;
+            const uint64_t b = ballot(has);
+            if (has) {
+                const int pos = place[wave][k] + lanes_below(b);
+                if (pos >= 0 && pos < edge_capacity) {
+                    if (pairs != nullptr)
+                        pairs[pos] = make_int2(stage[wave][lane * kStride + j], static_cast<int>(row));
+                    if (edge_ids != nullptr) edge_ids[pos] = first + __popc(mask & ((1u << k) - 1u));
+                }
+            }
+        }
+        __syncthreads();
     }
 }
 
@@ -900,6 +945,26 @@ extern "C" int lattice_hip_sparse_conv_input_grad(int dtype, const void* cot, in
     return LATTICE_OK;
 }
 
+namespace lattice {
+namespace {
+
+// Offset masks of a transposed map.
+int launch_transposed_masks(const int32_t* in_out_map, int in_capacity, int kernel_count, int32_t* row_masks,
+                            hipStream_t stream) {
+    const int words = (kernel_count + 31) / 32;
+    // At most 64 KB of map rows per block, and at most one row per lane.
+    const int rows_per_block = std::max(1, std::min(256, 16384 / kernel_count));
+    const size_t lds = static_cast<size_t>(rows_per_block) * kernel_count * sizeof(int32_t);
+    LATTICE_REQUIRE(lds <= 65536, "kernel count too large for the transposed masks.");
+    transposed_masks<<<grid_for(in_capacity, rows_per_block, 1u << 16), 256, lds, stream>>>(
+        in_out_map, in_capacity, kernel_count, words, rows_per_block, row_masks);
+    LATTICE_LAUNCH_CHECK();
+    return LATTICE_OK;
+}
+
+}  // namespace
+}  // namespace lattice
+
 extern "C" int lattice_hip_build_transposed_implicit_gemm_map(const int32_t* in_rows, const int32_t* out_rows,
                                                              const int32_t* kernel_ids, const int32_t* counts,
                                                              int edge_capacity, int in_capacity, int kernel_count,
@@ -915,7 +980,6 @@ extern "C" int lattice_hip_build_transposed_implicit_gemm_map(const int32_t* in_
     LATTICE_REQUIRE(in_out_map && row_masks && counts && (edge_capacity == 0 || (in_rows && out_rows && kernel_ids)),
                     "transposed map pointers must be non-null.");
     hipStream_t stream = as_stream(stream_ptr);
-    const int words = (kernel_count + 31) / 32;
     int rc = fill_i32(in_out_map, static_cast<long long>(in_capacity) * kernel_count, -1, stream);
     if (rc != LATTICE_OK) return rc;
     if (edge_capacity > 0) {
@@ -923,14 +987,31 @@ extern "C" int lattice_hip_build_transposed_implicit_gemm_map(const int32_t* in_
             in_rows, out_rows, kernel_ids, counts, edge_capacity, in_capacity, kernel_count, in_out_map, status);
         LATTICE_LAUNCH_CHECK();
     }
-    // At most 64 KB of map rows per block, and at most one row per lane.
-    const int rows_per_block = std::max(1, std::min(256, 16384 / kernel_count));
-    const size_t lds = static_cast<size_t>(rows_per_block) * kernel_count * sizeof(int32_t);
-    LATTICE_REQUIRE(lds <= 65536, "kernel count too large for the transposed masks.");
-    transposed_masks<<<grid_for(in_capacity, rows_per_block, 1u << 16), 256, lds, stream>>>(
-        in_out_map, in_capacity, kernel_count, words, rows_per_block, row_masks);
-    LATTICE_LAUNCH_CHECK();
-    return LATTICE_OK;
+    return launch_transposed_masks(in_out_map, in_capacity, kernel_count, row_masks, stream);
+}
+
+extern "C" int lattice_hip_build_transposed_map_from_dense(const int32_t* out_in_map, int out_capacity,
+                                                           int in_capacity, int kernel_count, int32_t* in_out_map,
+                                                           int32_t* row_masks, int32_t* status, void* stream_ptr) {
+    LATTICE_REQUIRE(out_capacity >= 0 && in_capacity >= 0 && kernel_count > 0,
+                    "transposed map shapes must be nonnegative with a positive kernel count.");
+    hipStream_t stream = as_stream(stream_ptr);
+    if (status != nullptr) {
+        const int rc = fill_i32(status, 1, 0, stream);
+        if (rc != LATTICE_OK) return rc;
+    }
+    if (in_capacity == 0) return LATTICE_OK;
+    LATTICE_REQUIRE(in_out_map && row_masks && (out_capacity == 0 || out_in_map),
+                    "transposed map pointers must be non-null.");
+    int rc = fill_i32(in_out_map, static_cast<long long>(in_capacity) * kernel_count, -1, stream);
+    if (rc != LATTICE_OK) return rc;
+    const long long entries = static_cast<long long>(out_capacity) * kernel_count;
+    if (entries > 0) {
+        transposed_dense_map<<<grid_for(entries, 256, 1u << 16), 256, 0, stream>>>(out_in_map, entries, kernel_count,
+                                                                                  in_capacity, in_out_map, status);
+        LATTICE_LAUNCH_CHECK();
+    }
+    return launch_transposed_masks(in_out_map, in_capacity, kernel_count, row_masks, stream);
 }
 
 extern "C" size_t lattice_hip_conv_weight_grad_workspace_bytes(int dtype, int kernel_count, int c_in, int c_out,
@@ -976,15 +1057,17 @@ extern "C" size_t lattice_hip_kernel_pairs_workspace_bytes(int rows) {
     return aligned_bytes(std::max<size_t>(group_blocks(rows), 1) * kGroupBins * sizeof(int32_t)) + 256;
 }
 
-extern "C" int lattice_hip_build_kernel_pairs(const int32_t* row_masks, const int32_t* row_offsets,
-                                              const int32_t* in_rows, int rows, int kernel_count, int edge_capacity,
-                                              int32_t* kernel_row_offsets, int32_t* pairs, int32_t* kernel_edge_ids,
-                                              void* workspace, size_t workspace_bytes, void* stream_ptr) {
+extern "C" int lattice_hip_build_kernel_pairs(const int32_t* row_masks, const int32_t* out_in_map,
+                                              const int32_t* row_offsets, int rows, int kernel_count,
+                                              int edge_capacity, int32_t* kernel_row_offsets, int32_t* pairs,
+                                              int32_t* kernel_edge_ids, void* workspace, size_t workspace_bytes,
+                                              void* stream_ptr) {
     LATTICE_REQUIRE(rows >= 0 && edge_capacity >= 0 && kernel_count > 0 && kernel_count <= kGroupBins,
                     "kernel pairs need nonnegative capacities and K <= 32.");
     LATTICE_REQUIRE(kernel_row_offsets != nullptr, "kernel pair pointers must be non-null.");
     LATTICE_REQUIRE(rows == 0 || edge_capacity == 0 ||
-                        (row_masks && row_offsets && in_rows && (pairs || kernel_edge_ids)),
+                        (row_masks && (pairs || kernel_edge_ids) && (!pairs || out_in_map) &&
+                         (!kernel_edge_ids || row_offsets)),
                     "kernel pair pointers must be non-null.");
     LATTICE_REQUIRE(reinterpret_cast<uintptr_t>(pairs) % 8 == 0, "kernel pairs must be 8-byte aligned.");
     LATTICE_REQUIRE(workspace != nullptr && workspace_bytes >= lattice_hip_kernel_pairs_workspace_bytes(rows),
@@ -999,8 +1082,9 @@ extern "C" int lattice_hip_build_kernel_pairs(const int32_t* row_masks, const in
     LATTICE_LAUNCH_CHECK();
     group_scan<<<1, 1024, 0, stream>>>(places, blocks, kernel_count, kernel_row_offsets);
     LATTICE_LAUNCH_CHECK();
-    group_emit<<<blocks, kGroupRows, 0, stream>>>(row_masks, row_offsets, in_rows, rows, kernel_count, edge_capacity,
-                                                  places, reinterpret_cast<int2*>(pairs), kernel_edge_ids);
+    group_emit<<<blocks, kGroupRows, 0, stream>>>(row_masks, out_in_map, row_offsets, rows, kernel_count,
+                                                  edge_capacity, places, reinterpret_cast<int2*>(pairs),
+                                                  kernel_edge_ids);
     LATTICE_LAUNCH_CHECK();
     return LATTICE_OK;
 }

@@ -321,8 +321,9 @@ query_map_blocks(BlockTable table, const int32_t* __restrict__ out_buckets, int 
         dst[0] = make_int4(v[0], v[1], v[2], v[3]);
         dst[1] = make_int4(v[4], v[5], v[6], v[7]);
         row_masks[row] = static_cast<int32_t>(mask);
-        degrees[row] = degree;
+        if (degrees != nullptr) degrees[row] = degree;
     }
+    if (block_totals == nullptr) return;
     int sum = degree;
 #pragma unroll
     for (int off = kWave / 2; off > 0; off >>= 1) sum += __shfl_xor(sum, off, kWave);
@@ -670,6 +671,23 @@ scan_block_totals(const int32_t* __restrict__ totals, int blocks, int32_t* __res
     }
 }
 
+// Degrees and per-block totals of a map whose query left them out: the bits
+// of each row's masks.
+__global__ void __launch_bounds__(kWave)
+count_degrees(const int32_t* __restrict__ row_masks, int out_capacity, int words, int32_t* __restrict__ degrees,
+              int32_t* __restrict__ block_totals) {
+    const long long row = static_cast<long long>(blockIdx.x) * kQueryRows + threadIdx.x;
+    int degree = 0;
+    if (row < out_capacity) {
+        for (int w = 0; w < words; ++w) degree += __popc(static_cast<uint32_t>(row_masks[row * words + w]));
+        degrees[row] = degree;
+    }
+    int sum = degree;
+#pragma unroll
+    for (int off = kWave / 2; off > 0; off >>= 1) sum += __shfl_xor(sum, off, kWave);
+    if (threadIdx.x == 0) block_totals[blockIdx.x] = sum;
+}
+
 // Edge emission in (out_row, kernel) order.  A block owns the same
 // kQueryRows rows as in the query: it turns their degrees (read from
 // row_offsets, where the query left them) into row offsets with its block
@@ -948,6 +966,17 @@ int launch_query(const QueryArgs& a, hipStream_t stream) {
     return LATTICE_OK;
 }
 
+// The same query again once a repeated coordinate has restored its first
+// row; a capped grid that returns at once otherwise.
+int launch_query_again(const QueryArgs& q, hipStream_t stream) {
+    QueryArgs again = q;
+    again.fix_rows = false;
+    again.rerun_if = q.repeat_status;
+    query_map_k3<<<static_cast<unsigned>(std::min(query_blocks(q.out_capacity), 1024)), kWave, 0, stream>>>(again);
+    LATTICE_LAUNCH_CHECK();
+    return LATTICE_OK;
+}
+
 int launch_emit(const int32_t* map, int out_capacity, int K, const int32_t* block_offsets,
                 const lattice_relation_outputs* out, hipStream_t stream) {
     const unsigned blocks = static_cast<unsigned>(query_blocks(out_capacity));
@@ -975,10 +1004,16 @@ int scan_groups(const int32_t* group_totals, int rows, int32_t* group_offsets, i
 
 // Common tail: query (degrees + per-block totals) -> scan of the block
 // totals -> emit (row offsets + edges) -> grouped views when requested.
+// edges false: the query alone (the dense map and the masks).
 int finish_relation(QueryArgs q, int in_capacity, const lattice_relation_outputs* out, Workspace& ws,
-                    hipStream_t stream) {
+                    hipStream_t stream, bool edges) {
     const int K = q.geom.volume;
     const int out_capacity = q.out_capacity;
+    if (!edges) {
+        int rc = launch_query(q, stream);
+        if (rc != LATTICE_OK || out_capacity <= 0 || !q.fix_rows) return rc;
+        return launch_query_again(q, stream);
+    }
     if (out_capacity <= 0) {
         int rc = fill_i32(out->row_offsets, 1, 0, stream);
         if (rc != LATTICE_OK) return rc;
@@ -994,13 +1029,8 @@ int finish_relation(QueryArgs q, int in_capacity, const lattice_relation_outputs
         int rc = launch_query(q, stream);
         if (rc != LATTICE_OK) return rc;
         if (q.fix_rows) {
-            // the same query again once a repeated coordinate has restored its
-            // first row; a capped grid that returns at once otherwise
-            QueryArgs again = q;
-            again.fix_rows = false;
-            again.rerun_if = q.repeat_status;
-            query_map_k3<<<static_cast<unsigned>(std::min(blocks, 1024)), kWave, 0, stream>>>(again);
-            LATTICE_LAUNCH_CHECK();
+            rc = launch_query_again(q, stream);
+            if (rc != LATTICE_OK) return rc;
         }
         scan_block_totals<<<1, kBlockScanThreads, 0, stream>>>(totals, blocks, offsets, out->counts);
         LATTICE_LAUNCH_CHECK();
@@ -1013,8 +1043,15 @@ int finish_relation(QueryArgs q, int in_capacity, const lattice_relation_outputs
                              ws, stream);
 }
 
-int check_outputs(const lattice_relation_outputs* out, bool need_coords, long long out_capacity, int K) {
+int check_outputs(const lattice_relation_outputs* out, bool need_coords, long long out_capacity, int K,
+                  bool edges = true) {
     LATTICE_REQUIRE(out != nullptr, "relation outputs are required.");
+    if (!edges) {
+        LATTICE_REQUIRE(out->counts && out->status, "relation output pointers must be non-null.");
+        LATTICE_REQUIRE(out_capacity == 0 || (out->out_in_map && out->row_masks && (!need_coords || out->out_coords)),
+                        "relation output pointers must be non-null.");
+        return LATTICE_OK;
+    }
     LATTICE_REQUIRE(out->row_offsets && out->counts && out->status, "relation output pointers must be non-null.");
     const bool views = out->in_edge_ids != nullptr || out->kernel_edge_ids != nullptr;
     LATTICE_REQUIRE(!views || (out->in_edge_ids && out->kernel_edge_ids && out->in_row_offsets &&
@@ -1097,13 +1134,16 @@ extern "C" int lattice_hip_build_kernel_relation(const int32_t* coords, int rows
         split ? bytes - tbytes : 0, stream_ptr);
 }
 
-extern "C" int lattice_hip_build_kernel_relation_with_table(
-    const int32_t* coords, int rows, const int32_t* active_rows, const int kernel_size[3], const int stride[3],
-    const int padding[3], const int dilation[3], const lattice_relation_outputs* out, void* table_mem,
-    size_t table_bytes, void* workspace, size_t workspace_bytes, void* stream_ptr) {
+namespace lattice {
+namespace {
+
+int build_forward(const int32_t* coords, int rows, const int32_t* active_rows, const int kernel_size[3],
+                  const int stride[3], const int padding[3], const int dilation[3],
+                  const lattice_relation_outputs* out, void* table_mem, size_t table_bytes, void* workspace,
+                  size_t workspace_bytes, void* stream_ptr, bool edges) {
     int rc = validate_geometry(kernel_size, stride, padding, dilation);
     if (rc != LATTICE_OK) return rc;
-    rc = check_outputs(out, true, rows, kernel_size[0] * kernel_size[1] * kernel_size[2]);
+    rc = check_outputs(out, true, rows, kernel_size[0] * kernel_size[1] * kernel_size[2], edges);
     if (rc != LATTICE_OK) return rc;
     LATTICE_REQUIRE(rows >= 0, "coords must have shape (N, 4).");
     LATTICE_REQUIRE(rows == 0 || coords != nullptr, "coords must be non-null.");
@@ -1210,17 +1250,16 @@ extern "C" int lattice_hip_build_kernel_relation_with_table(
         q.out_coords = out->out_coords;
         q.out_active = out->counts + 1;
     }
-    return finish_relation(q, rows, out, ws, stream);
+    return finish_relation(q, rows, out, ws, stream, edges);
 }
 
-extern "C" int lattice_hip_build_target_kernel_relation(
-    const int32_t* coords, int rows, const int32_t* active_rows, const int32_t* target_coords, int target_rows,
-    const int32_t* target_active_rows, const int kernel_size[3], const int stride[3], const int padding[3],
-    const int dilation[3], const lattice_relation_outputs* out, void* workspace, size_t workspace_bytes,
-    void* stream_ptr) {
+int build_target(const int32_t* coords, int rows, const int32_t* active_rows, const int32_t* target_coords,
+                 int target_rows, const int32_t* target_active_rows, const int kernel_size[3], const int stride[3],
+                 const int padding[3], const int dilation[3], const lattice_relation_outputs* out, void* workspace,
+                 size_t workspace_bytes, void* stream_ptr, bool edges) {
     int rc = validate_geometry(kernel_size, stride, padding, dilation);
     if (rc != LATTICE_OK) return rc;
-    rc = check_outputs(out, false, target_rows, kernel_size[0] * kernel_size[1] * kernel_size[2]);
+    rc = check_outputs(out, false, target_rows, kernel_size[0] * kernel_size[1] * kernel_size[2], edges);
     if (rc != LATTICE_OK) return rc;
     LATTICE_REQUIRE(rows >= 0 && target_rows >= 0, "coords must have shape (N, 4).");
     LATTICE_REQUIRE(active_rows != nullptr && target_active_rows != nullptr, "active_rows must be non-null.");
@@ -1245,7 +1284,78 @@ extern "C" int lattice_hip_build_target_kernel_relation(
     q.table = table;
     q.out_in_map = out->out_in_map;
     q.row_masks = out->row_masks;
-    return finish_relation(q, rows, out, ws, stream);
+    return finish_relation(q, rows, out, ws, stream, edges);
+}
+
+}  // namespace
+}  // namespace lattice
+
+extern "C" int lattice_hip_build_kernel_relation_with_table(
+    const int32_t* coords, int rows, const int32_t* active_rows, const int kernel_size[3], const int stride[3],
+    const int padding[3], const int dilation[3], const lattice_relation_outputs* out, void* table_mem,
+    size_t table_bytes, void* workspace, size_t workspace_bytes, void* stream_ptr) {
+    return build_forward(coords, rows, active_rows, kernel_size, stride, padding, dilation, out, table_mem,
+                         table_bytes, workspace, workspace_bytes, stream_ptr, true);
+}
+
+extern "C" int lattice_hip_build_kernel_map_with_table(
+    const int32_t* coords, int rows, const int32_t* active_rows, const int kernel_size[3], const int stride[3],
+    const int padding[3], const int dilation[3], const lattice_relation_outputs* out, void* table_mem,
+    size_t table_bytes, void* workspace, size_t workspace_bytes, void* stream_ptr) {
+    return build_forward(coords, rows, active_rows, kernel_size, stride, padding, dilation, out, table_mem,
+                         table_bytes, workspace, workspace_bytes, stream_ptr, false);
+}
+
+extern "C" int lattice_hip_build_target_kernel_relation(
+    const int32_t* coords, int rows, const int32_t* active_rows, const int32_t* target_coords, int target_rows,
+    const int32_t* target_active_rows, const int kernel_size[3], const int stride[3], const int padding[3],
+    const int dilation[3], const lattice_relation_outputs* out, void* workspace, size_t workspace_bytes,
+    void* stream_ptr) {
+    return build_target(coords, rows, active_rows, target_coords, target_rows, target_active_rows, kernel_size,
+                        stride, padding, dilation, out, workspace, workspace_bytes, stream_ptr, true);
+}
+
+extern "C" int lattice_hip_build_target_kernel_map(
+    const int32_t* coords, int rows, const int32_t* active_rows, const int32_t* target_coords, int target_rows,
+    const int32_t* target_active_rows, const int kernel_size[3], const int stride[3], const int padding[3],
+    const int dilation[3], const lattice_relation_outputs* out, void* workspace, size_t workspace_bytes,
+    void* stream_ptr) {
+    return build_target(coords, rows, active_rows, target_coords, target_rows, target_active_rows, kernel_size,
+                        stride, padding, dilation, out, workspace, workspace_bytes, stream_ptr, false);
+}
+
+extern "C" size_t lattice_hip_map_edges_workspace_bytes(int out_capacity) {
+    return 2 * aligned_bytes(static_cast<size_t>(query_blocks(std::max(out_capacity, 0)) + 1) * sizeof(int32_t)) + 256;
+}
+
+extern "C" int lattice_hip_build_map_edges(const int32_t* out_in_map, const int32_t* row_masks, int out_capacity,
+                                           int kernel_count, const lattice_relation_outputs* out, void* workspace,
+                                           size_t workspace_bytes, void* stream_ptr) {
+    LATTICE_REQUIRE(out_capacity >= 0 && kernel_count > 0, "map edges need a nonnegative capacity and offsets.");
+    LATTICE_REQUIRE(static_cast<long long>(out_capacity) * kernel_count < INT_MAX,
+                    "relation edge capacity exceeds int32.");
+    LATTICE_REQUIRE(out != nullptr && out->row_offsets && out->counts, "relation output pointers must be non-null.");
+    LATTICE_REQUIRE(out_capacity == 0 || (out_in_map && row_masks && out->in_rows && out->out_rows && out->kernel_ids),
+                    "relation output pointers must be non-null.");
+    hipStream_t stream = as_stream(stream_ptr);
+    if (out_capacity == 0) {
+        int rc = fill_i32(out->row_offsets, 1, 0, stream);
+        return rc != LATTICE_OK ? rc : fill_i32(out->counts, 1, 0, stream);
+    }
+    LATTICE_REQUIRE(workspace_bytes >= lattice_hip_map_edges_workspace_bytes(out_capacity),
+                    "map edges workspace too small.");
+    Workspace ws{static_cast<char*>(workspace), workspace_bytes};
+    const int blocks = query_blocks(out_capacity);
+    int32_t* totals = ws.take<int32_t>(blocks);
+    int32_t* offsets = ws.take<int32_t>(blocks);
+    LATTICE_REQUIRE(totals && offsets, "map edges workspace too small.");
+    count_degrees<<<static_cast<unsigned>(blocks), kWave, 0, stream>>>(row_masks, out_capacity,
+                                                                     (kernel_count + 31) / 32, out->row_offsets,
+                                                                     totals);
+    LATTICE_LAUNCH_CHECK();
+    scan_block_totals<<<1, kBlockScanThreads, 0, stream>>>(totals, blocks, offsets, out->counts);
+    LATTICE_LAUNCH_CHECK();
+    return launch_emit(out_in_map, out_capacity, kernel_count, offsets, out, stream);
 }
 
 extern "C" size_t lattice_hip_relation_grouped_views_workspace_bytes(int edge_capacity) {

@@ -82,17 +82,21 @@ def build_kernel_relation(coords: torch.Tensor,
                           stride: int | Sequence[int] = 1,
                           padding: int | Sequence[int] = 0,
                           dilation: int | Sequence[int] = 1, *,
-                          table: torch.Tensor | None = None) -> KernelRelation:
+                          table: torch.Tensor | None = None,
+                          map_only: bool = False) -> KernelRelation:
     """Forward sparse convolution relation (builders.py:156-191).  ``table``
     (optional): the ``block_table`` of an earlier relation over the same
     coordinates (built on the current stream), which the build then reuses
-    instead of hashing the coordinates again."""
+    instead of hashing the coordinates again.  ``map_only``: build the dense
+    map and leave the edges to their first use (``_map_only``)."""
     validate_coords(coords)
     spec = KernelSpec(size=kernel_size, stride=stride, padding=padding,
                       dilation=dilation)
     offsets = kernel_offsets(spec.size, spec.dilation)
     source_active = _active_rows(active_rows, coords)
-    native = _ext().build_kernel_relation_with_view(
+    build = (_ext().build_kernel_map if _map_only(map_only, offsets)
+             else _ext().build_kernel_relation_with_view)
+    native = build(
         coords, source_active, list(spec.size), list(spec.stride),
         list(spec.padding), list(spec.dilation), table=table)
     return _kernel_relation_from_native(
@@ -105,12 +109,13 @@ def build_submanifold_kernel_relation(
         coords: torch.Tensor, active_rows: torch.Tensor | None = None,
         kernel_size: int | Sequence[int] = 3,
         dilation: int | Sequence[int] = 1, *,
-        keep_table: bool = False) -> KernelRelation:
+        keep_table: bool = False,
+        map_only: bool = False) -> KernelRelation:
     """Submanifold relation whose output support is ``coords``
     (builders.py:194-233).  ``keep_table``: keep the build's block table of
     ``coords`` (a buffer of its own, about 96-192 B per row) as
     ``block_table`` for a later ``build_kernel_relation(..., table=...)``
-    over the same coordinates."""
+    over the same coordinates.  ``map_only``: as there."""
     validate_coords(coords)
     spec = KernelSpec(size=kernel_size, stride=1, padding=0,
                       dilation=dilation)
@@ -120,7 +125,10 @@ def build_submanifold_kernel_relation(
             'padding=0, and positive dilation.')
     offsets = kernel_offsets(spec.size, spec.dilation)
     source_active = _active_rows(active_rows, coords)
-    native = _ext().build_submanifold_kernel_relation_with_view(
+    build = (_ext().build_submanifold_kernel_map
+             if _map_only(map_only, offsets)
+             else _ext().build_submanifold_kernel_relation_with_view)
+    native = build(
         coords, source_active, list(spec.size), list(spec.dilation))
     return _kernel_relation_from_native(
         native, offsets=offsets, in_capacity=int(coords.shape[0]),
@@ -137,9 +145,10 @@ def build_target_kernel_relation(
         kernel_size: int | Sequence[int] = 3,
         stride: int | Sequence[int] = 1,
         padding: int | Sequence[int] = 0,
-        dilation: int | Sequence[int] = 1) -> KernelRelation:
+        dilation: int | Sequence[int] = 1,
+        map_only: bool = False) -> KernelRelation:
     """Relation from source coords to explicit target coords
-    (builders.py:82-127)."""
+    (builders.py:82-127).  ``map_only``: as in ``build_kernel_relation``."""
     validate_coords(coords)
     validate_coords(target_coords)
     if coords.dtype != target_coords.dtype:
@@ -149,7 +158,9 @@ def build_target_kernel_relation(
     offsets = kernel_offsets(spec.size, spec.dilation)
     source_active = _active_rows(active_rows, coords)
     target_active = _active_rows(target_active_rows, target_coords)
-    native = _ext().build_target_kernel_relation_with_view(
+    build = (_ext().build_target_kernel_map if _map_only(map_only, offsets)
+             else _ext().build_target_kernel_relation_with_view)
+    native = build(
         coords, source_active, target_coords, target_active,
         list(spec.size), list(spec.stride), list(spec.padding),
         list(spec.dilation))
@@ -248,17 +259,17 @@ def _kernel_relation_from_native(
     if in_row_offsets is None:
         n_kernels = len(offsets)
 
-        def grouped_views():
+        def grouped_views(edges=None):
+            rows, ids = ((in_rows, kernel_ids) if edges is None
+                         else (edges.in_rows, edges.kernel_ids))
             return _ext().build_relation_grouped_views(
-                in_rows, kernel_ids, counts, in_capacity, n_kernels)
+                rows, ids, counts, in_capacity, n_kernels)
     # The build's own row masks hold one bit per edge, in edge order.
     kernel_groups = None
     if implicit is not None and len(offsets) <= 32:
-        row_masks = implicit.row_masks
-
-        def kernel_groups(edge_ids):
-            return _ext().build_kernel_pairs(row_masks, row_offsets, in_rows,
-                                             len(offsets), edge_ids)
+        def kernel_groups(csr_offsets):
+            return _ext().build_kernel_pairs(
+                implicit.row_masks, implicit.out_in_map, csr_offsets)
     return KernelRelation(
         in_rows, out_rows, kernel_ids, row_offsets=row_offsets,
         counts=counts, in_row_offsets=in_row_offsets,
@@ -274,6 +285,14 @@ def _kernel_relation_from_native(
         repeated_edges=repeated_edges,
         direct_expansion=direct_expansion, repeated_coords=repeated_coords,
         block_table=block_table)
+
+
+def _map_only(wanted: bool, offsets: tuple[Triple, ...]) -> bool:
+    """Convs of at most 32 offsets read the dense map, not the edges: emitting
+    them at build time writes 12 bytes per edge and reads the map again (24 us
+    of the 250 us of a 3^3 build over 200,000 rows with 15 edges each).  More
+    offsets run over the edges."""
+    return wanted and len(offsets) <= 32
 
 
 def _require_positive(values: Triple, name: str) -> None:

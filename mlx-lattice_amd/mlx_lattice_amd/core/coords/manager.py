@@ -108,8 +108,11 @@ class CoordinateManager:
                         kernel_size: int | Sequence[int] = 3,
                         stride: int | Sequence[int] = 1,
                         padding: int | Sequence[int] = 0,
-                        dilation: int | Sequence[int] = 1) -> KernelRelation:
-        """Build or reuse a forward relation (manager.py:142-174)."""
+                        dilation: int | Sequence[int] = 1,
+                        map_only: bool = False) -> KernelRelation:
+        """Build or reuse a forward relation (manager.py:142-174).
+        ``map_only``: the consumer reads the dense map and not the edges,
+        which a relation built here then leaves to their first use."""
         spec = KernelSpec(size=kernel_size, stride=stride, padding=padding,
                           dilation=dilation)
         cache_key = (key, None, spec, 'forward')
@@ -118,7 +121,7 @@ class CoordinateManager:
                 self.coords(key), active_rows=self.active_rows(key),
                 kernel_size=spec.size, stride=spec.stride,
                 padding=spec.padding, dilation=spec.dilation,
-                table=self._take_block_table(key))
+                table=self._take_block_table(key), map_only=map_only)
         return self._kernel_relations[cache_key]
 
     def _take_block_table(self, key: CoordinateMapKey) -> torch.Tensor | None:
@@ -168,7 +171,8 @@ class CoordinateManager:
     def submanifold_kernel_relation(
             self, key: CoordinateMapKey, *,
             kernel_size: int | Sequence[int] = 3,
-            dilation: int | Sequence[int] = 1) -> KernelRelation:
+            dilation: int | Sequence[int] = 1,
+            map_only: bool = False) -> KernelRelation:
         """Build or reuse a submanifold relation (manager.py:200-229)."""
         spec = KernelSpec(size=kernel_size, stride=1, padding=0,
                           dilation=dilation)
@@ -177,7 +181,7 @@ class CoordinateManager:
             relation = build_submanifold_kernel_relation(
                 self.coords(key), active_rows=self.active_rows(key),
                 kernel_size=spec.size, dilation=spec.dilation,
-                keep_table=True)
+                keep_table=True, map_only=map_only)
             table = relation.block_table
             if table is not None:
                 stream = (torch.cuda.current_stream(table.device)
@@ -192,7 +196,8 @@ class CoordinateManager:
             kernel_size: int | Sequence[int] = 3,
             stride: int | Sequence[int] = 1,
             padding: int | Sequence[int] = 0,
-            dilation: int | Sequence[int] = 1) -> KernelRelation:
+            dilation: int | Sequence[int] = 1,
+            map_only: bool = False) -> KernelRelation:
         """Build or reuse a relation to explicit target coords
         (manager.py:266-305)."""
         if not self.owns(key) or not self.owns(target_key):
@@ -207,5 +212,6 @@ class CoordinateManager:
                 active_rows=self.active_rows(key),
                 target_active_rows=self.active_rows(target_key),
                 kernel_size=spec.size, stride=spec.stride,
-                padding=spec.padding, dilation=spec.dilation)
+                padding=spec.padding, dilation=spec.dilation,
+                map_only=map_only)
         return self._kernel_relations[cache_key]

@@ -167,6 +167,48 @@ class _StatusWord:
         return value
 
 
+class _MapEdges:
+    """The edges and their row offsets of a relation built as a dense map
+    alone, made from the map and its masks on first use.  They are kept with
+    the stream that wrote them: another stream waits for it.  Under graph
+    capture nothing is kept (the arrays hold values only once the graph
+    runs)."""
+
+    __slots__ = ('_view', '_counts', '_made')
+
+    def __init__(self, view: RelationImplicitGemmView,
+                 counts: torch.Tensor) -> None:
+        self._view = view
+        self._counts = counts
+        self._made = None
+
+    @property
+    def capacity(self) -> int:
+        return int(self._view.out_in_map.numel())
+
+    def get(self) -> tuple[RelationEdges, RelationCSRView]:
+        device = self._counts.device
+        if self._made is None:
+            from mlx_lattice_amd._native import ext
+
+            *edges, row_offsets = ext.build_map_edges(
+                self._view.out_in_map, self._view.row_masks, self._counts)
+            made = RelationEdges(*edges), RelationCSRView(row_offsets)
+            if torch.cuda.is_current_stream_capturing():
+                return made
+            stream = torch.cuda.current_stream(device)
+            self._made = (*made, stream, stream.record_event())
+            return made
+        edges, csr, stream, written = self._made
+        current = torch.cuda.current_stream(device)
+        if current != stream and not torch.cuda.is_current_stream_capturing():
+            current.wait_event(written)
+            for array in (edges.in_rows, edges.out_rows, edges.kernel_ids,
+                          csr.row_offsets):
+                array.record_stream(current)
+        return edges, csr
+
+
 @dataclass(frozen=True, slots=True)
 class SparseRelationContract:
     """Counts, capacities, coordinate context and geometry of a relation."""
@@ -243,16 +285,19 @@ class SparseRelationContract:
 class KernelRelation:
     """Sparse kernel relation with edge, CSR and implicit-GEMM views."""
 
-    contract: SparseRelationContract
-    edges: RelationEdges
-    output_csr: RelationCSRView
+    _contract: SparseRelationContract
+    _edges: RelationEdges | None
+    _output_csr: RelationCSRView | None
+    # Relations built as a dense map alone: makes the edges, the row offsets
+    # and the edge count on their first use.
+    _map_edges: _MapEdges | None
     _input_csr: RelationCSRView | None
     _kernel_csr: RelationCSRView | None
-    _grouped_views: Callable[[], tuple] | None
+    _grouped_views: Callable[..., tuple] | None
     # Builds the edges grouped by offset without a sort (dense-map relations
-    # of at most 32 offsets): called with whether to return the edge ids or
-    # the (input row, output row) pairs.
-    _kernel_groups: Callable[[bool], tuple] | None
+    # of at most 32 offsets): the edge ids when called with the row offsets,
+    # else the (input row, output row) pairs.
+    _kernel_groups: Callable[[torch.Tensor | None], tuple] | None
     _kernel_pairs: tuple[torch.Tensor, torch.Tensor] | None
     implicit_gemm: RelationImplicitGemmView | None = None
     sorted_implicit_gemm: RelationSortedImplicitGemmView | None = None
@@ -282,9 +327,9 @@ class KernelRelation:
 
     def __init__(
         self,
-        in_rows: torch.Tensor,
-        out_rows: torch.Tensor,
-        kernel_ids: torch.Tensor,
+        in_rows: torch.Tensor | None,
+        out_rows: torch.Tensor | None,
+        kernel_ids: torch.Tensor | None,
         *,
         row_offsets: torch.Tensor | None = None,
         counts: torch.Tensor | None = None,
@@ -306,8 +351,8 @@ class KernelRelation:
         kind: RelationKind = 'forward',
         implicit_gemm: RelationImplicitGemmView | None = None,
         sorted_implicit_gemm: RelationSortedImplicitGemmView | None = None,
-        grouped_views: Callable[[], tuple] | None = None,
-        kernel_groups: Callable[[bool], tuple] | None = None,
+        grouped_views: Callable[..., tuple] | None = None,
+        kernel_groups: Callable[[torch.Tensor | None], tuple] | None = None,
         repeated_edges: bool | torch.Tensor | None = None,
         direct_expansion: bool = False,
         repeated_coords: torch.Tensor | None = None,
@@ -318,8 +363,18 @@ class KernelRelation:
         returns ``(in_row_offsets, in_edge_ids, kernel_row_offsets,
         kernel_edge_ids)``; the forward convolution never reads those
         views, so they are only built for consumers that do.
-        ``kernel_groups`` likewise builds the grouping by offset alone."""
-        device = in_rows.device
+        ``kernel_groups`` likewise builds the grouping by offset alone.
+        The builders pass no edges (None, with ``counts``, ``implicit_gemm``
+        and ``grouped_views``) for a relation built as a dense map."""
+        map_edges = None
+        if in_rows is None:
+            if counts is None or implicit_gemm is None:
+                raise ValueError('a relation without edges needs its dense '
+                                 'map and counts.')
+            map_edges = _MapEdges(implicit_gemm, counts)
+            device = counts.device
+        else:
+            device = in_rows.device
         if counts is None:
             counts = torch.tensor(
                 [in_rows.shape[0],
@@ -335,12 +390,14 @@ class KernelRelation:
             target_coords=target_coords,
             target_active_rows=target_active_rows, stride=stride,
             padding=padding, kind=kind)
-        if row_offsets is None:
-            cap = int(contract.n_out_capacity or 0)
-            row_offsets = torch.zeros(cap + 1, dtype=torch.int32,
-                                      device=device)
-        _validate_row_offsets(row_offsets)
-        edges = RelationEdges(in_rows, out_rows, kernel_ids)
+        edges = csr = None
+        if map_edges is None:
+            if row_offsets is None:
+                cap = int(contract.n_out_capacity or 0)
+                row_offsets = torch.zeros(cap + 1, dtype=torch.int32,
+                                          device=device)
+            _validate_row_offsets(row_offsets)
+            edges = RelationEdges(in_rows, out_rows, kernel_ids)
         lazy_views = grouped_views is not None and in_row_offsets is None
         if lazy_views:
             pass
@@ -359,14 +416,17 @@ class KernelRelation:
             if kernel_edge_ids is None:
                 kernel_edge_ids = torch.zeros(edges.capacity,
                                               dtype=torch.int32, device=device)
-        if (contract.n_out_capacity is not None
-                and int(row_offsets.shape[0])
-                != int(contract.n_out_capacity) + 1):
-            raise ValueError(
-                'row_offsets must have length n_out_capacity + 1.')
-        object.__setattr__(self, 'contract', contract)
-        object.__setattr__(self, 'edges', edges)
-        object.__setattr__(self, 'output_csr', RelationCSRView(row_offsets))
+        if map_edges is None:
+            if (contract.n_out_capacity is not None
+                    and int(row_offsets.shape[0])
+                    != int(contract.n_out_capacity) + 1):
+                raise ValueError(
+                    'row_offsets must have length n_out_capacity + 1.')
+            csr = RelationCSRView(row_offsets)
+        object.__setattr__(self, '_contract', contract)
+        object.__setattr__(self, '_edges', edges)
+        object.__setattr__(self, '_output_csr', csr)
+        object.__setattr__(self, '_map_edges', map_edges)
         object.__setattr__(
             self, '_input_csr', None if lazy_views
             else RelationCSRView(in_row_offsets, in_edge_ids))
@@ -395,6 +455,33 @@ class KernelRelation:
         object.__setattr__(self, 'direct_expansion', bool(direct_expansion))
 
     @property
+    def edges(self) -> RelationEdges:
+        if self._map_edges is not None:
+            return self._map_edges.get()[0]
+        return self._edges
+
+    @property
+    def output_csr(self) -> RelationCSRView:
+        if self._map_edges is not None:
+            return self._map_edges.get()[1]
+        return self._output_csr
+
+    @property
+    def contract(self) -> SparseRelationContract:
+        """The contract, its edge count written."""
+        if self._map_edges is not None:
+            self._map_edges.get()
+        return self._contract
+
+    @property
+    def kind(self) -> RelationKind:
+        return self._contract.kind
+
+    @property
+    def source_active_rows(self) -> torch.Tensor | None:
+        return self._contract.source_active_rows
+
+    @property
     def input_csr(self) -> RelationCSRView:
         """Edges grouped by input row (stable in edge order)."""
         if self._input_csr is None:
@@ -405,7 +492,8 @@ class KernelRelation:
     def kernel_csr(self) -> RelationCSRView:
         """Edges grouped by kernel offset (stable in edge order)."""
         if self._kernel_csr is None and self._kernel_groups is not None:
-            k_offsets, _, k_ids = self._kernel_groups(True)
+            k_offsets, _, k_ids = self._kernel_groups(
+                self.output_csr.row_offsets)
             object.__setattr__(self, '_kernel_csr',
                                RelationCSRView(k_offsets, k_ids))
         elif self._kernel_csr is None:
@@ -417,12 +505,14 @@ class KernelRelation:
         every edge, grouped by kernel offset in the order of ``kernel_csr``,
         built on first use; None for relations that group by a sort."""
         if self._kernel_pairs is None and self._kernel_groups is not None:
-            k_offsets, pairs, _ = self._kernel_groups(False)
+            k_offsets, pairs, _ = self._kernel_groups(None)
             object.__setattr__(self, '_kernel_pairs', (k_offsets, pairs))
         return self._kernel_pairs
 
     def _materialize_grouped_views(self) -> None:
-        in_offsets, in_ids, k_offsets, k_ids = self._grouped_views()
+        in_offsets, in_ids, k_offsets, k_ids = (
+            self._grouped_views() if self._map_edges is None
+            else self._grouped_views(self.edges))
         object.__setattr__(self, '_input_csr',
                            RelationCSRView(in_offsets, in_ids))
         if self._kernel_csr is None:
@@ -431,7 +521,9 @@ class KernelRelation:
 
     @property
     def edge_capacity(self) -> int:
-        return self.edges.capacity
+        if self._map_edges is not None:
+            return self._map_edges.capacity
+        return self._edges.capacity
 
     @property
     def counts(self) -> torch.Tensor:
@@ -444,27 +536,27 @@ class KernelRelation:
 
     @property
     def out_count(self) -> torch.Tensor:
-        return self.contract.out_count
+        return self._contract.out_count
 
     @property
     def kernel_offsets(self) -> tuple[Triple, ...]:
-        return self.contract.kernel_offsets
+        return self._contract.kernel_offsets
 
     @property
     def out_coords(self) -> torch.Tensor | None:
-        return self.contract.out_coords
+        return self._contract.out_coords
 
     @property
     def n_in_capacity(self) -> int | None:
-        return self.contract.n_in_capacity
+        return self._contract.n_in_capacity
 
     @property
     def n_out_capacity(self) -> int | None:
-        return self.contract.n_out_capacity
+        return self._contract.n_out_capacity
 
     @property
     def n_kernels(self) -> int | None:
-        return self.contract.n_kernels
+        return self._contract.n_kernels
 
     @property
     def row_offsets(self) -> torch.Tensor:
@@ -506,7 +598,7 @@ class KernelRelation:
         """Return or lazily build the implicit-GEMM view (views.py:452-465)."""
         if self.implicit_gemm is not None:
             return self.implicit_gemm
-        if self.contract.kind in ('transposed', 'generative'):
+        if self._contract.kind in ('transposed', 'generative'):
             view = self._expanded_implicit_gemm()
             object.__setattr__(self, 'implicit_gemm', view)
             return view
@@ -525,7 +617,7 @@ class KernelRelation:
         generative relations hold it by construction (a target relation
         too: each (target row, offset) has one candidate input, its first
         row); a transposed relation does unless an input coordinate repeats."""
-        if self.contract.kind != 'transposed':
+        if self._contract.kind != 'transposed':
             return True
         if isinstance(self.repeated_edges, _StatusWord):
             # lattice_relation_flags: bit 2 = repeated (out_row, kernel_id)
@@ -544,7 +636,7 @@ class KernelRelation:
         submanifold relation does unless a coordinate repeats.  The first
         question reads the build's status word from pinned memory (copied
         when the relation was built), so it waits for that copy only."""
-        if self.contract.kind == 'target':
+        if self._contract.kind == 'target':
             return False
         if isinstance(self.repeated_coords, _StatusWord):
             # lattice_relation_flags: bit 8 = repeated coordinate
@@ -598,7 +690,7 @@ class KernelRelation:
         16,000 rows and 3 at 32,000, 6 for 16 -> 32 fp32 at 32,000 and 7 for
         64 -> 64 fp32 at 16,000, but 30 for 128 -> 128 fp32."""
         if (self.sorted_implicit_gemm is not None
-                or self.contract.kind not in ('forward', 'submanifold',
+                or self._contract.kind not in ('forward', 'submanifold',
                                               'target')
                 or not _tiled_pays(self.n_out_capacity, weight_bytes)):
             return self.require_sorted_implicit_gemm()
@@ -612,21 +704,27 @@ class KernelRelation:
                              ) -> RelationSortedImplicitGemmView:
         """``conv_view`` of the transposed relation."""
         if (self.transposed_sorted_implicit_gemm is not None
-                or self.contract.kind not in ('forward', 'submanifold')
+                or self._contract.kind not in ('forward', 'submanifold')
                 or self.n_in_capacity is None
                 or not _tiled_pays(self.n_in_capacity, weight_bytes)
                 or self.n_kernels is None or self.n_kernels > 32):
             return self.require_transposed_sorted_implicit_gemm()
         if self._transposed_tiled is None:
-            from mlx_lattice_amd._native import ext
-
-            in_out_map, row_masks, _ = ext.build_transposed_implicit_gemm_map(
-                self.edges.in_rows, self.edges.out_rows,
-                self.edges.kernel_ids, self.counts, int(self.n_in_capacity),
-                int(self.n_kernels))
             object.__setattr__(self, '_transposed_tiled',
-                               _tiled_view(in_out_map, row_masks))
+                               _tiled_view(*self._transposed_map()))
         return self._transposed_tiled
+
+    def _transposed_map(self) -> tuple[torch.Tensor, torch.Tensor]:
+        """(in_out_map, row_masks) of the transposed relation."""
+        from mlx_lattice_amd._native import ext
+
+        if self._map_edges is not None:
+            return ext.build_transposed_map_from_dense(
+                self.implicit_gemm.out_in_map, int(self.n_in_capacity))
+        in_out_map, row_masks, _ = ext.build_transposed_implicit_gemm_map(
+            self.edges.in_rows, self.edges.out_rows, self.edges.kernel_ids,
+            self.counts, int(self.n_in_capacity), int(self.n_kernels))
+        return in_out_map, row_masks
 
     def require_transposed_sorted_implicit_gemm(
             self) -> RelationSortedImplicitGemmView:
@@ -641,7 +739,7 @@ class KernelRelation:
         refused."""
         if self.transposed_sorted_implicit_gemm is not None:
             return self.transposed_sorted_implicit_gemm
-        if self.contract.kind not in ('forward', 'submanifold', 'transposed',
+        if self._contract.kind not in ('forward', 'submanifold', 'transposed',
                                       'generative'):
             raise ValueError('the transposed implicit-GEMM view needs a '
                              'forward, submanifold, transposed or generative '
@@ -653,11 +751,8 @@ class KernelRelation:
                 'sorted implicit GEMM view currently supports K <= 32.')
         from mlx_lattice_amd._native import ext
 
-        in_out_map, row_masks, _ = ext.build_transposed_implicit_gemm_map(
-            self.edges.in_rows, self.edges.out_rows, self.edges.kernel_ids,
-            self.counts, int(self.n_in_capacity), int(self.n_kernels))
         reorder, sorted_map, kv_map, tiles = ext.build_sorted_implicit_gemm_view(
-            in_out_map, row_masks)
+            *self._transposed_map())
         view = RelationSortedImplicitGemmView(
             sorted_out_in_map=sorted_map, sorted_kv_out_in_map=kv_map,
             reorder_rows=reorder, tile_masks=tiles)

@@ -68,6 +68,17 @@ def _small_dense_map(dtype: torch.dtype, c_in: int, c_out: int,
     return view.out_in_map
 
 
+def _dense_without_edges(feats: torch.Tensor,
+                         dense: torch.Tensor | None) -> bool:
+    """Whether the native entry, given this dense map, runs the dense-map
+    conv and so needs no edges (rows to write, feature rows aligned to their
+    size)."""
+    return (dense is not None and dense.numel() > 0
+            and (not feats.is_contiguous()
+                 or feats.data_ptr()
+                 % (int(feats.shape[1]) * feats.element_size()) == 0))
+
+
 # lattice_fragment_role: the weight of a padded conv
 _FORWARD, _TRANSPOSED, _MIRRORED = 0, 1, 2
 
@@ -91,7 +102,7 @@ def _padded_forward(feats: torch.Tensor, c_in: int, c_out: int,
     view costs more than it saves."""
     if not relation.dense_map_exact:
         return False
-    if feats.dtype == torch.float32 and relation.contract.kind in (
+    if feats.dtype == torch.float32 and relation.kind in (
             'transposed', 'generative'):
         return False
     return _padded_eligible(feats, c_out, relation, relation.n_out_capacity)
@@ -127,7 +138,7 @@ def _expand_eligible(feats: torch.Tensor, c_out: int,
     """A direct expanded relation (output row in * K + k = the single edge
     (in, k)) runs as a dense matrix-core GEMM without gathers."""
     return (relation.direct_expansion
-            and relation.contract.source_active_rows is not None
+            and relation.source_active_rows is not None
             and feats.dtype in (torch.float16, torch.bfloat16)
             and int(feats.shape[1]) in _EXPAND_CHANNELS
             and c_out in _EXPAND_CHANNELS
@@ -205,7 +216,7 @@ def _input_grad_matrix_core_eligible(cot: torch.Tensor, weight: torch.Tensor,
     columns."""
     c_in = int(weight.shape[1] if weight.ndim == 3 else weight.shape[4])
     c_out = int(cot.shape[1])
-    return (relation.contract.kind != 'target'
+    return (relation.kind != 'target'
             and cot.dtype in (torch.float16, torch.bfloat16)
             and c_out % 32 == 0 and c_out <= 512
             and c_in in _MATRIX_CORE_C_OUT
@@ -247,9 +258,9 @@ def _mirror_symmetric(relation: KernelRelation) -> bool:
     repeat: input row i then meets output row o at offset k exactly when
     o = out_in_map[i][K-1-k], so the transposed map is the forward map with
     its offsets reversed."""
-    if relation.contract.kind != 'submanifold':
+    if relation.kind != 'submanifold':
         return False
-    offs = relation.contract.kernel_offsets
+    offs = relation.kernel_offsets
     k = len(offs)
     return k > 0 and all(
         tuple(-v for v in offs[k - 1 - j]) == tuple(offs[j]) for j in range(k))
@@ -285,7 +296,7 @@ def sparse_conv_input_grad_from_relation(cot: torch.Tensor,
             in_capacity, relation.n_kernels, tile_order=view.tile_order(),
             weight_fragments=_weight_fragments(transposed))
     c_in = int(weight.shape[1] if weight.ndim == 3 else weight.shape[4])
-    if (relation.contract.kind != 'target' and relation.transposed_map_exact
+    if (relation.kind != 'target' and relation.transposed_map_exact
             and _padded_eligible(cot, c_in, relation, in_capacity)):
         mirrored = _mirror_symmetric(relation)
         size = _offset_bytes(weight)
@@ -333,7 +344,7 @@ def _conv_features(feats: torch.Tensor, weight: torch.Tensor,
     c_out = int(weight.shape[2] if weight.ndim == 3 else weight.shape[0])
     if feats.ndim == 2 and _expand_eligible(feats, c_out, relation):
         return ext.sparse_conv_features_expand(
-            feats, weight, relation.contract.source_active_rows,
+            feats, weight, relation.source_active_rows,
             relation.n_kernels, bias=bias, relu=relu)
     if feats.ndim == 2 and _matrix_core_eligible(
             feats.dtype, int(feats.shape[1]), c_out, relation,
@@ -350,11 +361,16 @@ def _conv_features(feats: torch.Tensor, weight: torch.Tensor,
         return _padded_conv(feats, _padded_fragments(weight, _FORWARD), 0,
                             c_out, relation.conv_view(_offset_bytes(weight)),
                             relation.n_out_capacity, relation, bias, relu)
+    if _dense_without_edges(feats, dense):
+        in_rows = kernel_ids = row_offsets = None
+    else:
+        edges = relation.edges
+        in_rows, kernel_ids = edges.in_rows, edges.kernel_ids
+        row_offsets = relation.output_csr.row_offsets
     return ext.sparse_conv_features_csr(
-        feats, weight, relation.edges.in_rows, relation.edges.kernel_ids,
-        relation.counts, relation.output_csr.row_offsets,
-        relation.n_out_capacity, relation.n_kernels, bias=bias, relu=relu,
-        out_in_map=dense)
+        feats, weight, in_rows, kernel_ids, relation._contract.counts,
+        row_offsets, relation.n_out_capacity, relation.n_kernels, bias=bias,
+        relu=relu, out_in_map=dense)
 
 
 def sparse_conv_features_sorted_from_relation(feats: torch.Tensor,
@@ -380,9 +396,7 @@ def sparse_conv_features_sorted_from_relation(feats: torch.Tensor,
     return ext.sparse_conv_features_sorted_implicit_gemm(
         feats, w5, view.sorted_out_in_map,
         view.sorted_kv_out_in_map, view.reorder_rows, view.tile_masks,
-        relation.edges.in_rows, relation.edges.out_rows,
-        relation.edges.kernel_ids, relation.counts,
-        relation.output_csr.row_offsets, None, None, None, None,
+        None, None, None, None, None, None, None, None, None,
         relation.n_out_capacity, relation.n_kernels,
         store_sorted=store_sorted, bias=bias, tile_order=view.tile_order(),
         relu=relu, weight_fragments=_weight_fragments(w5))
@@ -403,6 +417,7 @@ def sparse_quantized_conv_features_from_relation(
     kv = reorder = tiles = _empty_i32(device)
     order = fragments = None
     dense = None
+    mapped = False
     if _matrix_core_eligible(feats.dtype, weight.in_channels,
                              weight.out_channels, relation,
                              int(feats.shape[0])):
@@ -413,6 +428,9 @@ def sparse_quantized_conv_features_from_relation(
         tiles = view.tile_masks
         order = view.tile_order()
         fragments = _quantized_fragments(weight)
+        # an empty view (no rows) is no plan, and a shape without fragments
+        # runs the entry that takes the edges
+        mapped = relation.n_out_capacity > 0 and fragments.numel() > 0
     else:
         dense = _small_dense_map(feats.dtype, weight.in_channels,
                                  weight.out_channels, relation)
@@ -427,11 +445,18 @@ def sparse_quantized_conv_features_from_relation(
                 weight.out_channels, relation.conv_view(
                     weight.in_channels * weight.out_channels * 2),
                 relation.n_out_capacity, relation, bias, relu)
+        mapped = _dense_without_edges(feats, dense)
+    if mapped:
+        in_rows = out_rows = kernel_ids = row_offsets = None
+    else:
+        edges = relation.edges
+        in_rows, out_rows, kernel_ids = (edges.in_rows, edges.out_rows,
+                                         edges.kernel_ids)
+        row_offsets = relation.output_csr.row_offsets
     return ext.sparse_quantized_conv_features(
-        feats, weight.weight, weight.scales, weight.biases,
-        relation.edges.in_rows, relation.edges.out_rows,
-        relation.edges.kernel_ids, relation.counts,
-        relation.output_csr.row_offsets, kv, reorder, tiles,
+        feats, weight.weight, weight.scales, weight.biases, in_rows,
+        out_rows, kernel_ids, relation._contract.counts, row_offsets, kv,
+        reorder, tiles,
         relation.n_out_capacity, relation.n_kernels, weight.in_channels,
         weight.out_channels, weight.storage_in_channels, weight.group_size,
         weight.bits, bias=bias, tile_order=order, relu=relu,
@@ -479,7 +504,7 @@ class _SparsePoolFeatures(torch.autograd.Function):
     def backward(ctx, grad_out):
         feats, pooled = ctx.saved_tensors
         relation = ctx.relation
-        active = relation.contract.source_active_rows
+        active = relation.source_active_rows
         if ctx.input_exclusive and active is not None:
             grad = ext.sparse_pool_features_grad_exclusive(
                 grad_out.contiguous(), feats, pooled, relation.edges.in_rows,

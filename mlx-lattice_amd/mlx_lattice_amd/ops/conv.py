@@ -133,7 +133,9 @@ def _relation_conv(x: SparseTensor, weight, bias, spec: KernelSpec, *,
     _validate_feature_dtype(x.feats, weight)
     _validate_gpu_coord_dtype(x)
     _validate_weight_for_kernel(x, weight, spec.volume)
-    relation = _kernel_relation(x, spec, map_kind, target_key=target_key)
+    relation = _kernel_relation(
+        x, spec, map_kind, target_key=target_key,
+        map_only=_reads_map_only(x.feats, weight, spec.volume))
     if relation.n_out_capacity is None or relation.n_kernels is None:
         raise ValueError('kernel relation is missing static shape metadata.')
     # The bias is added in the conv kernels' store (after rounding, as a
@@ -172,16 +174,35 @@ def _relation_conv(x: SparseTensor, weight, bias, spec: KernelSpec, *,
                         active_rows=relation.out_count)
 
 
+def _reads_map_only(feats: torch.Tensor, weight, volume: int) -> bool:
+    """Whether the conv runs over the relation's dense map: feature rows of
+    whole 16-byte pieces (the matrix-core routes) or 16-bit rows of four
+    channels with 16 or 32 outputs (the dense-map conv).  Others read the
+    edges, which emitting with the map costs least."""
+    quantized = isinstance(weight, QuantizedWeight)
+    if feats.ndim != 2 or (quantized and feats.dtype == torch.float32):
+        return False
+    c_in = int(feats.shape[1])
+    if c_in * feats.element_size() % 16 == 0:
+        return True
+    c_out = (weight.out_channels if quantized
+             else int(weight.shape[0 if weight.ndim == 5 else 2]))
+    return (c_in == 4 and feats.element_size() == 2 and c_out in (16, 32)
+            and volume * c_in <= 256)
+
+
 def _kernel_relation(x: SparseTensor, spec: KernelSpec, map_kind: str, *,
-                     target_key: CoordinateMapKey | None = None):
+                     target_key: CoordinateMapKey | None = None,
+                     map_only: bool = False):
     manager = x.coord_manager
     if map_kind == 'forward':
         return manager.kernel_relation(
             x.coord_key, kernel_size=spec.size, stride=spec.stride,
-            padding=spec.padding, dilation=spec.dilation)
+            padding=spec.padding, dilation=spec.dilation, map_only=map_only)
     if map_kind == 'submanifold':
         return manager.submanifold_kernel_relation(
-            x.coord_key, kernel_size=spec.size, dilation=spec.dilation)
+            x.coord_key, kernel_size=spec.size, dilation=spec.dilation,
+            map_only=map_only)
     if map_kind == 'transposed':
         return manager.transposed_kernel_relation(
             x.coord_key, kernel_size=spec.size, stride=spec.stride,
@@ -194,7 +215,8 @@ def _kernel_relation(x: SparseTensor, spec: KernelSpec, map_kind: str, *,
             raise ValueError('target_key is required for target relations.')
         return manager.target_kernel_relation(
             x.coord_key, target_key, kernel_size=spec.size,
-            stride=spec.stride, padding=spec.padding, dilation=spec.dilation)
+            stride=spec.stride, padding=spec.padding, dilation=spec.dilation,
+            map_only=map_only)
     raise ValueError(
         "map_kind must be 'forward', 'submanifold', 'transposed', "
         "'generative', or 'target'.")

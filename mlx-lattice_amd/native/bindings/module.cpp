@@ -56,15 +56,18 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         },
         py::arg("kernel_size"), py::arg("dilation"));
 
-    auto forward = [](bool with_view) {
-        return [with_view](const at::Tensor& coords, const at::Tensor& active_rows,
+    // The *_map variants build the implicit-GEMM view alone: the tuple of
+    // *_with_view with None for the edges and their row offsets, which
+    // build_map_edges makes on demand.
+    auto forward = [](bool with_view, bool edges = true) {
+        return [with_view, edges](const at::Tensor& coords, const at::Tensor& active_rows,
                            const std::vector<int>& kernel_size, const std::vector<int>& stride,
                            const std::vector<int>& padding, const std::vector<int>& dilation,
                            const std::optional<at::Tensor>& table) {
             auto r = ln::make_kernel_relation(coords, active_rows, triple_from_values(kernel_size, "kernel_size"),
                                               triple_from_values(stride, "stride"),
                                               triple_from_values(padding, "padding"),
-                                              triple_from_values(dilation, "dilation"), !with_view, table);
+                                              triple_from_values(dilation, "dilation"), !with_view, table, edges);
             return with_view ? relation_tuple_with_view(r) : relation_tuple(r);
         };
     };
@@ -75,33 +78,46 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
           py::arg("kernel_size"), py::arg("stride"), py::arg("padding"), py::arg("dilation"), py::kw_only(),
           py::arg("table") = py::none());
 
-    auto subm = [](bool with_view) {
-        return [with_view](const at::Tensor& coords, const at::Tensor& active_rows,
+    m.def("build_kernel_map", forward(true, false), py::arg("coords"), py::arg("active_rows"),
+          py::arg("kernel_size"), py::arg("stride"), py::arg("padding"), py::arg("dilation"), py::kw_only(),
+          py::arg("table") = py::none());
+    m.def("build_map_edges", &ln::make_map_edges, py::arg("out_in_map"), py::arg("row_masks"), py::arg("counts"),
+          "(in_rows, out_rows, kernel_ids, row_offsets) of a *_map build; writes counts[0].");
+
+    auto subm = [](bool with_view, bool edges = true) {
+        return [with_view, edges](const at::Tensor& coords, const at::Tensor& active_rows,
                            const std::vector<int>& kernel_size, const std::vector<int>& dilation) {
             auto r = ln::make_submanifold_kernel_relation(coords, active_rows,
                                                           triple_from_values(kernel_size, "kernel_size"),
-                                                          triple_from_values(dilation, "dilation"), !with_view);
+                                                          triple_from_values(dilation, "dilation"), !with_view,
+                                                          edges);
             return with_view ? relation_tuple_with_view(r) : relation_tuple(r);
         };
     };
+    m.def("build_submanifold_kernel_map", subm(true, false), py::arg("coords"), py::arg("active_rows"),
+          py::arg("kernel_size"), py::arg("dilation"));
     m.def("build_submanifold_kernel_relation", subm(false), py::arg("coords"), py::arg("active_rows"),
           py::arg("kernel_size"), py::arg("dilation"),
           "Build a submanifold sparse kernel relation.");
     m.def("build_submanifold_kernel_relation_with_view", subm(true), py::arg("coords"), py::arg("active_rows"),
           py::arg("kernel_size"), py::arg("dilation"));
 
-    auto target = [](bool with_view) {
-        return [with_view](const at::Tensor& coords, const at::Tensor& active_rows, const at::Tensor& target_coords,
+    auto target = [](bool with_view, bool edges = true) {
+        return [with_view, edges](const at::Tensor& coords, const at::Tensor& active_rows, const at::Tensor& target_coords,
                            const at::Tensor& target_active_rows, const std::vector<int>& kernel_size,
                            const std::vector<int>& stride, const std::vector<int>& padding,
                            const std::vector<int>& dilation) {
             auto r = ln::make_target_kernel_relation(
                 coords, active_rows, target_coords, target_active_rows,
                 triple_from_values(kernel_size, "kernel_size"), triple_from_values(stride, "stride"),
-                triple_from_values(padding, "padding"), triple_from_values(dilation, "dilation"), !with_view);
+                triple_from_values(padding, "padding"), triple_from_values(dilation, "dilation"), !with_view,
+                edges);
             return with_view ? relation_tuple_with_view(r) : relation_tuple(r);
         };
     };
+    m.def("build_target_kernel_map", target(true, false), py::arg("coords"), py::arg("active_rows"),
+          py::arg("target_coords"), py::arg("target_active_rows"), py::arg("kernel_size"), py::arg("stride"),
+          py::arg("padding"), py::arg("dilation"));
     m.def("build_target_kernel_relation", target(false), py::arg("coords"), py::arg("active_rows"),
           py::arg("target_coords"), py::arg("target_active_rows"), py::arg("kernel_size"), py::arg("stride"),
           py::arg("padding"), py::arg("dilation"),
@@ -215,9 +231,11 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("in_edge_ids"), py::arg("kernel_row_offsets"), py::arg("kernel_edge_ids"), py::arg("out_capacity"),
         py::arg("n_kernels"), py::arg("store_sorted") = false, py::kw_only(), py::arg("bias") = py::none(),
         py::arg("tile_order") = py::none(), py::arg("relu") = false, py::arg("weight_fragments") = py::none());
-    m.def("build_kernel_pairs", &ln::build_kernel_pairs, py::arg("row_masks"), py::arg("row_offsets"),
-          py::arg("in_rows"), py::arg("n_kernels"), py::arg("edge_ids"),
-          "Return (kernel_row_offsets, pairs, kernel_edge_ids); edge_ids picks the ids, else the pairs.");
+    m.def("build_kernel_pairs", &ln::build_kernel_pairs, py::arg("row_masks"), py::arg("out_in_map"),
+          py::arg("row_offsets") = py::none(),
+          "Return (kernel_row_offsets, pairs, kernel_edge_ids): the ids when row_offsets is given, else the pairs.");
+    m.def("build_transposed_map_from_dense", &ln::build_transposed_map_from_dense, py::arg("out_in_map"),
+          py::arg("in_capacity"), "Return (in_out_map, row_masks) of a relation with a dense map.");
     m.def("sparse_conv_weight_grad_pairs", &ln::sparse_conv_weight_grad_pairs, py::arg("feats"),
           py::arg("cotangent"), py::arg("weights"), py::arg("pairs"), py::arg("kernel_row_offsets"),
           py::arg("n_kernels"));

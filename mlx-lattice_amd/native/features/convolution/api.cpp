@@ -144,9 +144,10 @@ at::Tensor sparse_conv_features(const at::Tensor& feats_in, const at::Tensor& we
     return out;
 }
 
-at::Tensor sparse_conv_features_csr(const at::Tensor& feats_in, const at::Tensor& weights_in, const at::Tensor& in_rows,
-                                    const at::Tensor& kernel_ids, const at::Tensor& counts,
-                                    const at::Tensor& row_offsets, int out_capacity, int n_kernels,
+at::Tensor sparse_conv_features_csr(const at::Tensor& feats_in, const at::Tensor& weights_in,
+                                    const std::optional<at::Tensor>& in_rows_in,
+                                    const std::optional<at::Tensor>& kernel_ids_in, const at::Tensor& counts,
+                                    const std::optional<at::Tensor>& row_offsets_in, int out_capacity, int n_kernels,
                                     const std::optional<at::Tensor>& bias, bool relu,
                                     const std::optional<at::Tensor>& out_in_map) {
     const char* op = "sparse_conv_features";
@@ -154,17 +155,25 @@ at::Tensor sparse_conv_features_csr(const at::Tensor& feats_in, const at::Tensor
         throw std::invalid_argument("out_capacity must be nonnegative and n_kernels must be positive.");
     }
     validate_weights(feats_in, weights_in, n_kernels, op);
-    require_i32_vector(in_rows, "relation rows and kernel_ids must be one-dimensional int32 arrays.");
-    require_i32_vector(kernel_ids, "relation rows and kernel_ids must be one-dimensional int32 arrays.");
-    if (in_rows.size(0) != kernel_ids.size(0)) {
-        throw std::invalid_argument("relation row arrays and kernel_ids must have equal capacity.");
+    const bool edges = in_rows_in.has_value() && kernel_ids_in.has_value() && row_offsets_in.has_value();
+    const at::Tensor in_rows = edges ? *in_rows_in : at::Tensor();
+    const at::Tensor kernel_ids = edges ? *kernel_ids_in : at::Tensor();
+    const at::Tensor row_offsets = edges ? *row_offsets_in : at::Tensor();
+    if (edges) {
+        require_i32_vector(in_rows, "relation rows and kernel_ids must be one-dimensional int32 arrays.");
+        require_i32_vector(kernel_ids, "relation rows and kernel_ids must be one-dimensional int32 arrays.");
+        if (in_rows.size(0) != kernel_ids.size(0)) {
+            throw std::invalid_argument("relation row arrays and kernel_ids must have equal capacity.");
+        }
     }
     if (counts.dim() != 1 || counts.size(0) != 2 || counts.scalar_type() != at::kInt) {
         throw std::invalid_argument("counts must have shape (2,) and int32 dtype.");
     }
-    require_i32_vector(row_offsets, "row_offsets must be a one-dimensional int32 array.");
-    if (row_offsets.size(0) != out_capacity + 1) {
-        throw std::invalid_argument("row_offsets length must match out_capacity + 1.");
+    if (edges) {
+        require_i32_vector(row_offsets, "row_offsets must be a one-dimensional int32 array.");
+        if (row_offsets.size(0) != out_capacity + 1) {
+            throw std::invalid_argument("row_offsets length must match out_capacity + 1.");
+        }
     }
     const at::Tensor feats = feats_in.contiguous();
     const at::Tensor weights = weights_in.contiguous();
@@ -182,6 +191,7 @@ at::Tensor sparse_conv_features_csr(const at::Tensor& feats_in, const at::Tensor
             out.data_ptr(), b, relu ? LATTICE_EPILOGUE_RELU : LATTICE_EPILOGUE_NONE, current_stream(feats)));
         return out;
     }
+    require(edges, "the conv over the edges needs in_rows, kernel_ids and row_offsets.");
     check_status(lattice_hip_sparse_conv_features(
         dtype_code(feats, op), feats.data_ptr(), static_cast<int>(feats.size(0)), static_cast<int>(feats.size(1)),
         weights.data_ptr(), layout, n_kernels, static_cast<int>(c_out), ci32(in_rows), ci32(kernel_ids),
@@ -501,9 +511,11 @@ at::Tensor conv_tile_order(const at::Tensor& tile_masks, int out_capacity) {
 
 at::Tensor sparse_quantized_conv_features(const at::Tensor& feats_in, const at::Tensor& weights_in,
                                           const at::Tensor& scales_in, const at::Tensor& biases_in,
-                                          const at::Tensor& in_rows, const at::Tensor& out_rows,
-                                          const at::Tensor& kernel_ids, const at::Tensor& counts,
-                                          const at::Tensor& row_offsets, const at::Tensor& sorted_kv_out_in_map,
+                                          const std::optional<at::Tensor>& in_rows_in,
+                                          const std::optional<at::Tensor>& out_rows_in,
+                                          const std::optional<at::Tensor>& kernel_ids_in, const at::Tensor& counts,
+                                          const std::optional<at::Tensor>& row_offsets_in,
+                                          const at::Tensor& sorted_kv_out_in_map,
                                           const at::Tensor& reorder_rows, const at::Tensor& tile_masks,
                                           int out_capacity, int n_kernels, int in_channels, int out_channels,
                                           int storage_in_channels, int group_size, int bits,
@@ -553,16 +565,23 @@ at::Tensor sparse_quantized_conv_features(const at::Tensor& feats_in, const at::
             throw std::invalid_argument("quantized convolution sorted plan shapes are invalid.");
         }
     }
-    if (in_rows.dim() != 1 || out_rows.dim() != 1 || kernel_ids.dim() != 1 || in_rows.scalar_type() != at::kInt ||
+    const bool edges = in_rows_in.has_value() && out_rows_in.has_value() && kernel_ids_in.has_value() &&
+                       row_offsets_in.has_value();
+    const at::Tensor in_rows = edges ? *in_rows_in : at::Tensor();
+    const at::Tensor out_rows = edges ? *out_rows_in : at::Tensor();
+    const at::Tensor kernel_ids = edges ? *kernel_ids_in : at::Tensor();
+    const at::Tensor row_offsets = edges ? *row_offsets_in : at::Tensor();
+    if (edges && (in_rows.dim() != 1 || out_rows.dim() != 1 || kernel_ids.dim() != 1 || in_rows.scalar_type() != at::kInt ||
         out_rows.scalar_type() != at::kInt || kernel_ids.scalar_type() != at::kInt ||
-        in_rows.sizes() != out_rows.sizes() || in_rows.sizes() != kernel_ids.sizes()) {
+        in_rows.sizes() != out_rows.sizes() || in_rows.sizes() != kernel_ids.sizes())) {
         throw std::invalid_argument(
             "quantized convolution relation edges must be equal-length one-dimensional int32 arrays.");
     }
     if (counts.dim() != 1 || counts.size(0) != 2 || counts.scalar_type() != at::kInt) {
         throw std::invalid_argument("quantized convolution counts must have shape (2,) and int32 dtype.");
     }
-    if (row_offsets.dim() != 1 || row_offsets.size(0) != out_capacity + 1 || row_offsets.scalar_type() != at::kInt) {
+    if (edges && (row_offsets.dim() != 1 || row_offsets.size(0) != out_capacity + 1 ||
+                  row_offsets.scalar_type() != at::kInt)) {
         throw std::invalid_argument(
             "quantized convolution row_offsets must have length out_capacity + 1 and int32 dtype.");
     }
@@ -620,6 +639,7 @@ at::Tensor sparse_quantized_conv_features(const at::Tensor& feats_in, const at::
             relu ? LATTICE_EPILOGUE_RELU : LATTICE_EPILOGUE_NONE, schedule_ptr(ws), ws_bytes, current_stream(feats)));
         return out;
     }
+    require(edges, "the quantized conv needs the relation's edges for this route.");
     check_status(lattice_hip_sparse_quantized_conv_features(
         dtype_code(feats, "quantized sparse convolution"), feats.data_ptr(), static_cast<int>(feats.size(0)),
         in_channels, reinterpret_cast<const uint32_t*>(weights.data_ptr()), scales.data_ptr(), biases.data_ptr(),
@@ -747,34 +767,58 @@ at::Tensor sparse_conv_weight_grad(const at::Tensor& feats_in, const at::Tensor&
 }
 
 std::tuple<at::Tensor, std::optional<at::Tensor>, std::optional<at::Tensor>> build_kernel_pairs(
-    const at::Tensor& row_masks_in, const at::Tensor& row_offsets, const at::Tensor& in_rows, int n_kernels,
-    bool edge_ids) {
+    const at::Tensor& row_masks_in, const at::Tensor& out_in_map_in, const std::optional<at::Tensor>& row_offsets) {
     if (row_masks_in.dim() != 2 || row_masks_in.size(1) != 1 || row_masks_in.scalar_type() != at::kInt) {
         throw std::invalid_argument("row_masks must have shape (N_out, 1) and int32 dtype.");
     }
-    require_i32_vector(row_offsets, "row_offsets must be a one-dimensional int32 array.");
-    require_i32_vector(in_rows, "relation rows must be one-dimensional int32 arrays.");
+    if (out_in_map_in.dim() != 2 || out_in_map_in.scalar_type() != at::kInt ||
+        out_in_map_in.size(0) != row_masks_in.size(0)) {
+        throw std::invalid_argument("out_in_map must have shape (N_out, K) and int32 dtype.");
+    }
+    const int n_kernels = static_cast<int>(out_in_map_in.size(1));
     if (n_kernels <= 0 || n_kernels > 32) throw std::invalid_argument("kernel pairs need 1 to 32 offsets.");
-    if (row_offsets.size(0) != row_masks_in.size(0) + 1) {
-        throw std::invalid_argument("row_offsets length must match the masks' rows + 1.");
+    at::Tensor offsets;
+    if (row_offsets.has_value()) {
+        require_i32_vector(*row_offsets, "row_offsets must be a one-dimensional int32 array.");
+        if (row_offsets->size(0) != row_masks_in.size(0) + 1) {
+            throw std::invalid_argument("row_offsets length must match the masks' rows + 1.");
+        }
+        require_device(*row_offsets, "row_offsets");
+        offsets = row_offsets->contiguous();
     }
     require_device(row_masks_in, "row_masks");
-    require_device(row_offsets, "row_offsets");
-    require_device(in_rows, "in_rows");
+    require_device(out_in_map_in, "out_in_map");
     const at::Tensor masks = row_masks_in.contiguous();
-    const at::Tensor offsets = row_offsets.contiguous();
-    const at::Tensor in = in_rows.contiguous();
+    const at::Tensor map = out_in_map_in.contiguous();
     const int rows = static_cast<int>(masks.size(0));
-    const int edges = static_cast<int>(in.size(0));
-    at::Tensor groups = empty_i32({n_kernels + 1}, in);
+    if (map.numel() >= INT32_MAX) throw std::invalid_argument("kernel pairs need fewer than 2^31 map entries.");
+    const int edges = static_cast<int>(map.numel());
+    at::Tensor groups = empty_i32({n_kernels + 1}, map);
     std::optional<at::Tensor> pairs, ids;
-    if (edge_ids) ids = empty_i32({edges}, in);
-    else pairs = empty_i32({edges, 2}, in);
-    at::Tensor ws = workspace(lattice_hip_kernel_pairs_workspace_bytes(rows), in);
-    check_status(lattice_hip_build_kernel_pairs(ci32(masks), ci32(offsets), ci32(in), rows, n_kernels, edges,
-                                                i32(groups), pairs ? i32(*pairs) : nullptr, ids ? i32(*ids) : nullptr,
-                                                ws.data_ptr(), static_cast<size_t>(ws.numel()), current_stream(in)));
+    if (offsets.defined()) ids = empty_i32({edges}, map);
+    else pairs = empty_i32({edges, 2}, map);
+    at::Tensor ws = workspace(lattice_hip_kernel_pairs_workspace_bytes(rows), map);
+    check_status(lattice_hip_build_kernel_pairs(
+        ci32(masks), ci32(map), offsets.defined() ? ci32(offsets) : nullptr, rows, n_kernels, edges, i32(groups),
+        pairs ? i32(*pairs) : nullptr, ids ? i32(*ids) : nullptr, ws.data_ptr(), static_cast<size_t>(ws.numel()),
+        current_stream(map)));
     return {groups, pairs, ids};
+}
+
+std::tuple<at::Tensor, at::Tensor> build_transposed_map_from_dense(const at::Tensor& out_in_map_in, int in_capacity) {
+    if (out_in_map_in.dim() != 2 || out_in_map_in.scalar_type() != at::kInt || out_in_map_in.size(1) <= 0) {
+        throw std::invalid_argument("out_in_map must have shape (N_out, K) and int32 dtype.");
+    }
+    if (in_capacity < 0) throw std::invalid_argument("in_capacity must be nonnegative.");
+    require_device(out_in_map_in, "out_in_map");
+    const at::Tensor dense = out_in_map_in.contiguous();
+    const int n_kernels = static_cast<int>(dense.size(1));
+    at::Tensor map = empty_i32({in_capacity, n_kernels}, dense);
+    at::Tensor masks = empty_i32({in_capacity, (n_kernels + 31) / 32}, dense);
+    check_status(lattice_hip_build_transposed_map_from_dense(ci32(dense), static_cast<int>(dense.size(0)),
+                                                             in_capacity, n_kernels, i32(map), i32(masks), nullptr,
+                                                             current_stream(dense)));
+    return {map, masks};
 }
 
 at::Tensor sparse_conv_weight_grad_pairs(const at::Tensor& feats_in, const at::Tensor& cot_in,

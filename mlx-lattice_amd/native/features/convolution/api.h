@@ -20,10 +20,12 @@ at::Tensor sparse_conv_features(const at::Tensor& feats, const at::Tensor& weigh
 // The CSR conv without the grouped plan views the reference signature
 // carries for its gradient (the forward reads only the output CSR).  With
 // the relation's dense map (out_in_map, (out_capacity, n_kernels)) and a
-// shape the dense-map conv takes (C_in 4 or 8), it runs that instead.
-at::Tensor sparse_conv_features_csr(const at::Tensor& feats, const at::Tensor& weights, const at::Tensor& in_rows,
-                                    const at::Tensor& kernel_ids, const at::Tensor& counts,
-                                    const at::Tensor& row_offsets, int out_capacity, int n_kernels,
+// shape the dense-map conv takes (C_in 4 or 8), it runs that instead and
+// does not need the edges.
+at::Tensor sparse_conv_features_csr(const at::Tensor& feats, const at::Tensor& weights,
+                                    const std::optional<at::Tensor>& in_rows,
+                                    const std::optional<at::Tensor>& kernel_ids, const at::Tensor& counts,
+                                    const std::optional<at::Tensor>& row_offsets, int out_capacity, int n_kernels,
                                     const std::optional<at::Tensor>& bias = std::nullopt, bool relu = false,
                                     const std::optional<at::Tensor>& out_in_map = std::nullopt);
 
@@ -51,11 +53,12 @@ at::Tensor conv_weight_fragments(const at::Tensor& weights);
 
 // Edges of a dense-map relation grouped by offset without a sort
 // (lattice_hip_build_kernel_pairs): (kernel_row_offsets, pairs (E, 2) or
-// none, kernel_edge_ids (E,) or none), and the weight gradient over the
-// pairs.
+// none, kernel_edge_ids (E,) or none; the ids when row_offsets is given,
+// else the pairs), and the weight gradient over the pairs.
 std::tuple<at::Tensor, std::optional<at::Tensor>, std::optional<at::Tensor>> build_kernel_pairs(
-    const at::Tensor& row_masks, const at::Tensor& row_offsets, const at::Tensor& in_rows, int n_kernels,
-    bool edge_ids);
+    const at::Tensor& row_masks, const at::Tensor& out_in_map, const std::optional<at::Tensor>& row_offsets);
+// (in_out_map (in_capacity, K), row_masks) of a relation with a dense map.
+std::tuple<at::Tensor, at::Tensor> build_transposed_map_from_dense(const at::Tensor& out_in_map, int in_capacity);
 at::Tensor sparse_conv_weight_grad_pairs(const at::Tensor& feats, const at::Tensor& cotangent,
                                          const at::Tensor& weights, const at::Tensor& pairs,
                                          const at::Tensor& kernel_row_offsets, int n_kernels);
@@ -79,9 +82,11 @@ at::Tensor sparse_conv_features_padded(const at::Tensor& feats, const at::Tensor
 
 at::Tensor sparse_quantized_conv_features(const at::Tensor& feats, const at::Tensor& weights,
                                           const at::Tensor& scales, const at::Tensor& biases,
-                                          const at::Tensor& in_rows, const at::Tensor& out_rows,
-                                          const at::Tensor& kernel_ids, const at::Tensor& counts,
-                                          const at::Tensor& row_offsets, const at::Tensor& sorted_kv_out_in_map,
+                                          const std::optional<at::Tensor>& in_rows,
+                                          const std::optional<at::Tensor>& out_rows,
+                                          const std::optional<at::Tensor>& kernel_ids, const at::Tensor& counts,
+                                          const std::optional<at::Tensor>& row_offsets,
+                                          const at::Tensor& sorted_kv_out_in_map,
                                           const at::Tensor& reorder_rows, const at::Tensor& tile_masks,
                                           int out_capacity, int n_kernels, int in_channels, int out_channels,
                                           int storage_in_channels, int group_size, int bits,

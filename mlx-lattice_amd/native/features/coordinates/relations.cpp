@@ -44,13 +44,15 @@ void validate_nonnegative(const Triple& v, const char* name) {
 }
 
 NativeKernelRelation allocate(const at::Tensor& like, int out_capacity, int in_capacity, int K, bool coords,
-                              bool views) {
+                              bool views, bool with_edges) {
     const int64_t edges = static_cast<int64_t>(out_capacity) * K;
     NativeKernelRelation r;
-    r.in_rows = empty_i32({edges}, like);
-    r.out_rows = empty_i32({edges}, like);
-    r.kernel_ids = empty_i32({edges}, like);
-    r.output_row_offsets = empty_i32({out_capacity + 1}, like);
+    if (with_edges) {
+        r.in_rows = empty_i32({edges}, like);
+        r.out_rows = empty_i32({edges}, like);
+        r.kernel_ids = empty_i32({edges}, like);
+        r.output_row_offsets = empty_i32({out_capacity + 1}, like);
+    }
     if (coords) r.out_coords = empty_i32({out_capacity, 4}, like);
     r.counts = empty_i32({2}, like);
     if (views) {
@@ -66,10 +68,12 @@ NativeKernelRelation allocate(const at::Tensor& like, int out_capacity, int in_c
 
 lattice_relation_outputs outputs_of(NativeKernelRelation& r, at::Tensor& status) {
     lattice_relation_outputs o{};
-    o.in_rows = i32(r.in_rows);
-    o.out_rows = i32(r.out_rows);
-    o.kernel_ids = i32(r.kernel_ids);
-    o.row_offsets = i32(r.output_row_offsets);
+    if (r.in_rows.defined()) {
+        o.in_rows = i32(r.in_rows);
+        o.out_rows = i32(r.out_rows);
+        o.kernel_ids = i32(r.kernel_ids);
+        o.row_offsets = i32(r.output_row_offsets);
+    }
     o.out_coords = r.out_coords.defined() ? i32(r.out_coords) : nullptr;
     o.counts = i32(r.counts);
     const bool views = r.in_edge_ids.defined();
@@ -98,7 +102,7 @@ std::vector<Triple> kernel_offsets(Triple kernel_size, Triple dilation) {
 
 NativeKernelRelation make_kernel_relation(const at::Tensor& coords_in, const at::Tensor& active_rows,
                                           Triple kernel_size, Triple stride, Triple padding, Triple dilation,
-                                          bool with_views, const std::optional<at::Tensor>& table) {
+                                          bool with_views, const std::optional<at::Tensor>& table, bool edges) {
     validate_coords(coords_in);
     validate_active_rows(active_rows);
     validate_positive(kernel_size, "kernel_size");
@@ -109,7 +113,7 @@ NativeKernelRelation make_kernel_relation(const at::Tensor& coords_in, const at:
     const at::Tensor coords = coords_in.contiguous();
     const int rows = static_cast<int>(coords.size(0));
     const int K = kernel_size[0] * kernel_size[1] * kernel_size[2];
-    NativeKernelRelation r = allocate(coords, rows, rows, K, true, with_views);
+    NativeKernelRelation r = allocate(coords, rows, rows, K, true, with_views && edges, edges);
     at::Tensor status = empty_i32({1}, coords);
     lattice_relation_outputs o = outputs_of(r, status);
     // The block table lives in a buffer of its own, so a caller keeping it
@@ -124,7 +128,8 @@ NativeKernelRelation make_kernel_relation(const at::Tensor& coords_in, const at:
     at::Tensor ws = workspace(need, coords);
     size_t tb_bytes = static_cast<size_t>(tb.numel());
     if (reuse) tb_bytes |= LATTICE_RELATION_TABLE_READY;
-    check_status(lattice_hip_build_kernel_relation_with_table(
+    auto* build = edges ? lattice_hip_build_kernel_relation_with_table : lattice_hip_build_kernel_map_with_table;
+    check_status(build(
         ci32(coords), rows, ci32(active_rows), kernel_size.data(), stride.data(), padding.data(), dilation.data(),
         &o, tb.data_ptr(), tb_bytes, ws.data_ptr(), static_cast<size_t>(ws.numel()), current_stream(coords)));
     r.status = status;
@@ -133,14 +138,16 @@ NativeKernelRelation make_kernel_relation(const at::Tensor& coords_in, const at:
 }
 
 NativeKernelRelation make_submanifold_kernel_relation(const at::Tensor& coords, const at::Tensor& active_rows,
-                                                      Triple kernel_size, Triple dilation, bool with_views) {
-    return make_kernel_relation(coords, active_rows, kernel_size, {1, 1, 1}, {0, 0, 0}, dilation, with_views);
+                                                      Triple kernel_size, Triple dilation, bool with_views,
+                                                      bool edges) {
+    return make_kernel_relation(coords, active_rows, kernel_size, {1, 1, 1}, {0, 0, 0}, dilation, with_views,
+                                std::nullopt, edges);
 }
 
 NativeKernelRelation make_target_kernel_relation(const at::Tensor& coords_in, const at::Tensor& active_rows,
                                                  const at::Tensor& target_in, const at::Tensor& target_active_rows,
                                                  Triple kernel_size, Triple stride, Triple padding,
-                                                 Triple dilation, bool with_views) {
+                                                 Triple dilation, bool with_views, bool edges) {
     validate_coords(coords_in);
     validate_coords(target_in, "target_coords");
     validate_active_rows(active_rows);
@@ -158,13 +165,14 @@ NativeKernelRelation make_target_kernel_relation(const at::Tensor& coords_in, co
     const int rows = static_cast<int>(coords.size(0));
     const int target_rows = static_cast<int>(target.size(0));
     const int K = kernel_size[0] * kernel_size[1] * kernel_size[2];
-    NativeKernelRelation r = allocate(coords, target_rows, rows, K, false, with_views);
+    NativeKernelRelation r = allocate(coords, target_rows, rows, K, false, with_views && edges, edges);
     r.out_coords = target;
     at::Tensor status = empty_i32({1}, coords);
     lattice_relation_outputs o = outputs_of(r, status);
     o.out_coords = nullptr;
     at::Tensor ws = workspace(lattice_hip_target_relation_workspace_bytes(rows, target_rows, K), coords);
-    check_status(lattice_hip_build_target_kernel_relation(
+    auto* build = edges ? lattice_hip_build_target_kernel_relation : lattice_hip_build_target_kernel_map;
+    check_status(build(
         ci32(coords), rows, ci32(active_rows), ci32(target), target_rows, ci32(target_active_rows),
         kernel_size.data(), stride.data(), padding.data(), dilation.data(), &o, ws.data_ptr(),
         static_cast<size_t>(ws.numel()), current_stream(coords)));
@@ -235,6 +243,40 @@ NativeKernelRelation make_expanded_relation(const at::Tensor& coords_in, const a
     }
     r.status = status;
     return r;
+}
+
+std::tuple<at::Tensor, at::Tensor, at::Tensor, at::Tensor> make_map_edges(const at::Tensor& out_in_map,
+                                                                           const at::Tensor& row_masks,
+                                                                           at::Tensor counts) {
+    if (out_in_map.dim() != 2 || out_in_map.scalar_type() != at::kInt || !out_in_map.is_contiguous()) {
+        throw std::invalid_argument("out_in_map must be a contiguous (Nout, K) int32 array.");
+    }
+    const int64_t words = (out_in_map.size(1) + 31) / 32;
+    if (row_masks.dim() != 2 || row_masks.scalar_type() != at::kInt || !row_masks.is_contiguous() ||
+        row_masks.size(0) != out_in_map.size(0) || row_masks.size(1) != words) {
+        throw std::invalid_argument("row_masks must be contiguous with ceil(K / 32) words per out_in_map row.");
+    }
+    if (counts.dim() != 1 || counts.size(0) != 2 || counts.scalar_type() != at::kInt || !counts.is_contiguous()) {
+        throw std::invalid_argument("counts must have shape (2,) and int32 dtype.");
+    }
+    require_on_device({{&out_in_map, "out_in_map"}, {&row_masks, "row_masks"}, {&counts, "counts"}});
+    const int rows = static_cast<int>(out_in_map.size(0));
+    const int64_t edges = out_in_map.numel();
+    at::Tensor in_rows = empty_i32({edges}, out_in_map);
+    at::Tensor out_rows = empty_i32({edges}, out_in_map);
+    at::Tensor kernel_ids = empty_i32({edges}, out_in_map);
+    at::Tensor row_offsets = empty_i32({rows + 1}, out_in_map);
+    lattice_relation_outputs o{};
+    o.in_rows = i32(in_rows);
+    o.out_rows = i32(out_rows);
+    o.kernel_ids = i32(kernel_ids);
+    o.row_offsets = i32(row_offsets);
+    o.counts = i32(counts);
+    at::Tensor ws = workspace(lattice_hip_map_edges_workspace_bytes(rows), out_in_map);
+    check_status(lattice_hip_build_map_edges(ci32(out_in_map), ci32(row_masks), rows,
+                                             static_cast<int>(out_in_map.size(1)), &o, ws.data_ptr(),
+                                             static_cast<size_t>(ws.numel()), current_stream(out_in_map)));
+    return {in_rows, out_rows, kernel_ids, row_offsets};
 }
 
 std::tuple<at::Tensor, at::Tensor, at::Tensor, at::Tensor> make_relation_grouped_views(

@@ -41,28 +41,37 @@ std::vector<Triple> kernel_offsets(Triple kernel_size, Triple dilation);
 // Builds never read device memory back: every int32 coordinate is accepted.
 // with_views: also build the grouped CSR views (otherwise their tensors
 // stay undefined and make_relation_grouped_views builds them on demand).
+// edges (with with_views false): also build the edges and their row offsets
+// (otherwise undefined, and counts[0] unset, until make_map_edges).
 // table (optional): the `table` of an earlier build over the same coords
 // and active_rows; its block table is reused instead of rebuilt.
 NativeKernelRelation make_kernel_relation(const at::Tensor& coords, const at::Tensor& active_rows,
                                           Triple kernel_size, Triple stride, Triple padding, Triple dilation,
                                           bool with_views = true,
-                                          const std::optional<at::Tensor>& table = std::nullopt);
+                                          const std::optional<at::Tensor>& table = std::nullopt,
+                                          bool edges = true);
 
 NativeKernelRelation make_submanifold_kernel_relation(const at::Tensor& coords, const at::Tensor& active_rows,
                                                       Triple kernel_size, Triple dilation,
-                                                      bool with_views = true);
+                                                      bool with_views = true, bool edges = true);
 
 NativeKernelRelation make_target_kernel_relation(const at::Tensor& coords, const at::Tensor& active_rows,
                                                  const at::Tensor& target_coords,
                                                  const at::Tensor& target_active_rows, Triple kernel_size,
                                                  Triple stride, Triple padding, Triple dilation,
-                                                 bool with_views = true);
+                                                 bool with_views = true, bool edges = true);
 
 // Generative (generative = true; padding and dilation ignored) and
 // transposed relations: output and edge capacities rows * K, no dense view.
 NativeKernelRelation make_expanded_relation(const at::Tensor& coords, const at::Tensor& active_rows,
                                             Triple kernel_size, Triple stride, Triple padding, Triple dilation,
                                             bool generative, bool with_views = true);
+
+// (in_rows, out_rows, kernel_ids, row_offsets) of a build without edges, from
+// its map and masks; counts[0] is written too (lattice_hip_build_map_edges).
+std::tuple<at::Tensor, at::Tensor, at::Tensor, at::Tensor> make_map_edges(const at::Tensor& out_in_map,
+                                                                           const at::Tensor& row_masks,
+                                                                           at::Tensor counts);
 
 // (in_row_offsets, in_edge_ids, kernel_row_offsets, kernel_edge_ids)
 std::tuple<at::Tensor, at::Tensor, at::Tensor, at::Tensor> make_relation_grouped_views(
