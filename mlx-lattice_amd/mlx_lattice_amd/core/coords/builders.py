@@ -9,6 +9,7 @@ query produced) into a ``KernelRelation``.
 from __future__ import annotations
 
 from collections.abc import Sequence
+from functools import lru_cache
 
 import torch
 
@@ -37,6 +38,11 @@ def kernel_offsets(kernel_size: int | Sequence[int],
     rate = triple(dilation, name='dilation')
     _require_positive(kernel, 'kernel_size')
     _require_positive(rate, 'dilation')
+    return _footprint(kernel, rate)
+
+
+@lru_cache(maxsize=64)
+def _footprint(kernel: Triple, rate: Triple) -> tuple[Triple, ...]:
     axes = []
     for size in kernel:
         if size % 2 == 1:
@@ -296,7 +302,7 @@ def _map_only(wanted: bool, offsets: tuple[Triple, ...]) -> bool:
 
 
 def _require_positive(values: Triple, name: str) -> None:
-    if any(value <= 0 for value in values):
+    if min(values) <= 0:
         raise ValueError(f'{name} values must be positive.')
 
 

@@ -57,10 +57,10 @@ class KernelSpec:
 
 
 def _require_positive(values: Triple, name: str) -> None:
-    if any(value <= 0 for value in values):
+    if min(values) <= 0:
         raise ValueError(f'{name} values must be positive.')
 
 
 def _require_nonnegative(values: Triple, name: str) -> None:
-    if any(value < 0 for value in values):
+    if min(values) < 0:
         raise ValueError(f'{name} values must be non-negative.')

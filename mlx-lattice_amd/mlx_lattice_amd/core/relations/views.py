@@ -142,24 +142,23 @@ class _StatusWord:
     for there; read() waits only for the copy's event (usually long
     complete by the time a backward pass asks)."""
 
+    __slots__ = ('_word',)
+
     def __init__(self, word: torch.Tensor) -> None:
         if word.is_cuda:
-            self._host = torch.empty(1, dtype=torch.int32, pin_memory=True)
-            self._host.copy_(word, non_blocking=True)
-            self._event = torch.cuda.Event()
-            self._event.record()
+            from mlx_lattice_amd._native import ext
+
+            self._word = ext.StatusWord(word)
         else:
-            self._host = word.clone()
-            self._event = None
+            self._word = word.clone()
 
     def read(self) -> int:
         """The word's value.  Raises RuntimeError when the builder's
         coordinate table overflowed (lattice_relation_flags bit 16): the
         table is sized above its key count, so this marks a sizing error
         and the relation's contents are void."""
-        if self._event is not None:
-            self._event.synchronize()
-        value = int(self._host[0])
+        value = (int(self._word[0]) if isinstance(self._word, torch.Tensor)
+                 else self._word.read())
         if value & 16:
             raise RuntimeError('relation build: the coordinate table '
                                'overflowed (status word bit 16); the '
@@ -249,12 +248,10 @@ class SparseRelationContract:
             raise ValueError(
                 "relation kind must be 'forward', 'target', "
                 "'submanifold', 'transposed', or 'generative'.")
-        offsets = tuple((int(x), int(y), int(z))
-                        for x, y, z in self.kernel_offsets)
+        offsets = _int_offsets(self.kernel_offsets)
         object.__setattr__(self, 'kernel_offsets', offsets)
-        object.__setattr__(self, 'stride', tuple(int(v) for v in self.stride))
-        object.__setattr__(self, 'padding',
-                           tuple(int(v) for v in self.padding))
+        object.__setattr__(self, 'stride', tuple(map(int, self.stride)))
+        object.__setattr__(self, 'padding', tuple(map(int, self.padding)))
         n_in = _optional_count(self.n_in_capacity, 'n_in_capacity')
         n_out = _optional_count(self.n_out_capacity, 'n_out_capacity')
         n_kernels = _optional_count(self.n_kernels, 'n_kernels')
@@ -761,6 +758,24 @@ class KernelRelation:
 
 
 # ---------------------------------------------------------------- helpers --
+
+
+def _int_offsets(offsets) -> tuple[Triple, ...]:
+    """The offsets as a tuple of int triples."""
+    return (_int_offset_tuple(offsets) if type(offsets) is tuple
+            else tuple((int(x), int(y), int(z)) for x, y, z in offsets))
+
+
+def _int_offset_tuple(offsets: tuple) -> tuple[Triple, ...]:
+    for offset in offsets:
+        if type(offset) is not tuple or len(offset) != 3:
+            break
+        x, y, z = offset
+        if type(x) is not int or type(y) is not int or type(z) is not int:
+            break
+    else:
+        return offsets
+    return tuple((int(x), int(y), int(z)) for x, y, z in offsets)
 
 
 def _tiled_pays(rows: int, weight_bytes: int) -> bool:

@@ -8,6 +8,10 @@ Triple = tuple[int, int, int]
 def triple(value: int | Sequence[int], *, name: str) -> Triple:
     """Normalize an integer or 3-item sequence into a spatial triple
     (mlx_lattice/core/types.py:8-16)."""
+    if type(value) is tuple and len(value) == 3:
+        x, y, z = value
+        if type(x) is int and type(y) is int and type(z) is int:
+            return value
     if isinstance(value, int):
         return (value, value, value)
     values = tuple(int(item) for item in value)

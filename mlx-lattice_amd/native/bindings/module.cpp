@@ -4,6 +4,7 @@
 // (coords.cpp:79-92); the *_with_view variants append the implicit-GEMM view
 // (out_in_map, row_masks) computed by the same pass.
 
+#include <hip/hip_runtime_api.h>
 #include <torch/extension.h>
 
 #include <array>
@@ -42,10 +43,49 @@ py::tuple relation_tuple_with_view(const ln::NativeKernelRelation& r) {
                           r.table);
 }
 
+// A device status word on its way to pinned host memory: the copy is queued
+// on the current stream, read() waits for it alone.
+class StatusWord {
+  public:
+    explicit StatusWord(const at::Tensor& word) {
+        ln::require_device(word, "status word");
+        if (word.numel() != 1 || word.scalar_type() != at::kInt) {
+            throw std::invalid_argument("a status word must have one int32 value.");
+        }
+        const c10::DeviceGuard guard(word.device());
+        host_ = at::empty({1}, at::TensorOptions().dtype(at::kInt).pinned_memory(true));
+        host_.copy_(word.reshape({1}), /*non_blocking=*/true);
+        check(hipEventCreateWithFlags(&event_, hipEventDisableTiming));
+        const hipError_t rc = hipEventRecord(event_, static_cast<hipStream_t>(ln::current_stream(word)));
+        if (rc != hipSuccess) {
+            (void)hipEventDestroy(event_);
+            check(rc);
+        }
+    }
+    ~StatusWord() { (void)hipEventDestroy(event_); }
+    StatusWord(const StatusWord&) = delete;
+    StatusWord& operator=(const StatusWord&) = delete;
+    int read() const {
+        {
+            py::gil_scoped_release release;
+            check(hipEventSynchronize(event_));
+        }
+        return host_.data_ptr<int32_t>()[0];
+    }
+
+  private:
+    static void check(hipError_t rc) {
+        if (rc != hipSuccess) throw std::runtime_error(std::string("status word: ") + hipGetErrorString(rc));
+    }
+    at::Tensor host_;
+    hipEvent_t event_ = nullptr;
+};
+
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.doc() = "MI355X-native sparse convolution hot path (gfx950 HIP kernels behind a C ABI).";
+    py::class_<StatusWord>(m, "StatusWord").def(py::init<const at::Tensor&>()).def("read", &StatusWord::read);
     m.def("version", []() { return std::string(lattice_hip_version()); });
     m.def("coord_hash_capacity", [](int rows) { return lattice_hip_coord_hash_capacity(rows); }, py::arg("rows"));
     m.def(
