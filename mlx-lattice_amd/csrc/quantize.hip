@@ -203,14 +203,20 @@ voxelize_csr(int mode, const float* __restrict__ feats, int channels, const int3
         Vec<V> acc{};
         const int lo = offsets[v];
         const int hi = offsets[v + 1];
-        int i = lo;
-        for (; i + 1 < hi; i += 2) {  // two gathers in flight
-            const Vec<V> a = Vec<V>::load(feats + static_cast<long long>(point_ids[i]) * channels + c);
-            const Vec<V> b = Vec<V>::load(feats + static_cast<long long>(point_ids[i + 1]) * channels + c);
-            add_scaled(acc, a, scale);
-            add_scaled(acc, b, scale);
+        for (int i = lo; i < hi; i += 4) {  // four gathers in flight (126 -> 113 us), added in their order
+            int id[4];
+            Vec<V> x[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) id[j] = i + j < hi ? point_ids[i + j] : -1;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                x[j] = i + j < hi ? Vec<V>::load(feats + static_cast<long long>(id[j]) * channels + c) : Vec<V>{};
+            }
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                if (i + j < hi) add_scaled(acc, x[j], scale);
+            }
         }
-        if (i < hi) add_scaled(acc, Vec<V>::load(feats + static_cast<long long>(point_ids[i]) * channels + c), scale);
         acc.store(out + static_cast<long long>(v) * channels + c);
     }
 }
@@ -428,7 +434,26 @@ interpolate_grad(const float* __restrict__ point_grad, int channels, const float
         const int v = static_cast<int>(t / chunks);
         const int c = static_cast<int>(t - static_cast<long long>(v) * chunks) * V;
         Vec<V> acc{};
-        for (int i = offsets[v]; i < offsets[v + 1]; ++i) {
+        const int end = offsets[v + 1];
+        int i = offsets[v];
+        // four entries' loads in flight, added in their order (64 channels,
+        // 1,000,000 points on 400,000 voxels: 247 -> 227 us, bound by the 2 GB
+        // of point rows gathered through the Infinity Cache)
+        for (; i + 4 <= end; i += 4) {
+            int e[4];
+            float w[4];
+            Vec<V> x[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) e[j] = entries[i + j];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                w[j] = weights[e[j]];
+                x[j] = Vec<V>::load(point_grad + static_cast<long long>(e[j] >> 3) * channels + c);
+            }
+#pragma unroll
+            for (int j = 0; j < 4; ++j) add_scaled(acc, x[j], w[j]);
+        }
+        for (; i < end; ++i) {
             const int e = entries[i];
             add_scaled(acc, Vec<V>::load(point_grad + static_cast<long long>(e >> 3) * channels + c), weights[e]);
         }

@@ -1,7 +1,7 @@
 // Stable LSD radix sort of (key, index) pairs with digits of up to 11 bits
 // (reduce-then-scan): a key of b bits takes ceil(b / 11) passes of equal
 // digit width (27 bits: 3 x 9, 20 bits: 2 x 10).  Per digit pass:
-//   1. sort_count: each tile of 2048 items counts its digits in LDS, writes
+//   1. sort_count: each tile of 2048 to 8192 items counts its digits in LDS, writes
 //      them digit-major, count[d * tiles + tile], and adds them to the
 //      per-digit totals;
 //   2. sort_scan: the count matrix becomes the output offset of every
@@ -68,6 +68,7 @@ __device__ inline void load_item(const PassInput& in, int i, int valid_src, uint
 // 16-byte vectors; the block of the last tile zeroes the padding.
 __host__ __device__ inline int padded_tiles(int tiles) { return (tiles + 3) & ~3; }
 
+template <int ITEMS>
 __global__ void __launch_bounds__(kSortThreads)
 sort_count(PassInput in, int n, PassPlan plan, int tiles, uint32_t* __restrict__ counts,
            uint32_t* __restrict__ digit_totals) {
@@ -78,12 +79,12 @@ sort_count(PassInput in, int n, PassPlan plan, int tiles, uint32_t* __restrict__
     const int valid_src = valid_items(in, n);
     const uint32_t digit_mask = (1u << plan.bits) - 1u;
 #pragma unroll
-    for (int r = 0; r < kSortItems; ++r) {
-        const int i = blockIdx.x * kSortTile + r * kSortThreads + threadIdx.x;
+    for (int r = 0; r < ITEMS; ++r) {
+        const long long i = (static_cast<long long>(blockIdx.x) * ITEMS + r) * kSortThreads + threadIdx.x;
         if (i < n) {
             uint32_t key;
             int32_t index;
-            load_item(in, i, valid_src, key, index);
+            load_item(in, static_cast<int>(i), valid_src, key, index);
             atomicAdd(&hist[(key >> plan.shift) & digit_mask], 1u);
         }
     }
@@ -270,6 +271,125 @@ sort_scatter(PassInput in, int n, PassPlan plan, int tiles, const uint32_t* __re
     }
 }
 
+// The scatter of large sorts, tiles of ITEMS * 1024 items.  Two-item tiles
+// clear and scan 16 waves' counts of every digit for 2048 items and scatter
+// two items per 10-bit digit; here the tile is ordered by digit in LDS first,
+// so that neighbouring lanes store to neighbouring places, and the counts are
+// 16 bits wide (a tile has fewer items).  Ranks as above.
+template <int ITEMS, int ROWS>
+__global__ void __launch_bounds__(kSortThreads)
+sort_scatter_large(PassInput in, int n, PassPlan plan, int tiles, const uint32_t* __restrict__ offsets, bool final,
+                   uint32_t* __restrict__ keys_out, int32_t* __restrict__ idx_out, int32_t* __restrict__ final_keys) {
+    if (in.src.run_if != nullptr && *in.src.run_if == 0) return;
+    constexpr int kTile = ITEMS * kSortThreads;
+    constexpr int kPer = ROWS / kSortThreads;  // digits per thread
+    static_assert(kTile <= 65536 && ROWS % kSortThreads == 0, "16-bit places; whole digits per thread");
+    __shared__ uint16_t wave_run[kSortWaves][ROWS];
+    __shared__ uint32_t dest[ROWS];
+    __shared__ uint32_t stage_key[kTile];
+    __shared__ int32_t stage_idx[kTile];
+    __shared__ uint32_t wave_sum[kSortWaves];
+    const int t = threadIdx.x;
+    const int wave = t / kWave;
+    const int lane = lane_id();
+    const int tile = blockIdx.x;
+    const long long tile0 = static_cast<long long>(tile) * kTile;
+    uint32_t* zero = reinterpret_cast<uint32_t*>(&wave_run[0][0]);
+    for (int i = t; i < kSortWaves * ROWS / 2; i += kSortThreads) zero[i] = 0;
+    uint32_t base[kPer];
+#pragma unroll
+    for (int j = 0; j < kPer; ++j) {
+        const int d = t * kPer + j;
+        base[j] = d < plan.rows ? offsets[static_cast<long long>(d) * padded_tiles(tiles) + tile] : 0u;
+    }
+    const int valid_src = valid_items(in, n);
+    const uint32_t digit_mask = (1u << plan.bits) - 1u;
+    uint32_t key[ITEMS];
+    int32_t index[ITEMS];
+    uint32_t rank[ITEMS];
+    const long long base_item = tile0 + wave * (ITEMS * kWave) + lane;
+#pragma unroll
+    for (int r = 0; r < ITEMS; ++r) {
+        key[r] = 0;
+        index[r] = 0;
+        rank[r] = 0;
+        const long long i = base_item + r * kWave;
+        if (i < n) load_item(in, static_cast<int>(i), valid_src, key[r], index[r]);
+    }
+    __syncthreads();
+    uint16_t* run = wave_run[wave];
+#pragma unroll
+    for (int r = 0; r < ITEMS; ++r) {
+        const bool has = base_item + r * kWave < n;
+        const int digit = static_cast<int>((key[r] >> plan.shift) & digit_mask);
+        uint64_t peers = ballot(has);
+        for (int b = 0; b < plan.bits; ++b) {
+            const bool bit = has && ((digit >> b) & 1);
+            const uint64_t ones = ballot(bit);
+            peers &= bit ? ones : ~ones;
+        }
+        const uint64_t below = peers & ((1ull << lane) - 1ull);
+        if (has) rank[r] = run[digit] + static_cast<uint32_t>(__popcll(below));
+        if (has && below == 0) run[digit] = static_cast<uint16_t>(run[digit] + __popcll(peers));
+    }
+    __syncthreads();
+    // Places in the ordered tile: digits in order, within one the waves.
+    uint32_t sum[kPer];
+    uint32_t all = 0;
+#pragma unroll
+    for (int j = 0; j < kPer; ++j) {
+        sum[j] = 0;
+#pragma unroll
+        for (int w = 0; w < kSortWaves; ++w) sum[j] += wave_run[w][t * kPer + j];
+        all += sum[j];
+    }
+    const uint32_t incl = wave_inclusive_scan(all, lane);
+    if (lane == kWave - 1) wave_sum[wave] = incl;
+    __syncthreads();
+    uint32_t place = incl - all;
+    for (int w = 0; w < wave; ++w) place += wave_sum[w];
+#pragma unroll
+    for (int j = 0; j < kPer; ++j) {
+        const int d = t * kPer + j;
+        dest[d] = base[j] - place;
+#pragma unroll
+        for (int w = 0; w < kSortWaves; ++w) {
+            const uint32_t c = wave_run[w][d];
+            wave_run[w][d] = static_cast<uint16_t>(place);
+            place += c;
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < ITEMS; ++r) {
+        if (base_item + r * kWave >= n) continue;
+        const uint32_t at = run[(key[r] >> plan.shift) & digit_mask] + rank[r];
+        stage_key[at] = key[r];
+        stage_idx[at] = index[r];
+    }
+    __syncthreads();
+    const int count = static_cast<int>(min(static_cast<long long>(kTile), n - tile0));
+    for (int j = t; j < count; j += kSortThreads) {
+        const uint32_t k = stage_key[j];
+        const uint32_t pos = dest[(k >> plan.shift) & digit_mask] + static_cast<uint32_t>(j);
+        idx_out[pos] = stage_idx[j];
+        if (!final) {
+            keys_out[pos] = k;
+        } else if (final_keys != nullptr) {
+            final_keys[pos] = static_cast<int32_t>(in.src.flip_sign ? k ^ 0x80000000u : k);
+        }
+    }
+}
+
+// Tiles: 2048 items below kLargeSort (400,000 row masks give 196 of them),
+// 4096 from there and 8192 from kHugeSort, each size as soon as it leaves
+// half of the CUs or more a tile.  Two 10-bit passes over 8,000,000 keys took
+// 148 + 76 (scatter + count) us each in tiles of 2048, 75 + 42 in 4096 and
+// 80 + 32 in 8192; over 1,000,000 keys 28 + 17 in 2048 and 12 + 13 in 4096.
+constexpr int kLargeSort = 1 << 19;
+constexpr int kHugeSort = 1 << 21;
+int tile_items(int n) { return kSortTile * (n >= kHugeSort ? 4 : n >= kLargeSort ? 2 : 1); }
+
 int pass_count(int end_bit) { return (end_bit + kMaxRadixBits - 1) / kMaxRadixBits; }
 
 // Pass p of `passes` over end_bit bits: equal widths, the remainder spread
@@ -292,7 +412,10 @@ int count_rows(int end_bit) {
 
 size_t radix_sort_workspace_bytes(int n, int end_bit) {
     const size_t items = static_cast<size_t>(std::max(n, 1));
-    const size_t tiles = (items + kSortTile - 1) / kSortTile;
+    const size_t tile = static_cast<size_t>(tile_items(n));
+    // never less than a smaller sort needs
+    const int floor = n >= kHugeSort ? kHugeSort / (2 * kSortTile) : n >= kLargeSort ? kLargeSort / kSortTile : 1;
+    const size_t tiles = std::max((items + tile - 1) / tile, static_cast<size_t>(floor));
     size_t bytes = 4 * aligned_bytes(items * sizeof(uint32_t));  // two (key, index) buffers
     bytes += aligned_bytes(static_cast<size_t>(padded_tiles(static_cast<int>(tiles))) * count_rows(end_bit) *
                            sizeof(uint32_t));  // digit x tile counts
@@ -305,7 +428,7 @@ int radix_sort_indices(const SortKeys& keys, int n, int end_bit, int32_t* sorted
     LATTICE_REQUIRE(end_bit >= 1 && end_bit <= 32, "radix sort end_bit must be in [1, 32].");
     if (n <= 0) return LATTICE_OK;
     const int passes = pass_count(end_bit);
-    const int tiles = (n + kSortTile - 1) / kSortTile;
+    const int tiles = static_cast<int>((static_cast<long long>(n) + tile_items(n) - 1) / tile_items(n));
     uint32_t* key_buf[2] = {ws.take<uint32_t>(n), ws.take<uint32_t>(n)};
     int32_t* idx_buf[2] = {ws.take<int32_t>(n), ws.take<int32_t>(n)};
     uint32_t* counts = ws.take<uint32_t>(static_cast<size_t>(padded_tiles(tiles)) * count_rows(end_bit));
@@ -321,14 +444,22 @@ int radix_sort_indices(const SortKeys& keys, int n, int end_bit, int32_t* sorted
         const int out = p % 2;
         const PassInput input{keys, p == 0 ? nullptr : key_buf[in], p == 0 ? nullptr : idx_buf[in], p == 0};
         uint32_t* pass_totals = totals + static_cast<size_t>(p) * kDigits;
-        sort_count<<<tiles, kSortThreads, 0, stream>>>(input, n, plan, tiles, counts, pass_totals);
+        auto* count = n >= kHugeSort    ? sort_count<4 * kSortItems>
+                      : n >= kLargeSort ? sort_count<2 * kSortItems>
+                                        : sort_count<kSortItems>;
+        count<<<tiles, kSortThreads, 0, stream>>>(input, n, plan, tiles, counts, pass_totals);
         LATTICE_LAUNCH_CHECK();
         sort_scan<<<plan.rows / kScanRows, kScanBlockThreads, 0, stream>>>(counts, pass_totals, tiles, keys.run_if);
         LATTICE_LAUNCH_CHECK();
-        sort_scatter<<<tiles, kSortThreads, 0, stream>>>(input, n, plan, tiles, counts, final,
-                                                          final ? nullptr : key_buf[out],
-                                                          final ? sorted_index : idx_buf[out],
-                                                          final ? sorted_keys : nullptr);
+        const bool narrow = plan.rows <= 1024;
+        auto* scatter = n < kLargeSort ? sort_scatter
+                        : n < kHugeSort
+                            ? narrow ? sort_scatter_large<2 * kSortItems, 1024> : sort_scatter_large<2 * kSortItems, 2048>
+                            : narrow ? sort_scatter_large<4 * kSortItems, 1024> : sort_scatter_large<4 * kSortItems, 2048>;
+        scatter<<<tiles, kSortThreads, 0, stream>>>(input, n, plan, tiles, counts, final,
+                                                    final ? nullptr : key_buf[out],
+                                                    final ? sorted_index : idx_buf[out],
+                                                    final ? sorted_keys : nullptr);
         LATTICE_LAUNCH_CHECK();
     }
     return LATTICE_OK;
