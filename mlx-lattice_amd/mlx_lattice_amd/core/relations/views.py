@@ -138,25 +138,41 @@ class RelationSortedImplicitGemmView:
 
 class _StatusWord:
     """A device status word copied to pinned host memory when the relation
-    is built: the copy is queued on the current stream and never waited
-    for there; read() waits only for the copy's event (usually long
-    complete by the time a backward pass asks)."""
+    is built, or by queue() (``deferred``) once something is known to ask
+    for it: the copy is queued on the current stream and never waited for
+    there; read() waits only for the copy's event (usually long complete by
+    the time a backward pass asks)."""
 
-    __slots__ = ('_word',)
+    __slots__ = ('_device', '_word')
 
-    def __init__(self, word: torch.Tensor) -> None:
-        if word.is_cuda:
+    def __init__(self, word: torch.Tensor, deferred: bool = False) -> None:
+        self._device = word
+        self._word = None
+        if not deferred:
+            self.queue()
+
+    @property
+    def unreadable(self) -> bool:
+        """Not queued, and under a graph capture, where nothing can be read."""
+        return (self._word is None and self._device.is_cuda
+                and torch.cuda.is_current_stream_capturing())
+
+    def queue(self) -> None:
+        if self._word is not None:
+            return
+        if self._device.is_cuda:
             from mlx_lattice_amd._native import ext
 
-            self._word = ext.StatusWord(word)
+            self._word = ext.StatusWord(self._device)
         else:
-            self._word = word.clone()
+            self._word = self._device.clone()
 
     def read(self) -> int:
         """The word's value.  Raises RuntimeError when the builder's
         coordinate table overflowed (lattice_relation_flags bit 16): the
         table is sized above its key count, so this marks a sizing error
         and the relation's contents are void."""
+        self.queue()
         value = (int(self._word[0]) if isinstance(self._word, torch.Tensor)
                  else self._word.read())
         if value & 16:
@@ -314,8 +330,9 @@ class KernelRelation:
     # Submanifold relations: whether an active row repeats an earlier row's
     # coordinate (each copy is an output row with the same neighbours, so
     # an input row can have several output rows at one offset).  Held as a
-    # _StatusWord copied to pinned memory at build time and read on the
-    # first question (transposed_map_exact).  None: no repeats possible.
+    # _StatusWord copied to pinned memory when a conv that needs gradients
+    # runs (expect_backward) and read on the first question
+    # (transposed_map_exact).  None: no repeats possible.
     repeated_coords: bool | _StatusWord | None = None
     # Submanifold relations built with their workspace: it starts with the
     # block table of the coordinates (the coordinate manager hands it to
@@ -446,8 +463,8 @@ class KernelRelation:
             if isinstance(repeated_edges, torch.Tensor) else repeated_edges)
         object.__setattr__(
             self, 'repeated_coords',
-            _StatusWord(repeated_coords) if repeated_coords is not None
-            else None)
+            _StatusWord(repeated_coords, deferred=True)
+            if repeated_coords is not None else None)
         object.__setattr__(self, 'block_table', block_table)
         object.__setattr__(self, 'direct_expansion', bool(direct_expansion))
 
@@ -632,14 +649,23 @@ class KernelRelation:
         output coordinates are distinct, or each output row has one edge); a
         submanifold relation does unless a coordinate repeats.  The first
         question reads the build's status word from pinned memory (copied
-        when the relation was built), so it waits for that copy only."""
+        when a forward that needs gradients ran), so it waits for that copy
+        only; under graph capture an unread word counts as a repeat."""
         if self._contract.kind == 'target':
             return False
         if isinstance(self.repeated_coords, _StatusWord):
+            if self.repeated_coords.unreadable:
+                return False
             # lattice_relation_flags: bit 8 = repeated coordinate
             flags = self.repeated_coords.read()
             object.__setattr__(self, 'repeated_coords', bool(flags & 8))
         return not self.repeated_coords
+
+    def expect_backward(self) -> None:
+        """Queue the copy that ``transposed_map_exact`` reads."""
+        if (isinstance(self.repeated_coords, _StatusWord)
+                and not self.repeated_coords.unreadable):
+            self.repeated_coords.queue()
 
     def _expanded_implicit_gemm(self) -> RelationImplicitGemmView:
         """Dense map of a generative or transposed relation, scattered from

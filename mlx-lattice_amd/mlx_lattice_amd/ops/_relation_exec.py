@@ -191,6 +191,7 @@ class _SparseConvFeatures(torch.autograd.Function):
     @staticmethod
     def forward(ctx, feats, weight, relation):
         ctx.relation = relation
+        relation.expect_backward()
         ctx.save_for_backward(feats, weight)
         return _conv_features(feats, weight, relation)
 

@@ -105,3 +105,48 @@ def test_edges_used_on_another_stream_and_under_capture():
     torch.cuda.synchronize()
     assert torch.equal(first, full.edges.in_rows[:e])
     assert torch.equal(second, full.edges.out_rows[:e])
+
+
+@pytest.mark.parametrize('repeat', [False, True])
+def test_repeat_flag_is_read_after_a_forward_without_gradients(repeat):
+    """The status word of a submanifold relation is copied when something
+    asks for it; a relation first used without gradients, then with them,
+    and under capture before any copy, takes a route that holds every edge."""
+    from mlx_lattice_amd import SparseTensor, ops
+
+    c = _coords(3000, 11)
+    if repeat:
+        c[17] = c[5]
+    rng = np.random.default_rng(4)
+    f = torch.as_tensor(rng.standard_normal((3000, 32)).astype(np.float32))
+    w = torch.as_tensor((rng.standard_normal((32, 3, 3, 3, 32)) / 17).astype(
+        np.float32)).to(DEV)
+    g = torch.as_tensor(rng.standard_normal((3000, 32)).astype(
+        np.float32)).to(DEV)
+
+    def grad(x, feats):
+        y = ops.subm_conv3d(x.replace(feats=feats), w)
+        return torch.autograd.grad(y.feats, feats, g)[0]
+
+    feats = f.to(DEV).requires_grad_()
+    want = grad(SparseTensor(c, f.to(DEV)), feats)
+    x = SparseTensor(c, f.to(DEV))
+    ops.subm_conv3d(x, w)                       # no gradient: no copy yet
+    relation = x.coord_manager.submanifold_kernel_relation(x.coord_key)
+    assert relation.repeated_coords.unreadable is False
+    torch.cuda.synchronize()
+    side = torch.cuda.Stream()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        captured = grad(x, feats)
+    for _ in range(3):
+        graph.replay()
+        torch.cuda.synchronize()
+        # fp32 sums of up to 27 * 32 products in another order
+        assert torch.allclose(captured, want, rtol=1e-5, atol=1e-4)
+    fresh = SparseTensor(c, f.to(DEV))
+    ops.subm_conv3d(fresh, w)
+    assert torch.equal(grad(fresh, feats), want)
+    relation = fresh.coord_manager.submanifold_kernel_relation(
+        fresh.coord_key)
+    assert relation.transposed_map_exact is not repeat
