@@ -184,9 +184,10 @@ def _add_bias(feats: torch.Tensor, bias: torch.Tensor) -> torch.Tensor:
 
 
 class _SparseConvFeatures(torch.autograd.Function):
-    """Sparse conv features with the reference's gradients: the input
-    gradient over the input-grouped CSR and the weight gradient over the
-    kernel-grouped CSR (cpu/algorithms.cpp:355-481)."""
+    """Sparse conv features with the reference's gradients
+    (cpu/algorithms.cpp:355-481): the input gradient over the transposed or
+    mirrored relation or the input-grouped CSR, the weight gradient over the
+    edges grouped by offset."""
 
     @staticmethod
     def forward(ctx, feats, weight, relation):
