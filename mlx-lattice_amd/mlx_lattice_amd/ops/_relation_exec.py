@@ -108,6 +108,20 @@ def _padded_forward(feats: torch.Tensor, c_in: int, c_out: int,
     return _padded_eligible(feats, c_out, relation, relation.n_out_capacity)
 
 
+def _weight_fits(weight: torch.Tensor, dtype: torch.dtype, c_in: int,
+                 c_out: int, relation: KernelRelation) -> bool:
+    """Whether the weight is that of a conv of these channels over the
+    relation.  The padded conv takes the weight as fragments, whose size does
+    not tell: any other weight goes to the entry that says what is wrong."""
+    if weight.ndim not in (3, 5) or weight.dtype != dtype:
+        return False
+    shape = tuple(weight.shape)
+    if weight.ndim == 3:
+        return shape == (relation.n_kernels, c_in, c_out)
+    return (shape[0] == c_out and shape[4] == c_in
+            and shape[1] * shape[2] * shape[3] == relation.n_kernels)
+
+
 def _offset_bytes(weight: torch.Tensor) -> int:
     """Bytes of the weight of one offset."""
     c_in = weight.shape[1] if weight.ndim == 3 else weight.shape[4]
@@ -298,7 +312,10 @@ def sparse_conv_input_grad_from_relation(cot: torch.Tensor,
             in_capacity, relation.n_kernels, tile_order=view.tile_order(),
             weight_fragments=_weight_fragments(transposed))
     c_in = int(weight.shape[1] if weight.ndim == 3 else weight.shape[4])
-    if (relation.kind != 'target' and relation.transposed_map_exact
+    if (relation.kind != 'target'
+            and _weight_fits(weight, cot.dtype, c_in, int(cot.shape[1]),
+                             relation)
+            and relation.transposed_map_exact
             and _padded_eligible(cot, c_in, relation, in_capacity)):
         mirrored = _mirror_symmetric(relation)
         size = _offset_bytes(weight)
@@ -356,10 +373,10 @@ def _conv_features(feats: torch.Tensor, weight: torch.Tensor,
                                                          relu=relu)
     dense = (_small_dense_map(feats.dtype, int(feats.shape[1]), c_out,
                               relation) if feats.ndim == 2 else None)
-    c_in = int(weight.shape[1] if weight.ndim == 3 else weight.shape[4])
-    if (dense is None and feats.ndim == 2 and c_in == int(feats.shape[1])
-            and feats.dtype == weight.dtype
-            and _padded_forward(feats, c_in, c_out, relation)):
+    if (dense is None and feats.ndim == 2
+            and _weight_fits(weight, feats.dtype, int(feats.shape[1]), c_out,
+                             relation)
+            and _padded_forward(feats, int(feats.shape[1]), c_out, relation)):
         return _padded_conv(feats, _padded_fragments(weight, _FORWARD), 0,
                             c_out, relation.conv_view(_offset_bytes(weight)),
                             relation.n_out_capacity, relation, bias, relu)
