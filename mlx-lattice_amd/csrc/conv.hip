@@ -1529,13 +1529,17 @@ __device__ inline void stream_store_padded(const float4_t (&acc)[RB][CB], T* sta
 // CSR kernels, whose lanes load both factors of every product: 96 -> 96 bf16
 // over 150,001 rows (4.6 edges each) 19,300 -> 43 us; 64 -> 64 float32 over
 // 60,001 rows 3,000 -> 46 us, its input gradient 629 -> 46 us.
-template <typename T, typename S, int NCH, int QB, bool PAD = false>
+// SPLIT (PAD, packed weights): the weight contracted unrounded, as two
+// fragments, as the edge kernel contracts it; without it rounded once, as in
+// the instances that fill their tiles.
+template <typename T, typename S, int NCH, int QB, bool PAD = false, bool SPLIT = false>
 __global__ void __launch_bounds__(S::THREADS, S::OCC)
 conv_igemm_stream(const T* __restrict__ feats, int n_in, int c_in, const T* __restrict__ wfrag, int kernel_count,
                   int c_out_total, const int32_t* __restrict__ kv_map, const int32_t* __restrict__ tile_masks,
                   const int32_t* __restrict__ reorder_rows, int rows, const int32_t* __restrict__ block_order,
                   T* __restrict__ out, Epilogue<T> epi, int halves) {
     static_assert(!PAD || NCH == 1, "padded chunks are stages of their own");
+    static_assert(!SPLIT || (PAD && QB != 0), "only padded packed weights are split");
     using V = typename MfmaOps<T>::vec;
     constexpr int RB = S::RB;
     constexpr int CB = S::CB;
@@ -1744,7 +1748,6 @@ conv_igemm_stream(const T* __restrict__ feats, int n_in, int c_in, const T* __re
                 idx_expand(d, ra);
             }
             wait_vm_b<W_B>(bcur);
-            constexpr bool SPLIT = PAD && QB != 0;
             V blo[SPLIT ? CB : 1][SPLIT ? ST : 1];
             if constexpr (SPLIT) {
 #pragma unroll
@@ -2362,14 +2365,14 @@ size_t padded_fragments_bytes(int dtype, int K, int c_in, int c_out) {
     return static_cast<size_t>(K) * ((c_in + step - 1) / step) * ((c_out + 31) / 32) * 2048;
 }
 
-template <typename T, typename S, int QB>
+template <typename T, typename S, int QB, bool SPLIT>
 void launch_padded_shape(const T* feats, int n_in, int c_in, const T* frag, int K, int c_out, const int32_t* kv_map,
                          const int32_t* tile_masks, const int32_t* reorder_rows, int rows, const int32_t* order,
                          T* out, Epilogue<T> epi, hipStream_t stream) {
     // an order's 128-row tiles are two 64-row or four 32-row ones
     const int tiles = (rows + kOrderTileRows - 1) / kOrderTileRows * (kOrderTileRows / S::ROWS);
     const int columns = (c_out + S::C_OUT - 1) / S::C_OUT;
-    conv_igemm_stream<T, S, 1, QB, true><<<static_cast<unsigned>(tiles) * columns, S::THREADS, 0, stream>>>(
+    conv_igemm_stream<T, S, 1, QB, true, SPLIT><<<static_cast<unsigned>(tiles) * columns, S::THREADS, 0, stream>>>(
         feats, n_in, c_in, frag, K, c_out, kv_map, tile_masks, reorder_rows, rows, order, out, epi, columns);
 }
 
@@ -2385,7 +2388,7 @@ bool few_rows(int rows, int c_out) {
     return rows * columns * columns <= kFewRows;
 }
 
-template <typename T, int QB = 0>
+template <typename T, int QB, bool SPLIT>
 int launch_padded(const T* feats, int n_in, int c_in, const T* frag, int K, int c_out, const int32_t* kv_map,
                   const int32_t* tile_masks, const int32_t* reorder_rows, int rows, int32_t* schedule, bool ready,
                   T* out, Epilogue<T> epi, hipStream_t stream) {
@@ -2397,8 +2400,8 @@ int launch_padded(const T* feats, int n_in, int c_in, const T* frag, int K, int 
         LATTICE_LAUNCH_CHECK();
     }
 #define LATTICE_PADDED(C, WR, ROWS)                                                                                \
-    launch_padded_shape<T, StreamShape<T, C, WR, ROWS>, QB>(feats, n_in, c_in, frag, K, c_out, kv_map, tile_masks, \
-                                                            reorder_rows, rows, schedule, out, epi, stream)
+    launch_padded_shape<T, StreamShape<T, C, WR, ROWS>, QB, SPLIT>(                                                \
+        feats, n_in, c_in, frag, K, c_out, kv_map, tile_masks, reorder_rows, rows, schedule, out, epi, stream)
     // Tile rows.  float32 is bound by its MFMAs: 32-row tiles (no more
     // gathers, a shorter longest tile) measured fastest at every size for
     // more than 32 columns (64 -> 64 over 60,001 / 128,000 rows 53 -> 46 /
@@ -2406,8 +2409,8 @@ int launch_padded(const T* feats, int n_in, int c_in, const T* frag, int K, int 
     // us), and 64 rows below (32 -> 32 at 128,000 rows 49 against 62 us).
     // 16 bits: 64 rows for few rows, and for one column tile of more than
     // 64 (96 -> 96 over 150,001 / 128,000 rows 48 -> 43 / 75 -> 73 us).
-    // Packed weights hold two fragments a piece, for which 128 rows and 128
-    // columns have no registers left: 64 rows.
+    // Split packed weights hold two fragments a piece, for which 128 rows and
+    // 128 columns have no registers left: 64 rows.
     if constexpr (sizeof(T) == 4) {
         if (c_out <= 32) {
             LATTICE_PADDED(32, 4, 64);
@@ -2416,7 +2419,7 @@ int launch_padded(const T* feats, int n_in, int c_in, const T* frag, int K, int 
         } else {
             LATTICE_PADDED(128, 1, 32);
         }
-    } else if (QB != 0 || few_rows(rows, c_out) || (c_out > 64 && c_out <= 128)) {
+    } else if (QB != 0 || few_rows(rows, c_out) || (c_out > 64 && c_out <= 128)) {  // (packed: split or few)
         if (c_out <= 32) {
             LATTICE_PADDED(32, 4, 64);
         } else if (c_out <= 64) {
@@ -2443,10 +2446,11 @@ int launch_stream(const T* feats, int n_in, int c_in, const T* frag, int K, int 
                   const int32_t* tile_masks, const int32_t* reorder_rows, int rows, int32_t* schedule, bool ready,
                   T* out, Epilogue<T> epi, hipStream_t stream) {
     if (rows <= 0) return LATTICE_OK;
-    // These shapes' fragments are the padded ones, with nothing to pad.
+    // These shapes' fragments are the padded ones, with nothing to pad; the
+    // smaller tiles change no result (the weight's rounding included).
     if (few_rows(rows, c_out)) {
-        return launch_padded<T, QB>(feats, n_in, c_in, frag, K, c_out, kv_map, tile_masks, reorder_rows, rows, schedule,
-                                    ready, out, epi, stream);
+        return launch_padded<T, QB, false>(feats, n_in, c_in, frag, K, c_out, kv_map, tile_masks, reorder_rows, rows,
+                                           schedule, ready, out, epi, stream);
     }
     const int tiles = (rows + kOrderTileRows - 1) / kOrderTileRows;
     if (tiles > kMaxScheduledTiles) schedule = nullptr;
@@ -2794,9 +2798,10 @@ extern "C" int lattice_hip_sparse_conv_features_padded(
     if (rc != LATTICE_OK) return rc;
     hipStream_t stream = as_stream(stream_ptr);
 #define LATTICE_PADDED_CALL(T, QB)                                                                                  \
-    launch_padded<T, QB>(static_cast<const T*>(feats), n_in, c_in, static_cast<const T*>(fragments), kernel_count,  \
-                         c_out, sorted_kv_out_in_map, tile_masks, reorder_rows, out_capacity, schedule, ready,     \
-                         static_cast<T*>(out), epilogue_of<T>(bias, epilogue), stream)
+    launch_padded<T, QB, QB != 0>(static_cast<const T*>(feats), n_in, c_in, static_cast<const T*>(fragments),       \
+                                  kernel_count, c_out, sorted_kv_out_in_map, tile_masks, reorder_rows,             \
+                                  out_capacity, schedule, ready, static_cast<T*>(out),                             \
+                                  epilogue_of<T>(bias, epilogue), stream)
     if (dtype == LATTICE_F32) return LATTICE_PADDED_CALL(float, 0);
     if (dtype == LATTICE_F16) {
         if (bits == 0) return LATTICE_PADDED_CALL(_Float16, 0);
