@@ -1281,7 +1281,7 @@ weight_fragments(const T* __restrict__ w, int K, int c_in, int c_out, T* __restr
 // ci = ks*STEP + lg*PE) in (k, ks, cg, cb) order, zeros past C_out and C_in.
 // role (LATTICE_FRAGMENTS_*): the weight itself, or that of the input
 // gradient: its channels swapped, and for a submanifold relation its offsets
-// reversed too.  One launch per weight version; bound by its own size.
+// reversed too.  One launch per conv; bound by its own size.
 template <typename T>
 __global__ void __launch_bounds__(256)
 padded_weight_fragments(const T* __restrict__ w, WeightIndex widx, int role, int c_in, int c_out,

@@ -129,19 +129,14 @@ def _offset_bytes(weight: torch.Tensor) -> int:
     return int(c_in) * int(c_out) * weight.element_size()
 
 
-def _padded_fragments(weight: torch.Tensor, role: int) -> torch.Tensor:
-    """The padded conv's fragment-ordered copy of a float weight, or of its
-    input gradient's weight, cached with the weight."""
-    return _cached_weight(weight, ('padded', role),
-                          lambda w: ext.conv_padded_fragments(w, role))
-
-
-def _padded_conv(feats, fragments, bits, c_out, view, rows, relation,
-                 bias=None, relu=False) -> torch.Tensor:
-    return ext.sparse_conv_features_padded(
-        feats, fragments, bits, c_out, view.sorted_kv_out_in_map,
-        view.reorder_rows, view.tile_masks, rows, relation.n_kernels,
-        bias=bias, tile_order=view.tile_order(), relu=relu)
+def _padded_conv(feats, weight, role, view, rows, relation, bias=None,
+                 relu=False) -> torch.Tensor:
+    """The padded conv over ``weight`` as it is now, or (``role``) over its
+    input gradient's weight: the kernel's order of it is made in the call."""
+    return ext.sparse_conv_padded(
+        feats, weight, role, view.sorted_kv_out_in_map, view.reorder_rows,
+        view.tile_masks, rows, relation.n_kernels, bias=bias,
+        tile_order=view.tile_order(), relu=relu)
 
 
 _EXPAND_CHANNELS = (32, 64, 128, 256)
@@ -321,10 +316,9 @@ def sparse_conv_input_grad_from_relation(cot: torch.Tensor,
         size = _offset_bytes(weight)
         view = (relation.conv_view(size) if mirrored
                 else relation.transposed_conv_view(size))
-        fragments = _padded_fragments(weight,
-                                      _MIRRORED if mirrored else _TRANSPOSED)
-        return _padded_conv(cot, fragments, 0, c_in, view, in_capacity,
-                            relation)
+        return _padded_conv(cot, weight,
+                            _MIRRORED if mirrored else _TRANSPOSED, view,
+                            in_capacity, relation)
     input_csr = relation.input_csr
     return ext.sparse_conv_input_grad(
         cot, weight, relation.edges.out_rows, relation.edges.kernel_ids,
@@ -377,8 +371,8 @@ def _conv_features(feats: torch.Tensor, weight: torch.Tensor,
             and _weight_fits(weight, feats.dtype, int(feats.shape[1]), c_out,
                              relation)
             and _padded_forward(feats, int(feats.shape[1]), c_out, relation)):
-        return _padded_conv(feats, _padded_fragments(weight, _FORWARD), 0,
-                            c_out, relation.conv_view(_offset_bytes(weight)),
+        return _padded_conv(feats, weight, _FORWARD,
+                            relation.conv_view(_offset_bytes(weight)),
                             relation.n_out_capacity, relation, bias, relu)
     if _dense_without_edges(feats, dense):
         in_rows = kernel_ids = row_offsets = None
@@ -459,11 +453,15 @@ def sparse_quantized_conv_features_from_relation(
                 and feats.dtype == weight.scales.dtype
                 and _padded_forward(feats, weight.in_channels,
                                     weight.out_channels, relation)):
-            return _padded_conv(
-                feats, _quantized_fragments(weight, padded=True), weight.bits,
-                weight.out_channels, relation.conv_view(
-                    weight.in_channels * weight.out_channels * 2),
-                relation.n_out_capacity, relation, bias, relu)
+            view = relation.conv_view(
+                weight.in_channels * weight.out_channels * 2)
+            return ext.sparse_quantized_conv_padded(
+                feats, weight.weight, weight.scales, weight.biases,
+                weight.in_channels, weight.out_channels,
+                weight.storage_in_channels, weight.group_size, weight.bits,
+                view.sorted_kv_out_in_map, view.reorder_rows, view.tile_masks,
+                relation.n_out_capacity, relation.n_kernels, bias=bias,
+                tile_order=view.tile_order(), relu=relu)
         mapped = _dense_without_edges(feats, dense)
     if mapped:
         in_rows = out_rows = kernel_ids = row_offsets = None
@@ -572,21 +570,17 @@ def _weight_fragments(weight5d: torch.Tensor) -> torch.Tensor:
     return _cached_weight(weight5d, 'fragments', ext.conv_weight_fragments)
 
 
-def _quantized_fragments(weight: QuantizedWeight,
-                         padded: bool = False) -> torch.Tensor:
+def _quantized_fragments(weight: QuantizedWeight) -> torch.Tensor:
     """The streamed matrix-core conv's fragment-ordered packed copy of a
     quantized weight (``ext.quantized_weight_fragments``: codes, scale and
     bias per 16-byte piece, dequantised in the kernel; empty when the shape
     takes the other matrix-core kernel), cached with the packed words and
     rebuilt when they, the scales or the biases change."""
-    kind = ('padded quantized fragments' if padded else 'quantized fragments',
-            id(weight.scales), weight.scales._version,
+    kind = ('quantized fragments', id(weight.scales), weight.scales._version,
             id(weight.biases), weight.biases._version)
-    fragments = (ext.quantized_padded_fragments if padded
-                 else ext.quantized_weight_fragments)
 
     def make(words):
-        return fragments(
+        return ext.quantized_weight_fragments(
             words, weight.scales, weight.biases, weight.in_channels,
             weight.out_channels, weight.storage_in_channels,
             weight.group_size, weight.bits)

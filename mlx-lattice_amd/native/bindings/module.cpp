@@ -289,6 +289,15 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
           py::arg("bits"), py::arg("out_channels"), py::arg("sorted_kv_out_in_map"), py::arg("reorder_rows"),
           py::arg("tile_masks"), py::arg("out_capacity"), py::arg("n_kernels"), py::kw_only(),
           py::arg("bias") = py::none(), py::arg("tile_order") = py::none(), py::arg("relu") = false);
+    m.def("sparse_conv_padded", &ln::sparse_conv_padded, py::arg("feats"), py::arg("weights"), py::arg("role"),
+          py::arg("sorted_kv_out_in_map"), py::arg("reorder_rows"), py::arg("tile_masks"), py::arg("out_capacity"),
+          py::arg("n_kernels"), py::kw_only(), py::arg("bias") = py::none(), py::arg("tile_order") = py::none(),
+          py::arg("relu") = false);
+    m.def("sparse_quantized_conv_padded", &ln::sparse_quantized_conv_padded, py::arg("feats"), py::arg("weights"),
+          py::arg("scales"), py::arg("biases"), py::arg("in_channels"), py::arg("out_channels"),
+          py::arg("storage_in_channels"), py::arg("group_size"), py::arg("bits"), py::arg("sorted_kv_out_in_map"),
+          py::arg("reorder_rows"), py::arg("tile_masks"), py::arg("out_capacity"), py::arg("n_kernels"),
+          py::kw_only(), py::arg("bias") = py::none(), py::arg("tile_order") = py::none(), py::arg("relu") = false);
     m.def("conv_weight_fragments", &ln::conv_weight_fragments, py::arg("weights"),
           "Fragment-ordered copy of a 5D fp16/bf16 weight for the streamed matrix-core conv (empty when the shape "
           "does not take it).");

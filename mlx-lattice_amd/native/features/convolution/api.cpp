@@ -496,6 +496,31 @@ at::Tensor sparse_conv_features_padded(const at::Tensor& feats_in, const at::Ten
     return out;
 }
 
+at::Tensor sparse_conv_padded(const at::Tensor& feats, const at::Tensor& weights, int role,
+                              const at::Tensor& sorted_kv_out_in_map, const at::Tensor& reorder_rows,
+                              const at::Tensor& tile_masks, int out_capacity, int n_kernels,
+                              const std::optional<at::Tensor>& bias, const std::optional<at::Tensor>& tile_order,
+                              bool relu) {
+    const at::Tensor fragments = conv_padded_fragments(weights, role);
+    const int64_t c_in = weights.dim() == 3 ? weights.size(1) : weights.size(4);
+    const int64_t columns = role == LATTICE_FRAGMENTS_FORWARD ? out_channels_of(weights) : c_in;
+    return sparse_conv_features_padded(feats, fragments, 0, static_cast<int>(columns), sorted_kv_out_in_map,
+                                       reorder_rows, tile_masks, out_capacity, n_kernels, bias, tile_order, relu);
+}
+
+at::Tensor sparse_quantized_conv_padded(const at::Tensor& feats, const at::Tensor& weights, const at::Tensor& scales,
+                                        const at::Tensor& biases, int in_channels, int out_channels,
+                                        int storage_in_channels, int group_size, int bits,
+                                        const at::Tensor& sorted_kv_out_in_map, const at::Tensor& reorder_rows,
+                                        const at::Tensor& tile_masks, int out_capacity, int n_kernels,
+                                        const std::optional<at::Tensor>& bias,
+                                        const std::optional<at::Tensor>& tile_order, bool relu) {
+    const at::Tensor fragments = quantized_padded_fragments(weights, scales, biases, in_channels, out_channels,
+                                                            storage_in_channels, group_size, bits);
+    return sparse_conv_features_padded(feats, fragments, bits, out_channels, sorted_kv_out_in_map, reorder_rows,
+                                       tile_masks, out_capacity, n_kernels, bias, tile_order, relu);
+}
+
 at::Tensor conv_tile_order(const at::Tensor& tile_masks, int out_capacity) {
     require_i32_vector(tile_masks, "tile_masks must have shape (ceil(N_out / 64) * 4,) and int32 dtype.");
     if (out_capacity < 0 || tile_masks.size(0) != ((out_capacity + 63) / 64) * 4) {

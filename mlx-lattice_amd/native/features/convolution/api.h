@@ -79,6 +79,23 @@ at::Tensor sparse_conv_features_padded(const at::Tensor& feats, const at::Tensor
                                        const std::optional<at::Tensor>& bias = std::nullopt,
                                        const std::optional<at::Tensor>& tile_order = std::nullopt,
                                        bool relu = false);
+// The same with the fragments made in the call, from the weight as it is
+// (one more launch, the size of the weight): what the operators run, since
+// no counter sees every write to a weight (through .data, by a graph replay)
+// and the edge kernels, which these stand in for, read the weight itself.
+at::Tensor sparse_conv_padded(const at::Tensor& feats, const at::Tensor& weights, int role,
+                              const at::Tensor& sorted_kv_out_in_map, const at::Tensor& reorder_rows,
+                              const at::Tensor& tile_masks, int out_capacity, int n_kernels,
+                              const std::optional<at::Tensor>& bias = std::nullopt,
+                              const std::optional<at::Tensor>& tile_order = std::nullopt, bool relu = false);
+at::Tensor sparse_quantized_conv_padded(const at::Tensor& feats, const at::Tensor& weights, const at::Tensor& scales,
+                                        const at::Tensor& biases, int in_channels, int out_channels,
+                                        int storage_in_channels, int group_size, int bits,
+                                        const at::Tensor& sorted_kv_out_in_map, const at::Tensor& reorder_rows,
+                                        const at::Tensor& tile_masks, int out_capacity, int n_kernels,
+                                        const std::optional<at::Tensor>& bias = std::nullopt,
+                                        const std::optional<at::Tensor>& tile_order = std::nullopt,
+                                        bool relu = false);
 
 at::Tensor sparse_quantized_conv_features(const at::Tensor& feats, const at::Tensor& weights,
                                           const at::Tensor& scales, const at::Tensor& biases,
