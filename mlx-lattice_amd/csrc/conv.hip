@@ -1436,10 +1436,18 @@ __device__ inline void dequant_fragments(typename MfmaOps<T>::vec raw, typename 
 // leave as 16-byte stores where rows are 16-byte aligned, float32 lanes hold
 // four consecutive columns and store them directly; other column counts
 // store value by value.
-template <typename T, typename S, int RB, int CB>
+// REDO: a NaN sum may come from a product that is no edge's (a missing
+// neighbour's zero times an infinite weight) or from a weight in two parts
+// (an infinite feature times a zero or opposite rest), and never does a wrong
+// sum look finite; with `redo` set such a value is summed again over its own
+// edges, by redo_sum(row, column).  One multiply-add per value tells whether
+// a lane has any.
+template <typename T, typename S, bool REDO, int RB, int CB, typename F>
 __device__ inline void stream_store_padded(const float4_t (&acc)[RB][CB], T* stage, const Epilogue<T>& epi, int col0,
                                            int c_out, int row0, int wr, int wc, int rows,
-                                           const int32_t* __restrict__ reorder_rows, T* __restrict__ out) {
+                                           const int32_t* __restrict__ reorder_rows, T* __restrict__ out, bool redo,
+                                           F redo_sum) {
+    static_assert(RB * CB * 4 <= 64, "one bit per value of a lane");
     const int lane = lane_id();
     const int lr = lane & 15;
     const int lg = lane >> 4;
@@ -1452,6 +1460,37 @@ __device__ inline void stream_store_padded(const float4_t (&acc)[RB][CB], T* sta
             const int co = col0 + wc * S::WCOLS + cb * 16 + lg * 4 + q;
             bcol[cb][q] = epi.bias != nullptr && co < c_out ? static_cast<float>(epi.bias[co]) : 0.0f;
         }
+    uint64_t nans = 0;
+    if constexpr (REDO) {
+        float probe = 0.0f;  // NaN once a value is not finite
+        if (redo) {
+#pragma unroll
+            for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+                for (int cb = 0; cb < CB; ++cb)
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) probe = __builtin_fmaf(acc[rb][cb][q], 0.0f, probe);
+        }
+        if (probe != probe) {
+#pragma unroll
+            for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+                for (int cb = 0; cb < CB; ++cb)
+#pragma unroll
+                    for (int q = 0; q < 4; ++q)
+                        if (acc[rb][cb][q] != acc[rb][cb][q]) nans |= 1ull << ((rb * CB + cb) * 4 + q);
+        }
+    }
+    // store(r, c, v): row r of the tile, column c of the tile's columns
+    const auto redo_all = [&](auto store) {
+        for (; nans != 0; nans &= nans - 1) {
+            const int bit = __builtin_ctzll(nans);
+            const int r = wr * S::WROWS + bit / (CB * 4) * 16 + lr;
+            const int c = wc * S::WCOLS + bit / 4 % CB * 16 + lg * 4 + bit % 4;
+            if (row0 + r < rows && col0 + c < c_out)
+                store(r, c, epi.apply(redo_sum(row0 + r, col0 + c), col0 + c));
+        }
+    };
     if constexpr (sizeof(T) == 4) {
 #pragma unroll
         for (int rb = 0; rb < RB; ++rb) {
@@ -1474,6 +1513,12 @@ __device__ inline void stream_store_padded(const float4_t (&acc)[RB][CB], T* sta
                 }
             }
         }
+        if constexpr (REDO) {
+            redo_all([&](int r, int c, T v) {
+                const long long orow = reorder_rows != nullptr ? reorder_rows[row0 + r] : row0 + r;
+                out[orow * c_out + col0 + c] = v;
+            });
+        }
     } else {
         constexpr int LDW = S::C_OUT + 8;
         static_assert(S::ROWS * LDW <= (S::LA + 1) * S::ABUF, "the staged tile fits the A ring");
@@ -1490,6 +1535,8 @@ __device__ inline void stream_store_padded(const float4_t (&acc)[RB][CB], T* sta
                     *reinterpret_cast<const uint2*>(v);
             }
         }
+        // (each lane its own staged values)
+        if constexpr (REDO) redo_all([&](int r, int c, T v) { stage[r * LDW + c] = v; });
         __syncthreads();
         const int cols = min(S::C_OUT, c_out - col0);
         if (whole) {
@@ -1516,6 +1563,46 @@ __device__ inline void stream_store_padded(const float4_t (&acc)[RB][CB], T* sta
     }
 }
 
+// One output value as the edge kernel sums it: the weight from its padded
+// fragments (QB: code * scale + bias in fp32), offset by offset of `mask`,
+// over the neighbours that the row has.
+template <typename T, int QB>
+__device__ inline float padded_edge_sum(const T* __restrict__ feats, int n_in, int c_in, const T* __restrict__ wfrag,
+                                        int ncg, const int32_t* __restrict__ kv_map, int rows, uint32_t mask, int row,
+                                        int co) {
+    constexpr int PE = 16 / static_cast<int>(sizeof(T));
+    const int ksteps = (c_in + 4 * PE - 1) / (4 * PE);
+    float sum = 0.0f;
+#pragma unroll 1  // (hardly ever run: no registers of the main loop's for it)
+    for (; mask != 0; mask &= mask - 1) {
+        const int k = __builtin_ctz(mask);
+        const int in = kv_map[static_cast<long long>(k) * rows + row];
+        if (in < 0 || in >= n_in) continue;
+        const T* f = feats + static_cast<long long>(in) * c_in;
+#pragma unroll 1
+        for (int ci = 0; ci < c_in; ci += PE) {
+            const long long p = fragment_piece(k, ci / (4 * PE), co / 32, co / 16 % 2, ci / PE % 4 * 16 + co % 16,
+                                               ksteps, ncg);
+            const uint4 raw = reinterpret_cast<const uint4*>(wfrag)[p];
+#pragma unroll
+            for (int j = 0; j < PE; ++j) {
+                float w;
+                if constexpr (QB != 0) {
+                    const uint32_t q = QB == 4 ? (raw.x >> (4 * j)) & 15u : ((j < 4 ? raw.x : raw.y) >> (8 * (j & 3))) & 255u;
+                    w = static_cast<float>(q) * static_cast<float>(__builtin_bit_cast(T, static_cast<uint16_t>(raw.z & 0xFFFFu))) +
+                        static_cast<float>(__builtin_bit_cast(T, static_cast<uint16_t>(raw.z >> 16)));
+                } else {
+                    T v[PE];
+                    __builtin_memcpy(v, &raw, 16);
+                    w = static_cast<float>(v[j]);
+                }
+                sum += static_cast<float>(f[ci + j]) * w;
+            }
+        }
+    }
+    return sum;
+}
+
 // PAD: channel counts that do not fill the tiles.  The fragments are padded
 // with zeros to whole 32-column groups and whole fragments of input
 // channels, a copy's pieces past C_in wrap past the buffer's range (zeros, no
@@ -1531,13 +1618,16 @@ __device__ inline void stream_store_padded(const float4_t (&acc)[RB][CB], T* sta
 // 60,001 rows 3,000 -> 46 us, its input gradient 629 -> 46 us.
 // SPLIT (PAD, packed weights): the weight contracted unrounded, as two
 // fragments, as the edge kernel contracts it; without it rounded once, as in
-// the instances that fill their tiles.
+// the instances that fill their tiles.  own_edges (PAD, not with a rounded
+// weight): sums that are NaN are made again edge by edge, for the shapes that
+// the edge kernels ran before: infinities and NaN reach the rows that they
+// have an edge to and no others.
 template <typename T, typename S, int NCH, int QB, bool PAD = false, bool SPLIT = false>
 __global__ void __launch_bounds__(S::THREADS, S::OCC)
 conv_igemm_stream(const T* __restrict__ feats, int n_in, int c_in, const T* __restrict__ wfrag, int kernel_count,
                   int c_out_total, const int32_t* __restrict__ kv_map, const int32_t* __restrict__ tile_masks,
                   const int32_t* __restrict__ reorder_rows, int rows, const int32_t* __restrict__ block_order,
-                  T* __restrict__ out, Epilogue<T> epi, int halves) {
+                  T* __restrict__ out, Epilogue<T> epi, int halves, bool own_edges) {
     static_assert(!PAD || NCH == 1, "padded chunks are stages of their own");
     static_assert(!SPLIT || (PAD && QB != 0), "only padded packed weights are split");
     using V = typename MfmaOps<T>::vec;
@@ -1824,7 +1914,11 @@ conv_igemm_stream(const T* __restrict__ feats, int n_in, int c_in, const T* __re
     }
 
     if constexpr (PAD) {
-        stream_store_padded<T, S>(acc, lds, epi, half * S::C_OUT, c_out_total, row0, wr, wc, rows, reorder_rows, out);
+        const auto edge_sum = [&](int row, int co) {
+            return padded_edge_sum<T, QB>(feats, n_in, c_in, wfrag, ncg, kv_map, rows, bmask, row, co);
+        };
+        stream_store_padded<T, S, QB == 0 || SPLIT>(acc, lds, epi, half * S::C_OUT, c_out_total, row0, wr, wc, rows,
+                                                    reorder_rows, out, own_edges, edge_sum);
     } else {
     // The finished tile goes through LDS (the A ring is free once every
     // wave's copies have landed) so that it leaves as 16-byte stores of
@@ -2317,7 +2411,7 @@ void launch_stream_nch(const T* feats, int n_in, int c_in, const T* frag, int K,
                        Epilogue<T> epi, int halves, hipStream_t stream) {
     const int tiles = (rows + S::ROWS - 1) / S::ROWS;
     conv_igemm_stream<T, S, NCH, QB><<<static_cast<unsigned>(tiles * halves), S::THREADS, 0, stream>>>(
-        feats, n_in, c_in, frag, K, c_out, kv_map, tile_masks, reorder_rows, rows, order, out, epi, halves);
+        feats, n_in, c_in, frag, K, c_out, kv_map, tile_masks, reorder_rows, rows, order, out, epi, halves, false);
 }
 
 template <typename T, typename S, int QB>
@@ -2368,12 +2462,13 @@ size_t padded_fragments_bytes(int dtype, int K, int c_in, int c_out) {
 template <typename T, typename S, int QB, bool SPLIT>
 void launch_padded_shape(const T* feats, int n_in, int c_in, const T* frag, int K, int c_out, const int32_t* kv_map,
                          const int32_t* tile_masks, const int32_t* reorder_rows, int rows, const int32_t* order,
-                         T* out, Epilogue<T> epi, hipStream_t stream) {
+                         T* out, Epilogue<T> epi, bool own_edges, hipStream_t stream) {
     // an order's 128-row tiles are two 64-row or four 32-row ones
     const int tiles = (rows + kOrderTileRows - 1) / kOrderTileRows * (kOrderTileRows / S::ROWS);
     const int columns = (c_out + S::C_OUT - 1) / S::C_OUT;
     conv_igemm_stream<T, S, 1, QB, true, SPLIT><<<static_cast<unsigned>(tiles) * columns, S::THREADS, 0, stream>>>(
-        feats, n_in, c_in, frag, K, c_out, kv_map, tile_masks, reorder_rows, rows, order, out, epi, columns);
+        feats, n_in, c_in, frag, K, c_out, kv_map, tile_masks, reorder_rows, rows, order, out, epi, columns,
+        own_edges);
 }
 
 // Few rows: a launch of at most about two 128-row tiles per CU lasts as long
@@ -2391,7 +2486,7 @@ bool few_rows(int rows, int c_out) {
 template <typename T, int QB, bool SPLIT>
 int launch_padded(const T* feats, int n_in, int c_in, const T* frag, int K, int c_out, const int32_t* kv_map,
                   const int32_t* tile_masks, const int32_t* reorder_rows, int rows, int32_t* schedule, bool ready,
-                  T* out, Epilogue<T> epi, hipStream_t stream) {
+                  T* out, Epilogue<T> epi, bool own_edges, hipStream_t stream) {
     if (rows <= 0) return LATTICE_OK;
     const int tiles = (rows + kOrderTileRows - 1) / kOrderTileRows;
     if (tiles > kMaxScheduledTiles) schedule = nullptr;
@@ -2401,7 +2496,7 @@ int launch_padded(const T* feats, int n_in, int c_in, const T* frag, int K, int 
     }
 #define LATTICE_PADDED(C, WR, ROWS)                                                                                \
     launch_padded_shape<T, StreamShape<T, C, WR, ROWS>, QB, SPLIT>(                                                \
-        feats, n_in, c_in, frag, K, c_out, kv_map, tile_masks, reorder_rows, rows, schedule, out, epi, stream)
+        feats, n_in, c_in, frag, K, c_out, kv_map, tile_masks, reorder_rows, rows, schedule, out, epi, own_edges, stream)
     // Tile rows.  float32 is bound by its MFMAs: 32-row tiles (no more
     // gathers, a shorter longest tile) measured fastest at every size for
     // more than 32 columns (64 -> 64 over 60,001 / 128,000 rows 53 -> 46 /
@@ -2450,7 +2545,7 @@ int launch_stream(const T* feats, int n_in, int c_in, const T* frag, int K, int 
     // smaller tiles change no result (the weight's rounding included).
     if (few_rows(rows, c_out)) {
         return launch_padded<T, QB, false>(feats, n_in, c_in, frag, K, c_out, kv_map, tile_masks, reorder_rows, rows,
-                                           schedule, ready, out, epi, stream);
+                                           schedule, ready, out, epi, false, stream);
     }
     const int tiles = (rows + kOrderTileRows - 1) / kOrderTileRows;
     if (tiles > kMaxScheduledTiles) schedule = nullptr;
@@ -2801,7 +2896,7 @@ extern "C" int lattice_hip_sparse_conv_features_padded(
     launch_padded<T, QB, QB != 0>(static_cast<const T*>(feats), n_in, c_in, static_cast<const T*>(fragments),       \
                                   kernel_count, c_out, sorted_kv_out_in_map, tile_masks, reorder_rows,             \
                                   out_capacity, schedule, ready, static_cast<T*>(out),                             \
-                                  epilogue_of<T>(bias, epilogue), stream)
+                                  epilogue_of<T>(bias, epilogue), true, stream)
     if (dtype == LATTICE_F32) return LATTICE_PADDED_CALL(float, 0);
     if (dtype == LATTICE_F16) {
         if (bits == 0) return LATTICE_PADDED_CALL(_Float16, 0);
