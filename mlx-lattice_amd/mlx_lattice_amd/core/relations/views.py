@@ -9,8 +9,9 @@ relation's device; counts stay on the device.
 
 from __future__ import annotations
 
+import threading
 from collections.abc import Callable
-from dataclasses import dataclass, field
+from dataclasses import dataclass, field, fields, is_dataclass
 from typing import Literal
 
 import torch
@@ -28,6 +29,64 @@ _ONE_ROUND_ROWS = 256 * 128
 _TILED_ROWS = 32768
 _TILED_WEIGHT_BYTES = 16384
 _TILED_WORK = 16384 * 16384
+_KEEP_LOCK = threading.RLock()
+
+
+def _arrays(value) -> list[torch.Tensor]:
+    """The tensors of a tensor, view or tuple of them."""
+    if isinstance(value, torch.Tensor):
+        return [value]
+    if isinstance(value, tuple):
+        return [t for item in value for t in _arrays(item)]
+    if is_dataclass(value):
+        return [t for f in fields(value)
+                for t in _arrays(getattr(value, f.name))]
+    return []
+
+
+def _kept(holder, name: str, device: torch.device, make: Callable):
+    """``holder.name``, device arrays that ``make`` builds on their first
+    use.  They are kept with the stream that wrote them, and another stream's
+    first use of them waits for it.  Under graph capture nothing is kept (the
+    arrays hold values only once the graph runs) but for the rest of that
+    capture's work on the stream; arrays made before a capture are used as
+    they are.  ``holder._written`` holds the streams ordered after each
+    array's writes, the writer first; a value given at construction is not in
+    it."""
+    value = getattr(holder, name)
+    if device.type != 'cuda':
+        if value is None:
+            value = make()
+            object.__setattr__(holder, name, value)
+        return value
+    from mlx_lattice_amd._native import ext
+
+    stream, capture = ext.stream_state(device.index)
+    written = holder._written
+    if value is not None:
+        streams = written.get(name)
+        if streams is None or capture or stream in streams:
+            return value
+        if not ext.join_stream(device.index, streams[0]):
+            return make()   # the writer is being captured: nothing to wait for
+        current = torch.cuda.current_stream(device)
+        for array in _arrays(value):
+            array.record_stream(current)
+        written[name] = (*streams, stream)
+        return value
+    if capture:
+        captured = written.get((name, 'captured'))
+        if captured is None or captured[:2] != (stream, capture):
+            captured = (stream, capture, make())
+            written[name, 'captured'] = captured
+        return captured[2]
+    with _KEEP_LOCK:
+        if getattr(holder, name) is None:
+            value = make()
+            written[name] = (stream,)
+            object.__setattr__(holder, name, value)
+            return value
+    return _kept(holder, name, device, make)   # another thread made it
 
 
 @dataclass(frozen=True, slots=True)
@@ -102,6 +161,8 @@ class RelationSortedImplicitGemmView:
     tile_masks: torch.Tensor
     _tile_order: torch.Tensor | None = field(default=None, compare=False,
                                              repr=False)
+    _written: dict = field(default_factory=dict, init=False, compare=False,
+                           repr=False)
 
     def __post_init__(self) -> None:
         if self.sorted_out_in_map.ndim != 2:
@@ -128,12 +189,14 @@ class RelationSortedImplicitGemmView:
         tiles all start at once."""
         if int(self.reorder_rows.shape[0]) <= _ONE_ROUND_ROWS:
             return None
-        if self._tile_order is None:
-            from mlx_lattice_amd._native import ext
+        return _kept(self, '_tile_order', self.tile_masks.device,
+                     self._order_tiles)
 
-            object.__setattr__(self, '_tile_order', ext.conv_tile_order(
-                self.tile_masks, int(self.reorder_rows.shape[0])))
-        return self._tile_order
+    def _order_tiles(self) -> torch.Tensor:
+        from mlx_lattice_amd._native import ext
+
+        return ext.conv_tile_order(self.tile_masks,
+                                   int(self.reorder_rows.shape[0]))
 
 
 class _StatusWord:
@@ -184,44 +247,30 @@ class _StatusWord:
 
 class _MapEdges:
     """The edges and their row offsets of a relation built as a dense map
-    alone, made from the map and its masks on first use.  They are kept with
-    the stream that wrote them: another stream waits for it.  Under graph
-    capture nothing is kept (the arrays hold values only once the graph
-    runs)."""
+    alone, made from the map and its masks on first use (``_kept``)."""
 
-    __slots__ = ('_view', '_counts', '_made')
+    __slots__ = ('_view', '_counts', '_made', '_written')
 
     def __init__(self, view: RelationImplicitGemmView,
                  counts: torch.Tensor) -> None:
         self._view = view
         self._counts = counts
         self._made = None
+        self._written = {}
 
     @property
     def capacity(self) -> int:
         return int(self._view.out_in_map.numel())
 
     def get(self) -> tuple[RelationEdges, RelationCSRView]:
-        device = self._counts.device
-        if self._made is None:
-            from mlx_lattice_amd._native import ext
+        return _kept(self, '_made', self._counts.device, self._make)
 
-            *edges, row_offsets = ext.build_map_edges(
-                self._view.out_in_map, self._view.row_masks, self._counts)
-            made = RelationEdges(*edges), RelationCSRView(row_offsets)
-            if torch.cuda.is_current_stream_capturing():
-                return made
-            stream = torch.cuda.current_stream(device)
-            self._made = (*made, stream, stream.record_event())
-            return made
-        edges, csr, stream, written = self._made
-        current = torch.cuda.current_stream(device)
-        if current != stream and not torch.cuda.is_current_stream_capturing():
-            current.wait_event(written)
-            for array in (edges.in_rows, edges.out_rows, edges.kernel_ids,
-                          csr.row_offsets):
-                array.record_stream(current)
-        return edges, csr
+    def _make(self) -> tuple[RelationEdges, RelationCSRView]:
+        from mlx_lattice_amd._native import ext
+
+        *edges, row_offsets = ext.build_map_edges(
+            self._view.out_in_map, self._view.row_masks, self._counts)
+        return RelationEdges(*edges), RelationCSRView(row_offsets)
 
 
 @dataclass(frozen=True, slots=True)
@@ -306,12 +355,16 @@ class KernelRelation:
     _map_edges: _MapEdges | None
     _input_csr: RelationCSRView | None
     _kernel_csr: RelationCSRView | None
+    # The (input, kernel) CSR views when `_grouped_views` makes them.
+    _grouped: tuple[RelationCSRView, RelationCSRView] | None
     _grouped_views: Callable[..., tuple] | None
     # Builds the edges grouped by offset without a sort (dense-map relations
     # of at most 32 offsets): the edge ids when called with the row offsets,
     # else the (input row, output row) pairs.
     _kernel_groups: Callable[[torch.Tensor | None], tuple] | None
+    _kernel_grouped: RelationCSRView | None
     _kernel_pairs: tuple[torch.Tensor, torch.Tensor] | None
+    _written: dict = field(compare=False, repr=False)
     implicit_gemm: RelationImplicitGemmView | None = None
     sorted_implicit_gemm: RelationSortedImplicitGemmView | None = None
     transposed_sorted_implicit_gemm: RelationSortedImplicitGemmView | None = None
@@ -451,7 +504,10 @@ class KernelRelation:
                            grouped_views if lazy_views else None)
         object.__setattr__(self, '_kernel_groups',
                            kernel_groups if lazy_views else None)
+        object.__setattr__(self, '_grouped', None)
+        object.__setattr__(self, '_kernel_grouped', None)
         object.__setattr__(self, '_kernel_pairs', None)
+        object.__setattr__(self, '_written', {})
         object.__setattr__(self, 'implicit_gemm', implicit_gemm)
         object.__setattr__(self, 'sorted_implicit_gemm', sorted_implicit_gemm)
         object.__setattr__(self, 'transposed_sorted_implicit_gemm', None)
@@ -495,43 +551,44 @@ class KernelRelation:
     def source_active_rows(self) -> torch.Tensor | None:
         return self._contract.source_active_rows
 
+    def _keep(self, name: str, make: Callable):
+        return _kept(self, name, self._contract.counts.device, make)
+
     @property
     def input_csr(self) -> RelationCSRView:
         """Edges grouped by input row (stable in edge order)."""
-        if self._input_csr is None:
-            self._materialize_grouped_views()
-        return self._input_csr
+        if self._input_csr is not None:
+            return self._input_csr
+        return self._keep('_grouped', self._group)[0]
 
     @property
     def kernel_csr(self) -> RelationCSRView:
         """Edges grouped by kernel offset (stable in edge order)."""
-        if self._kernel_csr is None and self._kernel_groups is not None:
-            k_offsets, _, k_ids = self._kernel_groups(
-                self.output_csr.row_offsets)
-            object.__setattr__(self, '_kernel_csr',
-                               RelationCSRView(k_offsets, k_ids))
-        elif self._kernel_csr is None:
-            self._materialize_grouped_views()
-        return self._kernel_csr
+        if self._kernel_csr is not None:
+            return self._kernel_csr
+        if self._kernel_groups is not None:
+            return self._keep('_kernel_grouped', self._group_by_kernel)
+        return self._keep('_grouped', self._group)[1]
 
     def kernel_pairs(self) -> tuple[torch.Tensor, torch.Tensor] | None:
         """(offsets (K + 1,), pairs (E, 2)): the (input row, output row) of
         every edge, grouped by kernel offset in the order of ``kernel_csr``,
         built on first use; None for relations that group by a sort."""
-        if self._kernel_pairs is None and self._kernel_groups is not None:
-            k_offsets, pairs, _ = self._kernel_groups(None)
-            object.__setattr__(self, '_kernel_pairs', (k_offsets, pairs))
-        return self._kernel_pairs
+        if self._kernel_groups is None:
+            return None
+        return self._keep('_kernel_pairs',
+                          lambda: self._kernel_groups(None)[:2])
 
-    def _materialize_grouped_views(self) -> None:
+    def _group_by_kernel(self) -> RelationCSRView:
+        offsets, _, ids = self._kernel_groups(self.output_csr.row_offsets)
+        return RelationCSRView(offsets, ids)
+
+    def _group(self) -> tuple[RelationCSRView, RelationCSRView]:
         in_offsets, in_ids, k_offsets, k_ids = (
             self._grouped_views() if self._map_edges is None
             else self._grouped_views(self.edges))
-        object.__setattr__(self, '_input_csr',
-                           RelationCSRView(in_offsets, in_ids))
-        if self._kernel_csr is None:
-            object.__setattr__(self, '_kernel_csr',
-                               RelationCSRView(k_offsets, k_ids))
+        return (RelationCSRView(in_offsets, in_ids),
+                RelationCSRView(k_offsets, k_ids))
 
     @property
     def edge_capacity(self) -> int:
@@ -610,19 +667,16 @@ class KernelRelation:
 
     def require_implicit_gemm(self) -> RelationImplicitGemmView:
         """Return or lazily build the implicit-GEMM view (views.py:452-465)."""
-        if self.implicit_gemm is not None:
-            return self.implicit_gemm
+        return self._keep('implicit_gemm', self._implicit_gemm)
+
+    def _implicit_gemm(self) -> RelationImplicitGemmView:
         if self._contract.kind in ('transposed', 'generative'):
-            view = self._expanded_implicit_gemm()
-            object.__setattr__(self, 'implicit_gemm', view)
-            return view
+            return self._expanded_implicit_gemm()
         from mlx_lattice_amd.core.coords.builders import (
             build_relation_implicit_gemm_view,
         )
 
-        view = build_relation_implicit_gemm_view(self)
-        object.__setattr__(self, 'implicit_gemm', view)
-        return view
+        return build_relation_implicit_gemm_view(self)
 
     @property
     def dense_map_exact(self) -> bool:
@@ -687,21 +741,14 @@ class KernelRelation:
         ``reorder_rows`` is the stable argsort of the row masks, the maps are
         gathered in that order and ``tile_masks`` ORs each 16-row quarter of
         every 64-row tile."""
-        if self.sorted_implicit_gemm is not None:
-            return self.sorted_implicit_gemm
+        return self._keep('sorted_implicit_gemm', self._sorted_implicit_gemm)
+
+    def _sorted_implicit_gemm(self) -> RelationSortedImplicitGemmView:
         view = self.require_implicit_gemm()
         if view.row_masks.shape[1] != 1:
             raise ValueError(
                 'sorted implicit GEMM view currently supports K <= 32.')
-        from mlx_lattice_amd._native import ext
-
-        reorder, sorted_map, kv_map, tiles = ext.build_sorted_implicit_gemm_view(
-            view.out_in_map, view.row_masks)
-        sorted_view = RelationSortedImplicitGemmView(
-            sorted_out_in_map=sorted_map, sorted_kv_out_in_map=kv_map,
-            reorder_rows=reorder, tile_masks=tiles)
-        object.__setattr__(self, 'sorted_implicit_gemm', sorted_view)
-        return sorted_view
+        return _sorted_view(view.out_in_map, view.row_masks)
 
     def conv_view(self, weight_bytes: int) -> RelationSortedImplicitGemmView:
         """The view a matrix-core conv whose weight has ``weight_bytes`` per
@@ -717,11 +764,11 @@ class KernelRelation:
                                               'target')
                 or not _tiled_pays(self.n_out_capacity, weight_bytes)):
             return self.require_sorted_implicit_gemm()
-        if self._tiled is None:
-            view = self.require_implicit_gemm()
-            object.__setattr__(self, '_tiled', _tiled_view(
-                view.out_in_map, view.row_masks))
-        return self._tiled
+        return self._keep('_tiled', self._tile)
+
+    def _tile(self) -> RelationSortedImplicitGemmView:
+        view = self.require_implicit_gemm()
+        return _tiled_view(view.out_in_map, view.row_masks)
 
     def transposed_conv_view(self, weight_bytes: int,
                              ) -> RelationSortedImplicitGemmView:
@@ -732,10 +779,8 @@ class KernelRelation:
                 or not _tiled_pays(self.n_in_capacity, weight_bytes)
                 or self.n_kernels is None or self.n_kernels > 32):
             return self.require_transposed_sorted_implicit_gemm()
-        if self._transposed_tiled is None:
-            object.__setattr__(self, '_transposed_tiled',
-                               _tiled_view(*self._transposed_map()))
-        return self._transposed_tiled
+        return self._keep('_transposed_tiled',
+                          lambda: _tiled_view(*self._transposed_map()))
 
     def _transposed_map(self) -> tuple[torch.Tensor, torch.Tensor]:
         """(in_out_map, row_masks) of the transposed relation."""
@@ -760,27 +805,23 @@ class KernelRelation:
         (``transposed_map_exact``, which the input gradient checks first);
         target relations (whose target may repeat a coordinate) are
         refused."""
-        if self.transposed_sorted_implicit_gemm is not None:
-            return self.transposed_sorted_implicit_gemm
-        if self._contract.kind not in ('forward', 'submanifold', 'transposed',
-                                      'generative'):
+        if (self.transposed_sorted_implicit_gemm is None
+                and self._contract.kind not in ('forward', 'submanifold',
+                                                'transposed', 'generative')):
             raise ValueError('the transposed implicit-GEMM view needs a '
                              'forward, submanifold, transposed or generative '
                              'relation.')
+        return self._keep('transposed_sorted_implicit_gemm',
+                          self._transposed_sorted_implicit_gemm)
+
+    def _transposed_sorted_implicit_gemm(
+            self) -> RelationSortedImplicitGemmView:
         if self.n_in_capacity is None or self.n_kernels is None:
             raise ValueError('kernel relation is missing static shape metadata.')
         if self.n_kernels > 32:
             raise ValueError(
                 'sorted implicit GEMM view currently supports K <= 32.')
-        from mlx_lattice_amd._native import ext
-
-        reorder, sorted_map, kv_map, tiles = ext.build_sorted_implicit_gemm_view(
-            *self._transposed_map())
-        view = RelationSortedImplicitGemmView(
-            sorted_out_in_map=sorted_map, sorted_kv_out_in_map=kv_map,
-            reorder_rows=reorder, tile_masks=tiles)
-        object.__setattr__(self, 'transposed_sorted_implicit_gemm', view)
-        return view
+        return _sorted_view(*self._transposed_map())
 
 
 # ---------------------------------------------------------------- helpers --
@@ -807,6 +848,17 @@ def _int_offset_tuple(offsets: tuple) -> tuple[Triple, ...]:
 def _tiled_pays(rows: int, weight_bytes: int) -> bool:
     return (rows <= _TILED_ROWS and weight_bytes <= _TILED_WEIGHT_BYTES
             and rows * weight_bytes <= _TILED_WORK)
+
+
+def _sorted_view(out_in_map: torch.Tensor, row_masks: torch.Tensor,
+                 ) -> RelationSortedImplicitGemmView:
+    from mlx_lattice_amd._native import ext
+
+    reorder, sorted_map, kv_map, tiles = ext.build_sorted_implicit_gemm_view(
+        out_in_map, row_masks)
+    return RelationSortedImplicitGemmView(
+        sorted_out_in_map=sorted_map, sorted_kv_out_in_map=kv_map,
+        reorder_rows=reorder, tile_masks=tiles)
 
 
 def _tiled_view(out_in_map: torch.Tensor, row_masks: torch.Tensor,

@@ -56,11 +56,13 @@ def _small_dense_map(dtype: torch.dtype, c_in: int, c_out: int,
     channels (C_in 4 or 8, C_out 16 or 32, fp16/bf16), when the relation
     already holds it: the native CSR entry then contracts a row's whole
     neighbourhood on the matrix cores instead of walking its edges."""
-    view = relation.implicit_gemm
-    if (view is None or dtype not in (torch.float16, torch.bfloat16)
+    if (relation.implicit_gemm is None
+            or dtype not in (torch.float16, torch.bfloat16)
             or c_in not in (4, 8) or c_out not in (16, 32)
-            or relation.n_kernels is None or relation.n_kernels * c_in > 256
-            or view.out_in_map.dtype != torch.int32
+            or relation.n_kernels is None or relation.n_kernels * c_in > 256):
+        return None
+    view = relation.require_implicit_gemm()
+    if (view.out_in_map.dtype != torch.int32
             or tuple(view.out_in_map.shape) != (relation.n_out_capacity,
                                                 relation.n_kernels)
             or not relation.dense_map_exact):

@@ -4,10 +4,13 @@
 // (coords.cpp:79-92); the *_with_view variants append the implicit-GEMM view
 // (out_in_map, row_masks) computed by the same pass.
 
+#include <c10/hip/HIPStream.h>
 #include <hip/hip_runtime_api.h>
 #include <torch/extension.h>
 
 #include <array>
+#include <cstdint>
+#include <utility>
 #include <vector>
 
 #include "features/convolution/api.h"
@@ -81,11 +84,44 @@ class StatusWord {
     hipEvent_t event_ = nullptr;
 };
 
+// The current stream and the id of the graph capture it is part of (0: none).
+std::pair<uintptr_t, uint64_t> stream_state(int device) {
+    hipStream_t stream = c10::hip::getCurrentHIPStream(static_cast<c10::DeviceIndex>(device)).stream();
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    unsigned long long id = 0;
+    if (hipStreamGetCaptureInfo(stream, &status, &id) != hipSuccess) {
+        (void)hipGetLastError();  // the legacy stream beside another stream's capture: not captured itself
+        status = hipStreamCaptureStatusNone;
+    }
+    return {reinterpret_cast<uintptr_t>(stream), status == hipStreamCaptureStatusNone ? 0 : id};
+}
+
+// Lets the current stream wait for the work on `writer` so far; false when
+// `writer` is being captured (or is no more): there is nothing to wait for.
+bool join_stream(int device, uintptr_t writer_handle) {
+    const c10::DeviceGuard guard(c10::Device(c10::kCUDA, static_cast<c10::DeviceIndex>(device)));
+    hipStream_t writer = reinterpret_cast<hipStream_t>(writer_handle);
+    hipStream_t current = c10::hip::getCurrentHIPStream(static_cast<c10::DeviceIndex>(device)).stream();
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    hipEvent_t event = nullptr;
+    bool ok = hipStreamIsCapturing(writer, &status) == hipSuccess && status == hipStreamCaptureStatusNone &&
+              hipEventCreateWithFlags(&event, hipEventDisableTiming) == hipSuccess;
+    if (ok) {
+        ok = hipEventRecord(event, writer) == hipSuccess && hipStreamWaitEvent(current, event, 0) == hipSuccess;
+        (void)hipEventDestroy(event);
+    }
+    if (!ok) (void)hipGetLastError();
+    return ok;
+}
+
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.doc() = "MI355X-native sparse convolution hot path (gfx950 HIP kernels behind a C ABI).";
     py::class_<StatusWord>(m, "StatusWord").def(py::init<const at::Tensor&>()).def("read", &StatusWord::read);
+    m.def("stream_state", &stream_state, py::arg("device"), "(current stream, id of its graph capture or 0).");
+    m.def("join_stream", &join_stream, py::arg("device"), py::arg("writer"),
+          "Let the current stream wait for `writer`; False when it is being captured.");
     m.def("version", []() { return std::string(lattice_hip_version()); });
     m.def("coord_hash_capacity", [](int rows) { return lattice_hip_coord_hash_capacity(rows); }, py::arg("rows"));
     m.def(
