@@ -383,8 +383,8 @@ class KernelRelation:
     # Submanifold relations: whether an active row repeats an earlier row's
     # coordinate (each copy is an output row with the same neighbours, so
     # an input row can have several output rows at one offset).  Held as a
-    # _StatusWord copied to pinned memory when a conv that needs gradients
-    # runs (expect_backward) and read on the first question
+    # _StatusWord copied to pinned memory when a conv of trainable features
+    # or weights runs (expect_backward) and read on the first question
     # (transposed_map_exact).  None: no repeats possible.
     repeated_coords: bool | _StatusWord | None = None
     # Submanifold relations built with their workspace: it starts with the
@@ -703,8 +703,9 @@ class KernelRelation:
         output coordinates are distinct, or each output row has one edge); a
         submanifold relation does unless a coordinate repeats.  The first
         question reads the build's status word from pinned memory (copied
-        when a forward that needs gradients ran), so it waits for that copy
-        only; under graph capture an unread word counts as a repeat."""
+        when a conv of trainable features or weights ran), so it waits for
+        that copy only; under graph capture a word that was not copied before
+        counts as a repeat."""
         if self._contract.kind == 'target':
             return False
         if isinstance(self.repeated_coords, _StatusWord):

@@ -172,6 +172,10 @@ def sparse_conv_features_from_relation(feats: torch.Tensor,
     ReLU after the bias into the store (the operators pass it only when
     autograd does not need the activation)."""
     _require_static(relation)
+    if feats.requires_grad or weight.requires_grad:
+        # (an evaluation of trainable layers too: a graph captured later
+        # cannot read what was not copied before)
+        relation.expect_backward()
     if torch.is_grad_enabled() and (feats.requires_grad
                                     or weight.requires_grad
                                     or (bias is not None
@@ -203,7 +207,6 @@ class _SparseConvFeatures(torch.autograd.Function):
     @staticmethod
     def forward(ctx, feats, weight, relation):
         ctx.relation = relation
-        relation.expect_backward()
         ctx.save_for_backward(feats, weight)
         return _conv_features(feats, weight, relation)
 

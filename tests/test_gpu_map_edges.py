@@ -150,3 +150,43 @@ def test_repeat_flag_is_read_after_a_forward_without_gradients(repeat):
     relation = fresh.coord_manager.submanifold_kernel_relation(
         fresh.coord_key)
     assert relation.transposed_map_exact is not repeat
+
+
+@pytest.mark.parametrize('trained', ['weight', 'feats'])
+def test_a_forward_without_grad_mode_prepares_a_captured_backward(trained):
+    """A trainable layer evaluated under ``no_grad`` first: a step captured
+    afterwards takes the input gradient that an eager one takes."""
+    from mlx_lattice_amd import SparseTensor, ops
+
+    c = _coords(3000, 12)
+    rng = np.random.default_rng(5)
+    f = torch.as_tensor(rng.standard_normal((3000, 64))).to(
+        DEV, torch.float16)
+    w = torch.as_tensor(rng.standard_normal((64, 3, 3, 3, 64)) / 24).to(
+        DEV, torch.float16)
+    g = torch.as_tensor(rng.standard_normal((3000, 64))).to(
+        DEV, torch.float16)
+
+    def grad(x, feats):
+        y = ops.subm_conv3d(x.replace(feats=feats), w)
+        return torch.autograd.grad(y.feats, feats, g)[0]
+
+    feats = f.clone().requires_grad_()
+    want = grad(SparseTensor(c, f), feats)
+    x = SparseTensor(c, f)
+    with torch.no_grad():
+        if trained == 'weight':
+            ops.subm_conv3d(x, w.clone().requires_grad_())
+        else:
+            ops.subm_conv3d(x.replace(feats=feats), w)
+    relation = x.coord_manager.submanifold_kernel_relation(x.coord_key)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=torch.cuda.Stream()):
+        assert not relation.repeated_coords.unreadable
+        captured = grad(x, feats)
+    for _ in range(3):
+        captured.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(captured, want)
