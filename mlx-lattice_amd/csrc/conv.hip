@@ -1412,9 +1412,11 @@ __device__ inline typename MfmaOps<T>::vec dequant_fragment(typename MfmaOps<T>:
 }
 
 // The same as two fragments whose sum is the fp32 weight but for 2^-16 (bf16)
-// or 2^-21 (fp16) of it: the padded instances contract both, as the edge
-// kernel contracts fp32 weights (one fragment alone raises the error of a
-// bf16 96 -> 96 int4 conv against 64 bits from 1.7e-3 to 2.3e-3).
+// or 2^-22 (fp16) of it, or, where the second is a subnormal fp16, 2^-25: the
+// padded instances contract both, as the edge kernel contracts fp32 weights
+// (one fragment alone raises the error of a bf16 96 -> 96 int4 conv against
+// 64 bits from 1.7e-3 to 2.3e-3).  Of a weight past the fp16 range the two
+// are infinities of opposite signs; stream_store_padded makes such sums again.
 template <typename T, int QB>
 __device__ inline void dequant_fragments(typename MfmaOps<T>::vec raw, typename MfmaOps<T>::vec& hi,
                                          typename MfmaOps<T>::vec& lo) {

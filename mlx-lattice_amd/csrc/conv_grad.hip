@@ -685,11 +685,6 @@ weight_grad_mfma(const T* __restrict__ feats, int n_in, int c_in, const T* __res
         for (int n = 0; n < NB; ++n) out[((wave * MB + m) * NB + n) * 64 + lane] = acc[m][n];
 }
 
-// dW[k] = sum of the partial tiles of offset k's blocks (XCD by XCD, then
-// turn by turn), one rounding, written in the weight's layout.  Blocks
-// (x, k): offset k's share is worked out once per thread, then the block
-// strides over the offset's C_in x C_out entries four at a time (16-byte
-// loads of the partials; each entry keeps its own summation order).
 constexpr int kReduceBatch = 8;  // partial loads in flight per thread
 constexpr int kReduceWaves = 4;
 
@@ -697,13 +692,13 @@ constexpr int kReduceWaves = 4;
 // turn by turn), one rounding, written in the weight's layout.  Blocks
 // (x, k): offset k's share is worked out once per thread, then the block
 // strides over the partial matrix's 4-float pieces, 64 at a time; its four
-// waves sum a quarter of the partials each, added in their order (one thread
-// per piece leaves a 64 x 64 weight 108 blocks of up to a hundred dependent
-// additions: 18 us for fp32 over 60,001 rows, in quarters 10) (fragment order of
-// weight_grad_mfma: piece (tile, wave, m, n, lane) holds ci = ci0 +
-// (TCI/2)*(wave&1) + 16m + 4(lane/16) + q, q < 4, and co = co0 +
-// (TCO/2)*(wave>>1) + 16n + lane%16); each entry keeps its own summation
-// order.
+// waves sum a quarter of the partials each, and the quarters are added in
+// their order, so each entry keeps one summation order.  One thread per
+// piece left a 64 x 64 weight 108 blocks of up to a hundred dependent
+// additions: 18 us for fp32 over 60,001 rows, in quarters 10.  The pieces
+// are in the fragment order of weight_grad_mfma: piece (tile, wave, m, n,
+// lane) holds ci = ci0 + (TCI/2)*(wave&1) + 16m + 4(lane/16) + q, q < 4, and
+// co = co0 + (TCO/2)*(wave>>1) + 16n + lane%16.
 template <typename T>
 __global__ void __launch_bounds__(kReduceWaves * kWave)
 weight_grad_reduce(const float* __restrict__ partial, const int32_t* __restrict__ koff, int slots,

@@ -209,11 +209,13 @@ def test_matrix_core_bf16():
     _close(to_np(out.feats.float()), ref, 2e-2, 3e-2, 'bf16 64->64')
 
 
-def test_csr_route_fp16_matches():
-    # Channel counts the matrix cores do not tile take the CSR route.
+@pytest.mark.parametrize('c_in', [24, 20])
+def test_csr_route_fp16_matches(c_in):
+    # Rows that are not whole 16-byte pieces (20 channels) take the CSR
+    # route, others that do not fill the tiles the padded instances.
     coords, rng = _shell(8000, 160, 3)
-    feats = rng.standard_normal((len(coords), 24)).astype(np.float16)
-    w = (rng.standard_normal((40, 3, 3, 3, 24)) * 0.05).astype(np.float16)
+    feats = rng.standard_normal((len(coords), c_in)).astype(np.float16)
+    w = (rng.standard_normal((40, 3, 3, 3, c_in)) * 0.05).astype(np.float16)
     out = _run_conv(coords, feats, w, torch.float16, subm=True, kernel_size=3)
     _, ref = _reference(coords, feats, w, dict(kernel_size=3))
     _close(to_np(out.feats.float()), ref, RTOL_F16, ATOL_F16, 'csr fp16')
@@ -360,7 +362,7 @@ def test_quantized_csr_route_matches_oracle(bits):
         in_channels=16, out_channels=12, storage_in_channels=32,
         group_size=q.group_size, bits=bits)
     _close(to_np(out.feats.float()), expected.astype(np.float32), 2e-3, 2e-3,
-           'quantized CSR vs oracle')
+           'quantized, 16 channels, vs oracle')
     del rng
 
 
@@ -531,10 +533,14 @@ def test_tile_schedule_does_not_change_results():
     (torch.bfloat16, 128, 256, None, 'subm'),    # 8-wave C_out = 256 shape
     (torch.float16, 32, 16, None, 'subm'),       # C_out = 16 shape
     (torch.float16, 64, 128, None, 'down'),      # k2s2: bias on rows past the active count too
-    (torch.float32, 16, 32, None, 'subm'),       # CSR fp32
-    (torch.float16, 24, 40, None, 'subm'),       # CSR fp16
+    (torch.float32, 16, 32, None, 'subm'),       # padded fp32
+    (torch.float16, 24, 40, None, 'subm'),       # padded fp16
+    (torch.float32, 5, 32, None, 'subm'),        # CSR rows (staged weights), fp32
+    (torch.float32, 6, 40, None, 'subm'),        # CSR fp32
+    (torch.float16, 20, 40, None, 'subm'),       # CSR fp16
     (torch.float16, 64, 64, 8, 'subm'),          # quantized, matrix cores
-    (torch.float16, 4, 32, 8, 'subm'),           # quantized CSR (staged weights)
+    (torch.float16, 4, 32, 8, 'subm'),           # quantized, dense map
+    (torch.float16, 12, 40, 8, 'subm'),          # quantized CSR
 ])
 def test_fused_bias_equals_separate_add(dtype, c_in, c_out, quant, kind):
     """The bias added in the conv store equals conv + bias done as a
@@ -577,10 +583,13 @@ def _bits(t):
     (torch.bfloat16, 128, 256, None, 'subm'),    # C_out = 256: two column halves
     (torch.float16, 32, 16, None, 'subm'),       # C_out = 16 shape
     (torch.float16, 64, 128, None, 'down'),      # k2s2: rows past the active count hold relu(bias)
-    (torch.float32, 16, 32, None, 'subm'),       # CSR rows (staged weights)
-    (torch.float16, 24, 40, None, 'subm'),       # CSR fp16
+    (torch.float32, 16, 32, None, 'subm'),       # padded fp32
+    (torch.float16, 24, 40, None, 'subm'),       # padded fp16
+    (torch.float32, 5, 32, None, 'subm'),        # CSR rows (staged weights)
+    (torch.float16, 20, 40, None, 'subm'),       # CSR fp16
     (torch.float16, 64, 64, 8, 'subm'),          # quantized, matrix cores
-    (torch.float16, 4, 32, 8, 'subm'),           # quantized CSR (staged weights)
+    (torch.float16, 4, 32, 8, 'subm'),           # quantized, dense map
+    (torch.float16, 12, 40, 8, 'subm'),          # quantized CSR
     (torch.float16, 64, 64, None, 'expand'),     # generative transposed: dense expansion
 ])
 def test_fused_relu_equals_separate_relu(dtype, c_in, c_out, quant, kind):

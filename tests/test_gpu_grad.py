@@ -108,8 +108,8 @@ CASES = [
     ('subm', 3, 1, 32, 128, torch.bfloat16, False),
     ('subm', 3, 1, 64, 32, torch.float16, True),       # mapped (K, C_in, C_out) weight
     ('forward', 2, 2, 64, 128, torch.float16, False),  # k2s2 downsample
-    ('subm', 3, 1, 16, 32, torch.float32, False),      # CSR input grad, simple weight grad
-    ('subm', 3, 1, 24, 40, torch.float16, False),      # CSR input grad (C_out % 32), MFMA weight grad
+    ('subm', 3, 1, 16, 32, torch.float32, False),      # padded input grad, fp32 MFMA weight grad
+    ('subm', 3, 1, 24, 40, torch.float16, False),      # padded input grad, MFMA weight grad
     ('forward', 2, 2, 8, 16, torch.float32, True),
     ('subm', 3, 1, 128, 128, torch.float16, False),    # 128 x 128 weight-grad tiles
     ('subm', 3, 1, 96, 136, torch.bfloat16, False),    # ragged 128-channel tiles

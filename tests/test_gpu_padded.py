@@ -144,6 +144,92 @@ def test_padded_quantized_conv_matches_the_unpacked_weight(dtype, bits, c_in,
            bound + 4 * HALF_ULP[dtype] ** 2 * mag, f'int{bits}')
 
 
+@pytest.mark.parametrize('dtype,c_in,c_out,rows', [
+    (torch.float32, 48, 72, 33001),    # an order of four 32-row tiles each
+    (torch.float32, 16, 32, 33001),    # two 64-row tiles
+    (torch.bfloat16, 96, 96, 40001),
+    (torch.float16, 24, 40, 66001),    # 128-row tiles of one column tile
+    (torch.bfloat16, 72, 200, 33001),  # and of two
+])
+def test_padded_conv_with_a_tile_order(dtype, c_in, c_out, rows):
+    """Enough rows for the longest-first order of the 128-row tiles, the last
+    tile ragged: the same bits in any order of the tiles."""
+    from mlx_lattice_amd import SparseTensor, ops
+    from mlx_lattice_amd._native import ext
+
+    coords, rng = _cloud(rows, c_in + c_out)
+    f = torch.as_tensor(rng.standard_normal((rows, c_in))).to(DEV, dtype)
+    w = torch.as_tensor(rng.standard_normal((c_out, 3, 3, 3, c_in))
+                        / np.sqrt(9 * c_in)).to(DEV, dtype)
+    print(f'tile order {dtype} {c_in}->{c_out} rows={rows}', flush=True)
+    x = SparseTensor(torch.as_tensor(coords).to(DEV), f)
+    y = ops.subm_conv3d(x, w, kernel_size=3).feats
+    rel = x.coord_manager.submanifold_kernel_relation(x.coord_key)
+    view = rel.sorted_implicit_gemm
+    order = view.tile_order()
+    tiles = (rows + 127) // 128
+    assert order is not None
+    listed = order.view(torch.int32)[:tiles]
+    assert torch.equal(listed.sort().values.cpu(),
+                       torch.arange(tiles, dtype=torch.int32))
+    # as they come, and shortest first
+    for other in (torch.arange(tiles, dtype=torch.int32, device=DEV),
+                  listed.flip(0)):
+        given = order.clone()
+        given.view(torch.int32)[:tiles] = other
+        z = ext.sparse_conv_features_padded(
+            f, ext.conv_padded_fragments(w, 0), 0, c_out,
+            view.sorted_kv_out_in_map, view.reorder_rows, view.tile_masks,
+            rows, 27, tile_order=given)
+        assert torch.equal(y, z)
+    torch.cuda.synchronize()
+    orel = O.kernel_relation(coords, kernel_size=3)
+    fd, wd = to_np(f.double()), to_np(w.double())
+    ref = O.conv_features_fp64(fd, O.mapped_weight(wd), orel)
+    _check(to_np(y.double()), ref,
+           _bound(fd, wd, orel, ref, dtype, c_in, 0.0), 'tile order')
+
+
+@pytest.mark.parametrize('dtype,bits,c_out', [
+    (torch.float16, 8, 96), (torch.float16, 4, 40), (torch.bfloat16, 8, 48),
+    (torch.bfloat16, 4, 96)])
+def test_padded_quantized_weight_is_not_rounded(dtype, bits, c_out):
+    """Rows with one edge whose features have the sign of what the rounding
+    of column 0's weight leaves, so that it adds up over the channels: within
+    the bound of two fragments, which a rounded weight exceeds."""
+    from mlx_lattice_amd import SparseTensor, dequantize_weight, ops
+    from mlx_lattice_amd import quantize_weight
+
+    rows, c_in = 65, 256
+    rng = np.random.default_rng(bits + c_out)
+    coords = np.zeros((rows, 4), np.int32)
+    coords[:, 1] = 4 * rng.permutation(rows)
+    q = quantize_weight(torch.as_tensor(
+        rng.standard_normal((c_out, 3, 3, 3, c_in)) / 32).to(DEV, dtype),
+        group_size=32, bits=bits)
+    exact = dequantize_weight(dataclasses.replace(
+        q, scales=q.scales.float(), biases=q.biases.float()))
+    w = to_np(exact.double()).reshape(c_out, 27, c_in)[:, 13]
+    left = w - to_np(exact.to(dtype).double()).reshape(c_out, 27, c_in)[:, 13]
+    f = np.sign(left[0]) * 2.0 ** rng.integers(-1, 2, (rows, 1))
+    print(f'unrounded int{bits} {dtype} {c_in}->{c_out}', flush=True)
+    x = SparseTensor(torch.as_tensor(coords).to(DEV),
+                     torch.as_tensor(f).to(DEV, dtype))
+    y = to_np(ops.subm_conv3d(x, q, kernel_size=3).feats.double())
+    ref, mag = f @ w.T, np.abs(f) @ np.abs(w).T
+    u = HALF_ULP[dtype]
+    # a weight's two fragments are off by u^2 of it, or, where the second is
+    # a subnormal float16, by half of the smallest one; fp32 sums of the two
+    # products of each channel; one rounding of the result
+    split = np.maximum(u * u * np.abs(w), 2.0 ** -25
+                       if dtype == torch.float16 else 0.0)
+    bound = (np.abs(f) @ split.T + (2 * c_in + 1) * 2.0 ** -24 * mag
+             + u * np.abs(ref) * (1 + u) + 2.0 ** -25)
+    _check(y, ref, bound, f'int{bits}')
+    rounded = np.abs(f @ left.T)[:, 0]
+    assert (rounded > 2 * bound[:, 0]).all()
+
+
 @pytest.mark.parametrize('dtype,c_in,c_out', [
     (torch.float32, 64, 64), (torch.float32, 12, 20),
     (torch.bfloat16, 96, 96)])
