@@ -16,6 +16,7 @@ from typing import Literal
 
 import torch
 
+from mlx_lattice_amd import _native
 from mlx_lattice_amd.core.types import Triple
 
 RelationKind = Literal['forward', 'target', 'submanifold', 'transposed',
@@ -59,13 +60,14 @@ def _kept(holder, name: str, device: torch.device, make: Callable):
             value = make()
             object.__setattr__(holder, name, value)
         return value
-    from mlx_lattice_amd._native import ext
-
-    stream, capture = ext.stream_state(device.index)
+    ext = _native.ext
     written = holder._written
     if value is not None:
         streams = written.get(name)
-        if streams is None or capture or stream in streams:
+        if streams is None or ext.current_stream(device.index) in streams:
+            return value
+        stream, capture = ext.stream_state(device.index)
+        if capture:
             return value
         if not ext.join_stream(device.index, streams[0]):
             return make()   # the writer is being captured: nothing to wait for
@@ -74,6 +76,7 @@ def _kept(holder, name: str, device: torch.device, make: Callable):
             array.record_stream(current)
         written[name] = (*streams, stream)
         return value
+    stream, capture = ext.stream_state(device.index)
     if capture:
         captured = written.get((name, 'captured'))
         if captured is None or captured[:2] != (stream, capture):

@@ -119,6 +119,10 @@ bool join_stream(int device, uintptr_t writer_handle) {
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.doc() = "MI355X-native sparse convolution hot path (gfx950 HIP kernels behind a C ABI).";
     py::class_<StatusWord>(m, "StatusWord").def(py::init<const at::Tensor&>()).def("read", &StatusWord::read);
+    m.def("current_stream", [](int device) {
+        return reinterpret_cast<uintptr_t>(
+            c10::hip::getCurrentHIPStream(static_cast<c10::DeviceIndex>(device)).stream());
+    }, py::arg("device"));
     m.def("stream_state", &stream_state, py::arg("device"), "(current stream, id of its graph capture or 0).");
     m.def("join_stream", &join_stream, py::arg("device"), py::arg("writer"),
           "Let the current stream wait for `writer`; False when it is being captured.");

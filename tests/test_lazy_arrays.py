@@ -18,6 +18,9 @@ class _Streams:
         self.captured = set()
         self.joins = []
 
+    def current_stream(self, device):
+        return self.now[0]
+
     def stream_state(self, device):
         return self.now
 
