@@ -534,6 +534,11 @@ class KernelRelation:
         return self._edges
 
     @property
+    def holds_edges(self) -> bool:
+        """Whether the edges were emitted by the build (or made since)."""
+        return self._map_edges is None or self._map_edges._made is not None
+
+    @property
     def output_csr(self) -> RelationCSRView:
         if self._map_edges is not None:
             return self._map_edges.get()[1]

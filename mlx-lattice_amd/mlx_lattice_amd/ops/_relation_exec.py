@@ -97,11 +97,38 @@ def _padded_eligible(feats: torch.Tensor, c_out: int,
                                           rows))
 
 
+def edges_pay(c_in: int, c_out: int, element_size: int, rows: int) -> bool:
+    """Whether a conv over a new relation runs faster over its edges than in
+    the padded instances: the edge kernels' time grows with rows and input
+    channels, while the view costs a launch up to 32,768 rows and a sort
+    above, and few outputs leave most of a 32-column group empty.  Map build
+    and 3^3 fp32 conv, edges / padded us:
+
+    rows     4 -> 3    4 -> 16   4 -> 24   4 -> 32   8 -> 8    8 -> 16
+    4,000    53 / 59   54 / 58   55 / 59   55 / 58   53 / 58   56 / 57
+    32,000   54 / 58   59 / 57             70 / 58             73 / 59
+    65,000   66 / 116  70 / 117  95 / 115  80 / 116  76 / 116  83 / 115
+    130,000  89 / 142  93 / 141  141 / 142 100 / 143 114 / 140 120 / 140
+    400,000  257 / 290 293 / 287           303 / 291           514 / 288
+
+    (8 -> 24 over 65,000 rows 154 / 116, 12 -> 3 91 / 117, 16 -> 16
+    109 / 114; 16 -> 32 over 20,000 117 / 58.)  Over a sorted view that is there the padded instances
+    are as fast or faster from 32,768 rows on (130,000 rows, 4 -> 16 35 / 36,
+    8 -> 16 63 / 36)."""
+    if rows <= 32768:
+        return c_in <= 8 and c_out <= (16 if c_in * element_size <= 16 else 8)
+    return rows * c_in <= 1 << 20 and (
+        c_out <= 16 and c_in <= 8 or c_out <= 4 and c_in <= 16
+        or c_out == 32 and c_in <= 4)
+
+
 def _padded_forward(feats: torch.Tensor, c_in: int, c_out: int,
                     relation: KernelRelation) -> bool:
     """The forward conv's use of the padded instances.  Expanded relations
-    keep the CSR route in fp32: their rows hold one edge each or few, so the
-    view costs more than it saves."""
+    keep the CSR route in fp32: their rows hold one edge each or few.  k2s2
+    from 30,000 rows, 16 -> 32 channels take 27 us over the edges, and 24 over
+    a view that takes 61 to build; from 32 channels on the padded instances
+    would be faster with the view too (64 -> 64: 2871 against 47 + 61)."""
     if not relation.dense_map_exact:
         return False
     if feats.dtype == torch.float32 and relation.kind in (
@@ -375,6 +402,11 @@ def _conv_features(feats: torch.Tensor, weight: torch.Tensor,
     if (dense is None and feats.ndim == 2
             and _weight_fits(weight, feats.dtype, int(feats.shape[1]), c_out,
                              relation)
+            and not (relation.holds_edges
+                     and relation.sorted_implicit_gemm is None
+                     and edges_pay(int(feats.shape[1]), c_out,
+                                   feats.element_size(),
+                                   relation.n_out_capacity))
             and _padded_forward(feats, int(feats.shape[1]), c_out, relation)):
         return _padded_conv(feats, weight, _FORWARD,
                             relation.conv_view(_offset_bytes(weight)),

@@ -21,6 +21,7 @@ from mlx_lattice_amd.core import (
 )
 from mlx_lattice_amd.core.types import Triple
 from mlx_lattice_amd.ops._relation_exec import (
+    edges_pay,
     sparse_conv_features_from_relation,
     sparse_quantized_conv_features_from_relation,
 )
@@ -135,7 +136,8 @@ def _relation_conv(x: SparseTensor, weight, bias, spec: KernelSpec, *,
     _validate_weight_for_kernel(x, weight, spec.volume)
     relation = _kernel_relation(
         x, spec, map_kind, target_key=target_key,
-        map_only=_reads_map_only(x.feats, weight, spec.volume))
+        map_only=_reads_map_only(x.feats, weight, spec.volume,
+                                 _out_rows(x, target_key)))
     if relation.n_out_capacity is None or relation.n_kernels is None:
         raise ValueError('kernel relation is missing static shape metadata.')
     # The bias is added in the conv kernels' store (after rounding, as a
@@ -174,21 +176,33 @@ def _relation_conv(x: SparseTensor, weight, bias, spec: KernelSpec, *,
                         active_rows=relation.out_count)
 
 
-def _reads_map_only(feats: torch.Tensor, weight, volume: int) -> bool:
-    """Whether the conv runs over the relation's dense map: feature rows of
-    whole 16-byte pieces (the matrix-core routes) or 16-bit rows of four
-    channels with 16 or 32 outputs (the dense-map conv).  Others read the
+def _out_rows(x: SparseTensor, target_key: CoordinateMapKey | None) -> int:
+    manager = x.coord_manager
+    coords = (manager.coords(target_key)
+              if target_key is not None and manager.owns(target_key)
+              else x.coords)
+    return int(coords.shape[0])
+
+
+def _reads_map_only(feats: torch.Tensor, weight, volume: int,
+                    rows: int) -> bool:
+    """Whether the conv runs over the relation's dense map: 16-bit rows of
+    four or eight channels with 16 or 32 outputs (the dense-map conv), or
+    feature rows of whole 16-byte pieces (the matrix-core routes) but for the
+    ``rows`` output rows that run over the edges faster.  Others read the
     edges, which emitting with the map costs least."""
     quantized = isinstance(weight, QuantizedWeight)
     if feats.ndim != 2 or (quantized and feats.dtype == torch.float32):
         return False
     c_in = int(feats.shape[1])
-    if c_in * feats.element_size() % 16 == 0:
-        return True
+    size = feats.element_size()
     c_out = (weight.out_channels if quantized
              else int(weight.shape[0 if weight.ndim == 5 else 2]))
-    return (c_in == 4 and feats.element_size() == 2 and c_out in (16, 32)
-            and volume * c_in <= 256)
+    if (c_in in (4, 8) and size == 2 and c_out in (16, 32)
+            and volume * c_in <= 256):
+        return True
+    return c_in * size % 16 == 0 and (
+        quantized or not edges_pay(c_in, c_out, size, rows))
 
 
 def _kernel_relation(x: SparseTensor, spec: KernelSpec, map_kind: str, *,

@@ -330,3 +330,46 @@ def test_weight_grad_matches_fp64(dtype, c_in, c_out, rows):
         got = to_np(got.double()).reshape(c_out, 27, c_in).transpose(1, 0, 2)
         _check(got, ref, bound, what)
     _check(to_np(mapped.double()).transpose(0, 2, 1), ref, bound, 'mapped')
+
+
+@pytest.mark.parametrize('dtype,c_in,c_out,rows,edges', [
+    (torch.float32, 4, 16, 32768, True), (torch.float32, 4, 17, 32768, False),
+    (torch.float32, 8, 8, 3000, True), (torch.float32, 8, 9, 3000, False),
+    (torch.float32, 8, 16, 32769, True), (torch.float32, 4, 32, 32769, True),
+    (torch.float32, 8, 32, 32769, False), (torch.float32, 12, 4, 3000, False),
+    (torch.float32, 12, 4, 32769, True), (torch.float32, 12, 5, 32769, False),
+    (torch.float16, 8, 12, 3000, True), (torch.float16, 8, 16, 3000, False),
+])
+def test_narrow_convs_of_new_relations_run_over_the_edges(dtype, c_in, c_out,
+                                                          rows, edges):
+    """At the borders of the rule; either route gives the sum, and a relation
+    that holds a sorted view keeps to the padded instances."""
+    from mlx_lattice_amd import SparseTensor, ops
+    from mlx_lattice_amd._native import ext
+
+    coords, rng = _cloud(rows, c_in + c_out)
+    f = torch.as_tensor(rng.standard_normal((rows, c_in))).to(DEV, dtype)
+    w = torch.as_tensor(rng.standard_normal((c_out, 3, 3, 3, c_in))
+                        / np.sqrt(9 * c_in)).to(DEV, dtype)
+    print(f'narrow {dtype} {c_in}->{c_out} rows={rows}', flush=True)
+    x = SparseTensor(torch.as_tensor(coords).to(DEV), f)
+    y = ops.subm_conv3d(x, w, kernel_size=3).feats
+    rel = x.coord_manager.submanifold_kernel_relation(x.coord_key)
+    assert rel.holds_edges == edges
+    dense_map = dtype == torch.float16 and c_out == 16
+    viewed = rel._tiled is not None or rel.sorted_implicit_gemm is not None
+    assert viewed == (not edges and not dense_map)
+    orel = O.kernel_relation(coords, kernel_size=3)
+    fd, wd = to_np(f.double()), to_np(w.double())
+    ref = O.conv_features_fp64(fd, O.mapped_weight(wd), orel)
+    bound = _bound(fd, wd, orel, ref, dtype, c_in, 0.0)
+    _check(to_np(y.double()), ref, bound, 'new')
+    view = rel.require_sorted_implicit_gemm()
+    z = ops.subm_conv3d(x, w, kernel_size=3).feats
+    _check(to_np(z.double()), ref, bound, 'sorted')
+    if not dense_map:
+        assert torch.equal(z, ext.sparse_conv_features_padded(
+            f, ext.conv_padded_fragments(w, 0), 0, c_out,
+            view.sorted_kv_out_in_map, view.reorder_rows, view.tile_masks,
+            rows, 27))
+    torch.cuda.synchronize()
