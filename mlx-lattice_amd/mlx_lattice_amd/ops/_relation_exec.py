@@ -7,8 +7,11 @@ the mask-sorted view, for every relation kind whose edges fit the dense
 (out_row, offset) map: fp16/bf16 with ``C_in % 32 == 0`` and ``C_out`` in
 {16, 32, 64, 128, 256} on the kernels tuned for those, other channel counts
 and fp32 on the streamed kernel's padded instances (rows of whole 16-byte
-pieces); everything else runs the CSR bandwidth kernel.  All routes compute
-the same sum with an fp32 accumulator.
+pieces); everything else, and the narrow rows of ``edges_pay``, runs the CSR
+bandwidth kernel.  All routes compute the same sum with an fp32 accumulator.
+Copies of a weight in a kernel's order are kept with it for the tuned widths
+alone, by its identity and version counter; the padded instances make theirs
+in the call.
 """
 
 from __future__ import annotations
@@ -112,9 +115,11 @@ def edges_pay(c_in: int, c_out: int, element_size: int, rows: int) -> bool:
     400,000  257 / 290 293 / 287           303 / 291           514 / 288
 
     (8 -> 24 over 65,000 rows 154 / 116, 12 -> 3 91 / 117, 16 -> 16
-    109 / 114; 16 -> 32 over 20,000 117 / 58.)  Over a sorted view that is there the padded instances
-    are as fast or faster from 32,768 rows on (130,000 rows, 4 -> 16 35 / 36,
-    8 -> 16 63 / 36)."""
+    109 / 114; 16 -> 32 over 20,000 117 / 58.)  Over a sorted view that is
+    there the padded instances are as fast or faster from 32,768 rows on
+    (130,000 rows, 4 -> 16 35 / 36, 8 -> 16 63 / 36).  Packed weights gain
+    more (int8 8 -> 8 over 32,000 rows 60 / 66, over 130,000 rows
+    124 / 158)."""
     if rows <= 32768:
         return c_in <= 8 and c_out <= (16 if c_in * element_size <= 16 else 8)
     return rows * c_in <= 1 << 20 and (
@@ -122,17 +127,35 @@ def edges_pay(c_in: int, c_out: int, element_size: int, rows: int) -> bool:
         or c_out == 32 and c_in <= 4)
 
 
+def _expanded_edges_pay(n_kernels: int, c_in: int, c_out: int) -> bool:
+    """``edges_pay`` of transposed and generative relations, whose rows hold
+    one edge or few.  fp16 over the edges / padded + its view, us, from 30,000
+    rows: k2s2 16 -> 16 11 / 20 + 68, 16 -> 24 40 / 21 + 68, 16 -> 32
+    22 / 20 + 68, 24 -> 24 53 / 20 + 68, 8 -> 64 89 / 23 + 68; k3s2 16 -> 16
+    67 / 36 + 207, 16 -> 32 169 / 38 + 207, 24 -> 16 335 / 37 + 207; packed
+    weights the same to 1.4 times as long on either side.  The last four of
+    these gain little from the edges, or lose much to a view that is there."""
+    rows_kernel = c_in <= 16 and c_out in (16, 32)
+    return n_kernels * c_in * c_out <= (8192 if rows_kernel else 3072)
+
+
 def _padded_forward(feats: torch.Tensor, c_in: int, c_out: int,
                     relation: KernelRelation) -> bool:
-    """The forward conv's use of the padded instances.  Expanded relations
-    keep the CSR route in fp32: their rows hold one edge each or few.  k2s2
-    from 30,000 rows, 16 -> 32 channels take 27 us over the edges, and 24 over
-    a view that takes 61 to build; from 32 channels on the padded instances
-    would be faster with the view too (64 -> 64: 2871 against 47 + 61)."""
+    """The forward conv's use of the padded instances: where they are
+    eligible and the edges do not run faster.  Expanded relations keep the
+    CSR route in fp32: k2s2 from 30,000 rows, 16 -> 32 channels take 27 us
+    over the edges, and 24 over a view that takes 61 to build; from 32
+    channels on the padded instances would be faster with the view too
+    (64 -> 64: 2871 against 47 + 61)."""
     if not relation.dense_map_exact:
         return False
-    if feats.dtype == torch.float32 and relation.kind in (
-            'transposed', 'generative'):
+    if relation.kind in ('transposed', 'generative'):
+        if (feats.dtype == torch.float32
+                or _expanded_edges_pay(int(relation.n_kernels), c_in, c_out)):
+            return False
+    elif (relation.holds_edges and relation.sorted_implicit_gemm is None
+            and edges_pay(c_in, c_out, feats.element_size(),
+                          relation.n_out_capacity)):
         return False
     return _padded_eligible(feats, c_out, relation, relation.n_out_capacity)
 
@@ -402,11 +425,6 @@ def _conv_features(feats: torch.Tensor, weight: torch.Tensor,
     if (dense is None and feats.ndim == 2
             and _weight_fits(weight, feats.dtype, int(feats.shape[1]), c_out,
                              relation)
-            and not (relation.holds_edges
-                     and relation.sorted_implicit_gemm is None
-                     and edges_pay(int(feats.shape[1]), c_out,
-                                   feats.element_size(),
-                                   relation.n_out_capacity))
             and _padded_forward(feats, int(feats.shape[1]), c_out, relation)):
         return _padded_conv(feats, weight, _FORWARD,
                             relation.conv_view(_offset_bytes(weight)),

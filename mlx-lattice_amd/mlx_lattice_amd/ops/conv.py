@@ -201,8 +201,7 @@ def _reads_map_only(feats: torch.Tensor, weight, volume: int,
     if (c_in in (4, 8) and size == 2 and c_out in (16, 32)
             and volume * c_in <= 256):
         return True
-    return c_in * size % 16 == 0 and (
-        quantized or not edges_pay(c_in, c_out, size, rows))
+    return c_in * size % 16 == 0 and not edges_pay(c_in, c_out, size, rows)
 
 
 def _kernel_relation(x: SparseTensor, spec: KernelSpec, map_kind: str, *,

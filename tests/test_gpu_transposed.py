@@ -12,6 +12,8 @@ Gradients follow tests/test_gpu_grad.py's tolerances.
 
 from __future__ import annotations
 
+import dataclasses
+
 import numpy as np
 import pytest
 import torch
@@ -494,3 +496,47 @@ def test_expansion_conv_matches_sorted_route_and_oracle(c_in, c_out, dtype):
     _close(f32(generic), ref, 2e-2, 1e-2, 'expansion vs oracle')
     assert torch.equal(out.feats[active * 8:],
                        bias.expand(n * 8 - active * 8, c_out))
+
+
+@pytest.mark.parametrize('ks,c_in,c_out,bits,edges', [
+    (2, 16, 32, 0, True), (2, 16, 24, 0, True), (2, 24, 24, 0, False),
+    (3, 16, 16, 0, True), (3, 16, 32, 0, False), (3, 24, 16, 0, False),
+    (2, 16, 32, 8, True), (3, 48, 24, 4, False),
+])
+def test_small_weights_of_expanded_relations_run_over_the_edges(
+        ks, c_in, c_out, bits, edges):
+    """At the borders of the rule (small weights over the edges, the others
+    in the padded instances): both are the same sum."""
+    from mlx_lattice_amd import dequantize_weight, quantize_weight
+
+    ops, SparseTensor = _ops()
+    rng = np.random.default_rng(ks * c_in + c_out)
+    flat = rng.choice(12 ** 3, 300, replace=False)
+    coords = np.stack([np.zeros_like(flat), flat // 144, flat // 12 % 12,
+                       flat % 12], 1).astype(np.int32)
+    f = torch.as_tensor(rng.standard_normal((300, c_in))).to(
+        DEV, torch.float16)
+    w = torch.as_tensor(rng.standard_normal((c_out, ks, ks, ks, c_in))
+                        / np.sqrt(2 * c_in)).to(DEV, torch.float16)
+    weight = quantize_weight(w, group_size=32, bits=bits) if bits else w
+    x = SparseTensor(torch.as_tensor(coords).to(DEV), f, stride=2)
+    print(f'expanded narrow k{ks} {c_in}->{c_out} int{bits}', flush=True)
+    y = ops.conv_transpose3d(x, weight, kernel_size=ks, stride=2)
+    rel = x.coord_manager.transposed_kernel_relation(
+        x.coord_key, kernel_size=ks, stride=2)
+    torch.cuda.synchronize()
+    assert (rel.sorted_implicit_gemm is None) == edges
+    orel = O.transposed_kernel_relation(coords, kernel_size=ks, stride=2)
+    if bits:
+        w = dequantize_weight(dataclasses.replace(
+            weight, scales=weight.scales.float(),
+            biases=weight.biases.float()))
+    fd, wd = to_np(f.double()), to_np(w.double())
+    ref = O.conv_features_fp64(fd, O.mapped_weight(wd), orel)
+    mag = O.conv_features_fp64(np.abs(fd), O.mapped_weight(np.abs(wd)), orel)
+    # fp32 sums of up to 27 edges' products, a weight rounded to half (the
+    # CSR route rounds packed float16 weights once), one rounding
+    bound = ((27 * c_in + 1) * 2.0 ** -24 * mag + 2.0 ** -11 * np.abs(ref)
+             + (2.0 ** -11 * mag if bits else 0.0) + 1e-7)
+    err = np.abs(to_np(y.feats.double())[:len(ref)] - ref)
+    assert (err <= bound).all(), float((err / bound).max())
