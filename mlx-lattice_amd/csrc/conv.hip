@@ -6,9 +6,9 @@
 //    accumulator; lanes of a row read the same feature values (broadcast)
 //    and consecutive output channels of the weight (coalesced).  Follows
 //    the output-stationary loop of cpu/algorithms.cpp:180-302 and, for packed
-//    weights, cpu/quantized.cpp:64-141.  Used for input rows
-//    that are not whole 16-byte pieces, K > 32 and relations the dense map
-//    cannot hold.
+//    weights, cpu/quantized.cpp:64-141.  Used for input rows that are not
+//    whole 16-byte pieces, K > 32, relations the dense map cannot hold, float32
+//    over expanded relations and a few narrow shapes of new relations.
 //  * Implicit-GEMM route (MFMA path): output rows are visited in the
 //    mask-sorted order of the sorted view (core/relations/views.py:467-510),
 //    64 rows per 256-thread block.  For every kernel offset that any row of
