@@ -256,10 +256,14 @@ def _kernel_relation_from_native(
                            else out_coords)
     implicit = (RelationImplicitGemmView(view[0], row_masks=view[1])
                 if len(view) >= 2 else None)
-    # The status word of a submanifold relation flags repeated coordinates;
-    # its workspace holds the block table of its coordinates.
-    repeated_coords = (view[2] if len(view) >= 3 and kind == 'submanifold'
-                       else None)
+    # The status word of a relation whose output rows are its input rows (a
+    # submanifold one, or a forward one of unit stride without padding) flags
+    # repeated coordinates; a submanifold build's workspace holds the block
+    # table of its coordinates.
+    own_rows = kind == 'submanifold' or (
+        kind == 'forward' and tuple(stride) == (1, 1, 1)
+        and tuple(padding) == (0, 0, 0))
+    repeated_coords = view[2] if len(view) >= 3 and own_rows else None
     block_table = view[3] if len(view) >= 4 and keep_table else None
     grouped_views = None
     if in_row_offsets is None:

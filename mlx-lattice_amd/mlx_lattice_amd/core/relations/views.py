@@ -383,8 +383,8 @@ class KernelRelation:
     # Generative, and transposed relations whose stride exceeds the offsets'
     # extent: output row in * K + k holds the single edge (in, k).
     direct_expansion: bool = False
-    # Submanifold relations: whether an active row repeats an earlier row's
-    # coordinate (each copy is an output row with the same neighbours, so
+    # Submanifold relations, and forward ones of unit stride without padding:
+    # whether an active row repeats an earlier row's coordinate (each copy is an output row with the same neighbours, so
     # an input row can have several output rows at one offset).  Held as a
     # _StatusWord copied to pinned memory when a conv of trainable features
     # or weights runs (expect_backward) and read on the first question
@@ -709,7 +709,9 @@ class KernelRelation:
         every edge: at most one edge per (in_row, kernel_id).  Forward,
         generative and transposed relations hold it by construction (their
         output coordinates are distinct, or each output row has one edge); a
-        submanifold relation does unless a coordinate repeats.  The first
+        submanifold relation, and a forward one of unit stride without
+        padding, whose output rows are the input rows too, does unless a
+        coordinate repeats.  The first
         question reads the build's status word from pinned memory (copied
         when a conv of trainable features or weights ran), so it waits for
         that copy only; under graph capture a word that was not copied before
@@ -808,10 +810,11 @@ class KernelRelation:
         """Mask-sorted view of the transposed relation (input row -> output
         row per offset), built on first use and cached: the matrix-core
         route of the input gradient runs the forward's implicit GEMM over
-        it.  Forward relations have at most one output row per (input row,
-        offset), generative and transposed relations exactly one, and
-        submanifold relations too unless a coordinate repeats
-        (``transposed_map_exact``, which the input gradient checks first);
+        it.  Strided forward relations have at most one output row per (input
+        row, offset), generative and transposed relations exactly one, and
+        relations whose output rows are their input rows too unless a
+        coordinate repeats (``transposed_map_exact``, which the input
+        gradient checks first);
         target relations (whose target may repeat a coordinate) are
         refused."""
         if (self.transposed_sorted_implicit_gemm is None

@@ -267,6 +267,59 @@ def test_gradients_with_repeated_coordinates(ks):
     assert _relation(y, 'subm', ks, 1).transposed_map_exact
 
 
+@pytest.mark.parametrize('dtype,c_in,c_out', [
+    (torch.float32, 48, 40), (torch.float16, 32, 32), (torch.bfloat16, 40, 72),
+    (torch.float32, 32, 33)])            # the last over the edges
+@pytest.mark.parametrize('ks', [3, (3, 2, 1), 2])
+@pytest.mark.parametrize('repeats', [True, False])
+def test_unit_stride_convs_of_repeated_coords(dtype, c_in, c_out, ks, repeats):
+    """A conv of unit stride without padding keeps the input rows as its
+    output rows, repeats included, so an input row can have several output
+    rows at one offset, as in a submanifold conv."""
+    ops, _ = _imports()
+    rng = np.random.default_rng(c_in + c_out)
+    flat = rng.choice(12 ** 3, 900, replace=False)
+    base = np.stack([np.zeros_like(flat), flat // 144, flat // 12 % 12,
+                     flat % 12], 1).astype(np.int32)
+    coords = base.copy()
+    if repeats:
+        coords[rng.integers(0, 900, 150)] = base[rng.integers(0, 900, 150)]
+    n = len(coords)
+    shape = (ks,) * 3 if isinstance(ks, int) else ks
+    feats = torch.as_tensor(rng.standard_normal((n, c_in))).to(
+        DEV, dtype).requires_grad_()
+    w = torch.as_tensor(rng.standard_normal((c_out, *shape, c_in))
+                        / np.sqrt(9 * c_in)).to(DEV, dtype)
+    x = _sparse(coords, feats)
+    print(f'unit stride {dtype} {c_in}->{c_out} {shape} {repeats}', flush=True)
+    y = ops.conv3d(x, w, kernel_size=ks, stride=1)
+    cot = torch.as_tensor(rng.standard_normal((n, c_out))).to(DEV, dtype)
+    grad, = torch.autograd.grad(y.feats, feats, cot)
+    rel = x.coord_manager.kernel_relation(x.coord_key, kernel_size=ks,
+                                          stride=1)
+    torch.cuda.synchronize()
+    assert rel.transposed_map_exact is not repeats
+    orel = _oracle_relation(rel)
+    f64 = lambda t: to_np(t.double())  # noqa: E731
+    e = int(rel.counts[0])
+    i, o, k = (np.asarray(orel[v])[:e]
+               for v in ('in_rows', 'out_rows', 'kernel_ids'))
+    wk = f64(w).reshape(c_out, -1, c_in)
+    ref, mag, edges = np.zeros((n, c_in)), np.zeros((n, c_in)), np.zeros(n)
+    for j in range(wk.shape[1]):
+        at = k == j
+        np.add.at(ref, i[at], f64(cot)[o[at]] @ wk[:, j])
+        np.add.at(mag, i[at], np.abs(f64(cot))[o[at]] @ np.abs(wk[:, j]))
+        np.add.at(edges, i[at], 1)
+    half = {torch.float32: 2.0 ** -24, torch.float16: 2.0 ** -11,
+            torch.bfloat16: 2.0 ** -8}[dtype]
+    # a fp32 sum over the row's edges and channels, one rounding
+    bound = ((edges[:, None] * c_out + 1) * 2.0 ** -24 * mag
+             + half * np.abs(ref) * (1 + half) + 1e-7)
+    err = np.abs(f64(grad) - ref)
+    assert (err <= bound).all(), float((err / bound).max())
+
+
 def test_weight_grad_with_no_edges():
     """An empty relation gives a zero weight gradient on every route."""
     from mlx_lattice_amd.ops._relation_exec import (
