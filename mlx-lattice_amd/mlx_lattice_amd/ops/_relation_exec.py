@@ -10,7 +10,7 @@ and fp32 on the streamed kernel's padded instances (rows of whole 16-byte
 pieces); everything else, and the narrow rows of ``edges_pay``, runs the CSR
 bandwidth kernel.  All routes compute the same sum with an fp32 accumulator.
 Copies of a weight in a kernel's order are kept with it for the tuned widths
-alone, by its identity and version counter; the padded instances make theirs
+alone, by its identity, storage and version counter; the padded instances make theirs
 in the call.
 """
 
@@ -25,9 +25,10 @@ from mlx_lattice_amd.core.quantized import QuantizedWeight
 from mlx_lattice_amd.core.relations import KernelRelation
 
 _MATRIX_CORE_C_OUT = (16, 32, 64, 128, 256)
-# (id(weight), kind) -> (weak reference, shape, dtype, version, value)
+# (id(weight), kind) -> (weak reference, (storage, shape, dtype, version),
+# value)
 _WEIGHT_CACHE: dict[tuple[int, str], tuple[weakref.ReferenceType, tuple,
-                                           torch.dtype, int, torch.Tensor]] = {}
+                                           torch.Tensor]] = {}
 
 
 def _empty_i32(device) -> torch.Tensor:
@@ -593,19 +594,17 @@ class _SparsePoolFeatures(torch.autograd.Function):
 
 
 def _cached_weight(weight: torch.Tensor, kind: str, make) -> torch.Tensor:
-    """``make(weight)``, cached by the weight's identity, shape, dtype and
-    version counter (so an in-place update, as an optimizer step makes,
-    rebuilds it), like the reference's ``_mapped_weight``
+    """``make(weight)``, cached by the weight's identity, storage, shape,
+    dtype and version counter (so an in-place update, as an optimizer step
+    makes, and an assignment to ``.data`` rebuild it; a write through
+    ``.data`` is not seen), like the reference's ``_mapped_weight``
     (_relation_exec.py:217-250)."""
     key = (id(weight), kind)
-    shape = tuple(weight.shape)
+    state = (weight.data_ptr(), tuple(weight.shape), weight.dtype,
+             weight._version)
     cached = _WEIGHT_CACHE.get(key)
-    if cached is not None:
-        ref, cached_shape, cached_dtype, version, value = cached
-        if (ref() is weight and cached_shape == shape
-                and cached_dtype == weight.dtype
-                and version == weight._version):
-            return value
+    if cached is not None and cached[0]() is weight and cached[1] == state:
+        return cached[2]
     value = make(weight)
 
     def _drop(ref, key=key):
@@ -613,8 +612,7 @@ def _cached_weight(weight: torch.Tensor, kind: str, make) -> torch.Tensor:
         if entry is not None and entry[0] is ref:
             _WEIGHT_CACHE.pop(key, None)
 
-    _WEIGHT_CACHE[key] = (weakref.ref(weight, _drop), shape, weight.dtype,
-                          weight._version, value)
+    _WEIGHT_CACHE[key] = (weakref.ref(weight, _drop), state, value)
     return value
 
 
@@ -631,8 +629,9 @@ def _quantized_fragments(weight: QuantizedWeight) -> torch.Tensor:
     bias per 16-byte piece, dequantised in the kernel; empty when the shape
     takes the other matrix-core kernel), cached with the packed words and
     rebuilt when they, the scales or the biases change."""
-    kind = ('quantized fragments', id(weight.scales), weight.scales._version,
-            id(weight.biases), weight.biases._version)
+    kind = ('quantized fragments',
+            *((id(t), t.data_ptr(), t._version)
+              for t in (weight.scales, weight.biases)))
 
     def make(words):
         return ext.quantized_weight_fragments(

@@ -119,3 +119,33 @@ def test_a_captured_step_and_eager_calls_between_replays(dtype, c_in, c_out):
         torch.cuda.synchronize()
         assert torch.equal(now[0], fresh[0]) and torch.equal(now[1], fresh[1])
         assert not torch.equal(now[0], y)
+
+
+@pytest.mark.parametrize('mapped', [False, True])
+def test_kept_copies_follow_a_new_storage(mapped):
+    """The tuned 16-bit widths keep a copy of the weight in the kernel's
+    order; one made of other storage (an assignment to ``.data``) is not
+    taken for it."""
+    from mlx_lattice_amd import ops, quantize_weight
+
+    dtype = torch.float16
+    x, rng = _tensor(600, 64, dtype, 5)
+    w, other = (_weight(rng, 64, 64, dtype) for _ in range(2))
+    if mapped:
+        w, other = (v.permute(1, 2, 3, 4, 0).reshape(27, 64, 64).contiguous()
+                    for v in (w, other))
+    cot = torch.as_tensor(rng.standard_normal((600, 64))).to(DEV, dtype)
+    print(f'kept copies mapped={mapped}', flush=True)
+    w.requires_grad_()
+    _both(x, w, cot)
+    w.data = other.clone()
+    now, want = _both(x, w, cot), _both(x, other, cot)
+    q, r = (quantize_weight(_weight(rng, 64, 64, dtype), group_size=32,
+                            bits=4) for _ in range(2))
+    ops.subm_conv3d(x, q)
+    for name in ('weight', 'scales', 'biases'):
+        getattr(q, name).data = getattr(r, name).clone()
+    a, b = ops.subm_conv3d(x, q), ops.subm_conv3d(x, r)
+    torch.cuda.synchronize()
+    assert torch.equal(now[0], want[0]) and torch.equal(now[1], want[1])
+    assert torch.equal(a.feats, b.feats)
